@@ -402,7 +402,7 @@ struct ReduceCall {
     int out_dtype;
 };
 
-static ReduceCall prepare_reduce(int entry_id, const hpt_view* in, const int64_t* axes, int naxes) {
+static ReduceCall prepare_reduce(int entry_id, const hpt_view* in, const int64_t* axes, int naxes, bool spare_scratch = true) {
     check_view(in, "reduce input", false);
     if (naxes < 0 || naxes > kMaxRank || (naxes > 0 && !axes))
         fail(HPT_ERR_PARAM, "reduce: bad axes argument");
@@ -416,15 +416,28 @@ static ReduceCall prepare_reduce(int entry_id, const hpt_view* in, const int64_t
     const bool heavy = (entry_id == HPT_LOGSUMEXP && dtype_size(c.out_dtype) > 2) ||
                        ((entry_id == HPT_SUM_SQUARE || entry_id == HPT_REDUCEL2) && in->dtype == HPT_F32);
     c.plan = plan_reduce(in->data, in->shape, in->strides, in->ndim, norm, naxes,
-                         dtype_size(in->dtype), c.entry->acc_size[in->dtype], heavy);
+                         dtype_size(in->dtype), c.entry->acc_size[in->dtype], heavy, spare_scratch);
     return c;
+}
+
+// Whether work on `st` is being recorded (or may not be asked about because another stream's is): scratch must
+// not be allocated then, and a recorded call outlives the buffer's next owner.
+static bool capturing(hipStream_t st) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &status) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;
+    }
+    return status != hipStreamCaptureStatusNone;
 }
 
 // use_static: the partials go to the library's static device array instead of allocated
 // scratch; a plan that needs more than the array holds is refused.
+// Small inputs that are split for speed alone are reduced in one launch where scratch is not to be had for the
+// asking: for the static entry (whose one array is shared by all streams), under capture, and when the device is full.
 static void run_reduce(int dev, void* stream, int entry_id, const hpt_view* in, const int64_t* axes,
                        int naxes, int init_out, hpt_view* out, bool use_static = false) {
-    ReduceCall c = prepare_reduce(entry_id, in, axes, naxes);
+    ReduceCall c = prepare_reduce(entry_id, in, axes, naxes, !use_static);
     check_out(out, c.out_dtype, c.plan.K, "reduce output");
     check_alias(in, out, false, "reduce", "the input");
     if (c.plan.kind == ReduceKind::Empty) return;
@@ -432,7 +445,7 @@ static void run_reduce(int dev, void* stream, int entry_id, const hpt_view* in, 
         fail(HPT_ERR_PARAM, "reduce input: data pointer is null");
     if (!init_out && !(entry_id == HPT_SUM || entry_id == HPT_NANSUM))
         fail(HPT_ERR_PARAM, "init_out = 0 (accumulate into out) is only defined for sum and nansum");
-    const size_t pbytes = scratch_need(c.plan, c.entry->acc_size[in->dtype]);
+    size_t pbytes = scratch_need(c.plan, c.entry->acc_size[in->dtype]);
     if (use_static && pbytes > kStaticScratchBytes)
         fail(HPT_ERR_MEMORY,
              "reduce_static: this reduction needs %zu bytes of scratch, the static scratch holds %zu; "
@@ -441,6 +454,10 @@ static void run_reduce(int dev, void* stream, int entry_id, const hpt_view* in, 
     use_device(dev);
     hipStream_t st = (hipStream_t)stream;
     ReduceLaunchFn fn = c.entry->launch[in->dtype];
+    if (c.plan.small_split && capturing(st)) {
+        c = prepare_reduce(entry_id, in, axes, naxes, false);
+        pbytes = 0;
+    }
     if (pbytes && use_static) {
         ReduceScratch sc;
         sc.partial = static_scratch_of(dev);
@@ -450,7 +467,12 @@ static void run_reduce(int dev, void* stream, int entry_id, const hpt_view* in, 
         StreamScratch& s = scratch_entry(dev, st);
         std::lock_guard<std::mutex> g(s.mu);
         ReduceScratch sc;
-        sc.partial = scratch_reserve(dev, s, pbytes);
+        try {
+            sc.partial = scratch_reserve(dev, s, pbytes);
+        } catch (const Error&) {
+            if (!c.plan.small_split) throw;
+            c = prepare_reduce(entry_id, in, axes, naxes, false);
+        }
         fn(c.plan, in->data, out->data, sc, st, init_out);
         check_launch("reduce");
     } else {

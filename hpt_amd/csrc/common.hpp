@@ -108,15 +108,17 @@ struct ReducePlan {
     int flat_xb = 0;    // > 0: a period of the flat walk is wider than a workgroup and spans this many of them;
                         // `split` then counts the partials per output (slices x row phases)
     int flat_phases = 1;  // rows per period in that case
+    bool small_split = false;  // Col: split although the input is small, for speed alone; a plan without partials exists (spare_scratch = false)
 };
 
 // Build the plan for reducing `axes` (already normalised) of a view.
 // `elem_size` and `data` decide whether 128-bit loads are legal; `acc_size` is
 // the size of one accumulator (bounds the LDS a column kernel may use). `heavy`: the op spends many
 // instructions per element (an exponential, f64 arithmetic on f32 data), which wants more wavefronts
-// per compute unit than a plain sum.
+// per compute unit than a plain sum. `spare_scratch`: small inputs may be split too, which takes a little scratch;
+// without it they are reduced in one launch.
 ReducePlan plan_reduce(const void* data, const int64_t* shape, const int64_t* strides, int ndim,
-                       const int64_t* axes, int naxes, size_t elem_size, size_t acc_size, bool heavy = false);
+                       const int64_t* axes, int naxes, size_t elem_size, size_t acc_size, bool heavy = false, bool spare_scratch = true);
 
 std::string describe(const ReducePlan& p);
 

@@ -104,9 +104,13 @@ static int legal_vec(const void* data, size_t elem_size, int64_t inner_len, cons
 // hold 8 such blocks.
 constexpr int64_t kBlocksToFill = 2048;
 constexpr int64_t kComputeUnits = 256;  // MI355X
+// Column reductions below this take the plans for small inputs; the partials of those that are split stay below
+// the second figure.
+constexpr int64_t kSmallColBytes = 8ll << 20;
+constexpr size_t kSmallColScratch = 1u << 20;
 
 ReducePlan plan_reduce(const void* data, const int64_t* shape, const int64_t* strides, int ndim,
-                       const int64_t* axes, int naxes, size_t elem_size, size_t acc_size, bool heavy) {
+                       const int64_t* axes, int naxes, size_t elem_size, size_t acc_size, bool heavy, bool spare_scratch) {
     ReducePlan p;
     bool is_red[kMaxRank] = {};
     for (int i = 0; i < naxes; ++i) is_red[axes[i]] = true;
@@ -246,7 +250,7 @@ ReducePlan plan_reduce(const void* data, const int64_t* shape, const int64_t* st
                 p.kept.size[0] >= 256 && p.K * p.R * (int64_t)elem_size >= (4ll << 20) && ((uintptr_t)data & 15) == 0) {
                 const int64_t L = p.kept.size[1];
                 const int64_t shp[2] = {p.kept.size[0], p.R * L}, str[2] = {p.R * L, 1}, ax[1] = {1};
-                ReducePlan q = plan_reduce(data, shp, str, 2, ax, 1, elem_size, acc_size, heavy);
+                ReducePlan q = plan_reduce(data, shp, str, 2, ax, 1, elem_size, acc_size, heavy, spare_scratch);
                 if (q.kind == ReduceKind::Row && q.lean && q.vec == full && !q.ragged && !q.unaligned && q.sstride == 1 &&
                     q.split == 1 && !q.row_tile) {
                     q.interleave = (int)L;
@@ -387,8 +391,12 @@ ReducePlan plan_reduce(const void* data, const int64_t* shape, const int64_t* st
         // times the bytes in flight per lane for f16. The last lane of a row loads its few elements singly.
         // (Worth it when a row is a few wavefronts of such lanes and enough is reduced into each output
         // that the lane's outputs, which it then writes one by one, are a small part of the traffic.)
-        if (p.lean && nk && p.vec == 1 && p.sstride == 1 && full > 1 && p.kept.stride[nk - 1] == 1 && kin >= 256 &&
-            p.R >= 256 && (uintptr_t)data % elem_size == 0) {
+        // (Small inputs, whose time is the chain of loads of one lane, gain from two lanes per row on: their column
+        // blocks are narrow, below.)
+        const int64_t bytes = p.K * p.R * (int64_t)elem_size;
+        const bool small = p.lean && bytes < kSmallColBytes;
+        if (p.lean && nk && p.vec == 1 && p.sstride == 1 && full > 1 && p.kept.stride[nk - 1] == 1 &&
+            (small ? kin >= 2 * full && p.R >= 64 : kin >= 256 && p.R >= 256) && (uintptr_t)data % elem_size == 0) {
             p.unaligned = true;
             p.vec = full;
         }
@@ -404,6 +412,39 @@ ReducePlan plan_reduce(const void* data, const int64_t* shape, const int64_t* st
                 if (waste(p.bx) * 8 > kv && waste(b) < waste(p.bx)) p.bx = b;
         }
         int64_t xblocks = (kv + p.bx - 1) / p.bx * (p.lean ? outer : 1);
+        if (small) {
+            // Below 8 MiB the time is the chain of dependent batches of loads of one lane, and the compute units that
+            // stand idle: 16-lane column blocks (256-byte segments of each row) make more workgroups of them, and up
+            // to 1024 threads share a block's rows. Where that still leaves a lane more than 24 rows (three batches of
+            // eight loads; a second launch costs as much: f32 [1216, 225], 19 rows, 6.4 us in one launch, 7.3 in two),
+            // the rows are dealt over workgroups too, about 12 to a lane. Over axis 0, us before -> now:
+            // f32 [12608, 128] 109 -> 8.9, f16 [2315, 363] 197 -> 8.2 (in one launch 16.1), bf16 [34112, 40] 57 -> 9.0,
+            // f32 [5440, 45] 28.3 -> 7.4; one launch is enough for f32 [1578, 2101][:, ::2], 17.6 -> 8.3.
+            while (p.bx > 16 && xblocks < kComputeUnits && p.R >= 32) {
+                p.bx /= 2;
+                xblocks = (kv + p.bx - 1) / p.bx * outer;
+            }
+            const int rows_per_wave = 64 / p.bx, uv = p.vec / p.sstride;
+            int64_t by = pow2_ceil((p.R + 7) / 8);
+            by = std::min(by, rows_per_wave * pow2_ceil((2048 + xblocks - 1) / xblocks));
+            by = std::max<int64_t>(rows_per_wave, std::min<int64_t>(by, 1024 / p.bx));
+            while (by > rows_per_wave && (size_t)p.bx * by * uv * acc_size > (64u << 10)) by /= 2;
+            p.by = (int)by;
+            p.split = 1;
+            if ((p.R + by - 1) / by > 24 && spare_scratch) {
+                // workgroups of 256 threads: the more rows share a workgroup, the longer its fold through LDS
+                const int64_t sby = std::min<int64_t>(by, std::max(rows_per_wave, 256 / p.bx));
+                const int64_t cap = (int64_t)(kSmallColScratch / acc_size) / p.K;
+                const int64_t split = std::min({(p.R + sby * 12 - 1) / (sby * 12), (1024 + xblocks - 1) / xblocks, cap});
+                if (split * sby > 2 * by) {
+                    p.by = (int)sby;
+                    p.split = (int)split;
+                    p.small_split = true;
+                }
+            }
+            p.chunk = (p.R + p.split - 1) / p.split;
+            return p;
+        }
         // One wavefront per 64 vector columns streams best when there are enough
         // columns (measured: 832 wavefronts with 128 loads each reach 5.9 TB/s);
         // with fewer, thread rows and then workgroups split the reduced range.
@@ -417,8 +458,7 @@ ReducePlan plan_reduce(const void* data, const int64_t* shape, const int64_t* st
         const int64_t can = std::max<int64_t>(1, p.R / 16);
         const int64_t rp = std::min(need, can);
         if (rp > 1) {
-            const int64_t bytes = p.K * p.R * (int64_t)elem_size;
-            if (bytes >= (8ll << 20)) {
+            if (bytes >= kSmallColBytes) {
                 // Large input: partition over WORKGROUPS first, so that the partitions land
                 // on different CUs (48 workgroups of 1024 threads leave 208 CUs idle), and
                 // fold the partials in a second launch.
