@@ -392,11 +392,11 @@ ReducePlan plan_reduce(const void* data, const int64_t* shape, const int64_t* st
         // (Worth it when a row is a few wavefronts of such lanes and enough is reduced into each output
         // that the lane's outputs, which it then writes one by one, are a small part of the traffic.)
         // (Small inputs, whose time is the chain of loads of one lane, gain from two lanes per row on: their column
-        // blocks are narrow, below.)
+        // blocks are narrow, below. Under 16 KiB a lane has a dozen loads in all either way.)
         const int64_t bytes = p.K * p.R * (int64_t)elem_size;
         const bool small = p.lean && bytes < kSmallColBytes;
         if (p.lean && nk && p.vec == 1 && p.sstride == 1 && full > 1 && p.kept.stride[nk - 1] == 1 &&
-            (small ? kin >= 2 * full && p.R >= 64 : kin >= 256 && p.R >= 256) && (uintptr_t)data % elem_size == 0) {
+            (small ? kin >= 2 * full && p.R >= 64 && bytes >= (16 << 10) : kin >= 256 && p.R >= 256) && (uintptr_t)data % elem_size == 0) {
             p.unaligned = true;
             p.vec = full;
         }
