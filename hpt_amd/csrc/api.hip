@@ -524,12 +524,20 @@ static NormCall prepare_norm(const hpt_view* in, const void* out_data, int64_t a
 }
 
 // Launch a normalisation; plans that need scratch (partial row statistics) get
-// the per-stream buffer, held under its lock from lookup to launch.
+// the per-stream buffer, held under its lock from lookup to launch. Transposed rows off the vector grid have a form
+// without scratch too (one group of lanes per row): it is taken under capture and on a full device.
 static void launch_norm(int dev, hipStream_t st, NormLaunchFn fn, NormCall& c, const char* what) {
+    const bool spare = c.plan.kind == NormKind::Transposed && c.plan.shift;
+    if (spare && capturing(st)) demote_to_generic(c.plan);
     if (c.plan.scratch_bytes) {
         StreamScratch& s = scratch_entry(dev, st);
         std::lock_guard<std::mutex> g(s.mu);
-        c.args.scratch = scratch_reserve(dev, s, c.plan.scratch_bytes);
+        try {
+            c.args.scratch = scratch_reserve(dev, s, c.plan.scratch_bytes);
+        } catch (const Error&) {
+            if (!spare) throw;
+            demote_to_generic(c.plan);
+        }
         fn(c.plan, c.args, st);
         check_launch(what);
     } else {

@@ -675,31 +675,51 @@ NormPlan plan_normalize(const void* in_data, const void* out_data, const int64_t
 
     if (p.norm_in.n == 1 && p.out_axis_stride == 1) {
         // rows are contiguous in the output
-        // input contiguous along the rows, output along the axis (a transposed view):
-        // statistics pass + register-tile transpose, when 128-bit access is legal both ways
+        // input contiguous along the rows, output along the axis (a transposed view): register tiles in
+        // one pass, or statistics pass + register-tile transpose; unaligned vectors (shift) where a pitch, a
+        // length or a base is off the 16-byte grid. The rows went element by element then, one cache line per
+        // lane and load: us, rows x columns, softmax and layernorm: f16 15552 x 1470 206 and 226 -> 24 and 22,
+        // f16 2066 x 11011 248 and 262 -> 46 and 42, f32 2557 x 2644 97 and 102 -> 21 and 21, f32 6966 x 368
+        // 32 and 36 -> 10.6 and 11, f16 1279 x 432 9.6 and 10.6 -> 7.4 and 6.4.
         const int nk = p.kept_in.n;
         const int v = max_vec;
-        bool transposed = sa > 1 && nk >= 1 && nk <= 2 && p.kept_in.stride[nk - 1] == 1 && v > 1 &&
-                          p.kept_in.size[nk - 1] % v == 0 && p.cols % v == 0 && sa % v == 0 &&
-                          (nk == 1 || (p.kept_in.stride[0] % v == 0 && p.kept_in.size[0] <= 65535)) &&
-                          ((uintptr_t)in_data % 16) == 0 && ((uintptr_t)out_data % 16) == 0 &&
-                          p.kept_in.size[nk - 1] <= (1 << 30) && p.cols <= (1 << 30) &&  // 32-bit positions
-                          p.kept_in.size[nk - 1] >= 8 * v && p.cols >= 8 * v;
-        if (transposed) {
+        const bool lies_transposed = sa > 1 && nk >= 1 && nk <= 2 && p.kept_in.stride[nk - 1] == 1 && v > 1 &&
+                                     (nk == 1 || p.kept_in.size[0] <= 65535) &&
+                                     p.kept_in.size[nk - 1] <= (1 << 30) && p.cols <= (1 << 30) &&  // 32-bit positions
+                                     p.kept_in.size[nk - 1] >= 8 * v && p.cols >= 8 * v;
+        const bool on_grid = lies_transposed && p.kept_in.size[nk - 1] % v == 0 && p.cols % v == 0 && sa % v == 0 &&
+                             (nk == 1 || p.kept_in.stride[0] % v == 0) &&
+                             ((uintptr_t)in_data % 16) == 0 && ((uintptr_t)out_data % 16) == 0;
+        // (columns that overlap, of a view made by hand, keep the forms below)
+        if (lies_transposed && (on_grid || sa >= p.kept_in.size[nk - 1])) {
             p.vec = v;
+            p.shift = on_grid ? 0 : 1;
             {
                 // Single pass when 16 vectors per thread hold (16 * rgN bytes of rows) x (all
                 // columns): rgN lanes along the rows, 1024 / rgN thread columns of 16 columns
-                // each. Prefer long row segments, but keep at least ~one workgroup per
-                // compute unit; below 64-byte segments the three-pass form is used.
+                // each, 4096 columns at most. Long row segments where they leave enough workgroups; a
+                // matrix too small for that is cut into segments of 64 and 32 bytes, which still beats three launches
+                // by far (us, three passes -> one; rows x columns): f32 3200 x 224 softmax 21.5 -> 5.2, layernorm
+                // 12.6 -> 4.9; f16 5184 x 2048 24.7 -> 14.7, 21 -> 13; f32 300 x 1001 18.6 -> 6.3; bf16 511 x 2001
+                // 22 -> 13.0. It loses where few workgroups walk many columns of a layernorm whose statistics are
+                // cheap (f32 129 x 4000: 12.0 -> 13.9). Beyond 4096 columns 32-byte segments gain nothing (f16
+                // 2048 x 8192 28.0 -> 26.3, f32 333 x 8000 layernorm 17 -> 25): three passes. So do
+                // matrices below 16384 elements, whose plan is pinned.
                 const int64_t R = p.kept_in.size[nk - 1];
                 const int64_t batch = nk > 1 ? p.kept_in.size[0] : 1;
                 const int64_t cgroups = (p.cols + 15) / 16;
+                auto blocks_of = [&](int rg) { return (R + rg * v - 1) / (rg * v) * batch; };
                 int rgN = 16;
                 while (rgN >= 4 && cgroups * rgN > 1024) rgN >>= 1;
-                while (rgN > 8 && (R + rgN * v - 1) / (rgN * v) * batch < 256) rgN >>= 1;
-                const int64_t blocks = rgN >= 4 ? (R + rgN * v - 1) / (rgN * v) * batch : 0;
-                if (rgN >= 4 && blocks >= 128) {
+                if (rgN > 8 && blocks_of(rgN) < 256) rgN = 8;
+                // Sums of exponentials of f32 rows: f64, but for matrices on the vector grid that fill the chip with long
+                // segments, where a thread's 16 of a row are added in f32 and the conversions would show (f32
+                // 6080 x 2752 38.3 -> 39.6 us).
+                p.wide_sum = p.shift || blocks_of(rgN) < 128;
+                if (rgN > 4 && blocks_of(rgN) < 192) rgN = 4;
+                if (rgN == 4 && blocks_of(rgN) < 128) rgN = 2;
+                const bool cheap_passes = n_norm_dims > 0 && elem_size >= 4 && p.cols > 2048 && blocks_of(rgN) < 32;
+                if (cgroups * 4 <= 1024 && !cheap_passes && (blocks_of(rgN) >= 128 || total >= 16384)) {
                     p.kind = NormKind::TransposedTile;
                     p.tpr = rgN;
                     const int64_t cols_per_wave = 16 * (64 / rgN);
@@ -1232,7 +1252,7 @@ std::string describe(const NormPlan& p) {
     static const char* names[] = {"empty", "rowreg", "rowstream", "rowsplit", "col", "col-split", "transposed", "transposed-tile", "col-reg", "generic"};
     char buf[256];
     snprintf(buf, sizeof buf, "%s%s%s rows=%lld cols=%lld vec=%d tpr=%d rpb=%d nchunk=%d ostride=%lld ",
-             names[(int)p.kind], p.sstride == 2 ? "-step2" : (p.flat_t ? (p.shift ? "-flat-unaligned" : "-flat") : (p.shift ? ((p.kind == NormKind::RowSplit || p.kind == NormKind::ColReg || p.kind == NormKind::ColSplit) ? "-unaligned" : (p.lds_rows ? "-lds-shift" : "-shift")) : (p.gb_lds == 2 ? "-l2gb" : p.gb_lds ? "-ldsgb" : (p.raw_rows ? "-raw" : (p.lds_rows ? "-lds" : ""))))), p.tile_rows ? "+tile" : (p.interleave > 1 ? "-interleaved" : p.interleave < 0 ? "-modular" : p.group_tile ? "-group-tile" : (p.slab_tile ? "-slab" : "")), (long long)p.rows, (long long)p.cols, p.vec, p.tpr, p.rpb,
+             names[(int)p.kind], p.sstride == 2 ? "-step2" : (p.flat_t ? (p.shift ? "-flat-unaligned" : "-flat") : (p.shift ? ((p.kind == NormKind::RowSplit || p.kind == NormKind::ColReg || p.kind == NormKind::ColSplit || p.kind == NormKind::Transposed || p.kind == NormKind::TransposedTile) ? "-unaligned" : (p.lds_rows ? "-lds-shift" : "-shift")) : (p.gb_lds == 2 ? "-l2gb" : p.gb_lds ? "-ldsgb" : (p.raw_rows ? "-raw" : (p.lds_rows ? "-lds" : ""))))), p.tile_rows ? "+tile" : (p.interleave > 1 ? "-interleaved" : p.interleave < 0 ? "-modular" : p.group_tile ? "-group-tile" : (p.slab_tile ? "-slab" : "")), (long long)p.rows, (long long)p.cols, p.vec, p.tpr, p.rpb,
              p.nchunk, (long long)p.out_axis_stride);
     std::string s = buf;
     if (p.kind == NormKind::RowReg) s += "max_blocks=" + std::to_string(p.max_blocks) + " ";  // (layernorm walks its rows)

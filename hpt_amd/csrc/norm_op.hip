@@ -175,6 +175,16 @@ template <class T> void launch_transposed(const NormPlan& p, const NormArgs& a, 
         t.rg_log2 = ilog2(p.tpr);
         t.share_log2 = p.tpr >= 8 ? 0 : (p.tpr == 4 ? 1 : 2);
         const unsigned blocks = (unsigned)((t.R + p.tpr * FULL - 1) / (p.tpr * FULL));
+        if (p.shift) {
+            transposed_tile_kernel<KIND, T, true><<<dim3(blocks, batch), dim3(64u * (unsigned)p.rpb), 0, st>>>(t);
+            return;
+        }
+        if constexpr (std::is_same<T, float>::value && KIND != NORM_LAYERNORM) {
+            if (p.wide_sum) {
+                transposed_tile_kernel<KIND, T, false, true><<<dim3(blocks, batch), dim3(64u * (unsigned)p.rpb), 0, st>>>(t);
+                return;
+            }
+        }
         transposed_tile_kernel<KIND, T><<<dim3(blocks, batch), dim3(64u * (unsigned)p.rpb), 0, st>>>(t);
         return;
     }
@@ -203,10 +213,14 @@ template <class T> void launch_transposed(const NormPlan& p, const NormArgs& a, 
         const unsigned rg = (unsigned)((t.R + 64 * FULL - 1) / (64 * FULL));
         using Part = typename RowPartial<KIND, T>::type;
         const unsigned nw = (unsigned)p.tpr;  // wavefronts per workgroup of the statistics pass
-        transposed_stats_kernel<KIND, T>
-            <<<dim3(rg, (unsigned)t.S, batch), dim3(64 * nw), (size_t)nw * FULL * 64 * sizeof(Part), st>>>(t);
+        const dim3 sgrid(rg, (unsigned)t.S, batch);
+        const size_t slds = (size_t)nw * FULL * 64 * sizeof(Part);
+        if (p.shift) transposed_stats_kernel<KIND, T, FULL, true><<<sgrid, dim3(64 * nw), slds, st>>>(t);
+        else transposed_stats_kernel<KIND, T><<<sgrid, dim3(64 * nw), slds, st>>>(t);
         transposed_finalize_kernel<KIND, T><<<dim3((unsigned)((t.R + 15) / 16), 1, batch), dim3(16, 16), 0, st>>>(t);
-        transposed_apply_kernel<KIND, T><<<dim3((rt + 3) / 4, (unsigned)((tiles + 1) / 2), batch), dim3(256), 0, st>>>(t);
+        const dim3 agrid((rt + 3) / 4, (unsigned)((tiles + 1) / 2), batch);
+        if (p.shift) transposed_apply_kernel<KIND, T, true><<<agrid, dim3(256), 0, st>>>(t);
+        else transposed_apply_kernel<KIND, T><<<agrid, dim3(256), 0, st>>>(t);
         return;
     }
 }

@@ -258,7 +258,9 @@ __global__ void __launch_bounds__(256) transposed_finalize_kernel(const Transpos
 // wavefronts of a workgroup take neighbouring row tiles (512 contiguous bytes of the input per
 // column) and each wavefront takes two neighbouring column tiles (256 contiguous bytes of
 // the output per row).
-template <int KIND, class T>
+// UA: rows or columns that are not whole, aligned vectors: unaligned vectors, the last one of either taken from the
+// end backwards (what two lanes hold is stored twice, the same bits).
+template <int KIND, class T, bool UA = false>
 __global__ void __launch_bounds__(256) transposed_apply_kernel(const TransposedArgs a) {
     using CT = typename Elem<T>::Wide;
     constexpr int VEC = 16 / sizeof(T);
@@ -266,38 +268,42 @@ __global__ void __launch_bounds__(256) transposed_apply_kernel(const TransposedA
 
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int rg = lane & 7, cl = lane >> 3;
-    const int r0 = (blockIdx.x * 4 + w) * TR + rg * VEC;
+    int r0 = (blockIdx.x * 4 + w) * TR + rg * VEC;
     const int c_base = blockIdx.y * (NC * TC) + cl * VEC;
     if (r0 >= a.R || c_base >= a.cols) return;
+    if constexpr (UA) r0 = min(r0, a.R - VEC);
 
     const CT* pp = (const CT*)a.params + (int64_t)blockIdx.z * 3 * a.R + r0;
-    const Pack<CT, VEC> p0 = *reinterpret_cast<const Pack<CT, VEC>*>(pp);
-    const Pack<CT, VEC> p1 = *reinterpret_cast<const Pack<CT, VEC>*>(pp + a.R);
+    auto params = [](const CT* p) { return UA ? load_pack_unaligned<CT, VEC>(p) : load_pack<CT, VEC>(p); };
+    auto load = [](const T* p) { return UA ? load_pack_unaligned<T, VEC>(p) : load_pack<T, VEC>(p); };
+    const Pack<CT, VEC> p0 = params(pp);
+    const Pack<CT, VEC> p1 = params(pp + a.R);
     Pack<CT, VEC> p2 = p0;
-    if constexpr (KIND == NORM_LAYERNORM) p2 = *reinterpret_cast<const Pack<CT, VEC>*>(pp + 2 * (int64_t)a.R);
+    if constexpr (KIND == NORM_LAYERNORM) p2 = params(pp + 2 * (int64_t)a.R);
 
     const T* base = (const T*)a.in + (int64_t)blockIdx.z * a.bi + r0;
     Pack<T, VEC> v[NC][VEC], gam[NC], bet[NC];
     bool have[NC];
+    int col[NC];
 #pragma unroll
     for (int s = 0; s < NC; ++s) {
-        const int c0 = c_base + s * TC;
-        have[s] = c0 < a.cols;
+        have[s] = c_base + s * TC < a.cols;
+        const int c0 = col[s] = UA ? min(c_base + s * TC, a.cols - VEC) : c_base + s * TC;
         if (!have[s]) continue;
 #pragma unroll
-        for (int i = 0; i < VEC; ++i) v[s][i] = load_pack<T, VEC>(base + (int64_t)(c0 + i) * a.sa);
+        for (int i = 0; i < VEC; ++i) v[s][i] = load(base + (int64_t)(c0 + i) * a.sa);
         if constexpr (KIND == NORM_LAYERNORM) {
 #pragma unroll
             for (int i = 0; i < VEC; ++i) {
                 gam[s].v[i] = Elem<T>::narrow((CT)1);
                 bet[s].v[i] = Elem<T>::narrow((CT)0);
             }
-            if (a.gamma) gam[s] = load_pack<T, VEC>((const T*)a.gamma + c0);
-            if (a.beta) bet[s] = load_pack<T, VEC>((const T*)a.beta + c0);
+            if (a.gamma) gam[s] = load((const T*)a.gamma + c0);
+            if (a.beta) bet[s] = load((const T*)a.beta + c0);
         }
     }
 
-    T* out = (T*)a.out + ((int64_t)blockIdx.z * a.R + r0) * a.cols + c_base;
+    T* out = (T*)a.out + ((int64_t)blockIdx.z * a.R + r0) * a.cols;
 #pragma unroll
     for (int k = 0; k < VEC; ++k)
 #pragma unroll
@@ -316,7 +322,8 @@ __global__ void __launch_bounds__(256) transposed_apply_kernel(const TransposedA
                     y = (x - p0.v[k]) - p1.v[k];
                 o.v[i] = Elem<T>::narrow(y);
             }
-            store_pack_stream<T, VEC>(out + (int64_t)k * a.cols + s * TC, o);
+            if constexpr (UA) store_pack_unaligned<T, VEC>(out + (int64_t)k * a.cols + col[s], o);
+            else store_pack_stream<T, VEC>(out + (int64_t)k * a.cols + col[s], o);
         }
 }
 
@@ -797,7 +804,12 @@ template <class T, int VEC> __device__ __forceinline__ void forget_values(Pack<T
     }
 }
 
-template <int KIND, class T>
+// UA: rows or columns that are not whole, aligned vectors. The same vectors are loaded and stored unaligned; the
+// last row vector and the last column vector are taken from the end backwards, so nothing outside the tensor is
+// touched. Rows held twice give the same bits twice; columns held twice are left out of the sums the second time.
+// WIDE: softmax of f32 rows adds every exponential in f64. (A kernel of its own: with both loops in one kernel f32
+// 6080 x 2752 takes 44 us instead of 38.)
+template <int KIND, class T, bool UA = false, bool WIDE = UA>
 __global__ void __launch_bounds__(1024) transposed_tile_kernel(const TileArgs a) {
     using CT = typename Elem<T>::Wide;
     using ST = typename StatType<T>::type;
@@ -820,13 +832,19 @@ __global__ void __launch_bounds__(1024) transposed_tile_kernel(const TileArgs a)
         const int x = b & 7, q = b >> 3;
         b = ((x + 8 * (q >> a.share_log2)) << a.share_log2) | (q & ((1 << a.share_log2) - 1));
     }
-    const int r0 = (b * rgN + rg) * VEC;
-    const bool row_ok = r0 < a.R;
+    const bool row_ok = (b * rgN + rg) * VEC < a.R;
+    const int r0 = UA ? min((b * rgN + rg) * VEC, a.R - VEC) : (b * rgN + rg) * VEC;
     const int gw = VEC * cgw;                       // columns a wavefront covers per group
     const int c_first = w * 16 * cgw + cgl * VEC;   // first column of group 0
     bool col_ok[H];
+    int col[H], twice[H];  // UA: first column of the group's vector, how many of its columns another thread counts
 #pragma unroll
-    for (int h = 0; h < H; ++h) col_ok[h] = c_first + h * gw < a.cols;
+    for (int h = 0; h < H; ++h) {
+        const int c = c_first + h * gw;
+        col_ok[h] = c < a.cols;
+        col[h] = UA ? min(c, a.cols - VEC) : c;
+        twice[h] = UA ? c - col[h] : 0;
+    }
 
     const CT one = std::is_same<T, f16_t>::value ? (CT)opaque_one() : (CT)1;  // see widen_fma
 
@@ -841,9 +859,9 @@ __global__ void __launch_bounds__(1024) transposed_tile_kernel(const TileArgs a)
         const T* base = (const T*)a.in + (int64_t)blockIdx.y * a.bi + (row_ok ? r0 : 0);
 #pragma unroll
         for (int h = 0; h < H; ++h) {
-            const T* p = base + (col_ok[h] ? (int64_t)(c_first + h * gw) * a.sa : (int64_t)0);
+            const T* p = base + (col_ok[h] ? (int64_t)col[h] * a.sa : (int64_t)0);
 #pragma unroll
-            for (int i = 0; i < VEC; ++i) v[h * VEC + i] = load_pack<T, VEC>(p + i * a.sa);
+            for (int i = 0; i < VEC; ++i) v[h * VEC + i] = UA ? load_pack_unaligned<T, VEC>(p + i * a.sa) : load_pack<T, VEC>(p + i * a.sa);
         }
     }
     // gamma / beta of this thread's columns, fetched before anything is stored: a load
@@ -855,11 +873,11 @@ __global__ void __launch_bounds__(1024) transposed_tile_kernel(const TileArgs a)
     // then replaced: a load under a branch would make the compiler wait for it, and for
     // every load issued before it, at the end of the branch)
     auto load_affine = [&](int h, Pack<T, VEC>& gp, Pack<T, VEC>& bp) {
-        const int c = col_ok[h] ? c_first + h * gw : 0;
+        const int c = col_ok[h] ? col[h] : 0;
         const T* gsrc = a.gamma ? (const T*)a.gamma + c : (const T*)a.in;
         const T* bsrc = a.beta ? (const T*)a.beta + c : (const T*)a.in;
-        gp = load_pack<T, VEC>(gsrc);
-        bp = load_pack<T, VEC>(bsrc);
+        gp = UA ? load_pack_unaligned<T, VEC>(gsrc) : load_pack<T, VEC>(gsrc);
+        bp = UA ? load_pack_unaligned<T, VEC>(bsrc) : load_pack<T, VEC>(bsrc);
         Pack<T, VEC> ones, zeros;
 #pragma unroll
         for (int i = 0; i < VEC; ++i) {
@@ -922,15 +940,20 @@ __global__ void __launch_bounds__(1024) transposed_tile_kernel(const TileArgs a)
         }
         forget_values(v);
         tile_all_reduce<MaxC<CT>, CT, VEC>(m, rgN, rg, cgl, w, nw, (CT*)part, (CT*)res);
-        CT s[VEC], nml[VEC];
+        ST s[VEC];
+        CT nml[VEC];
 #pragma unroll
         for (int k = 0; k < VEC; ++k) {
             s[k] = 0;
             nml[k] = -m[k] * (CT)1.4426950408889634;  // -max * log2(e), see tile_exp
         }
+        using AT = typename std::conditional<WIDE, ST, CT>::type;  // what the thread's own sums are taken in
+        AT t[VEC];
+#pragma unroll
+        for (int k = 0; k < VEC; ++k) t[k] = 0;
 #pragma unroll
         for (int h = 0; h < H; ++h) {
-            CT sh[VEC];
+            AT sh[VEC];
 #pragma unroll
             for (int k = 0; k < VEC; ++k) sh[k] = 0;
 #pragma unroll
@@ -938,20 +961,22 @@ __global__ void __launch_bounds__(1024) transposed_tile_kernel(const TileArgs a)
 #pragma unroll
                 for (int k = 0; k < VEC; ++k) {
                     const CT e = tile_exp<T>(v[h * VEC + i].v[k], m[k], nml[k]);
-                    sh[k] += e;
+                    sh[k] += (AT)(UA && i < twice[h] ? (CT)0 : e);
                     if constexpr (kKeepExp && KIND == NORM_SOFTMAX) v[h * VEC + i].v[k] = Elem<T>::narrow(e);
                 }
             if (col_ok[h]) {
 #pragma unroll
-                for (int k = 0; k < VEC; ++k) s[k] += sh[k];
+                for (int k = 0; k < VEC; ++k) t[k] += sh[k];
             }
         }
+#pragma unroll
+        for (int k = 0; k < VEC; ++k) s[k] = (ST)t[k];
         forget_values(v);
-        tile_all_reduce<SumC<CT>, CT, VEC>(s, rgN, rg, cgl, w, nw, (CT*)part, (CT*)res);
+        tile_all_reduce<SumC<ST>, ST, VEC>(s, rgN, rg, cgl, w, nw, part, res);
 #pragma unroll
         for (int k = 0; k < VEC; ++k) {
             p0[k] = m[k];
-            p1[k] = KIND == NORM_SOFTMAX ? (CT)1 / s[k] : log_ct<T>(s[k]);
+            p1[k] = KIND == NORM_SOFTMAX ? (CT)1 / (CT)s[k] : log_ct<T>((CT)s[k]);
             p2[k] = nml[k];
         }
     } else {
@@ -969,7 +994,7 @@ __global__ void __launch_bounds__(1024) transposed_tile_kernel(const TileArgs a)
 #pragma unroll
                 for (int i = 0; i < VEC; ++i)
 #pragma unroll
-                    for (int k = 0; k < VEC; ++k) th[k] += (ST)Elem<T>::widen(v[h * VEC + i].v[k]);
+                    for (int k = 0; k < VEC; ++k) th[k] += (ST)(UA && i < twice[h] ? (CT)0 : Elem<T>::widen(v[h * VEC + i].v[k]));
                 if (col_ok[h]) {
 #pragma unroll
                     for (int k = 0; k < VEC; ++k) sum[k] += th[k];
@@ -987,7 +1012,10 @@ __global__ void __launch_bounds__(1024) transposed_tile_kernel(const TileArgs a)
 #pragma unroll
                 for (int i = 0; i < VEC; ++i)
 #pragma unroll
-                    for (int k = 0; k < VEC; ++k) th[k] = widen_fma(v[h * VEC + i].v[k], one, th[k]);
+                    for (int k = 0; k < VEC; ++k) {
+                        const CT t1 = widen_fma(v[h * VEC + i].v[k], one, th[k]);
+                        th[k] = UA && i < twice[h] ? th[k] : t1;
+                    }
                 if (col_ok[h]) {
 #pragma unroll
                     for (int k = 0; k < VEC; ++k) t[k] += th[k];
@@ -1023,6 +1051,7 @@ __global__ void __launch_bounds__(1024) transposed_tile_kernel(const TileArgs a)
                     for (int k = 0; k < VEC; ++k) {
                         CT d = widen_fma(v[h * VEC + i].v[k], one, -p0[k]);
                         if constexpr (sizeof(ST) > sizeof(CT)) d -= p1[k];
+                        if (UA && i < twice[h]) d = 0;
                         th[k] += d * d;
                     }
                 if (col_ok[h]) {
@@ -1050,7 +1079,7 @@ __global__ void __launch_bounds__(1024) transposed_tile_kernel(const TileArgs a)
             asm volatile("" : "+v"(*reinterpret_cast<u32x4*>(&bet[h])));
         }
     }
-    T* out = (T*)a.out + ((int64_t)blockIdx.y * a.R + r0) * a.cols + c_first;
+    T* out = (T*)a.out + ((int64_t)blockIdx.y * a.R + r0) * a.cols;
 #pragma unroll
     for (int h = 0; h < H; ++h) {
         if (!col_ok[h]) continue;
@@ -1089,7 +1118,9 @@ __global__ void __launch_bounds__(1024) transposed_tile_kernel(const TileArgs a)
                 }
                 o.v[i] = Elem<T>::narrow(y);
             }
-            store_pack_stream<T, VEC>(out + (int64_t)k * a.cols + h * gw, o);
+            // (unaligned: the lines shared with the neighbouring stores meet in L2)
+            if constexpr (UA) store_pack_unaligned<T, VEC>(out + (int64_t)k * a.cols + col[h], o);
+            else store_pack_stream<T, VEC>(out + (int64_t)k * a.cols + col[h], o);
             // one output vector at a time: interleaving several only adds live registers
             __builtin_amdgcn_sched_barrier(0);
         }
