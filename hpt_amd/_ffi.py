@@ -63,6 +63,8 @@ SIGNATURES = {
     "hpt_hip_device_count": (C.c_int32, [C.POINTER(C.c_int32)]),
     "hpt_hip_alloc": (C.c_int32, [C.c_int32, C.c_size_t, C.c_size_t, C.c_int32, C.POINTER(C.c_void_p)]),
     "hpt_hip_free": (C.c_int32, [C.c_int32, C.c_void_p, C.c_size_t, C.c_size_t]),
+    "hpt_hip_alloc_ordered": (C.c_int32, [C.c_int32, C.c_size_t, C.c_size_t, C.POINTER(C.c_void_p)]),
+    "hpt_hip_free_ordered": (C.c_int32, [C.c_int32, C.c_void_p, C.c_size_t, C.c_size_t]),
     "hpt_hip_forget": (C.c_int32, [C.c_int32, C.c_void_p]),
     "hpt_hip_cache_resize": (C.c_int32, [C.c_int32, C.c_size_t]),
     "hpt_hip_cache_clear": (C.c_int32, [C.c_int32]),
@@ -128,15 +130,19 @@ def check(status: int) -> None:
         raise _ERRORS.get(status, HptError)(status, msg)
 
 
+# (ctypes builds an array type on every multiplication unless its cache still holds it)
+_I64_ARRAY = [C.c_int64 * max(1, n) for n in range(9)]
+_I64_P = C.POINTER(C.c_int64)
+
+
 def i64_array(values):
-    values = list(values)
-    return (C.c_int64 * max(1, len(values)))(*values)
+    values = tuple(values)
+    return _I64_ARRAY[len(values)](*values) if len(values) < len(_I64_ARRAY) else (C.c_int64 * len(values))(*values)
 
 
 def make_view(ptr: int, shape, strides, dtype: int):
     """Build an hpt_view; returns (view, keepalive) — keep both alive during the call."""
     sh = i64_array(shape)
     st = i64_array(strides)
-    v = View(C.c_void_p(ptr), C.cast(sh, C.POINTER(C.c_int64)), C.cast(st, C.POINTER(C.c_int64)),
-             len(list(shape)), int(dtype))
+    v = View(ptr, C.cast(sh, _I64_P), C.cast(st, _I64_P), len(shape), dtype)
     return v, (sh, st)

@@ -59,6 +59,25 @@ static void use_device(int dev) {
         hip_check(hipSetDevice(dev), HPT_ERR_DEVICE, "hipSetDevice");
 }
 
+// Whether work on `st` is being recorded (or may not be asked about because another stream's is): scratch must
+// not be allocated then, and a recorded call outlives the buffer's next owner.
+static bool capturing(hipStream_t st) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &status) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;
+    }
+    return status != hipStreamCaptureStatusNone;
+}
+
+// Lets the calling thread make runtime calls that a capture in progress (its own or another thread's, on streams that
+// these calls do not touch) would otherwise refuse.
+struct RelaxedCapture {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+    ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
 // ---- device caching allocator ------------------------------------------------
 // Same policy as the reference's CudaAllocator
 // (hpt-allocator/src/allocators/cuda.rs:41-322, utils/allocate.rs:15-130,
@@ -66,6 +85,10 @@ static void use_device(int dev) {
 // layout; a freed block is kept in an LRU cache of layouts; evicting a layout
 // releases all of its blocks; when the device is out of memory, layouts are
 // evicted least-recently-used first and the allocation is retried.
+// A block may come back while work on the DEFAULT stream still uses it (hpt_hip_free_ordered): it is numbered, and
+// handed on at once only to a caller whose first use of it is queued on the same stream (hpt_hip_alloc_ordered), so the
+// queue itself keeps the two apart. Anybody else waits for the default stream first, which makes every block numbered
+// so far idle. (Waiting at every free instead kept the host and the device taking turns: about 25 us of a pass.)
 
 struct LayoutKey {
     size_t bytes, align;
@@ -74,11 +97,17 @@ struct LayoutKey {
     }
 };
 
+struct CachedBlock {
+    void* p;
+    uint64_t number;  // of the free that left work queued on the default stream; 0: idle
+};
+
 struct DeviceAllocator {
     std::mutex mu;
+    uint64_t last_number = 0, idle_upto = 0;  // blocks numbered up to idle_upto are known to be idle
     size_t capacity = 100;  // cached layouts; the CPU allocator's default (allocators/cpu.rs:22)
     std::list<LayoutKey> lru;  // front = most recently used
-    std::map<LayoutKey, std::pair<std::list<LayoutKey>::iterator, std::vector<void*>>> cache;
+    std::map<LayoutKey, std::pair<std::list<LayoutKey>::iterator, std::vector<CachedBlock>>> cache;
     std::unordered_map<void*, LayoutKey> live;
     uint64_t device_mallocs = 0;
     size_t internal_blocks = 0;  // live blocks the library itself holds (scratch), not a caller
@@ -88,19 +117,46 @@ struct DeviceAllocator {
         for (auto& kv : cache) n += kv.second.second.size();
         return n;
     }
+    // Requires `mu` and the device to be current. False where the stream cannot be waited for: while another stream
+    // that it orders itself with is being captured.
+    bool wait_default_stream() {
+        if (idle_upto == last_number) return true;
+        if (capturing(nullptr)) return false;
+        RelaxedCapture relaxed;
+        if (hipStreamSynchronize(nullptr) != hipSuccess) {
+            (void)hipGetLastError();
+            return false;
+        }
+        idle_upto = last_number;
+        return true;
+    }
     void evict_one() {  // requires a non-empty cache
         LayoutKey k = lru.back();
         auto it = cache.find(k);
-        for (void* p : it->second.second) (void)hipFree(p);
+        for (const CachedBlock& b : it->second.second) {
+            if (b.number > idle_upto) (void)wait_default_stream();
+            (void)hipFree(b.p);
+        }
         cache.erase(it);
         lru.pop_back();
     }
-    void* allocate(size_t bytes, size_t align) {
+    // `ordered`: the block's first use will be queued on the default stream.
+    void* allocate(size_t bytes, size_t align, bool ordered = false) {
         LayoutKey k{bytes, align};
         auto it = cache.find(k);
-        if (it != cache.end() && !it->second.second.empty()) {
-            void* p = it->second.second.back();
-            it->second.second.pop_back();
+        size_t take = 0;  // one more than the index of the block to hand out
+        if (it != cache.end()) {
+            const std::vector<CachedBlock>& blocks = it->second.second;
+            take = blocks.size();
+            if (!ordered) {
+                while (take && blocks[take - 1].number > idle_upto) --take;
+                if (!take && wait_default_stream()) take = blocks.size();
+            }
+        }
+        if (take) {
+            std::vector<CachedBlock>& blocks = it->second.second;
+            void* p = blocks[take - 1].p;
+            blocks.erase(blocks.begin() + (take - 1));
             lru.splice(lru.begin(), lru, it->second.first);
             if (it->second.second.empty()) {
                 lru.erase(it->second.first);
@@ -110,6 +166,7 @@ struct DeviceAllocator {
             return p;
         }
         void* p = nullptr;
+        RelaxedCapture relaxed;
         for (;;) {
             hipError_t e = hipMalloc(&p, bytes ? bytes : 1);
             if (e == hipSuccess) break;
@@ -127,7 +184,8 @@ struct DeviceAllocator {
         live[p] = k;
         return p;
     }
-    void deallocate(void* p, size_t bytes, size_t align) {
+    // `ordered`: work queued on the default stream, and on no other, may still use the block.
+    void deallocate(void* p, size_t bytes, size_t align, bool ordered = false) {
         auto it = live.find(p);
         if (it == live.end()) fail(HPT_ERR_MEMORY, "pointer %p was not allocated by hpt_hip_alloc", p);
         if (it->second.bytes != bytes || it->second.align != align)
@@ -135,17 +193,19 @@ struct DeviceAllocator {
                  it->second.bytes, it->second.align, bytes, align);
         LayoutKey k = it->second;
         live.erase(it);
+        const CachedBlock b{p, ordered ? ++last_number : 0};
         if (capacity == 0) {
+            if (ordered) (void)wait_default_stream();
             (void)hipFree(p);
             return;
         }
         auto c = cache.find(k);
         if (c == cache.end()) {
             lru.push_front(k);
-            cache[k] = {lru.begin(), {p}};
+            cache[k] = {lru.begin(), {b}};
             while (cache.size() > capacity) evict_one();
         } else {
-            c->second.second.push_back(p);
+            c->second.second.push_back(b);
             lru.splice(lru.begin(), lru, c->second.first);
         }
     }
@@ -420,17 +480,6 @@ static ReduceCall prepare_reduce(int entry_id, const hpt_view* in, const int64_t
     return c;
 }
 
-// Whether work on `st` is being recorded (or may not be asked about because another stream's is): scratch must
-// not be allocated then, and a recorded call outlives the buffer's next owner.
-static bool capturing(hipStream_t st) {
-    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(st, &status) != hipSuccess) {
-        (void)hipGetLastError();
-        return true;
-    }
-    return status != hipStreamCaptureStatusNone;
-}
-
 // use_static: the partials go to the library's static device array instead of allocated
 // scratch; a plan that needs more than the array holds is refused.
 // Small inputs that are split for speed alone are reduced in one launch where scratch is not to be had for the
@@ -591,6 +640,27 @@ int32_t hpt_hip_free(int32_t dev, void* p, size_t bytes, size_t align) {
         DeviceAllocator& a = allocator_of(dev);
         std::lock_guard<std::mutex> g(a.mu);
         a.deallocate(p, bytes, align);
+    });
+}
+
+int32_t hpt_hip_alloc_ordered(int32_t dev, size_t bytes, size_t align, void** out) {
+    return guarded([&] {
+        if (!out) fail(HPT_ERR_PARAM, "alloc: null output");
+        if (align == 0 || (align & (align - 1))) fail(HPT_ERR_PARAM, "alloc: align %zu is not a power of two", align);
+        use_device(dev);
+        DeviceAllocator& a = allocator_of(dev);
+        std::lock_guard<std::mutex> g(a.mu);
+        *out = a.allocate(bytes, align, true);
+    });
+}
+
+int32_t hpt_hip_free_ordered(int32_t dev, void* p, size_t bytes, size_t align) {
+    return guarded([&] {
+        if (!p) return;
+        use_device(dev);
+        DeviceAllocator& a = allocator_of(dev);
+        std::lock_guard<std::mutex> g(a.mu);
+        a.deallocate(p, bytes, align, true);
     });
 }
 

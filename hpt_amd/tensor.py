@@ -19,6 +19,7 @@ hpt/src/backends/common/shape_manipulate.rs:144-167 and hpt-common/src/slice.rs:
 from __future__ import annotations
 
 import ctypes as C
+import math
 from typing import Iterable, Optional, Sequence
 
 import numpy as np
@@ -88,10 +89,14 @@ def _stream_key(stream) -> int:
     return int(getattr(stream, "value", None) or 0)
 
 
+_DEFAULT_STREAM_ONLY = {0}
+
+
 class _StreamTracked:
     """Which streams have work queued that reads or writes this memory. The library's free hands a
     block to the next caller at once (include/hpt_hip.h), and the synchronous copies only wait for
-    the default stream, so the owner waits for these streams itself before it frees or copies."""
+    the default stream, so the owner waits for these streams itself before it frees or copies (memory used
+    on the default stream alone is freed without a wait, through hpt_hip_free_ordered)."""
 
     device = 0
 
@@ -118,25 +123,36 @@ class _StreamTracked:
 
 
 class _DeviceStorage(_StreamTracked):
-    """A block owned through the library's caching allocator (hpt-allocator's Backend<B>)."""
+    """A block owned through the library's caching allocator (hpt-allocator's Backend<B>).
+    ordered: the block's first use is a call on the default stream, so it may be one that earlier work on that
+    stream is still using (hpt_hip_alloc_ordered); until somebody waits, it counts as used there."""
 
-    def __init__(self, device: int, nbytes: int, zeroed: bool = False):
+    def __init__(self, device: int, nbytes: int, zeroed: bool = False, ordered: bool = False):
         p = C.c_void_p()
-        check(_ffi.lib().hpt_hip_alloc(device, nbytes, ALIGN, int(zeroed), C.byref(p)))
+        if ordered:
+            check(_ffi.lib().hpt_hip_alloc_ordered(device, nbytes, ALIGN, C.byref(p)))
+        else:
+            check(_ffi.lib().hpt_hip_alloc(device, nbytes, ALIGN, int(zeroed), C.byref(p)))
         self.ptr = p.value or 0
         self.nbytes, self.device = nbytes, device
         self._init_streams()
+        if ordered:
+            self.touch(0)
 
     def __del__(self):
         if not self.ptr:
             return
-        try:
-            self.wait()  # kernels still queued on a caller's stream may use the block
-        except Exception:
-            pass  # (interpreter shutdown, or the device is gone: nothing more can be waited for)
+        free = "hpt_hip_free"
+        if self.pending == _DEFAULT_STREAM_ONLY:
+            free = "hpt_hip_free_ordered"  # the next owner's work queues up behind what is still running
+        else:
+            try:
+                self.wait()  # kernels still queued on a caller's stream may use the block
+            except Exception:
+                pass  # (interpreter shutdown, or the device is gone: nothing more can be waited for)
         try:
             # the block always goes back to the allocator, whatever the wait did
-            _ffi.lib().hpt_hip_free(self.device, C.c_void_p(self.ptr), self.nbytes, ALIGN)
+            getattr(_ffi.lib(), free)(self.device, C.c_void_p(self.ptr), self.nbytes, ALIGN)
         except Exception:
             pass
         self.ptr = 0
@@ -171,6 +187,19 @@ def _touch(stream, *tensors) -> None:
         st = getattr(t, "_storage", None) if t is not None else None
         if isinstance(st, _StreamTracked):
             st.touch(stream)
+
+
+_OUT_DTYPES = {}
+
+
+def _reduce_out_dtype(op: int, dtype: DType) -> DType:
+    """The output dtype of a reduce op (a constant of the library for each pair, asked for once)."""
+    od = _OUT_DTYPES.get((op, dtype.code))
+    if od is None:
+        out = C.c_int32()
+        check(_ffi.lib().hpt_hip_reduce_out_dtype(op, dtype.code, C.byref(out)))
+        od = _OUT_DTYPES[op, dtype.code] = DTYPES[out.value]
+    return od
 
 
 def _as_axes(axes) -> list:
@@ -210,8 +239,13 @@ class Tensor:
     def empty(cls, shape, dtype: DType, device: int = 0, zeroed: bool = False) -> "Tensor":
         """TensorCreator::empty for the Hip backend (cuda/tensor_internal/normal_creation.rs:34-69)."""
         shape = [int(s) for s in shape]
-        n = int(np.prod(shape, dtype=np.int64)) if shape else 1
-        st = _DeviceStorage(device, n * dtype.size, zeroed)
+        st = _DeviceStorage(device, math.prod(shape) * dtype.size, zeroed)
+        return cls(st, st.ptr, shape, _contiguous_strides(shape), dtype, "hip", device)
+
+    @classmethod
+    def _result(cls, shape, dtype: DType, device: int, stream) -> "Tensor":
+        """empty() for the output of a call that is about to be queued on `stream`."""
+        st = _DeviceStorage(device, math.prod(shape) * dtype.size, ordered=_stream_key(stream) == 0)
         return cls(st, st.ptr, shape, _contiguous_strides(shape), dtype, "hip", device)
 
     @classmethod
@@ -276,7 +310,7 @@ class Tensor:
         return h.astype(np.float64)
 
     def size(self) -> int:
-        return int(np.prod(self.shape, dtype=np.int64)) if self.shape else 1
+        return math.prod(self.shape)
 
     @property
     def ndim(self) -> int:
@@ -438,13 +472,11 @@ class Tensor:
         self._require_hip("reduce")
         l = _ffi.lib()
         axes = _as_axes(axes)
-        od = C.c_int32()
-        check(l.hpt_hip_reduce_out_dtype(op, self.dtype.code, C.byref(od)))
-        out_dtype = DTYPES[od.value]
+        out_dtype = _reduce_out_dtype(op, self.dtype)
         flat_shape = self._reduce_shape(axes, False)
-        final_shape = self._reduce_shape(axes, keep_dims)
+        final_shape = self._reduce_shape(axes, True) if keep_dims else flat_shape
         if out is None:
-            res = Tensor.empty(flat_shape, out_dtype, self.device)
+            res = Tensor._result(flat_shape, out_dtype, self.device, stream)
         else:
             if not out.is_contiguous():
                 raise ShapeError(_ffi.ERR_SHAPE, "out tensor must be contiguous")
@@ -460,6 +492,8 @@ class Tensor:
         check(entry(self.device, stream, op, C.byref(vin), ax, len(axes), int(init_out), C.byref(vout)))
         _touch(stream, self, res)
         del k1, k2
+        if out is None and not keep_dims:
+            return res
         return Tensor(res._storage, res.ptr, final_shape, _contiguous_strides(final_shape), res.dtype, "hip",
                       self.device)
 
@@ -470,13 +504,15 @@ class Tensor:
         if len(axes) != 1:
             raise ParamError(_ffi.ERR_PARAM, "argmax/argmin reduce exactly one axis")
         flat_shape = self._reduce_shape(axes, False)
-        final_shape = self._reduce_shape(axes, keep_dims)
-        res = Tensor.empty(flat_shape, i64, self.device)
+        final_shape = self._reduce_shape(axes, True) if keep_dims else flat_shape
+        res = Tensor._result(flat_shape, i64, self.device, stream)
         vin, k1 = self._c_view()
         vout, k2 = res._c_view()
         check(l.hpt_hip_argreduce(self.device, stream, int(is_max), C.byref(vin), axes[0], C.byref(vout)))
         _touch(stream, self, res)
         del k1, k2
+        if not keep_dims:
+            return res
         return Tensor(res._storage, res.ptr, final_shape, _contiguous_strides(final_shape), i64, "hip", self.device)
 
     # ---- NormalReduce (hpt-traits/src/ops/reduce.rs:45-176) ----------------------
@@ -538,11 +574,11 @@ class Tensor:
         return self._argreduce(False, axis, keep_dims, **kw)
 
     # ---- NormalizationOps (hpt-traits/src/ops/normalization.rs:6-64) ------------
-    def _norm_out(self, out: Optional["Tensor"], dtype: DType) -> "Tensor":
+    def _norm_out(self, out: Optional["Tensor"], dtype: DType, stream) -> "Tensor":
         """The result tensor of a normalisation: fresh, or the caller's `out` (which may be `self`: the
         ABI allows a normalisation in place over one contiguous tensor)."""
         if out is None:
-            return Tensor.empty(self.shape, dtype, self.device)
+            return Tensor._result(self.shape, dtype, self.device, stream)
         out._require_hip("out")
         return out
 
@@ -550,7 +586,7 @@ class Tensor:
         self._require_hip("softmax")
         # NormalizationOps::Output = Tensor<FloatBinaryType<T>>: a non-float input is promoted inside the
         # kernel (one launch, no promoted copy), as the reference promotes inside the op
-        res = self._norm_out(out, self._float_binary_type())
+        res = self._norm_out(out, self._float_binary_type(), stream)
         vin, k1 = self._c_view()
         vout, k2 = res._c_view()
         check(_ffi.lib().hpt_hip_softmax(self.device, stream, int(log), C.byref(vin), int(axis), C.byref(vout)))
@@ -579,7 +615,7 @@ class Tensor:
             # (the fused add + layernorm takes float tensors; the promoted copy is kept alive by `_touch`)
             return self.astype(ft, stream=stream).layernorm(normalized_shape, gamma, beta, eps, stream=stream,
                                                             residual=residual, out=out)
-        res = self._norm_out(out, ft)
+        res = self._norm_out(out, ft, stream)
         vin, k1 = self._c_view()
         vout, k2 = res._c_view()
         keep = [k1, k2]
@@ -613,7 +649,7 @@ class Tensor:
         `scores.mul_(scaling)`, fill -inf where key > query, `softmax(-1)` of
         hpt-examples/examples/transformer/main.rs:233-246 in one pass; the masked part is never read."""
         self._require_hip("softmax_causal")
-        res = Tensor.empty(self.shape, self.dtype, self.device)
+        res = Tensor._result(self.shape, self.dtype, self.device, stream)
         vin, k1 = self._c_view()
         vout, k2 = res._c_view()
         check(_ffi.lib().hpt_hip_softmax_causal(self.device, stream, int(log), C.byref(vin), float(scale),
@@ -631,7 +667,7 @@ class Tensor:
     def astype(self, dtype: DType, stream=None) -> "Tensor":
         """astype (hpt/src/backends/cuda/tensor_impls.rs:129-140) to a float dtype (or to the same dtype)."""
         self._require_hip("astype")
-        res = Tensor.empty(self.shape, dtype, self.device)
+        res = Tensor._result(self.shape, dtype, self.device, stream)
         vin, k1 = self._c_view()
         vout, k2 = res._c_view()
         check(_ffi.lib().hpt_hip_cast(self.device, stream, C.byref(vin), C.byref(vout)))
@@ -641,15 +677,13 @@ class Tensor:
 
     def _float_binary_type(self) -> DType:
         """FloatBinaryType<T> (hpt-types/src/type_promote.rs): the output dtype of the float-valued entries."""
-        out = C.c_int32()
-        check(_ffi.lib().hpt_hip_reduce_out_dtype(MEAN, self.dtype.code, C.byref(out)))
-        return DTYPES[out.value]
+        return _reduce_out_dtype(MEAN, self.dtype)
 
     def contiguous(self, stream=None) -> "Tensor":
         """Contiguous::contiguous (hpt/src/backends/cuda/tensor_internal/normal_out_unary.rs:286-310):
         a new contiguous tensor with this view's elements."""
         self._require_hip("contiguous")
-        res = Tensor.empty(self.shape, self.dtype, self.device)
+        res = Tensor._result(self.shape, self.dtype, self.device, stream)
         vin, k1 = self._c_view()
         vout, k2 = res._c_view()
         check(_ffi.lib().hpt_hip_contiguous(self.device, stream, C.byref(vin), C.byref(vout)))
@@ -711,7 +745,7 @@ class Tensor:
                 raise ShapeError(_ffi.ERR_SHAPE, f"broadcast failed: lhs shape {self.shape}, rhs shape {rhs.shape}")
             shape.append(max(x, y) if min(x, y) != 0 else 0)
         a, b = self.expand(shape), rhs.expand(shape)
-        res = out if out is not None else Tensor.empty(shape, self.dtype, self.device)
+        res = out if out is not None else Tensor._result(shape, self.dtype, self.device, stream)
         va, k1 = a._c_view()
         vb, k2 = b._c_view()
         vo, k3 = res._c_view()

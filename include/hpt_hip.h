@@ -118,6 +118,14 @@ int32_t hpt_hip_alloc(int32_t dev, size_t bytes, size_t align, int32_t zeroed, v
  * The block may be handed out again at once: free it only after the stream that
  * last used it has finished with it. */
 int32_t hpt_hip_free(int32_t dev, void* p, size_t bytes, size_t align);
+/* The same two for callers whose work goes to the DEFAULT stream, without a wait (they have no counterpart in the
+ * reference, whose device tensors are freed after a synchronisation). hpt_hip_free_ordered takes a block that work
+ * already queued on the default stream, and on no other, may still use. hpt_hip_alloc_ordered may return such a
+ * block: the caller queues its own first use of it on the default stream, too, and gives the block back with
+ * hpt_hip_free_ordered, or with hpt_hip_free after waiting for that stream. hpt_hip_alloc never returns a block
+ * that is still in use: where only such blocks are cached it waits for the default stream. */
+int32_t hpt_hip_alloc_ordered(int32_t dev, size_t bytes, size_t align, void** out);
+int32_t hpt_hip_free_ordered(int32_t dev, void* p, size_t bytes, size_t align);
 /* Allocator::forget (hpt-allocator/src/allocators/cuda.rs:140-146; called by Tensor::forget,
  * hpt/src/backends/cuda/tensor_impls.rs:277-306): the allocator stops tracking `p`, which the
  * caller owns from now on (it came from hipMalloc: release it with hipFree). A pointer the
