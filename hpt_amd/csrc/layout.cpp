@@ -11,7 +11,6 @@
 // group (kept or reduced) owns the smallest stride decides which way the lanes
 // of a wavefront run, so that they always walk memory in address order.
 #include <algorithm>
-#include <cstdlib>
 #include <cstring>
 
 #include "common.hpp"
@@ -1016,6 +1015,41 @@ NormPlan plan_normalize(const void* in_data, const void* out_data, const int64_t
         // When it is in the input too, three passes spread over the whole chip: partial statistics
         // (lanes along the inner dim, the axis dealt over wavefronts and workgroups), finalize, apply.
         const int nk = p.kept_in.n;
+        const int64_t slab_bytes = p.cols * sa * (int64_t)elem_size, slabs = nk == 2 ? p.kept_in.size[0] : 0;
+        const bool is_slab = nk == 2 && max_vec > 1 && p.cols >= 2 && sa == p.kept_in.size[1] && p.kept_in.stride[1] == 1 &&
+                             p.kept_out.stride[1] == 1 && p.kept_in.size[1] == p.out_axis_stride &&
+                             p.kept_in.stride[0] == p.cols * sa && p.kept_out.stride[0] == p.cols * sa &&
+                             ((uintptr_t)in_data % elem_size) == 0 && ((uintptr_t)out_data % elem_size) == 0;
+        // One workgroup per slab, the slab in its registers: the fewest threads (a multiple of L / gcd(L, vector) of them
+        // take part) that hold it in four vectors each, up to eight of 1024 threads. (Two vectors and twice the threads:
+        // f32 [5592, 2000, 3] 49.2 -> 70.2 us, [500, 512, 16] 11.0 -> 13.0, nothing gains more than noise.)
+        auto slab_shape = [&]() {
+            const int64_t nv = (p.cols * sa + max_vec - 1) / max_vec;
+            int64_t g = sa, b = max_vec;
+            while (b) { const int64_t t = g % b; g = b; b = t; }
+            const int64_t lp = sa / g;
+            for (int64_t t = 64; t <= 1024; t <<= 1) {
+                const int64_t act = t / lp * lp;
+                if (sa > t || act == 0) continue;
+                int64_t nc = (nv + act - 1) / act;
+                if (nc > 8 || (nc > 4 && t < 1024)) continue;
+                if (nc == 5 || nc == 7) ++nc;  // (kernels exist for 1, 2, 3, 4, 6 and 8)
+                p.kind = NormKind::Col;
+                p.inner = p.out_axis_stride;
+                p.slab_tile = (int)t;
+                p.nchunk = (int)nc;
+                p.vec = max_vec;
+                return true;
+            }
+            return false;
+        };
+        // A very narrow inner dim. The general forms leave lanes idle or walk an axis serially there, and take three
+        // launches below 4 MiB. us before -> slab: f32 [201, 1639, 4] 92 -> 6.5, bf16 [112, 4044, 8] 128 -> 11.0,
+        // f16 [112, 3904, 6] 43 -> 8.8, f32 [2048, 128, 2] 17.3 -> 4.0, bf16 [693, 488, 5] 14.4 -> 6.2, f32 [2511, 963, 8]
+        // 45 -> 34, bf16 [8, 4000, 4] 12.3 -> 7.0. Up to 64 KiB, and to the 128 KiB that fit a workgroup where the alternative
+        // is not the flat walk (f32 [32, 4096, 8] 38.8 -> 10.9).
+        const bool narrow = is_slab && sa <= 8 && p.cols >= 64 && slabs <= (1 << 30) &&
+                            slab_bytes <= (slabs * slab_bytes < (8ll << 20) ? (128 << 10) : (64 << 10));
         // Small groups laid back to back (a contiguous [batch, cols, L] tensor with cols * L elements of at
         // most 2 KiB: softmax over 4 heads of 64, over the 2 of [N, 2, 3]): lanes along L would idle and a
         // lane per (batch, inner) pair reads single elements at a stride. A workgroup stages 16 KiB of whole
@@ -1025,7 +1059,10 @@ NormPlan plan_normalize(const void* in_data, const void* out_data, const int64_t
             p.kept_out.stride[1] == 1 && p.kept_in.size[1] == p.out_axis_stride &&
             p.kept_in.stride[0] == p.cols * sa && p.kept_out.stride[0] == p.cols * sa &&
             p.cols * sa * (int64_t)elem_size <= 2048 && sa * (int64_t)elem_size < 512 && p.kept_in.size[0] >= 1024 &&
-            p.rows * p.cols * (int64_t)elem_size >= (4ll << 20) && (((uintptr_t)in_data | (uintptr_t)out_data) & 15) == 0) {
+            p.rows * p.cols * (int64_t)elem_size >= (4ll << 20) && (((uintptr_t)in_data | (uintptr_t)out_data) & 15) == 0 &&
+            // (a lane walks its column alone: the longer ones are better off with a wavefront per group, as slabs -
+            // us: bf16 [9408, 216, 4] 25.5 -> 12.3, [5986, 125, 3] 15.1 -> 8.3, f32 [13254, 87, 5] 18.0 -> 13.0)
+            !(narrow && (elem_size == 2 ? p.cols > 96 : elem_size == 4 && sa >= 3))) {
             int64_t groups = (16 << 10) / (p.cols * sa * (int64_t)elem_size);
             groups -= groups % max_vec;  // tiles start on 16-byte boundaries
             if (groups >= max_vec) {
@@ -1060,38 +1097,24 @@ NormPlan plan_normalize(const void* in_data, const void* out_data, const int64_t
                 // An inner dim of 3, 5, 6 or 7: the largest multiple of it of a row's lanes take part, so that all of a
                 // lane's vectors start at the same place modulo the inner dim; the lane keeps a (max, sum) per vector
                 // place and the places are rotated into softmaxes, folded, and rotated back.
+                // (Large inputs with an inner dim of 5, 6 or 7 are faster as slabs, us: f32 [4000, 512, 7] 29.3 -> 23.2,
+                // f16 [11264, 488, 6] 39.7 -> 31.2, [11008, 576, 5] 44.5 -> 30.2; with 3 there is no difference: f32
+                // [5592, 2000, 3] 48.9 and 49.2. Smaller ones stay, their plan is pinned.)
                 const int64_t act = q.tpr / sa * sa, nvr = p.cols * sa / max_vec;
                 const int64_t nc = (nvr + act - 1) / act;
-                if (nc <= 8) {
+                const bool as_slab = narrow && sa >= 5 && slabs * slab_bytes >= (40ll << 20);
+                if (nc <= 8 && !as_slab) {
                     q.interleave = -(int)sa;
                     q.nchunk = (int)nc;
                     return q;
                 }
             }
         }
-        // Mid-sized slabs with a very narrow inner dim ([B, 1000, 3], [B, 2048, 5]): one workgroup per slab through LDS.
-        // (From 16 bytes of inner dim on the register kernel, which serves axes up to 1024, is as fast or faster:
-        // f32 [2048, 1024, 8] 4.0 against 2.6 TB/s; beyond 1024 the alternative is the three-pass flat walk.
-        // Four-byte inner dims of 5 ... 11 elements that are not whole vectors are the exception - the register kernel
-        // loads them one or two elements at a time: f32, % of the HBM peak, registers -> slab: [4000, 512, 5] 29.5 -> 45.7,
-        // [4000, 512, 7] 31.6 -> 46.8, [4000, 300, 10] 37.1 -> 45.3, [4000, 300, 11] 34.0 -> 43.9, [8000, 100, 6] 23.3 -> 33.1.
-        // Two-byte inner dims of 7 ... 20 elements go either way by a few points and stay; f64 gains nothing.)
-        if (nk == 2 && max_vec > 1 && p.cols > 64 && sa == p.kept_in.size[1] && p.kept_in.stride[1] == 1 &&
-            p.kept_out.stride[1] == 1 && p.kept_in.size[1] == p.out_axis_stride &&
-            p.kept_in.stride[0] == p.cols * sa && p.kept_out.stride[0] == p.cols * sa &&
-            p.cols * sa * (int64_t)elem_size <= (64 << 10) && sa * (int64_t)elem_size <= ((p.cols > 1024 || (elem_size == 4 && sa % max_vec != 0)) ? (elem_size == 4 && sa % max_vec != 0 ? 48 : 32) : 12) &&
-            p.kept_in.size[0] >= 256 &&
-            p.rows * p.cols * (int64_t)elem_size >= (4ll << 20) && ((uintptr_t)in_data % elem_size) == 0 &&
-            ((uintptr_t)out_data % elem_size) == 0) {
-            p.kind = NormKind::Col;
-            p.inner = p.out_axis_stride;
-            // lanes per column: as many as 256 threads leave for each of the L columns, a wavefront at most
-            int64_t tpc = 64;
-            while (tpc > 1 && tpc * sa > 256) tpc >>= 1;
-            p.slab_tile = (int)tpc;
-            p.vec = max_vec;
-            return p;
-        }
+        // Wider ones, at least 256 of them. (Two-byte inner dims of 9 ... 20 elements, and four-byte ones of whole vectors,
+        // go either way by a few points and keep the register columns.)
+        const bool mid_slab = is_slab && p.cols > 64 && slab_bytes <= (64 << 10) && slabs >= 256 && slabs * slab_bytes >= (4ll << 20) &&
+                              sa * (int64_t)elem_size <= ((p.cols > 1024 || (elem_size == 4 && sa % max_vec != 0)) ? (elem_size == 4 && sa % max_vec != 0 ? 48 : 32) : 12);
+        if ((narrow || mid_slab) && slab_shape()) return p;
         if (nk >= 1 && nk <= 2 && p.kept_in.stride[nk - 1] == 1 && p.kept_out.stride[nk - 1] == 1 &&
             p.kept_in.size[nk - 1] == p.out_axis_stride && p.kept_in.size[nk - 1] <= (1 << 30) && p.cols <= (1 << 30) &&
             (nk == 1 || p.kept_in.size[0] <= 65535)) {

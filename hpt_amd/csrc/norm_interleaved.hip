@@ -2,6 +2,7 @@
 // narrow L) for one softmax kind and the four float dtypes. Compiled with -DHPT_NORM_KIND=<0 or 1>.
 #include "norm_interleaved.hpp"
 #include "norm_kernels.hpp"
+#include "norm_slab.hpp"
 
 #ifndef HPT_NORM_KIND
 #error "compile with -DHPT_NORM_KIND=<kind>"
@@ -76,6 +77,38 @@ template <class T> static void launch_interleaved_t(const NormPlan& p, const Nor
         default: fail(HPT_ERR_KERNEL, "interleaved rows: %d softmaxes per row", p.interleave);
     }
 }
+
+template <class T> static void launch_slabs_t(const NormPlan& p, const NormArgs& a, hipStream_t st) {
+    constexpr int VEC = 16 / sizeof(T);
+    const int L = (int)p.kept_in.size[1], C = (int)p.cols, threads = p.slab_tile;
+    int g = L, b = VEC;
+    while (b) { const int r = g % b; g = b; b = r; }
+    const int lp = L / g, act = threads / lp * lp;  // a multiple of lp: act * VEC is one of L
+    const int64_t nvec = ((int64_t)C * L + VEC - 1) / VEC;
+    if (threads < 64 || threads > 1024 || act < 1 || L > threads || (int64_t)C * L < VEC || nvec > (int64_t)act * p.nchunk)
+        fail(HPT_ERR_KERNEL, "slab plan: %d x %d elements do not fit %d threads of %d vectors", C, L, threads, p.nchunk);
+    int g_log2 = 0;
+    while (g_log2 < 6 && (L << (g_log2 + 1)) <= threads) ++g_log2;
+    using ST = typename StatType<T>::type;
+    const size_t smem = (size_t)act * VEC * sizeof(ST) + 2 * (size_t)L * sizeof(typename Elem<T>::Wide);
+    const dim3 grid((unsigned)p.kept_in.size[0]), block((unsigned)threads);
+    const T* in = (const T*)a.in;
+    T* out = (T*)a.out;
+    switch (p.nchunk) {
+        case 1: norm_slab_kernel<KIND, T, 1><<<grid, block, smem, st>>>(in, out, C, L, act, g_log2); return;
+        case 2: norm_slab_kernel<KIND, T, 2><<<grid, block, smem, st>>>(in, out, C, L, act, g_log2); return;
+        case 3: norm_slab_kernel<KIND, T, 3><<<grid, block, smem, st>>>(in, out, C, L, act, g_log2); return;
+        case 4: norm_slab_kernel<KIND, T, 4><<<grid, block, smem, st>>>(in, out, C, L, act, g_log2); return;
+        case 6: norm_slab_kernel<KIND, T, 6><<<grid, block, smem, st>>>(in, out, C, L, act, g_log2); return;
+        case 8: norm_slab_kernel<KIND, T, 8><<<grid, block, smem, st>>>(in, out, C, L, act, g_log2); return;
+        default: fail(HPT_ERR_KERNEL, "slab plan: no kernel for %d vectors per thread", p.nchunk);
+    }
+}
+
+template <> void launch_slabs<HPT_NORM_KIND, f16_t>(const NormPlan& p, const NormArgs& a, hipStream_t st) { launch_slabs_t<f16_t>(p, a, st); }
+template <> void launch_slabs<HPT_NORM_KIND, bf16_t>(const NormPlan& p, const NormArgs& a, hipStream_t st) { launch_slabs_t<bf16_t>(p, a, st); }
+template <> void launch_slabs<HPT_NORM_KIND, float>(const NormPlan& p, const NormArgs& a, hipStream_t st) { launch_slabs_t<float>(p, a, st); }
+template <> void launch_slabs<HPT_NORM_KIND, double>(const NormPlan& p, const NormArgs& a, hipStream_t st) { launch_slabs_t<double>(p, a, st); }
 
 template <> void launch_interleaved_rows<HPT_NORM_KIND, f16_t>(const NormPlan& p, const NormArgs& a, dim3 grid, dim3 block, hipStream_t st) {
     launch_interleaved_t<f16_t>(p, a, grid, block, st);

@@ -13,4 +13,7 @@ struct NormArgs;
 template <int KIND, class T>
 void launch_interleaved_rows(const NormPlan& p, const NormArgs& a, dim3 grid, dim3 block, hipStream_t st);
 
+// Launch the plan `p` (kind Col, slab_tile > 0): one workgroup per contiguous [cols, L] slab.
+template <int KIND, class T> void launch_slabs(const NormPlan& p, const NormArgs& a, hipStream_t st);
+
 }  // namespace hpt
