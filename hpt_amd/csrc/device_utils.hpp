@@ -193,6 +193,26 @@ __device__ __forceinline__ void store_pack_unaligned(T* p, const Pack<T, N>& v) 
     __builtin_memcpy(p, &v, sizeof(T) * N);
 }
 
+// The same, non-temporal (the vector type says how little alignment the compiler may count on). For results that
+// are written once, in runs of whole lines: the softmax kernels whose rows lie off the vector grid were
+// held up by their ordinary stores. us, ordinary -> non-temporal: over axis 0 f32 [8190, 4097] 97 -> 82, f16 53 -> 48, bf16
+// [2700, 12001] 48.5 -> 43.8; over axis 1 f16 [20, 2500, 1001] 71 -> 64, f32 [64, 128, 3249] 61.5 -> 54.9, bf16 [400, 64, 1235]
+// 42 -> 33, f32 [2240, 1408, 8] 47 -> 42, f16 [11264, 488, 6] 37 -> 28; no difference below 8 MiB or in the flat walks of
+// narrow inner dims, which keep the ordinary form.
+template <class T, int N>
+__device__ __forceinline__ void store_pack_unaligned_stream(T* p, const Pack<T, N>& v) {
+    static_assert(sizeof(T) >= 2, "elements of two bytes or more");
+#if HPT_STREAMING_ACCESS
+    if constexpr (sizeof(T) * N == 16) {
+        typedef u32x4 u32x4_loose __attribute__((aligned(2)));
+        union { u32x4 u; Pack<T, N> v; } c;
+        c.v = v;
+        __builtin_nontemporal_store(c.u, reinterpret_cast<u32x4_loose*>(p));
+    } else
+#endif
+        store_pack_unaligned<T, N>(p, v);
+}
+
 // ---- exponential ---------------------------------------------------------------
 // e^x for f32 data. The error of the hardware route exp2(x * log2 e) grows with |x| (the product
 // is rounded before the exponential sees it: |x| * 6e-8 relative). Here x = n ln 2 + r is split

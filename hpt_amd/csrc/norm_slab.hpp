@@ -126,7 +126,7 @@ __global__ void __launch_bounds__(1024) norm_slab_kernel(const T* in, T* outp, i
         }
         const int iv = t + c * act;
         if (iv < nvec) {
-            store_pack_unaligned<T, VEC>(dst + (int64_t)iv * VEC, o);
+            store_pack_unaligned_stream<T, VEC>(dst + (int64_t)iv * VEC, o);
         } else {
 #pragma unroll
             for (int j = 0; j < VEC; ++j)

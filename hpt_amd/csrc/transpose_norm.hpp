@@ -353,7 +353,7 @@ __global__ void __launch_bounds__(256) col_apply_kernel(const TransposedArgs a, 
             const CT d = Elem<T>::widen(v.v[k]) - p0.v[k];
             o.v[k] = Elem<T>::narrow(kLog ? d - p1.v[k] : exp_ct<T>(d) * p1.v[k]);
         }
-        if constexpr (UA) store_pack_unaligned<T, VEC>(out + (int64_t)c * a.R, o);
+        if constexpr (UA) store_pack_unaligned_stream<T, VEC>(out + (int64_t)c * a.R, o);
         else if constexpr (VEC > 1) store_pack_stream<T, VEC>(out + (int64_t)c * a.R, o);
         else out[(int64_t)c * a.R] = o.v[0];
     };
@@ -549,7 +549,7 @@ __global__ void __launch_bounds__(256) col_reg_kernel(const ColRegArgs a) {
             T* dst = out + (int64_t)(ty_st + (i << a.ty_log2)) * a.L;
             if constexpr (UA) {
                 if (skip == 0) {
-                    store_pack_unaligned<T, EV>(dst, o);
+                    store_pack_unaligned_stream<T, EV>(dst, o);
                 } else {
 #pragma unroll
                     for (int k = 0; k < EV; ++k)
