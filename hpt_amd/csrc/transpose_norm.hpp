@@ -332,6 +332,9 @@ __global__ void __launch_bounds__(256) transposed_apply_kernel(const TransposedA
 // "columns" the axis); the last pass keeps the layout: lanes along the inner dim, each thread
 // holds the VEC per-row numbers in registers and walks a slice of the axis with batches of
 // loads in flight. out is contiguous: [batch][cols][R].
+// UA: the last vector of an inner row is taken from the row's end backwards and stores only the elements that the vector
+// before it does not cover. Each element has one writer: `out` may be `in`, and the vector before may belong to another
+// workgroup, which then reads what this one must not have touched.
 template <int KIND, class T, int VEC, bool UA = false>
 __global__ void __launch_bounds__(256) col_apply_kernel(const TransposedArgs a, int chunk) {
     using CT = typename Elem<T>::Wide;
@@ -339,7 +342,8 @@ __global__ void __launch_bounds__(256) col_apply_kernel(const TransposedArgs a, 
     const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
     int r0 = (blockIdx.x * 64 + tx) * VEC;
     if (r0 >= a.R) return;
-    if constexpr (UA) r0 = min(r0, a.R - VEC);  // the row's last vector, from its end backwards
+    const int skip = UA ? max(r0 - (a.R - VEC), 0) : 0;  // leading elements that belong to the vector before
+    r0 -= skip;
     const CT* pp = (const CT*)a.params + (int64_t)blockIdx.z * 3 * a.R + r0;
     const Pack<CT, VEC> p0 = UA ? load_pack_unaligned<CT, VEC>(pp) : *reinterpret_cast<const Pack<CT, VEC>*>(pp);
     const Pack<CT, VEC> p1 = UA ? load_pack_unaligned<CT, VEC>(pp + a.R) : *reinterpret_cast<const Pack<CT, VEC>*>(pp + a.R);
@@ -353,8 +357,15 @@ __global__ void __launch_bounds__(256) col_apply_kernel(const TransposedArgs a, 
             const CT d = Elem<T>::widen(v.v[k]) - p0.v[k];
             o.v[k] = Elem<T>::narrow(kLog ? d - p1.v[k] : exp_ct<T>(d) * p1.v[k]);
         }
-        if constexpr (UA) store_pack_unaligned_stream<T, VEC>(out + (int64_t)c * a.R, o);
-        else if constexpr (VEC > 1) store_pack_stream<T, VEC>(out + (int64_t)c * a.R, o);
+        if constexpr (UA) {
+            if (skip == 0) {
+                store_pack_unaligned_stream<T, VEC>(out + (int64_t)c * a.R, o);
+            } else {
+#pragma unroll
+                for (int k = 0; k < VEC; ++k)
+                    if (k >= skip) out[(int64_t)c * a.R + k] = o.v[k];
+            }
+        } else if constexpr (VEC > 1) store_pack_stream<T, VEC>(out + (int64_t)c * a.R, o);
         else out[(int64_t)c * a.R] = o.v[0];
     };
     auto fetch = [&](int c) {
