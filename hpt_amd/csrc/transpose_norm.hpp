@@ -89,7 +89,7 @@ __global__ void __launch_bounds__(1024) transposed_stats_kernel(const Transposed
     CT m[VEC], s[VEC], s2[VEC];
     ST se[VEC];  // softmax: the sum of exponentials
     if constexpr (KIND == NORM_LAYERNORM) {
-        Pack<T, VEC> f = load_pack<T, VEC>(base);
+        Pack<T, VEC> f = UA ? load_pack_unaligned<T, VEC>(base) : load_pack<T, VEC>(base);
 #pragma unroll
         for (int k = 0; k < VEC; ++k) m[k] = Elem<T>::widen(f.v[k]);
     } else {
