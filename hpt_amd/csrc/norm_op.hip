@@ -207,7 +207,7 @@ template <class T> void launch_transposed(const NormPlan& p, const NormArgs& a, 
         t.bi = nk > 1 ? p.kept_in.stride[0] : 0;
         t.eps = a.eps;
         t.inv_cols = a.inv_cols;
-        t.cols_per_split = (t.cols + t.S - 1) / t.S;
+        t.nw = p.tpr;
         const int tiles = (t.cols + TILE - 1) / TILE;
         const unsigned rt = (unsigned)((t.R + TILE - 1) / TILE);
         const unsigned rg = (unsigned)((t.R + 64 * FULL - 1) / (64 * FULL));

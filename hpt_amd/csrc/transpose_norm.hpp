@@ -5,8 +5,8 @@
 //
 //   transposed_stats_kernel     walks the input in address order (lanes along the
 //       rows, 1 KiB per wavefront and column) and keeps VEC running row
-//       statistics per lane (online max + rescaled sum, or shifted sums ->
-//       (n, mean, M2)); S workgroups share the axis so that the chip is full.
+//       statistics per lane (online max + rescaled sum, or mean and sum of squared
+//       deviations); S workgroups share the axis so that the chip is full.
 //   transposed_finalize_kernel  folds the S partials of each row into the three
 //       numbers the last pass needs.
 //   transposed_apply_kernel     reads the input a second time (it is still in the
@@ -38,23 +38,40 @@ struct TransposedArgs {
     int R;            // rows per batch (contiguous in the input)
     int cols;         // length of the normalised axis
     int S;            // workgroups sharing the axis in the statistics pass
-    int cols_per_split;
+    int nw;           // wavefronts per workgroup of the statistics pass
 };
+
+// Columns that wavefront `pid` of the P that share a row's columns takes (it starts at column pid and steps by P), and
+// columns that the nw wavefronts of workgroup y take together.
+__device__ __forceinline__ int columns_of_wave(int cols, int P, int pid) { return cols / P + (pid < cols % P ? 1 : 0); }
+__device__ __forceinline__ int columns_of_group(int cols, int P, int nw, int y) {
+    return cols / P * nw + min(max(cols % P - y * nw, 0), nw);
+}
 
 // A partial row statistic over some of the columns.
 //   softmax  : (max, sum of exp(x - max)), the sum in StatType; merged with SoftStatOp.
-//   layernorm: (sum of (x - k), sum of (x - k)^2) with k the row's FIRST element,
-//              the same shift for every partial of the row, so that partials
-//              merge by plain addition and only the last step divides.
-template <class CT> struct ShiftedSums {
-    CT s1, s2;
+//   layernorm: (mean, sum of squared deviations from it), in f64 for every type; how many columns
+//              they are of follows from where they lie. Merged with MomentStatOp.
+// (Sums of (x - k) and (x - k)^2 around the row's first element k, which merge by plain addition, lose what a far k has
+// in common with every term: 2^-24 of n (k - mean)^2, against a sum that is no larger than that divided by n. f32
+// [5001, 131] transposed with first elements at 100: 65 % of the results off by more than 1e-5, f16 by a unit of the last place.)
+struct RowMoments {
+    double mean, m2;
 };
+// sum + lo += x, the rounding of the sum kept in lo
+__device__ __forceinline__ void carry_add(double& sum, double& lo, double x) {
+    const double t = sum + x, b = t - sum;
+    lo += (sum - (t - b)) + (x - b);
+    sum = t;
+}
 template <int KIND, class T> struct RowPartial {
     using CT = typename Elem<T>::Wide;
     using ST = typename StatType<T>::type;  // the sum of exponentials of f32 rows is carried in f64
-    using type = typename std::conditional<KIND == NORM_LAYERNORM, ShiftedSums<CT>, SoftStat<CT, ST>>::type;
+    using type = typename std::conditional<KIND == NORM_LAYERNORM, RowMoments, SoftStat<CT, ST>>::type;
 };
 
+// (What the moments cost against the sums around the row's first element, stored [columns, rows], us: f32 [5001, 1001] 18.9 ->
+// 20.0, [5000, 8000] 110.8 -> 112.2, f16 [5001, 8001] 54.1 -> 56.5, [8192, 16384] 128.4 -> 137.3, f64 [5001, 4001] 98.8 -> 101.0.)
 // Pass 1: partial row statistics. Lanes run along the rows (a wavefront reads 1 KiB
 // of consecutive rows per column), so every lane owns its VEC rows outright: no
 // cross-lane merge. Every wavefront takes its own columns; the wavefronts of a
@@ -85,34 +102,70 @@ __global__ void __launch_bounds__(1024) transposed_stats_kernel(const Transposed
     const int pid = blockIdx.y * NW + w;
     const T* base = (const T*)a.in + (int64_t)blockIdx.z * a.bi + r0;
 
-    // per row: softmax (m, s); layernorm s = sum (x - k), s2 = sum (x - k)^2, k = x[row][0]
-    CT m[VEC], s[VEC], s2[VEC];
-    ST se[VEC];  // softmax: the sum of exponentials
-    if constexpr (KIND == NORM_LAYERNORM) {
-        Pack<T, VEC> f = UA ? load_pack_unaligned<T, VEC>(base) : load_pack<T, VEC>(base);
-#pragma unroll
-        for (int k = 0; k < VEC; ++k) m[k] = Elem<T>::widen(f.v[k]);
-    } else {
-#pragma unroll
-        for (int k = 0; k < VEC; ++k) m[k] = neg_inf<CT>();
-    }
+    // per row: softmax (max m, sum of exponentials se); layernorm, of the n columns folded so far:
+    //   f32  f64 sums of (x - org) and (x - org)^2, org the first element that the lane sees
+    //   f16, bf16  the mean in f64 and the squared deviations from it in f32, a merge per batch of columns (f64 sums:
+    //        f16 [8192, 16384] transposed 190 us, this 137)
+    //   f64  the same with the roundings of both carried along: the type leaves no bits to spare, and a lane may
+    //        fold a thousand batches one after the other
+    constexpr bool kSums = std::is_same<T, float>::value;
+    CT m[VEC], s2[VEC];
+    ST se[VEC];
+    double org[VEC], mean[VEC], m2[VEC], mean_lo[VEC], m2_lo[VEC];
+    int n = 0;
 #pragma unroll
     for (int k = 0; k < VEC; ++k) {
-        s[k] = 0;
+        m[k] = neg_inf<CT>();
+        org[k] = mean[k] = m2[k] = mean_lo[k] = m2_lo[k] = 0;
         s2[k] = 0;
         se[k] = 0;
+    }
+    if constexpr (KIND == NORM_LAYERNORM && kSums) {
+        const T* p0 = base + (int64_t)min(pid, a.cols - 1) * a.sa;
+        const Pack<T, VEC> f = UA ? load_pack_unaligned<T, VEC>(p0) : load_pack<T, VEC>(p0);
+#pragma unroll
+        for (int k = 0; k < VEC; ++k) org[k] = (double)Elem<T>::widen(f.v[k]);
     }
     auto fold = [&](const Pack<T, VEC>* v, auto cnt_tag) {
         constexpr int CNT = decltype(cnt_tag)::value;
         if constexpr (KIND == NORM_LAYERNORM) {
+            if constexpr (kSums) {
 #pragma unroll
-            for (int i = 0; i < CNT; ++i)
+                for (int i = 0; i < CNT; ++i)
+#pragma unroll
+                    for (int k = 0; k < VEC; ++k) {
+                        const double d = (double)Elem<T>::widen(v[i].v[k]) - org[k];
+                        mean[k] += d;
+                        m2[k] = fma(d, d, m2[k]);
+                    }
+            } else {
+                // the batch's own mean and deviations, then a merge per batch and row (the weights are the same in every lane)
+                const CT share = (CT)CNT / (CT)(n + CNT), cross = share * (CT)n;
 #pragma unroll
                 for (int k = 0; k < VEC; ++k) {
-                    const CT d = Elem<T>::widen(v[i].v[k]) - m[k];
-                    s[k] += d;
-                    s2[k] += d * d;
+                    const CT x0 = Elem<T>::widen(v[0].v[k]);
+                    CT sum = 0, sq = 0;
+#pragma unroll
+                    for (int i = 1; i < CNT; ++i) sum += Elem<T>::widen(v[i].v[k]) - x0;
+                    const CT mb = x0 + sum * (CT)(1.0 / CNT);
+#pragma unroll
+                    for (int i = 0; i < CNT; ++i) {
+                        const CT d = Elem<T>::widen(v[i].v[k]) - mb;
+                        sq += d * d;
+                    }
+                    if constexpr (sizeof(CT) == 8) {
+                        const double delta = (mb - mean[k]) - mean_lo[k];
+                        carry_add(mean[k], mean_lo[k], delta * share);
+                        carry_add(m2[k], m2_lo[k], sq + delta * delta * cross);
+                    } else {
+                        const double delta = (double)mb - mean[k];
+                        mean[k] = fma(delta, (double)share, mean[k]);
+                        const CT df = (CT)delta;
+                        s2[k] += sq + df * df * cross;
+                    }
                 }
+            }
+            n += CNT;
         } else {
 #pragma unroll
             for (int k = 0; k < VEC; ++k) {
@@ -156,8 +209,14 @@ __global__ void __launch_bounds__(1024) transposed_stats_kernel(const Transposed
     for (int k = 0; k < VEC; ++k) {
         Part t;
         if constexpr (KIND == NORM_LAYERNORM) {
-            t.s1 = s[k];
-            t.s2 = s2[k];
+            if constexpr (kSums) {
+                const double d = n > 0 ? mean[k] / n : 0, q = m2[k] - mean[k] * d;
+                t.mean = org[k] + d;
+                t.m2 = q < 0 ? 0 : q;  // (a NaN stays one)
+            } else {
+                t.mean = mean[k] + mean_lo[k];
+                t.m2 = sizeof(CT) == 8 ? m2[k] + m2_lo[k] : (double)s2[k];
+            }
         } else {
             t.m = m[k];
             t.s = se[k];
@@ -169,14 +228,23 @@ __global__ void __launch_bounds__(1024) transposed_stats_kernel(const Transposed
     Part* dst = (Part*)a.stats + ((int64_t)blockIdx.z * a.S + blockIdx.y) * a.R + r0;
     for (int k = w; k < VEC; k += NW) {
         Part t = sm[k * 64 + lane];
-        for (int o = 1; o < NW; ++o) {
-            const Part u = sm[(o * VEC + k) * 64 + lane];
-            if constexpr (KIND == NORM_LAYERNORM) {
-                t.s1 += u.s1;
-                t.s2 += u.s2;
-            } else {
-                t = SoftStatOp<T, CT, ST>::comb(t, u);
+        if constexpr (KIND == NORM_LAYERNORM) {
+            // the mean first, as differences from the first wavefront's (f64 elements: and once more from the result, which
+            // takes out what a first one far from the others has cost), then the deviations from it
+            auto cnt = [&](int o) { return (double)columns_of_wave(a.cols, P, blockIdx.y * NW + o); };
+#pragma unroll
+            for (int pass = 0; pass < (sizeof(CT) == 8 ? 2 : 1); ++pass) {
+                double shift = 0;
+                for (int o = 0; o < NW; ++o) shift += cnt(o) * (sm[(o * VEC + k) * 64 + lane].mean - t.mean);
+                t.mean += shift / (double)columns_of_group(a.cols, P, NW, blockIdx.y);
             }
+            t.m2 = 0;
+            for (int o = 0; o < NW; ++o) {
+                const Part u = sm[(o * VEC + k) * 64 + lane];
+                t.m2 += u.m2 + cnt(o) * (u.mean - t.mean) * (u.mean - t.mean);
+            }
+        } else {
+            for (int o = 1; o < NW; ++o) t = SoftStatOp<T, CT, ST>::comb(t, sm[(o * VEC + k) * 64 + lane]);
         }
         dst[k] = t;
     }
@@ -192,65 +260,62 @@ __global__ void __launch_bounds__(256) transposed_finalize_kernel(const Transpos
     using ST = typename StatType<T>::type;
     using Part = typename RowPartial<KIND, T>::type;
     constexpr int LY = 16;
-    __shared__ ST sm0[LY][16], sm1[LY][16];
     const int r = blockIdx.x * 16 + threadIdx.x;
     const bool ok = r < a.R;
     const int P = a.S;
-    ST acc0, acc1;  // layernorm: sums of s1, s2; softmax: running max, rescaled sum
-    if constexpr (KIND == NORM_LAYERNORM) { acc0 = 0; acc1 = 0; }
-    else { acc0 = (ST)neg_inf<CT>(); acc1 = 0; }
-    if (ok) {
-        const Part* sp = (const Part*)a.stats + (int64_t)blockIdx.z * P * a.R + r;
-        auto take = [&](const Part& t) {
-            if constexpr (KIND == NORM_LAYERNORM) {
-                acc0 += (ST)t.s1;
-                acc1 += (ST)t.s2;
-            } else {
-                SoftStat<CT, ST> x{(CT)acc0, acc1};
-                x = SoftStatOp<T, CT, ST>::comb(x, t);
-                acc0 = x.m;
-                acc1 = x.s;
-            }
-        };
+    const Part* sp = (const Part*)a.stats + (int64_t)blockIdx.z * P * a.R + (ok ? r : 0);
+    // four partials in flight (the kernel is a chain of load latencies)
+    auto each = [&](auto take) {
         int p = threadIdx.y;
-        for (; p + 3 * LY < P; p += 4 * LY) {  // four partials in flight (the kernel is a chain of load latencies)
+        for (; p + 3 * LY < P; p += 4 * LY) {
             Part t[4];
 #pragma unroll
             for (int u = 0; u < 4; ++u) t[u] = sp[(int64_t)(p + u * LY) * a.R];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) take(t[u]);
+            for (int u = 0; u < 4; ++u) take(t[u], p + u * LY);
         }
-        for (; p < P; p += LY) take(sp[(int64_t)p * a.R]);
-    }
-    sm0[threadIdx.y][threadIdx.x] = acc0;
-    sm1[threadIdx.y][threadIdx.x] = acc1;
-    __syncthreads();
-    if (threadIdx.y > 0 || !ok) return;
-    for (int y = 1; y < LY; ++y) {
-        if constexpr (KIND == NORM_LAYERNORM) {
-            acc0 += sm0[y][threadIdx.x];
-            acc1 += sm1[y][threadIdx.x];
-        } else {
-            SoftStat<CT, ST> x{(CT)acc0, acc1}, t{(CT)sm0[y][threadIdx.x], sm1[y][threadIdx.x]};
-            x = SoftStatOp<T, CT, ST>::comb(x, t);
-            acc0 = x.m;
-            acc1 = x.s;
-        }
-    }
-    CT* p = (CT*)a.params + (int64_t)blockIdx.z * 3 * a.R + r;
+        for (; p < P; p += LY) take(sp[(int64_t)p * a.R], p);
+    };
+    CT* params = (CT*)a.params + (int64_t)blockIdx.z * 3 * a.R + r;
     if constexpr (KIND == NORM_LAYERNORM) {
-        const ST k = (ST)Elem<T>::widen(((const T*)a.in)[(int64_t)blockIdx.z * a.bi + r]);
-        const ST mean = k + acc0 * (ST)a.inv_cols;
-        ST m2 = acc1 - acc0 * acc0 * (ST)a.inv_cols;
-        if (m2 < (ST)0) m2 = 0;
+        // the mean first, as differences from the first partial's (f64 elements: twice, as above), then the squared
+        // deviations from it
+        __shared__ double sm[LY][16];
+        auto total = [&](double x) {
+            __syncthreads();
+            sm[threadIdx.y][threadIdx.x] = x;
+            __syncthreads();
+            double s = sm[0][threadIdx.x];
+            for (int y = 1; y < LY; ++y) s += sm[y][threadIdx.x];
+            return s;
+        };
+        auto cnt = [&](int y) { return (double)columns_of_group(a.cols, P * a.nw, a.nw, y); };
+        double mean = sp[0].mean, m2 = 0;
+#pragma unroll
+        for (int pass = 0; pass < (sizeof(CT) == 8 ? 2 : 1); ++pass) {
+            double shift = 0;
+            each([&](const Part& t, int y) { shift += cnt(y) * (t.mean - mean); });
+            mean += total(shift) / (double)a.cols;
+        }
+        each([&](const Part& t, int y) { m2 += t.m2 + cnt(y) * (t.mean - mean) * (t.mean - mean); });
+        m2 = total(m2);
+        if (threadIdx.y > 0 || !ok) return;
         const CT hi = (CT)mean;
-        p[0] = hi;
-        p[a.R] = (CT)(mean - (ST)hi);
-        p[2 * (int64_t)a.R] = rsqrt_ct((CT)(m2 * (ST)a.inv_cols) + (CT)a.eps);
+        params[0] = hi;
+        params[a.R] = (CT)(mean - (double)hi);
+        params[2 * (int64_t)a.R] = rsqrt_ct((CT)(m2 * a.inv_cols) + (CT)a.eps);
     } else {
-        p[0] = (CT)acc0;
-        p[a.R] = KIND == NORM_SOFTMAX ? (CT)1 / (CT)acc1 : log_ct<T>((CT)acc1);
-        p[2 * (int64_t)a.R] = 0;
+        using Op = SoftStatOp<T, CT, ST>;
+        __shared__ Part sm[LY][16];
+        Part acc{neg_inf<CT>(), (ST)0};
+        if (ok) each([&](const Part& t, int) { acc = Op::comb(acc, t); });
+        sm[threadIdx.y][threadIdx.x] = acc;
+        __syncthreads();
+        if (threadIdx.y > 0 || !ok) return;
+        for (int y = 1; y < LY; ++y) acc = Op::comb(acc, sm[y][threadIdx.x]);
+        params[0] = acc.m;
+        params[a.R] = KIND == NORM_SOFTMAX ? (CT)1 / (CT)acc.s : log_ct<T>((CT)acc.s);
+        params[2 * (int64_t)a.R] = 0;
     }
 }
 
