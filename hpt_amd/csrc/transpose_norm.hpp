@@ -856,14 +856,19 @@ struct alignas(16) HalfPairs {
     half2_t p[4];
 };
 
-// exp(x - m) of a tile element. f16: exp2(x * log2(e) - m * log2(e)) with the
+// exp(x - m) of a tile element. f16 softmax: exp2(x * log2(e) - m * log2(e)) with the
 // scaling folded into the one multiply-add that also widens x (`nml` = -m * log2(e));
-// a row of -inf only still yields NaN (-inf + inf). Other types: as everywhere else.
-template <class T>
-__device__ __forceinline__ typename Elem<T>::Wide tile_exp(T x, typename Elem<T>::Wide m, typename Elem<T>::Wide nml) {
+// a row of -inf only still yields NaN (-inf + inf). The rounding of nml is common to the
+// row: a softmax divides it out. A log_softmax keeps it (rows at 16000: 7e-4, where a
+// result near zero has units of 1e-5), so it subtracts first (`one`: see widen_fma). Other types: as everywhere else.
+template <int KIND, class T>
+__device__ __forceinline__ typename Elem<T>::Wide tile_exp(T x, typename Elem<T>::Wide m, typename Elem<T>::Wide nml,
+                                                                  typename Elem<T>::Wide one) {
     using CT = typename Elem<T>::Wide;
-    if constexpr (std::is_same<T, f16_t>::value) {
+    if constexpr (std::is_same<T, f16_t>::value && KIND == NORM_SOFTMAX) {
         return __builtin_amdgcn_exp2f(widen_fma(x, (CT)1.4426950408889634, nml));
+    } else if constexpr (std::is_same<T, f16_t>::value) {
+        return exp_ct<T>(widen_fma(x, one, -m));
     } else {
         return exp_ct<T>(Elem<T>::widen(x) - m);
     }
@@ -1036,7 +1041,7 @@ __global__ void __launch_bounds__(1024) transposed_tile_kernel(const TileArgs a)
             for (int i = 0; i < VEC; ++i)
 #pragma unroll
                 for (int k = 0; k < VEC; ++k) {
-                    const CT e = tile_exp<T>(v[h * VEC + i].v[k], m[k], nml[k]);
+                    const CT e = tile_exp<KIND, T>(v[h * VEC + i].v[k], m[k], nml[k], one);
                     sh[k] += (AT)(UA && i < twice[h] ? (CT)0 : e);
                     if constexpr (kKeepExp && KIND == NORM_SOFTMAX) v[h * VEC + i].v[k] = Elem<T>::narrow(e);
                 }
@@ -1188,7 +1193,7 @@ __global__ void __launch_bounds__(1024) transposed_tile_kernel(const TileArgs a)
                     y = y * p2[k] * g[i] + bt[i];
                 } else if constexpr (KIND == NORM_SOFTMAX) {
                     if constexpr (kKeepExp) y = Elem<T>::widen(v[h * VEC + i].v[k]) * p1[k];
-                    else y = tile_exp<T>(v[h * VEC + i].v[k], p0[k], p2[k]) * p1[k];
+                    else y = tile_exp<KIND, T>(v[h * VEC + i].v[k], p0[k], p2[k], one) * p1[k];
                 } else {
                     y = d - p1[k];
                 }

@@ -1,5 +1,6 @@
 """Rows that a careless statistic gets wrong: layernorm rows whose first element lies far from the rest (nothing may be summed
-around that element alone in 32 bits). Against numpy in more than 64 bits."""
+around that element alone in 32 bits), and f16 log_softmax rows with a large common offset (nothing may round the offset
+before it is subtracted). Against numpy in 64 bits or more."""
 import numpy as np
 import pytest
 
@@ -66,3 +67,23 @@ def test_layernorm_of_transposed_rows_with_a_far_first_element(hpt, dev, shape, 
     some = slice(None) if len(shape) == 2 else slice(0, shape[0], 37)  # (batches: a sample)
     v = values.swapaxes(-1, -2)
     _check_layernorm(hpt, got[some], v[some], dtype, f"{shape} {dtype} first {first}: {plan}")
+
+
+@pytest.mark.parametrize("offset,step", [(0, 8), (1000, 8), (-1000, 8), (16000, 8), (-16000, 8)])
+@pytest.mark.parametrize("shape", [(200, 1001), (200, 1000), (2000, 4099)], ids=lambda v: "x".join(map(str, v)))
+def test_f16_log_softmax_of_transposed_rows_with_a_large_offset(hpt, dev, shape, offset, step):
+    """One element `step` above the others, all far from zero: the result there is close to zero and shows every error of
+    the logarithm of the sum. Allowed: half a unit of the last f16 place, and 1e-6 for the sum and its logarithm in f32."""
+    x = np.full(shape, offset, np.float32)
+    x[7] += step
+    x[11::3] -= step
+    a = x.astype(np.float16)
+    assert np.array_equal(a.astype(np.float32), x)  # (the values are f16 numbers)
+    t = hpt.Tensor.from_numpy(a).to_hip(dev).permute([1, 0])
+    plan = hpt.normalize_plan(t, 1)
+    assert plan.startswith("transposed-tile"), plan
+    got = t.log_softmax(1).numpy().astype(np.float64)
+    v = x.T.astype(np.float64)
+    d = v - v.max(1, keepdims=True)
+    want = d - np.log(np.exp(d).sum(1, keepdims=True))
+    assert_close(got, want, 2.0 ** -11, 1e-6, f"{shape} offset {offset}: {plan}")
