@@ -218,9 +218,12 @@ template <class T> void launch_transposed(const NormPlan& p, const NormArgs& a, 
         if (p.shift) transposed_stats_kernel<KIND, T, FULL, true><<<sgrid, dim3(64 * nw), slds, st>>>(t);
         else transposed_stats_kernel<KIND, T><<<sgrid, dim3(64 * nw), slds, st>>>(t);
         transposed_finalize_kernel<KIND, T><<<dim3((unsigned)((t.R + 15) / 16), 1, batch), dim3(16, 16), 0, st>>>(t);
-        const dim3 agrid((rt + 3) / 4, (unsigned)((tiles + 1) / 2), batch);
-        if (p.shift) transposed_apply_kernel<KIND, T, true><<<agrid, dim3(256), 0, st>>>(t);
-        else transposed_apply_kernel<KIND, T><<<agrid, dim3(256), 0, st>>>(t);
+        // (more column blocks than a grid has in y, from 2^22 four-byte columns on: one launch after the other)
+        for (int blocks = (tiles + 1) / 2; t.y0 < blocks; t.y0 += 65535) {
+            const dim3 agrid((rt + 3) / 4, (unsigned)std::min(blocks - t.y0, 65535), batch);
+            if (p.shift) transposed_apply_kernel<KIND, T, true><<<agrid, dim3(256), 0, st>>>(t);
+            else transposed_apply_kernel<KIND, T><<<agrid, dim3(256), 0, st>>>(t);
+        }
         return;
     }
 }

@@ -39,6 +39,7 @@ struct TransposedArgs {
     int cols;         // length of the normalised axis
     int S;            // workgroups sharing the axis in the statistics pass
     int nw;           // wavefronts per workgroup of the statistics pass
+    int y0;           // last pass: column block of blockIdx.y = 0 (a grid has at most 65535 of them)
 };
 
 // Columns that wavefront `pid` of the P that share a row's columns takes (it starts at column pid and steps by P), and
@@ -334,7 +335,7 @@ __global__ void __launch_bounds__(256) transposed_apply_kernel(const TransposedA
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int rg = lane & 7, cl = lane >> 3;
     int r0 = (blockIdx.x * 4 + w) * TR + rg * VEC;
-    const int c_base = blockIdx.y * (NC * TC) + cl * VEC;
+    const int c_base = (blockIdx.y + a.y0) * (NC * TC) + cl * VEC;
     if (r0 >= a.R || c_base >= a.cols) return;
     if constexpr (UA) r0 = min(r0, a.R - VEC);
 

@@ -116,3 +116,21 @@ def test_transposed_unaligned_captured(hpt, dev):
         hip.hipGraphExecDestroy(gexec)
         hip.hipGraphDestroy(graph)
         hip.hipStreamDestroy(s)
+
+
+@pytest.mark.parametrize("dtype,rows,cols", [("f64", 17, 2097121), ("f64", 16, 2097152), ("f32", 33, 4194241)])
+def test_transposed_of_millions_of_columns(hpt, dev, dtype, rows, cols):
+    """Just past 65535 column blocks of the last pass (32 eight-byte columns each, 64 four-byte ones)."""
+    np_dtype = np.float64 if dtype == "f64" else np.float32
+    x = np.random.default_rng(21).random((cols, rows), dtype=np_dtype)
+    t = hpt.Tensor.from_numpy(x).to_hip(dev).permute([1, 0])
+    assert hpt.normalize_plan(t, 1).startswith("transposed"), hpt.normalize_plan(t, 1)
+    e = np.exp(x.T.astype(np.float64))
+    # (results of 5e-7: compared as shares of the largest; f64 sums of cols terms in any order are 1e-10 apart at most)
+    got = t.softmax(1).numpy()
+    assert_close(got * cols, e / e.sum(1, keepdims=True) * cols, 1e-9 if dtype == "f64" else F32_RTOL, F32_ATOL, "softmax")
+    del e, got
+    d = x.T.astype(np.float64)
+    d -= d.mean(1, keepdims=True)
+    d /= np.sqrt((d * d).mean(1, keepdims=True) + 1e-5)
+    assert_close(t.layernorm([cols], None, None, 1e-5).numpy(), d, 1e-9 if dtype == "f64" else F32_RTOL, F32_ATOL, "layernorm")
