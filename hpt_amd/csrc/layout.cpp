@@ -1022,8 +1022,10 @@ NormPlan plan_normalize(const void* in_data, const void* out_data, const int64_t
                              ((uintptr_t)in_data % elem_size) == 0 && ((uintptr_t)out_data % elem_size) == 0;
         // One workgroup per slab, the slab in its registers: the fewest threads (a multiple of L / gcd(L, vector) of them
         // take part) that hold it in four vectors each, up to eight of 1024 threads. (Two vectors and twice the threads:
-        // f32 [5592, 2000, 3] 49.2 -> 70.2 us, [500, 512, 16] 11.0 -> 13.0, nothing gains more than noise.)
-        auto slab_shape = [&]() {
+        // f32 [5592, 2000, 3] 49.2 -> 70.2 us, [500, 512, 16] 11.0 -> 13.0, nothing gains more than noise.) Not where the
+        // slabs times their threads reach the 2^32 work-items that a launch may have.
+        int slab_threads = 0, slab_chunk = 0;
+        auto slab_fits = [&]() {
             const int64_t nv = (p.cols * sa + max_vec - 1) / max_vec;
             int64_t g = sa, b = max_vec;
             while (b) { const int64_t t = g % b; g = b; b = t; }
@@ -1034,12 +1036,9 @@ NormPlan plan_normalize(const void* in_data, const void* out_data, const int64_t
                 int64_t nc = (nv + act - 1) / act;
                 if (nc > 8 || (nc > 4 && t < 1024)) continue;
                 if (nc == 5 || nc == 7) ++nc;  // (kernels exist for 1, 2, 3, 4, 6 and 8)
-                p.kind = NormKind::Col;
-                p.inner = p.out_axis_stride;
-                p.slab_tile = (int)t;
-                p.nchunk = (int)nc;
-                p.vec = max_vec;
-                return true;
+                slab_threads = (int)t;
+                slab_chunk = (int)nc;
+                return slabs < (1ll << 32) / t;
             }
             return false;
         };
@@ -1048,8 +1047,8 @@ NormPlan plan_normalize(const void* in_data, const void* out_data, const int64_t
         // f16 [112, 3904, 6] 43 -> 8.8, f32 [2048, 128, 2] 17.3 -> 4.0, bf16 [693, 488, 5] 14.4 -> 6.2, f32 [2511, 963, 8]
         // 45 -> 34, bf16 [8, 4000, 4] 12.3 -> 7.0. Up to 64 KiB, and to the 128 KiB that fit a workgroup where the alternative
         // is not the flat walk (f32 [32, 4096, 8] 38.8 -> 10.9).
-        const bool narrow = is_slab && sa <= 8 && p.cols >= 64 && slabs <= (1 << 30) &&
-                            slab_bytes <= (slabs * slab_bytes < (8ll << 20) ? (128 << 10) : (64 << 10));
+        const bool narrow = is_slab && sa <= 8 && p.cols >= 64 &&
+                            slab_bytes <= (slabs * slab_bytes < (8ll << 20) ? (128 << 10) : (64 << 10)) && slab_fits();
         // Small groups laid back to back (a contiguous [batch, cols, L] tensor with cols * L elements of at
         // most 2 KiB: softmax over 4 heads of 64, over the 2 of [N, 2, 3]): lanes along L would idle and a
         // lane per (batch, inner) pair reads single elements at a stride. A workgroup stages 16 KiB of whole
@@ -1114,7 +1113,14 @@ NormPlan plan_normalize(const void* in_data, const void* out_data, const int64_t
         // go either way by a few points and keep the register columns.)
         const bool mid_slab = is_slab && p.cols > 64 && slab_bytes <= (64 << 10) && slabs >= 256 && slabs * slab_bytes >= (4ll << 20) &&
                               sa * (int64_t)elem_size <= ((p.cols > 1024 || (elem_size == 4 && sa % max_vec != 0)) ? (elem_size == 4 && sa % max_vec != 0 ? 48 : 32) : 12);
-        if ((narrow || mid_slab) && slab_shape()) return p;
+        if (narrow || (mid_slab && slab_fits())) {
+            p.kind = NormKind::Col;
+            p.inner = p.out_axis_stride;
+            p.slab_tile = slab_threads;
+            p.nchunk = slab_chunk;
+            p.vec = max_vec;
+            return p;
+        }
         if (nk >= 1 && nk <= 2 && p.kept_in.stride[nk - 1] == 1 && p.kept_out.stride[nk - 1] == 1 &&
             p.kept_in.size[nk - 1] == p.out_axis_stride && p.kept_in.size[nk - 1] <= (1 << 30) && p.cols <= (1 << 30) &&
             (nk == 1 || p.kept_in.size[0] <= 65535)) {
