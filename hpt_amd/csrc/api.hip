@@ -8,6 +8,7 @@
 #include <list>
 #include <map>
 #include <mutex>
+#include <optional>
 #include <unordered_map>
 #include <vector>
 
@@ -166,12 +167,15 @@ struct DeviceAllocator {
             return p;
         }
         void* p = nullptr;
-        RelaxedCapture relaxed;
+        // Device memory is not allocated while a capture refuses it (scratch least of all: its address would be recorded, and
+        // hpt_hip_cache_clear hands it on) - except in the place of a cached block that is only not idle yet.
+        std::optional<RelaxedCapture> relaxed;
+        if (it != cache.end()) relaxed.emplace();
         for (;;) {
             hipError_t e = hipMalloc(&p, bytes ? bytes : 1);
             if (e == hipSuccess) break;
             (void)hipGetLastError();  // clear the sticky error before retrying
-            if (cache.empty())
+            if (e != hipErrorOutOfMemory || cache.empty())
                 fail(HPT_ERR_MEMORY, "Failed to allocate %zu bytes on device: %s", bytes,
                      hipGetErrorString(e));
             evict_one();
