@@ -90,6 +90,8 @@ struct RelaxedCapture {
 // handed on at once only to a caller whose first use of it is queued on the same stream (hpt_hip_alloc_ordered), so the
 // queue itself keeps the two apart. Anybody else waits for the default stream first, which makes every block numbered
 // so far idle. (Waiting at every free instead kept the host and the device taking turns: about 25 us of a pass.)
+// That wait lasts as long as the stream has work: it is made without the lock, and ordered callers take blocks in use
+// before idle ones, so that whoever needs an idle block mostly finds one.
 
 struct LayoutKey {
     size_t bytes, align;
@@ -119,16 +121,20 @@ struct DeviceAllocator {
         return n;
     }
     // Requires `mu` and the device to be current. False where the stream cannot be waited for: while another stream
-    // that it orders itself with is being captured.
-    bool wait_default_stream() {
-        if (idle_upto == last_number) return true;
+    // that it orders itself with is being captured. `lock` (on mu) is let go for the wait: the cache may be another after.
+    bool wait_default_stream(std::unique_lock<std::mutex>* lock = nullptr) {
+        const uint64_t upto = last_number;
+        if (idle_upto >= upto) return true;
         if (capturing(nullptr)) return false;
         RelaxedCapture relaxed;
-        if (hipStreamSynchronize(nullptr) != hipSuccess) {
+        if (lock) lock->unlock();
+        const hipError_t e = hipStreamSynchronize(nullptr);
+        if (lock) lock->lock();
+        if (e != hipSuccess) {
             (void)hipGetLastError();
             return false;
         }
-        idle_upto = last_number;
+        idle_upto = std::max(idle_upto, upto);
         return true;
     }
     void evict_one() {  // requires a non-empty cache
@@ -141,18 +147,17 @@ struct DeviceAllocator {
         cache.erase(it);
         lru.pop_back();
     }
-    // `ordered`: the block's first use will be queued on the default stream.
-    void* allocate(size_t bytes, size_t align, bool ordered = false) {
+    // `lock` holds mu. `ordered`: the block's first use will be queued on the default stream.
+    void* allocate(std::unique_lock<std::mutex>& lock, size_t bytes, size_t align, bool ordered = false) {
         LayoutKey k{bytes, align};
         auto it = cache.find(k);
         size_t take = 0;  // one more than the index of the block to hand out
-        if (it != cache.end()) {
+        for (bool waited = false; it != cache.end(); waited = true, it = cache.find(k)) {
             const std::vector<CachedBlock>& blocks = it->second.second;
             take = blocks.size();
-            if (!ordered) {
-                while (take && blocks[take - 1].number > idle_upto) --take;
-                if (!take && wait_default_stream()) take = blocks.size();
-            }
+            while (take && (blocks[take - 1].number > idle_upto) != ordered) --take;
+            if (!take && ordered) take = blocks.size();
+            if (take || waited || !wait_default_stream(&lock)) break;
         }
         if (take) {
             std::vector<CachedBlock>& blocks = it->second.second;
@@ -265,8 +270,8 @@ static void* scratch_reserve(int dev, StreamScratch& s, size_t bytes) {
         DeviceAllocator& a = allocator_of(dev);
         void* p;
         {
-            std::lock_guard<std::mutex> g(a.mu);
-            p = a.allocate(want, kScratchAlign);
+            std::unique_lock<std::mutex> g(a.mu);
+            p = a.allocate(g, want, kScratchAlign);
             ++a.internal_blocks;
         }
         if (s.base) s.retired.emplace_back(s.base, s.bytes);
@@ -624,8 +629,8 @@ int32_t hpt_hip_alloc(int32_t dev, size_t bytes, size_t align, int32_t zeroed, v
         if (align == 0 || (align & (align - 1))) fail(HPT_ERR_PARAM, "alloc: align %zu is not a power of two", align);
         use_device(dev);
         DeviceAllocator& a = allocator_of(dev);
-        std::lock_guard<std::mutex> g(a.mu);
-        void* p = a.allocate(bytes, align);
+        std::unique_lock<std::mutex> g(a.mu);
+        void* p = a.allocate(g, bytes, align);
         if (zeroed && bytes) {
             hipError_t e = hipMemset(p, 0, bytes);
             if (e != hipSuccess) {
@@ -653,8 +658,8 @@ int32_t hpt_hip_alloc_ordered(int32_t dev, size_t bytes, size_t align, void** ou
         if (align == 0 || (align & (align - 1))) fail(HPT_ERR_PARAM, "alloc: align %zu is not a power of two", align);
         use_device(dev);
         DeviceAllocator& a = allocator_of(dev);
-        std::lock_guard<std::mutex> g(a.mu);
-        *out = a.allocate(bytes, align, true);
+        std::unique_lock<std::mutex> g(a.mu);
+        *out = a.allocate(g, bytes, align, true);
     });
 }
 

@@ -127,3 +127,59 @@ def test_allocation_under_capture_beside_a_busy_block(hpt, dev, hip):
     hip.hipGraphExecDestroy(gexec)
     hip.hipGraphDestroy(graph)
     hip.hipStreamDestroy(s)
+
+
+def test_a_waiting_allocation_holds_nobody_up(hpt, dev, hip):
+    """An ordinary allocation that finds only a block in use waits for the default stream; meanwhile other threads take and
+    give back blocks."""
+    import time
+    from hpt_amd import _ffi
+    l, n, m = hpt.lib(), 23456 * 64, 34567 * 64
+    p, q, r = P(), P(), P()
+    _ffi.check(l.hpt_hip_cache_clear(dev))
+    _ffi.check(l.hpt_hip_alloc_ordered(dev, n, 64, C.byref(p)))
+    _ffi.check(l.hpt_hip_alloc_ordered(dev, m, 64, C.byref(q)))
+    _ffi.check(l.hpt_hip_free_ordered(dev, q, m, 64))
+    keep = hpt.Tensor.empty([1 << 28], hpt.f32, dev)
+    keep.add_(keep, out=keep)
+    hpt.synchronize(dev)
+    for _ in range(200):  # about a tenth of a second
+        keep.add_(keep, out=keep)
+    _ffi.check(l.hpt_hip_free_ordered(dev, p, n, 64))
+    waiting = threading.Thread(target=lambda: _ffi.check(l.hpt_hip_alloc(dev, n, 64, 0, C.byref(r))))
+    waiting.start()
+    time.sleep(0.01)
+    for _ in range(20):
+        _ffi.check(l.hpt_hip_alloc_ordered(dev, m, 64, C.byref(q)))
+        _ffi.check(l.hpt_hip_free_ordered(dev, q, m, 64))
+    busy = hip.hipStreamQuery(None) != 0
+    hip.hipGetLastError()  # (not ready)
+    still = waiting.is_alive()
+    waiting.join()
+    assert hip.hipStreamQuery(None) == 0 and r.value == p.value
+    assert busy and still, "allocations on another thread waited for the default stream too"
+    _ffi.check(l.hpt_hip_free(dev, r, n, 64))
+    _ffi.check(l.hpt_hip_cache_clear(dev))
+
+
+def test_idle_blocks_are_left_for_those_who_need_one(hpt, dev, hip):
+    from hpt_amd import _ffi
+    l, n = hpt.lib(), 45678 * 64
+    p, q, r = P(), P(), P()
+    _ffi.check(l.hpt_hip_cache_clear(dev))
+    for x in (p, q):
+        _ffi.check(l.hpt_hip_alloc(dev, n, 64, 0, C.byref(x)))
+    keep = _busy(hpt, dev)
+    _ffi.check(l.hpt_hip_free_ordered(dev, p, n, 64))
+    _ffi.check(l.hpt_hip_free(dev, q, n, 64))  # idle, and freed last
+    _ffi.check(l.hpt_hip_alloc_ordered(dev, n, 64, C.byref(r)))
+    assert r.value == p.value
+    _ffi.check(l.hpt_hip_free_ordered(dev, r, n, 64))
+    _ffi.check(l.hpt_hip_alloc(dev, n, 64, 0, C.byref(r)))
+    assert r.value == q.value
+    _ffi.check(l.hpt_hip_alloc_ordered(dev, n, 64, C.byref(q)))
+    assert q.value == p.value
+    for x in (r, q):
+        _ffi.check(l.hpt_hip_free_ordered(dev, x, n, 64))
+    del keep
+    _ffi.check(l.hpt_hip_cache_clear(dev))
