@@ -814,7 +814,7 @@ NormPlan plan_normalize(const void* in_data, const void* out_data, const int64_t
                 if (S >= 2) {
                     p.kind = NormKind::RowSplit;
                     p.tsplit = (int)S;
-                    p.scratch_bytes = (size_t)p.rows * S * 16;
+                    p.scratch_bytes = (size_t)p.rows * S * 24;
                     return p;
                 }
                 if (p.shift) {  // not worth splitting: back to element-wise rows

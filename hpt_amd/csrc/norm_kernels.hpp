@@ -1402,7 +1402,7 @@ __global__ void __launch_bounds__(1024) row_stream_kernel(const NormArgs a) {
 // One workgroup per row leaves most of the chip idle when there are fewer rows than compute
 // units (a batch of 32 rows of 131072 logits). Here S workgroups take a slice of the row each:
 //   row_split_stats_kernel     partial statistics of a slice: softmax (max, sum of exp(x - max)),
-//                              layernorm sums of (x - k), (x - k)^2 with k the row's first element
+//                              layernorm (count, mean, squared deviations)
 //   row_split_apply_kernel     folds the S partials of its row into (max, 1/sum or ln sum) or
 //                              (mean_hi, mean_lo, rstd), re-reads the slice and writes the result
 // Input rows are contiguous along the axis (any row offsets), the output is contiguous.
@@ -1412,19 +1412,12 @@ struct RowSplitArgs {
     const void* gamma;
     const void* beta;
     const void* residual;  // NORM_ADD_LAYERNORM
-    void* part;            // [rows][S] partials (16 bytes each at most)
+    void* part;            // [rows][S] partials (24 bytes each at most)
     Dims kept_in;
     int64_t rows, cols;
     int64_t chunk_v;       // vectors per slice
     double eps, inv_cols;
     int S;
-};
-
-template <class ST> struct SumPair {
-    ST a, b;
-};
-template <class ST> struct SumPairOp {
-    __device__ static __forceinline__ SumPair<ST> comb(SumPair<ST> x, SumPair<ST> y) { return SumPair<ST>{x.a + y.a, x.b + y.b}; }
 };
 
 // UA: rows whose length or start is off the 16-byte grid. The vectors are unaligned, and a row's last
@@ -1459,7 +1452,7 @@ template <int KIND, class T, int VEC, bool UA>
 __global__ void __launch_bounds__(256) row_split_stats_kernel(const RowSplitArgs a) {
     using CT = typename Elem<T>::Wide;
     using ST = typename StatType<T>::type;
-    __shared__ __align__(16) unsigned char smem_raw[16 * 2 * sizeof(double)];
+    __shared__ __align__(16) unsigned char smem_raw[16 * 3 * sizeof(double)];
     const int64_t row = blockIdx.y;
     const T* in_row = (const T*)a.in + offset_of(a.kept_in, row);
     const int64_t nv = row_split_vectors<VEC, UA>(a.cols);
@@ -1493,19 +1486,18 @@ __global__ void __launch_bounds__(256) row_split_stats_kernel(const RowSplitArgs
         st = block_reduce<SoftStatOp<T, CT, ST>>(st, (SoftStat<CT, ST>*)smem_raw);
         if (threadIdx.x == 0) ((SoftStat<CT, ST>*)a.part)[row * a.S + blockIdx.x] = st;
     } else {
-        // the shift k is the row's first element (after the residual, if any): the same for every slice
-        CT k;
-        {
-            CT x0[VEC];
-            row_split_load<KIND, T, VEC, UA>(a, in_row, row, 0, x0);
-            k = x0[0];
-        }
-        CT s1 = 0, s2 = 0;
+        // Per thread: sums around an element of its own (the last of its first vector, which is no other thread's), turned into
+        // (count, mean, squared deviations) at the end. (One origin for the row, its first element, would have to be read
+        // again by every workgroup of the last pass: in place, one of them has overwritten it by then.)
+        CT k = 0, s1 = 0, s2 = 0;
+        int64_t n = 0;
         for (int64_t iv = v0 + threadIdx.x; iv < v1; iv += 256) {
             CT x[VEC];
             const int64_t e0 = row_split_start<VEC, UA>(iv, a.cols);
             row_split_load<KIND, T, VEC, UA>(a, in_row, row, e0, x);
             const int skip = UA ? (int)(iv * VEC - e0) : 0;
+            if (n == 0) k = x[VEC - 1];
+            n += VEC - skip;
 #pragma unroll
             for (int j = 0; j < VEC; ++j) {
                 const CT d = (!UA || j >= skip) ? x[j] - k : (CT)0;
@@ -1513,9 +1505,15 @@ __global__ void __launch_bounds__(256) row_split_stats_kernel(const RowSplitArgs
                 s2 += d * d;
             }
         }
-        SumPair<ST> sp{(ST)s1, (ST)s2};
-        sp = block_reduce<SumPairOp<ST>>(sp, (SumPair<ST>*)smem_raw);
-        if (threadIdx.x == 0) ((SumPair<ST>*)a.part)[row * a.S + blockIdx.x] = sp;
+        MomentStat<ST> st{(ST)0, (ST)0, (ST)0};
+        if (n > 0) {
+            st.n = (ST)n;
+            st.mean = (ST)k + (ST)s1 / st.n;
+            st.m2 = (ST)s2 - (ST)s1 * (ST)s1 / st.n;
+            if (st.m2 < (ST)0) st.m2 = 0;
+        }
+        st = block_reduce<MomentStatOp<ST>>(st, (MomentStat<ST>*)smem_raw);
+        if (threadIdx.x == 0) ((MomentStat<ST>*)a.part)[row * a.S + blockIdx.x] = st;
     }
 }
 
@@ -1526,7 +1524,7 @@ template <int KIND, class T, int VEC, bool UA>
 __global__ void __launch_bounds__(256) row_split_apply_kernel(const RowSplitArgs a) {
     using CT = typename Elem<T>::Wide;
     using ST = typename StatType<T>::type;
-    __shared__ __align__(16) unsigned char smem_raw[16 * 2 * sizeof(double)];
+    __shared__ __align__(16) unsigned char smem_raw[16 * 3 * sizeof(double)];
     const int64_t row = blockIdx.y;
     const T* in_row = (const T*)a.in + offset_of(a.kept_in, row);
     T* out_row = (T*)a.out + row * a.cols;
@@ -1539,17 +1537,12 @@ __global__ void __launch_bounds__(256) row_split_apply_kernel(const RowSplitArgs
         p1 = norm_is_log(KIND) ? log_ct<T>((CT)st.s) : (CT)((ST)1 / st.s);
         p2 = 0;
     } else {
-        SumPair<ST> sp{(ST)0, (ST)0};
-        for (int i = threadIdx.x; i < a.S; i += 256) sp = SumPairOp<ST>::comb(sp, ((const SumPair<ST>*)a.part)[row * a.S + i]);
-        sp = block_reduce<SumPairOp<ST>>(sp, (SumPair<ST>*)smem_raw);
-        CT x0[VEC];
-        row_split_load<KIND, T, VEC, UA>(a, in_row, row, 0, x0);
-        const ST mean = (ST)x0[0] + sp.a * (ST)a.inv_cols;
-        ST m2 = sp.b - sp.a * sp.a * (ST)a.inv_cols;
-        if (m2 < (ST)0) m2 = 0;
-        p0 = (CT)mean;
-        p1 = (CT)(mean - (ST)p0);
-        p2 = rsqrt_ct((CT)(m2 * (ST)a.inv_cols) + (CT)a.eps);
+        MomentStat<ST> st{(ST)0, (ST)0, (ST)0};
+        for (int i = threadIdx.x; i < a.S; i += 256) st = MomentStatOp<ST>::comb(st, ((const MomentStat<ST>*)a.part)[row * a.S + i]);
+        st = block_reduce<MomentStatOp<ST>>(st, (MomentStat<ST>*)smem_raw);
+        p0 = (CT)st.mean;
+        p1 = (CT)(st.mean - (ST)p0);
+        p2 = rsqrt_ct((CT)(st.m2 * (ST)a.inv_cols) + (CT)a.eps);
     }
     const int64_t nv = row_split_vectors<VEC, UA>(a.cols);
     const int64_t v0 = (int64_t)blockIdx.x * a.chunk_v, v1 = min(nv, v0 + a.chunk_v);

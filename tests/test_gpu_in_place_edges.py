@@ -29,3 +29,20 @@ def test_softmax_over_odd_columns_in_place(hpt, dev, dtype, shape, log):
     want = run(axis).numpy()
     run(axis, out=t)
     assert np.array_equal(t.numpy(), want), plan
+
+
+@pytest.mark.parametrize("dtype", ["f32", "f16", "f64"])
+@pytest.mark.parametrize("shape", [(1, 1 << 22), (5, 1 << 20), (4, 300007), (100, 65539)], ids=lambda v: "x".join(map(str, v)))
+def test_layernorm_of_shared_rows_in_place(hpt, dev, dtype, shape):
+    a, dt = _values(hpt, shape, dtype)
+    a[:, 0] = 50
+    t, r = hpt.Tensor.from_numpy(a, dt).to_hip(dev), hpt.Tensor.from_numpy(a[:, ::-1].copy(), dt).to_hip(dev)
+    plan = hpt.normalize_plan(t, 0, 1)
+    assert plan.startswith("rowsplit"), plan
+    n = [shape[1]]
+    want, want_sum = t.layernorm(n, None, None, 1e-5).numpy(), t.layernorm(n, None, None, 1e-5, residual=r).numpy()
+    u = hpt.Tensor.from_numpy(a, dt).to_hip(dev)
+    t.layernorm(n, None, None, 1e-5, out=t)
+    assert np.array_equal(t.numpy(), want), plan
+    u.layernorm(n, None, None, 1e-5, residual=r, out=u)
+    assert np.array_equal(u.numpy(), want_sum), plan
