@@ -1448,6 +1448,18 @@ __device__ __forceinline__ void row_split_load(const RowSplitArgs& a, const T* i
     }
 }
 
+// The moments of every thread of a workgroup of four wavefronts as one, in every thread. Sums of differences from the first
+// thread's mean, then of the deviations from the result: a merge per step of the reduction would divide in each.
+__device__ __forceinline__ MomentStat<double> block_moments(MomentStat<double> v, double* smem) {
+    auto sum = [&](double x) { return block_reduce<SumC<double>>(x, smem); };
+    __syncthreads();
+    if (threadIdx.x == 0) smem[16] = v.mean;
+    __syncthreads();
+    const double first = smem[16], n = sum(v.n), shift = sum(v.n > 0 ? v.n * (v.mean - first) : 0.0);
+    const double mean = n > 0 ? first + shift / n : 0, d = v.mean - mean;
+    return {n, mean, sum(v.n > 0 ? v.m2 + v.n * d * d : 0.0)};
+}
+
 template <int KIND, class T, int VEC, bool UA>
 __global__ void __launch_bounds__(256) row_split_stats_kernel(const RowSplitArgs a) {
     using CT = typename Elem<T>::Wide;
@@ -1486,34 +1498,36 @@ __global__ void __launch_bounds__(256) row_split_stats_kernel(const RowSplitArgs
         st = block_reduce<SoftStatOp<T, CT, ST>>(st, (SoftStat<CT, ST>*)smem_raw);
         if (threadIdx.x == 0) ((SoftStat<CT, ST>*)a.part)[row * a.S + blockIdx.x] = st;
     } else {
-        // Per thread: sums around an element of its own (the last of its first vector, which is no other thread's), turned into
-        // (count, mean, squared deviations) at the end. (One origin for the row, its first element, would have to be read
-        // again by every workgroup of the last pass: in place, one of them has overwritten it by then.)
-        CT k = 0, s1 = 0, s2 = 0;
+        // Per thread: f64 sums around an element of its own (the last of its first vector, which is no other thread's), turned
+        // into (count, mean, squared deviations) at the end. (One origin for the row, its first element, would have to be read
+        // again by every workgroup of the last pass: in place, one of them has overwritten it by then. In f32 such
+        // sums lost what a far first element had in common with every term: f32 [2, 300007] with 1000 there, half of the
+        // results off by more than 1e-5; f16 [3, 1048576] 1.2e-2 of the norm, 30 times what rounding the results costs.)
+        double k = 0, s1 = 0, s2 = 0;
         int64_t n = 0;
         for (int64_t iv = v0 + threadIdx.x; iv < v1; iv += 256) {
             CT x[VEC];
             const int64_t e0 = row_split_start<VEC, UA>(iv, a.cols);
             row_split_load<KIND, T, VEC, UA>(a, in_row, row, e0, x);
             const int skip = UA ? (int)(iv * VEC - e0) : 0;
-            if (n == 0) k = x[VEC - 1];
+            if (n == 0) k = (double)x[VEC - 1];
             n += VEC - skip;
 #pragma unroll
             for (int j = 0; j < VEC; ++j) {
-                const CT d = (!UA || j >= skip) ? x[j] - k : (CT)0;
+                const double d = (!UA || j >= skip) ? (double)x[j] - k : 0.0;
                 s1 += d;
-                s2 += d * d;
+                s2 = fma(d, d, s2);
             }
         }
-        MomentStat<ST> st{(ST)0, (ST)0, (ST)0};
+        MomentStat<double> st{0, 0, 0};
         if (n > 0) {
-            st.n = (ST)n;
-            st.mean = (ST)k + (ST)s1 / st.n;
-            st.m2 = (ST)s2 - (ST)s1 * (ST)s1 / st.n;
-            if (st.m2 < (ST)0) st.m2 = 0;
+            st.n = (double)n;
+            st.mean = k + s1 / st.n;
+            st.m2 = s2 - s1 * s1 / st.n;
+            if (st.m2 < 0) st.m2 = 0;
         }
-        st = block_reduce<MomentStatOp<ST>>(st, (MomentStat<ST>*)smem_raw);
-        if (threadIdx.x == 0) ((MomentStat<ST>*)a.part)[row * a.S + blockIdx.x] = st;
+        st = block_moments(st, (double*)smem_raw);
+        if (threadIdx.x == 0) ((MomentStat<double>*)a.part)[row * a.S + blockIdx.x] = st;
     }
 }
 
@@ -1537,12 +1551,12 @@ __global__ void __launch_bounds__(256) row_split_apply_kernel(const RowSplitArgs
         p1 = norm_is_log(KIND) ? log_ct<T>((CT)st.s) : (CT)((ST)1 / st.s);
         p2 = 0;
     } else {
-        MomentStat<ST> st{(ST)0, (ST)0, (ST)0};
-        for (int i = threadIdx.x; i < a.S; i += 256) st = MomentStatOp<ST>::comb(st, ((const MomentStat<ST>*)a.part)[row * a.S + i]);
-        st = block_reduce<MomentStatOp<ST>>(st, (MomentStat<ST>*)smem_raw);
+        MomentStat<double> st{0, 0, 0};
+        for (int i = threadIdx.x; i < a.S; i += 256) st = MomentStatOp<double>::comb(st, ((const MomentStat<double>*)a.part)[row * a.S + i]);
+        st = block_moments(st, (double*)smem_raw);
         p0 = (CT)st.mean;
-        p1 = (CT)(st.mean - (ST)p0);
-        p2 = rsqrt_ct((CT)(st.m2 * (ST)a.inv_cols) + (CT)a.eps);
+        p1 = (CT)(st.mean - (double)p0);
+        p2 = rsqrt_ct((CT)(st.m2 * a.inv_cols) + (CT)a.eps);
     }
     const int64_t nv = row_split_vectors<VEC, UA>(a.cols);
     const int64_t v0 = (int64_t)blockIdx.x * a.chunk_v, v1 = min(nv, v0 + a.chunk_v);

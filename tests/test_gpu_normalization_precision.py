@@ -69,6 +69,23 @@ def test_layernorm_of_transposed_rows_with_a_far_first_element(hpt, dev, shape, 
     _check_layernorm(hpt, got[some], v[some], dtype, f"{shape} {dtype} first {first}: {plan}")
 
 
+@pytest.mark.parametrize("first", [0, 100, 1000, 30000])
+@pytest.mark.parametrize("shape", [(3, 1 << 20), (2, 300007), (100, 65539)], ids=lambda v: "x".join(map(str, v)))
+@pytest.mark.parametrize("dtype", ["f32", "f16", "bf16", "f64"])
+def test_layernorm_of_shared_rows_with_a_far_first_element(hpt, dev, shape, dtype, first):
+    x = np.random.default_rng(4).standard_normal(shape)
+    x[:, 0] += first
+    a, dt, values = _stored(hpt, x, dtype)
+    t = hpt.Tensor.from_numpy(a, dt).to_hip(dev)
+    plan = hpt.normalize_plan(t, 0, 1)
+    assert plan.startswith("rowsplit"), plan
+    got = t.layernorm([shape[1]], None, None, 1e-5).numpy()
+    if dtype == "bf16":
+        got = hpt.bf16_bits_to_f32(got)
+    # (f64: the thread that holds the first element sums up to 32 elements around it)
+    _check_layernorm(hpt, got, values, dtype, f"{shape} {dtype} first {first}: {plan}", f64_units=128)
+
+
 @pytest.mark.parametrize("offset,step", [(0, 8), (1000, 8), (-1000, 8), (16000, 8), (-16000, 8)])
 @pytest.mark.parametrize("shape", [(200, 1001), (200, 1000), (2000, 4099)], ids=lambda v: "x".join(map(str, v)))
 def test_f16_log_softmax_of_transposed_rows_with_a_large_offset(hpt, dev, shape, offset, step):
