@@ -387,7 +387,8 @@ ReducePlan plan_reduce(const void* data, const int64_t* shape, const int64_t* st
         // Rows that are not whole, aligned vectors (an odd inner length, a base or pitch off 16 bytes):
         // a lane still takes `full` neighbouring outputs, with unaligned 128-bit loads (global memory
         // takes them; now and then one touches two lines) instead of one element at a time - eight
-        // times the bytes in flight per lane for f16. The last lane of a row loads its few elements singly.
+        // times the bytes in flight per lane for f16. The last lane of a row takes its vector from the row's end
+        // backwards, so a row holds one at least (kin >= full).
         // (Worth it when a row is a few wavefronts of such lanes and enough is reduced into each output
         // that the lane's outputs, which it then writes one by one, are a small part of the traffic.)
         // (Small inputs, whose time is the chain of loads of one lane, gain from two lanes per row on: their column

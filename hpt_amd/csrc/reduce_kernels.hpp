@@ -1307,6 +1307,7 @@ if (p.unaligned)             col_flat_kernel<Op, FULL, true><<<dim3(1, (unsigned
                 // every lane's first output index, outer * kin + cv * uv, must be a multiple of uv: kin is
                 a.vec_out = init_out && !p.kept_swapped && uv > 1 && kin % uv == 0 && ((uintptr_t)out % chunk) == 0;
             }
+            if (p.unaligned && kin < p.vec) fail(HPT_ERR_KERNEL, "unaligned columns: a row of %d elements holds no vector of %d", a.kin, p.vec);
             dim3 grid((unsigned)((a.kin_v + p.bx - 1) / p.bx), (unsigned)outer, (unsigned)p.split);
             if (vec && p.sstride == 2) col_lean_kernel<Op, FULL, 2><<<grid, block, smem, st>>>(a);
             else if (vec && p.unaligned) {

@@ -78,7 +78,7 @@ static View random_view(size_t elem, int64_t budget, bool allow_zero, bool allow
 }
 
 static int failures = 0;
-static long seen_transposed_binary = 0, seen_lds_rows = 0;
+static long seen_transposed_binary = 0, seen_lds_rows = 0, seen_small_split = 0;
 #define CHECK(cond, ...)                       \
     do {                                       \
         if (!(cond)) {                         \
@@ -135,6 +135,17 @@ static void fuzz_reduce() {
         CHECK(pow2(p.vec) && (size_t)p.vec * elem <= 16, "%s plan=%s", show(v).c_str(), d.c_str());
         CHECK(p.split >= 1 && p.split_q >= 1 && p.split_i >= 1, "%s plan=%s", show(v).c_str(), d.c_str());
         CHECK(p.interleave >= 1, "%s plan=%s", show(v).c_str(), d.c_str());
+        {   // without scratch to spare: the same plan, or one launch in the place of a split made for speed alone
+            const ReducePlan q = plan_reduce((const void*)v.base, v.shape.data(), v.strides.data(), ndim, axes.data(),
+                                             (int)axes.size(), elem, acc, false, false);
+            CHECK(!q.small_split && (p.small_split ? p.split > 1 && q.split == 1 : describe(q) == d), "%s plan=%s without=%s",
+                  show(v).c_str(), d.c_str(), describe(q).c_str());
+            CHECK(!p.small_split || K * p.split * (int64_t)acc <= (1 << 20), "%s plan=%s", show(v).c_str(), d.c_str());
+            seen_small_split += p.small_split;
+        }
+        // unaligned column vectors: an inner row holds one at least
+        if (p.kind == ReduceKind::Col && p.unaligned && !p.flat_t && !p.flat_xb)
+            CHECK(p.kept.n && p.kept.size[p.kept.n - 1] >= p.vec, "%s plan=%s", show(v).c_str(), d.c_str());
         if (p.interleave > 1)  // rows that are [R, interleave] slabs: whole aligned vectors, one workgroup per row
             CHECK(p.kind == ReduceKind::Row && p.lean && p.split == 1 && (size_t)p.vec * elem == 16 && p.vec % p.interleave == 0 &&
                       p.interleave <= 8 && p.K % p.interleave == 0 && (p.R * p.interleave) % p.vec == 0 && !p.ragged && !p.unaligned &&
@@ -302,7 +313,7 @@ int main(int argc, char** argv) {
         fuzz_elementwise();
         if (failures > 20) break;
     }
-    std::printf("planner_fuzz: %ld iterations, %d failures (%ld transposing binary plans, %ld register + LDS row plans)\n", iters,
-                failures, seen_transposed_binary, seen_lds_rows);
+    std::printf("planner_fuzz: %ld iterations, %d failures (%ld transposing binary plans, %ld register + LDS row plans, %ld small split reductions)\n",
+                iters, failures, seen_transposed_binary, seen_lds_rows, seen_small_split);
     return failures ? 1 : 0;
 }
