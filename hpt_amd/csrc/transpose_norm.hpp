@@ -416,37 +416,49 @@ __global__ void __launch_bounds__(256) col_apply_kernel(const TransposedArgs a, 
     const T* in = (const T*)a.in + (int64_t)blockIdx.z * a.bi + r0;
     T* out = (T*)a.out + (int64_t)blockIdx.z * a.cols * a.R + r0;
     const int c_end = min(a.cols, (int)(blockIdx.y + 1) * chunk);
-    auto apply = [&](const Pack<T, VEC>& v, int c) {
-        Pack<T, VEC> o;
-#pragma unroll
-        for (int k = 0; k < VEC; ++k) {
-            const CT d = Elem<T>::widen(v.v[k]) - p0.v[k];
-            o.v[k] = Elem<T>::narrow(kLog ? d - p1.v[k] : exp_ct<T>(d) * p1.v[k]);
-        }
-        if constexpr (UA) {
-            if (skip == 0) {
-                store_pack_unaligned_stream<T, VEC>(out + (int64_t)c * a.R, o);
-            } else {
-#pragma unroll
-                for (int k = 0; k < VEC; ++k)
-                    if (k >= skip) out[(int64_t)c * a.R + k] = o.v[k];
-            }
-        } else if constexpr (VEC > 1) store_pack_stream<T, VEC>(out + (int64_t)c * a.R, o);
-        else out[(int64_t)c * a.R] = o.v[0];
-    };
     auto fetch = [&](int c) {
         if constexpr (UA) return load_pack_unaligned<T, VEC>(in + (int64_t)c * a.sa);
         else return load_pack<T, VEC>(in + (int64_t)c * a.sa);
     };
-    int c = blockIdx.y * chunk + ty;
-    for (; c + 12 < c_end; c += 16) {  // four positions in flight per thread (thread rows are 4 apart)
-        Pack<T, VEC> v[4];
+    auto walk = [&](auto row_end) {
+        auto apply = [&](const Pack<T, VEC>& v, int c) {
+            Pack<T, VEC> o;
 #pragma unroll
-        for (int u = 0; u < 4; ++u) v[u] = fetch(c + 4 * u);
+            for (int k = 0; k < VEC; ++k) {
+                const CT d = Elem<T>::widen(v.v[k]) - p0.v[k];
+                o.v[k] = Elem<T>::narrow(kLog ? d - p1.v[k] : exp_ct<T>(d) * p1.v[k]);
+            }
+            T* dst = out + (int64_t)c * a.R;
+            if constexpr (decltype(row_end)::value) {
+                if (skip == 0) {
+                    store_pack_unaligned_stream<T, VEC>(dst, o);
+                } else {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) apply(v[u], c + 4 * u);
+                    for (int k = 0; k < VEC; ++k)
+                        if (k >= skip) dst[k] = o.v[k];
+                }
+            } else if constexpr (UA) store_pack_unaligned_stream<T, VEC>(dst, o);
+            else if constexpr (VEC > 1) store_pack_stream<T, VEC>(dst, o);
+            else dst[0] = o.v[0];
+        };
+        int c = blockIdx.y * chunk + ty;
+        for (; c + 12 < c_end; c += 16) {  // four positions in flight per thread (thread rows are 4 apart)
+            Pack<T, VEC> v[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) v[u] = fetch(c + 4 * u);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) apply(v[u], c + 4 * u);
+        }
+        for (; c < c_end; c += 4) apply(fetch(c), c);
+    };
+    // (a walk of its own for the workgroups at the rows' ends: with the test in every store f32 [8190, 4097] takes 2.5 us more)
+    if constexpr (UA) {
+        if (blockIdx.x == gridDim.x - 1) {
+            walk(std::true_type{});
+            return;
+        }
     }
-    for (; c < c_end; c += 4) apply(fetch(c), c);
+    walk(std::false_type{});
 }
 
 // ---- a SHORT strided axis: the whole axis in registers ---------------------------------------
