@@ -392,7 +392,8 @@ ReducePlan plan_reduce(const void* data, const int64_t* shape, const int64_t* st
         // (Worth it when a row is a few wavefronts of such lanes and enough is reduced into each output
         // that the lane's outputs, which it then writes one by one, are a small part of the traffic.)
         // (Small inputs, whose time is the chain of loads of one lane, gain from two lanes per row on: their column
-        // blocks are narrow, below. Under 16 KiB a lane has a dozen loads in all either way.)
+        // blocks are narrow, below. Under 16 KiB a lane has a dozen loads in all either way: f32 [100, 33] 4.3 us in both forms,
+        // f16 [200, 33] 4.5 and 4.9.)
         const int64_t bytes = p.K * p.R * (int64_t)elem_size;
         const bool small = p.lean && bytes < kSmallColBytes;
         if (p.lean && nk && p.vec == 1 && p.sstride == 1 && full > 1 && p.kept.stride[nk - 1] == 1 &&
@@ -416,10 +417,11 @@ ReducePlan plan_reduce(const void* data, const int64_t* shape, const int64_t* st
             // Below 8 MiB the time is the chain of dependent batches of loads of one lane, and the compute units that
             // stand idle: 16-lane column blocks (256-byte segments of each row) make more workgroups of them, and up
             // to 1024 threads share a block's rows. Where that still leaves a lane more than 24 rows (three batches of
-            // eight loads; a second launch costs as much: f32 [1216, 225], 19 rows, 6.4 us in one launch, 7.3 in two),
+            // eight loads; a second launch costs as much: f32 [1216, 225], 19 rows, 6.4 us in one launch, 7.3 in two, in cache),
             // the rows are dealt over workgroups too, about 12 to a lane. Over axis 0, us before -> now:
-            // f32 [12608, 128] 109 -> 8.9, f16 [2315, 363] 197 -> 8.2 (in one launch 16.1), bf16 [34112, 40] 57 -> 9.0,
-            // f32 [5440, 45] 28.3 -> 7.4; one launch is enough for f32 [1578, 2101][:, ::2], 17.6 -> 8.3.
+            // f32 [12608, 128] 109 -> 8.3 (in one launch 33.9), f16 [2315, 363] 197 -> 8.8 (16.1), f32 [5440, 45] 28.3 -> 7.3
+            // (15.5), f32 [1578, 2101][:, ::2], 25 rows per lane, 17.6 -> 11.1 (12.1), bf16 [34112, 40] 57 -> 8.2. (Device time
+            // of both launches.)
             while (p.bx > 16 && xblocks < kComputeUnits && p.R >= 32) {
                 p.bx /= 2;
                 xblocks = (kv + p.bx - 1) / p.bx * outer;
@@ -678,9 +680,9 @@ NormPlan plan_normalize(const void* in_data, const void* out_data, const int64_t
         // input contiguous along the rows, output along the axis (a transposed view): register tiles in
         // one pass, or statistics pass + register-tile transpose; unaligned vectors (shift) where a pitch, a
         // length or a base is off the 16-byte grid. The rows went element by element then, one cache line per
-        // lane and load: us, rows x columns, softmax and layernorm: f16 15552 x 1470 206 and 226 -> 24 and 22,
-        // f16 2066 x 11011 248 and 262 -> 46 and 42, f32 2557 x 2644 97 and 102 -> 21 and 21, f32 6966 x 368
-        // 32 and 36 -> 10.6 and 11, f16 1279 x 432 9.6 and 10.6 -> 7.4 and 6.4.
+        // lane and load: device us, rows x columns, softmax and layernorm: f16 15552 x 1470 206 and 226 -> 31.7 and 30.7,
+        // f16 2066 x 11011 248 and 262 -> 50.7 and 49.7, f32 2557 x 2644 97 and 102 -> 25.7 and 24.4, f32 6966 x 368
+        // 32 and 36 -> 11.4 and 11.3, f16 1279 x 432 9.6 and 10.6 -> 6.9 and 6.6.
         const int nk = p.kept_in.n;
         const int v = max_vec;
         const bool lies_transposed = sa > 1 && nk >= 1 && nk <= 2 && p.kept_in.stride[nk - 1] == 1 && v > 1 &&
@@ -699,12 +701,13 @@ NormPlan plan_normalize(const void* in_data, const void* out_data, const int64_t
                 // columns): rgN lanes along the rows, 1024 / rgN thread columns of 16 columns
                 // each, 4096 columns at most. Long row segments where they leave enough workgroups; a
                 // matrix too small for that is cut into segments of 64 and 32 bytes, which still beats three launches
-                // by far (us, three passes -> one; rows x columns): f32 3200 x 224 softmax 21.5 -> 5.2, layernorm
-                // 12.6 -> 4.9; f16 5184 x 2048 24.7 -> 14.7, 21 -> 13; f32 300 x 1001 18.6 -> 6.3; bf16 511 x 2001
-                // 22 -> 13.0. It loses where few workgroups walk many columns of a layernorm whose statistics are
-                // cheap (f32 129 x 4000: 12.0 -> 13.9). Beyond 4096 columns 32-byte segments gain nothing (f16
-                // 2048 x 8192 28.0 -> 26.3, f32 333 x 8000 layernorm 17 -> 25): three passes. So do
-                // matrices below 16384 elements, whose plan is pinned.
+                // by far (device us, three passes -> one; rows x columns): f32 3200 x 224 softmax 21.5 -> 5.6, layernorm
+                // 12.6 -> 4.9; f16 5184 x 2048 24.7 -> 17.2, 21 -> 16.0; f32 300 x 1001 18.6 -> 7.5; bf16 511 x 2001
+                // 22 -> 12.6; f32 200 x 3300 layernorm 14.2 -> 10.8 and, where the few workgroups have most columns to
+                // walk, 129 x 4000 14.0 (and two gaps between launches) -> 14.6. Beyond 4096 columns 32-byte segments gain
+                // nothing (f16 2048 x 8192 28.0 -> 26.3, f32 333 x 8000 layernorm 17 -> 25): three passes. Matrices below 16384
+                // elements keep three passes only because tests name that plan; in time they lose as well
+                // (f32 64 x 100 softmax 13.8 -> 4.8, f16 100 x 120 18.8 -> 5.2).
                 const int64_t R = p.kept_in.size[nk - 1];
                 const int64_t batch = nk > 1 ? p.kept_in.size[0] : 1;
                 const int64_t cgroups = (p.cols + 15) / 16;
@@ -718,8 +721,7 @@ NormPlan plan_normalize(const void* in_data, const void* out_data, const int64_t
                 p.wide_sum = p.shift || blocks_of(rgN) < 128;
                 if (rgN > 4 && blocks_of(rgN) < 192) rgN = 4;
                 if (rgN == 4 && blocks_of(rgN) < 128) rgN = 2;
-                const bool cheap_passes = n_norm_dims > 0 && elem_size >= 4 && p.cols > 2048 && blocks_of(rgN) < 32;
-                if (cgroups * 4 <= 1024 && !cheap_passes && (blocks_of(rgN) >= 128 || total >= 16384)) {
+                if (cgroups * 4 <= 1024 && (blocks_of(rgN) >= 128 || total >= 16384)) {
                     p.kind = NormKind::TransposedTile;
                     p.tpr = rgN;
                     const int64_t cols_per_wave = 16 * (64 / rgN);
@@ -1044,10 +1046,10 @@ NormPlan plan_normalize(const void* in_data, const void* out_data, const int64_t
             return false;
         };
         // A very narrow inner dim. The general forms leave lanes idle or walk an axis serially there, and take three
-        // launches below 4 MiB. us before -> slab: f32 [201, 1639, 4] 92 -> 6.5, bf16 [112, 4044, 8] 128 -> 11.0,
-        // f16 [112, 3904, 6] 43 -> 8.8, f32 [2048, 128, 2] 17.3 -> 4.0, bf16 [693, 488, 5] 14.4 -> 6.2, f32 [2511, 963, 8]
-        // 45 -> 34, bf16 [8, 4000, 4] 12.3 -> 7.0. Up to 64 KiB, and to the 128 KiB that fit a workgroup where the alternative
-        // is not the flat walk (f32 [32, 4096, 8] 38.8 -> 10.9).
+        // launches below 4 MiB. us before -> slab: f32 [201, 1639, 4] 92 -> 6.3, bf16 [112, 4044, 8] 128 -> 10.0,
+        // f16 [112, 3904, 6] 43 -> 8.6, f32 [2048, 128, 2] 17.3 -> 4.1, bf16 [693, 488, 5] 14.4 -> 6.0, f32 [2511, 963, 8]
+        // 45 -> 29.5, bf16 [8, 4000, 4] 12.3 -> 6.5. Up to 64 KiB, and to the 128 KiB that fit a workgroup where the alternative
+        // is not the flat walk (f32 [32, 4096, 8] 38.8 -> 9.2).
         const bool narrow = is_slab && sa <= 8 && p.cols >= 64 &&
                             slab_bytes <= (slabs * slab_bytes < (8ll << 20) ? (128 << 10) : (64 << 10)) && slab_fits();
         // Small groups laid back to back (a contiguous [batch, cols, L] tensor with cols * L elements of at
@@ -1061,7 +1063,8 @@ NormPlan plan_normalize(const void* in_data, const void* out_data, const int64_t
             p.cols * sa * (int64_t)elem_size <= 2048 && sa * (int64_t)elem_size < 512 && p.kept_in.size[0] >= 1024 &&
             p.rows * p.cols * (int64_t)elem_size >= (4ll << 20) && (((uintptr_t)in_data | (uintptr_t)out_data) & 15) == 0 &&
             // (a lane walks its column alone: the longer ones are better off with a wavefront per group, as slabs -
-            // us: bf16 [9408, 216, 4] 25.5 -> 12.3, [5986, 125, 3] 15.1 -> 8.3, f32 [13254, 87, 5] 18.0 -> 13.0)
+            // us: bf16 [5986, 125, 3] 15.1 -> 8.2, f32 [13254, 87, 5] 18.0 -> 13.1; with an inner dim that divides the vector
+            // as interleaved rows, below: bf16 [9408, 216, 4] 25.5 -> 9.7)
             !(narrow && (elem_size == 2 ? p.cols > 96 : elem_size == 4 && sa >= 3))) {
             int64_t groups = (16 << 10) / (p.cols * sa * (int64_t)elem_size);
             groups -= groups % max_vec;  // tiles start on 16-byte boundaries
@@ -1097,9 +1100,11 @@ NormPlan plan_normalize(const void* in_data, const void* out_data, const int64_t
                 // An inner dim of 3, 5, 6 or 7: the largest multiple of it of a row's lanes take part, so that all of a
                 // lane's vectors start at the same place modulo the inner dim; the lane keeps a (max, sum) per vector
                 // place and the places are rotated into softmaxes, folded, and rotated back.
-                // (Large inputs with an inner dim of 5, 6 or 7 are faster as slabs, us: f32 [4000, 512, 7] 29.3 -> 23.2,
-                // f16 [11264, 488, 6] 39.7 -> 31.2, [11008, 576, 5] 44.5 -> 30.2; with 3 there is no difference: f32
-                // [5592, 2000, 3] 48.9 and 49.2. Smaller ones stay, their plan is pinned.)
+                // (Inputs with an inner dim of 5, 6 or 7 are faster as slabs, us: f32 [4000, 512, 7] 29.3 -> 23.2,
+                // f16 [11264, 488, 6] 39.7 -> 25.2, [11008, 576, 5] 44.5 -> 25.3; with 3 there is no difference: f32
+                // [5592, 2000, 3] 48.9 and 49.2. The line at 40 MiB is not where the times cross: tests name the plan of smaller
+                // ones, f16 [700, 4000, 6] of 32 MiB the largest, and they are faster as slabs as well - that one 32.0 -> 19.4,
+                // f32 [2900, 512, 7] 24.2 -> 18.3, [300, 512, 7] 9.8 -> 5.7, f16 [4000, 576, 5] 19.9 -> 13.1.)
                 const int64_t act = q.tpr / sa * sa, nvr = p.cols * sa / max_vec;
                 const int64_t nc = (nvr + act - 1) / act;
                 const bool as_slab = narrow && sa >= 5 && slabs * slab_bytes >= (40ll << 20);

@@ -10,8 +10,8 @@ namespace hpt {
 // a workgroup's places meet in LDS, where groups of 2^g_log2 lanes share a column. One read and one write, whole
 // vectors, no per-element walk through LDS at stride L (which bounded the form before: three dependent loops over the
 // axis per column). Bound by latency up to a few MB - load, two folds, store - and by memory beyond.
-// us, softmax over C of [batch, C, L], staged slab -> now: bf16 [432, 2596, 8] 32 -> 15.2, bf16 [640, 3286, 6] 41 -> 22.7,
-// f32 [2240, 1408, 8] 80 -> 42.5 (4.75 TB/s), f32 [2688, 1931, 6] 85 -> 50.4 (4.95 TB/s), f32 [1024, 3692, 3] 36 -> 22.6.
+// us, softmax over C of [batch, C, L], staged slab -> now: bf16 [432, 2596, 8] 32 -> 14.4, bf16 [640, 3286, 6] 41 -> 19.5,
+// f32 [2240, 1408, 8] 80 -> 38.1 (5.3 TB/s), f32 [2688, 1931, 6] 85 -> 46.8 (5.3 TB/s), f32 [1024, 3692, 3] 36 -> 21.8.
 template <int KIND, class T, int NC>
 __global__ void __launch_bounds__(1024) norm_slab_kernel(const T* in, T* outp, int C, int L, int act, int g_log2) {
     static_assert(KIND == NORM_SOFTMAX || KIND == NORM_LOGSOFTMAX, "a softmax kernel");
