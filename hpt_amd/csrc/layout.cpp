@@ -694,52 +694,65 @@ NormPlan plan_normalize(const void* in_data, const void* out_data, const int64_t
                              ((uintptr_t)in_data % 16) == 0 && ((uintptr_t)out_data % 16) == 0;
         // (columns that overlap, of a view made by hand, keep the forms below)
         if (lies_transposed && (on_grid || sa >= p.kept_in.size[nk - 1])) {
-            p.vec = v;
-            p.shift = on_grid ? 0 : 1;
-            {
-                // Single pass when 16 vectors per thread hold (16 * rgN bytes of rows) x (all
-                // columns): rgN lanes along the rows, 1024 / rgN thread columns of 16 columns
-                // each, 4096 columns at most. Long row segments where they leave enough workgroups; a
-                // matrix too small for that is cut into segments of 64 and 32 bytes, which still beats three launches
-                // by far (device us, three passes -> one; rows x columns): f32 3200 x 224 softmax 21.5 -> 5.6, layernorm
-                // 12.6 -> 4.9; f16 5184 x 2048 24.7 -> 17.2, 21 -> 16.0; f32 300 x 1001 18.6 -> 7.5; bf16 511 x 2001
-                // 22 -> 12.6; f32 200 x 3300 layernorm 14.2 -> 10.8 and, where the few workgroups have most columns to
-                // walk, 129 x 4000 14.0 (and two gaps between launches) -> 14.6. Beyond 4096 columns 32-byte segments gain
-                // nothing (f16 2048 x 8192 28.0 -> 26.3, f32 333 x 8000 layernorm 17 -> 25): three passes. Matrices below 16384
-                // elements keep three passes only because tests name that plan; in time they lose as well
-                // (f32 64 x 100 softmax 13.8 -> 4.8, f16 100 x 120 18.8 -> 5.2).
-                const int64_t R = p.kept_in.size[nk - 1];
-                const int64_t batch = nk > 1 ? p.kept_in.size[0] : 1;
-                const int64_t cgroups = (p.cols + 15) / 16;
-                auto blocks_of = [&](int rg) { return (R + rg * v - 1) / (rg * v) * batch; };
-                int rgN = 16;
-                while (rgN >= 4 && cgroups * rgN > 1024) rgN >>= 1;
-                if (rgN > 8 && blocks_of(rgN) < 256) rgN = 8;
-                // Sums of exponentials of f32 rows: f64, but for matrices on the vector grid that fill the chip with long
-                // segments, where a thread's 16 of a row are added in f32 and the conversions would show (f32
-                // 6080 x 2752 38.3 -> 39.6 us).
-                p.wide_sum = p.shift || blocks_of(rgN) < 128;
-                if (rgN > 4 && blocks_of(rgN) < 192) rgN = 4;
-                if (rgN == 4 && blocks_of(rgN) < 128) rgN = 2;
-                if (cgroups * 4 <= 1024 && (blocks_of(rgN) >= 128 || total >= 16384)) {
+            // Single pass when 16 vectors per thread hold (16 * rgN bytes of rows) x (all
+            // columns): rgN lanes along the rows, 1024 / rgN thread columns of 16 columns
+            // each, 4096 columns at most. Long row segments where they leave enough workgroups; a
+            // matrix too small for that is cut into segments of 64 and 32 bytes, which still beats three launches
+            // by far (device us, three passes -> one; rows x columns): f32 3200 x 224 softmax 21.5 -> 5.6, layernorm
+            // 12.6 -> 4.9; f16 5184 x 2048 24.7 -> 17.2, 21 -> 16.0; f32 300 x 1001 18.6 -> 7.5; bf16 511 x 2001
+            // 22 -> 12.6; f32 200 x 3300 layernorm 14.2 -> 10.8 and, where the few workgroups have most columns to
+            // walk, 129 x 4000 14.0 (and two gaps between launches) -> 14.6. Beyond 4096 columns 32-byte segments gain
+            // nothing (f16 2048 x 8192 28.0 -> 26.3, f32 333 x 8000 layernorm 17 -> 25): three passes. Matrices on the grid
+            // below 16384 elements keep three passes only because tests name that plan; in time they lose as well
+            // (f32 64 x 100 softmax 13.8 -> 4.8).
+            const int64_t R = p.kept_in.size[nk - 1];
+            const int64_t batch = nk > 1 ? p.kept_in.size[0] : 1;
+            const int64_t cgroups = (p.cols + 15) / 16;
+            auto blocks_of = [&](int rg) { return (R + rg * v - 1) / (rg * v) * batch; };
+            int rgN = 16;
+            while (rgN >= 4 && cgroups * rgN > 1024) rgN >>= 1;
+            if (rgN > 8 && blocks_of(rgN) < 256) rgN = 8;
+            // Sums of exponentials of f32 rows: f64, but for matrices on the vector grid that fill the chip with long
+            // segments, where a thread's 16 of a row are added in f32 and the conversions would show (f32
+            // 6080 x 2752 38.3 -> 39.6 us).
+            const bool wide_sum = !on_grid || blocks_of(rgN) < 128;
+            if (rgN > 4 && blocks_of(rgN) < 192) rgN = 4;
+            if (rgN == 4 && blocks_of(rgN) < 128) rgN = 2;
+            const bool tile = cgroups * 4 <= 1024 && (!on_grid || blocks_of(rgN) >= 128 || total >= 16384);
+            // Few rows off the grid: a group of lanes per row (the general form) reads single elements at a stride, but has
+            // every row in a workgroup of its own at once. It is ahead of few tiles of two-byte rows beyond 256 columns, whose 16
+            // rows share a workgroup (device us, lanes and tile: bf16 85 x 3255 softmax 10.1 and 15.6, 207 x 1238 7.4 and 9.6, 107 x
+            // 288 5.6 and 7.5, f16 138 x 3583 12.5 and 15.0; layernorm bf16 183 x 1189 8.0 and 9.6, f16 goes either way, 137 x 579 6.5
+            // and 7.0, 176 x 1854 9.7 and 7.7; 24 tiles and more gain mostly: f16 478 x 339 7.1 and 6.6, bf16 504 x 1201 11.2 and 8.7,
+            // but 492 x 288 softmax 6.3 and 7.6; wider types always: f32 163 x 1691 10.2 and 9.9, f64 493 x 16 6.2 and 5.0), and of three
+            // launches for few and not too long rows (f32 83 x 5029 softmax 16.2 and 20.9, 40 x 6207 17.2 and 20.0, 35 x 15104
+            // 30.8 and 26.2; layernorm 51 x 4736 15.3 and 14.8, 96 x 7241 19.8 and 16.7; two-byte 113 x 4181 layernorm 13.8 and 20.3,
+            // 122 x 12359 28.0 and 22.2, softmax 88 x 9461 21.2 and 24.1, 90 x 13253 27.6 and 27.4; f64 18 x 5625 17.4 and 15.0). From
+            // 129 to about 256 rows the lanes are still ahead (f32 146 x 5018 17.1 and 22.1, 207 x 6398 22.7 and 23.4), but tests
+            // name the three passes there.
+            const int64_t longest = (n_norm_dims > 0 ? 4608 : 6656) * (elem_size == 2 ? 3 : 2) / 2;
+            const bool lanes = !on_grid && elem_size <= 4 && (tile ? elem_size == 2 && p.cols > 256 && blocks_of(rgN) < 24 : p.rows <= 128 && p.cols < longest);
+            if (!lanes) {
+                p.vec = v;
+                p.shift = on_grid ? 0 : 1;
+                if (tile) {
                     p.kind = NormKind::TransposedTile;
+                    p.wide_sum = wide_sum;
                     p.tpr = rgN;
                     const int64_t cols_per_wave = 16 * (64 / rgN);
                     p.rpb = (int)((p.cols + cols_per_wave - 1) / cols_per_wave);
                     return p;
                 }
+                p.kind = NormKind::Transposed;
+                // statistics pass: a wavefront covers 64*v rows; enough column splits for
+                // about 2048 wavefronts, each keeping at least 32 columns
+                const int64_t groups = (R + 64 * v - 1) / (64 * v) * batch;
+                int64_t S = std::max<int64_t>(1, std::min<int64_t>(512 / groups, p.cols / 128));
+                p.tsplit = (int)std::min<int64_t>(S, 64);
+                p.tpr = 4;  // wavefronts per workgroup of the statistics pass
+                p.scratch_bytes = (size_t)p.rows * p.tsplit * 16 + (size_t)p.rows * 3 * 8;
+                return p;
             }
-            p.kind = NormKind::Transposed;
-            // statistics pass: a wavefront covers 64*v rows; enough column splits for
-            // about 2048 wavefronts, each keeping at least 32 columns
-            const int64_t R = p.kept_in.size[nk - 1];
-            const int64_t batch = nk > 1 ? p.kept_in.size[0] : 1;
-            const int64_t groups = (R + 64 * v - 1) / (64 * v) * batch;
-            int64_t S = std::max<int64_t>(1, std::min<int64_t>(512 / groups, p.cols / 128));
-            p.tsplit = (int)std::min<int64_t>(S, 64);
-            p.tpr = 4;  // wavefronts per workgroup of the statistics pass
-            p.scratch_bytes = (size_t)p.rows * p.tsplit * 16 + (size_t)p.rows * 3 * 8;
-            return p;
         }
         if (sa >= 1 && sa <= 4) {
             // vector width: input and output must both allow it
