@@ -391,37 +391,68 @@ ReducePlan plan_reduce(const void* data, const int64_t* shape, const int64_t* st
         // backwards, so a row holds one at least (kin >= full).
         // (Worth it when a row is a few wavefronts of such lanes and enough is reduced into each output
         // that the lane's outputs, which it then writes one by one, are a small part of the traffic.)
-        // (Small inputs, whose time is the chain of loads of one lane, gain from two lanes per row on: their column
-        // blocks are narrow, below. Under 16 KiB a lane has a dozen loads in all either way: f32 [100, 33] 4.3 us in both forms,
-        // f16 [200, 33] 4.5 and 4.9.)
         const int64_t bytes = p.K * p.R * (int64_t)elem_size;
         const bool small = p.lean && bytes < kSmallColBytes;
-        if (p.lean && nk && p.vec == 1 && p.sstride == 1 && full > 1 && p.kept.stride[nk - 1] == 1 &&
-            (small ? kin >= 2 * full && p.R >= 64 && bytes >= (16 << 10) : kin >= 256 && p.R >= 256) && (uintptr_t)data % elem_size == 0) {
-            p.unaligned = true;
-            p.vec = full;
-        }
-        int64_t kv = ((p.lean ? kin : p.K) + (p.unaligned ? full - 1 : 0)) / (p.vec / p.sstride);  // vector columns the lanes spread over
-        p.bx = (int)std::min<int64_t>(64, pow2_ceil(kv));
-        // A row of vector columns that is not a whole number of wavefronts (96: hidden size 768 in two-byte
-        // elements) would leave the last wavefront of every row partly idle: narrower column blocks
-        // (32 or 16 lanes, two or four reduced positions per wavefront) that divide it better.
-        // Over axis 1, TB/s: f16 [128, 512, 1280] 4.7 -> 6.1, [512, 197, 768] 5.0 -> 5.7, f32 [256, 512, 320] 5.0 -> 6.2.
-        if (kv > 64) {
-            auto waste = [&](int64_t b) { return (kv + b - 1) / b * b - kv; };
-            for (int b = 32; b >= 16; b >>= 1)
-                if (waste(p.bx) * 8 > kv && waste(b) < waste(p.bx)) p.bx = b;
-        }
-        int64_t xblocks = (kv + p.bx - 1) / p.bx * (p.lean ? outer : 1);
+        const bool ua_ok = p.lean && nk && p.vec == 1 && p.sstride == 1 && full > 1 && p.kept.stride[nk - 1] == 1 && (uintptr_t)data % elem_size == 0;
+        int64_t kv = 0, xblocks = 0;  // vector columns the lanes spread over, column blocks
+        auto columns = [&](bool ua) {
+            p.unaligned = ua;
+            if (ua) p.vec = full;
+            kv = ((p.lean ? kin : p.K) + (ua ? full - 1 : 0)) / (p.vec / p.sstride);
+            p.bx = (int)std::min<int64_t>(64, pow2_ceil(kv));
+            // A row of vector columns that is not a whole number of wavefronts (96: hidden size 768 in two-byte
+            // elements) would leave the last wavefront of every row partly idle: narrower column blocks
+            // (32 or 16 lanes, two or four reduced positions per wavefront) that divide it better.
+            // Over axis 1, TB/s: f16 [128, 512, 1280] 4.7 -> 6.1, [512, 197, 768] 5.0 -> 5.7, f32 [256, 512, 320] 5.0 -> 6.2.
+            if (kv > 64) {
+                auto waste = [&](int64_t b) { return (kv + b - 1) / b * b - kv; };
+                for (int b = 32; b >= 16; b >>= 1)
+                    if (waste(p.bx) * 8 > kv && waste(b) < waste(p.bx)) p.bx = b;
+            }
+            xblocks = (kv + p.bx - 1) / p.bx * (p.lean ? outer : 1);
+        };
+        // One wavefront per 64 vector columns streams best when there are enough
+        // columns (measured: 832 wavefronts with 128 loads each reach 5.9 TB/s);
+        // with fewer, thread rows and then workgroups split the reduced range:
+        // r-partitions so that about 768 wavefronts run, each with >= 16 loads.
+        const int64_t kWavesWanted = 768;
+        auto need_of = [&]() { return (kWavesWanted + xblocks - 1) / xblocks; };
+        const int64_t can = std::max<int64_t>(1, p.R / 16);
+        // One launch, thread rows meet in LDS: a workgroup is at least one wavefront.
+        auto rows_in_one_launch = [&]() {
+            const int64_t base = 64 / p.bx, rp = std::min(need_of(), can);
+            if (rp <= 1) return base;
+            int64_t by = std::min<int64_t>(pow2_ceil(rp), 1024 / p.bx / base) * base;
+            while (by > base && (size_t)p.bx * by * (p.vec / p.sstride) * acc_size > (64u << 10)) by /= 2;
+            return by;
+        };
+        columns(ua_ok && kin >= 256 && p.R >= 256);
         if (small) {
             // Below 8 MiB the time is the chain of dependent batches of loads of one lane, and the compute units that
             // stand idle: 16-lane column blocks (256-byte segments of each row) make more workgroups of them, and up
             // to 1024 threads share a block's rows. Where that still leaves a lane more than 24 rows (three batches of
-            // eight loads; a second launch costs as much: f32 [1216, 225], 19 rows, 6.4 us in one launch, 7.3 in two, in cache),
+            // eight loads; a second launch costs as much: f32 [1216, 225], 19 rows, 6.4 us in one launch, 7.3 in two, in cache;
+            // 48 single elements, [7482, 3] 5.3 and 7.1, [10304, 4] 5.8 and 7.2),
             // the rows are dealt over workgroups too, about 12 to a lane. Over axis 0, us before -> now:
             // f32 [12608, 128] 109 -> 8.3 (in one launch 33.9), f16 [2315, 363] 197 -> 8.8 (16.1), f32 [5440, 45] 28.3 -> 7.3
-            // (15.5), f32 [1578, 2101][:, ::2], 25 rows per lane, 17.6 -> 11.1 (12.1), bf16 [34112, 40] 57 -> 8.2. (Device time
-            // of both launches.)
+            // (15.5), bf16 [34112, 40] 57 -> 8.2. (Device time of both launches.)
+            // Where the plan above already leaves a lane few rows with less than 1024 threads to fold, the narrower blocks
+            // only add to the fold: it stays from 4 (fewer mean more threads than the rows need) to 12 rows of vectors or 20 of
+            // single elements per lane, and single elements become unaligned vectors, from two lanes per row on, beyond 24
+            // (us, as was and in narrow blocks: f64 [9, 3008] 2.7 and 3.6, i32 [33, 118] 2.3 and 3.5, u8 [136, 3096] 3.8 and 5.8, f32
+            // [960, 199] 5.4 and 7.0; but f32 [676, 120], 21 rows, 9.8 and 7.6, [176, 4992], 11 rows by 1024 threads, 6.8 and
+            // 5.7, i32 [187, 8], one row, 3.7 and 2.6).
+            if (!p.unaligned) {
+                const int64_t by = rows_in_one_launch(), rows = (p.R + by - 1) / by;
+                if (ua_ok && kin >= 2 * full && p.R >= 64 && rows > 24) {
+                    columns(true);
+                } else if (p.bx * by < 1024 && rows >= 4 && rows <= (p.vec > 1 ? 12 : 20)) {
+                    p.by = (int)by;
+                    p.split = 1;
+                    p.chunk = p.R;
+                    return p;
+                }
+            }
             while (p.bx > 16 && xblocks < kComputeUnits && p.R >= 32) {
                 p.bx /= 2;
                 xblocks = (kv + p.bx - 1) / p.bx * outer;
@@ -433,7 +464,7 @@ ReducePlan plan_reduce(const void* data, const int64_t* shape, const int64_t* st
             while (by > rows_per_wave && (size_t)p.bx * by * uv * acc_size > (64u << 10)) by /= 2;
             p.by = (int)by;
             p.split = 1;
-            if ((p.R + by - 1) / by > 24 && spare_scratch) {
+            if ((p.R + by - 1) / by > (p.vec > 1 ? 24 : 48) && spare_scratch) {
                 // workgroups of 256 threads: the more rows share a workgroup, the longer its fold through LDS
                 const int64_t sby = std::min<int64_t>(by, std::max(rows_per_wave, 256 / p.bx));
                 const int64_t cap = (int64_t)(kSmallColScratch / acc_size) / p.K;
@@ -447,18 +478,11 @@ ReducePlan plan_reduce(const void* data, const int64_t* shape, const int64_t* st
             p.chunk = (p.R + p.split - 1) / p.split;
             return p;
         }
-        // One wavefront per 64 vector columns streams best when there are enough
-        // columns (measured: 832 wavefronts with 128 loads each reach 5.9 TB/s);
-        // with fewer, thread rows and then workgroups split the reduced range.
         const int base_by = 64 / p.bx;  // a workgroup is at least one wavefront
-        const int64_t kWavesWanted = 768;
         const int uv = p.vec / p.sstride;
         p.by = base_by;
         p.split = 1;
-        // r-partitions wanted so that about 768 wavefronts run, each with >= 16 loads
-        const int64_t need = (kWavesWanted + xblocks - 1) / xblocks;
-        const int64_t can = std::max<int64_t>(1, p.R / 16);
-        const int64_t rp = std::min(need, can);
+        const int64_t need = need_of(), rp = std::min(need, can);
         if (rp > 1) {
             if (bytes >= kSmallColBytes) {
                 // Large input: partition over WORKGROUPS first, so that the partitions land
@@ -491,10 +515,7 @@ ReducePlan plan_reduce(const void* data, const int64_t* shape, const int64_t* st
                     p.by = (int)by * base_by;
                 }
             } else {
-                // Small input: one launch, thread rows meet in LDS
-                int64_t by = std::min<int64_t>(pow2_ceil(rp), 1024 / p.bx / base_by) * base_by;
-                while (by > base_by && (size_t)p.bx * by * uv * acc_size > (64u << 10)) by /= 2;
-                p.by = (int)by;
+                p.by = (int)rows_in_one_launch();
             }
         }
         // Workgroups of several wavefronts each live as long as the launch does, one (or two ...) per
