@@ -31,6 +31,23 @@ def test_softmax_over_odd_columns_in_place(hpt, dev, dtype, shape, log):
     assert np.array_equal(t.numpy(), want), plan
 
 
+# the other forms with unaligned vectors: slabs in one workgroup's registers, register columns, the flat walk
+MIDDLE = [("col-slab", (201, 1639, 5)), ("col-slab", (3, 4095, 7)), ("col-reg-unaligned", (16, 128, 3249)), ("col-split-flat-unaligned", (9, 2501, 1001))]
+
+
+@pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("plan,shape", MIDDLE, ids=lambda v: v if isinstance(v, str) else "x".join(map(str, v)))
+def test_softmax_over_the_middle_axis_in_place(hpt, dev, dtype, plan, shape):
+    a, dt = _values(hpt, shape, dtype)
+    for log in (False, True):
+        t = hpt.Tensor.from_numpy(a, dt).to_hip(dev)
+        assert hpt.normalize_plan(t, 1).startswith(plan), hpt.normalize_plan(t, 1)
+        run = t.log_softmax if log else t.softmax
+        want = run(1).numpy()
+        run(1, out=t)
+        assert np.array_equal(t.numpy(), want), log
+
+
 @pytest.mark.parametrize("dtype", ["f32", "f16", "f64"])
 @pytest.mark.parametrize("shape", [(1, 1 << 22), (5, 1 << 20), (4, 300007), (100, 65539)], ids=lambda v: "x".join(map(str, v)))
 def test_layernorm_of_shared_rows_in_place(hpt, dev, dtype, shape):
