@@ -620,6 +620,23 @@ static bool lds_row_shape(NormPlan& p, int64_t nvec, size_t elem_size, bool shif
     return true;
 }
 
+// Slices of the axis for `groups` column groups: the count that fills one, two, three or four rounds of compute units to nine
+// tenths, or the one that comes closest.
+static int64_t stats_split(int64_t groups) {
+    int64_t best = 1;
+    double best_fill = 0;
+    for (int64_t r = 1; r <= 4; ++r) {
+        const int64_t S = r * kComputeUnits / groups;
+        const double fill = (double)(S * groups) / (double)(r * kComputeUnits);
+        if (S >= 1 && fill > best_fill) {
+            best = S;
+            best_fill = fill;
+        }
+        if (fill >= 0.9) break;
+    }
+    return best;
+}
+
 NormPlan plan_normalize(const void* in_data, const void* out_data, const int64_t* shape,
                         const int64_t* strides, int ndim, int64_t axis, int n_norm_dims,
                         size_t elem_size, bool fused) {
@@ -1232,7 +1249,19 @@ NormPlan plan_normalize(const void* in_data, const void* out_data, const int64_t
             p.vec = v;
             // A narrow inner dim (or one that is not whole vectors) leaves most lanes idle: walk the
             // contiguous [cols, L] slab as a flat array of aligned vectors instead.
-            if (max_vec > 1 && (!vec_ok || L <= 1024 * max_vec) && sa == L && ((uintptr_t)in_data % elem_size) == 0 &&
+            // (Lanes along the inner dim, below, once it is some wavefronts of vectors: one read of the statistics pass deep in
+            // flight and stores in address order beat the flat walk's one large workgroup per compute unit. Softmax over axis 0,
+            // us, flat and below: f32 128 MiB, inner 1280 75.3 and 71.0, 2048 73.4 and 65.8, 3000 82.3 and 75.1, 1001 81.3 and 77.7; 32 MiB,
+            // 512 25.5 and 24.3, 1000 28.3 and 25.3, 2000 29.5 and 23.4, 384 27.1 and 28.4; two-byte 64 MiB, 384 43.5 and 41.9, 600 (a second
+            // wavefront that is nearly empty) 48.3 and 50.9, 1024 42.3 and 37.5, 3000 50.8 and 41.2, 1001 48.8 and 43.0; 24 MiB, 320 29.6 and
+            // 23.4, 600 28.6 and 25.3, 257 27.7 and 37.8. From 64 MiB on f32 of 512 ... 1024 goes either way (512 72.6 and 69.2, 704 75.0 and 74.3, 1000
+            // 74.2 and 75.7, 1024 72.6 and 67.8), and tests name the flat walk there and for odd slabs of 1001.)
+            const int64_t all_bytes = batch * p.cols * L * (int64_t)elem_size;
+            const int64_t lanes = L / max_vec;
+            bool wide = vec_ok && L > 1024 * max_vec;
+            if (elem_size == 4) wide = vec_ok ? L > 1024 || (L >= 512 && all_bytes < (64ll << 20)) : L >= 768 && batch == 1;
+            else if (elem_size == 2) wide = vec_ok ? L >= 320 && (all_bytes < (48ll << 20) || lanes * 3 >= (lanes + 63) / 64 * 64 * 2) : L >= 768 && batch == 1;
+            if (max_vec > 1 && !wide && sa == L && ((uintptr_t)in_data % elem_size) == 0 &&
                 ((uintptr_t)out_data % elem_size) == 0 && batch * p.cols * L * (int64_t)elem_size >= (8ll << 20)) {
                 // (slabs that start off 16-byte boundaries take the same vectors unaligned: `shift`)
                 const bool aligned = ((uintptr_t)in_data % 16) == 0 && ((uintptr_t)out_data % 16) == 0 &&
@@ -1264,10 +1293,13 @@ NormPlan plan_normalize(const void* in_data, const void* out_data, const int64_t
                 p.vec = v;
                 p.shift = 1;
             }
+            // One workgroup per compute unit for the statistics pass (its loads are in flight two batches deep), or the
+            // few rounds of them that leave the fewest units idle.
             const int64_t groups = (L + 64 * v - 1) / (64 * v) * batch;
-            int64_t S = std::max<int64_t>(1, std::min<int64_t>(512 / groups, p.cols / 32));
-            p.tsplit = (int)std::min<int64_t>(S, 64);
-            p.tpr = 4;  // wavefronts per workgroup of the statistics pass
+            p.tsplit = (int)std::min(stats_split(groups), std::max<int64_t>(1, p.cols / 32));
+            // (beyond 64 partials per row the finalize pass grows: 64 columns each then, f32 [4100, 63] 11.7 -> 10.6 us)
+            if (p.tsplit > 64) p.tsplit = (int)std::max<int64_t>(64, std::min<int64_t>(p.tsplit, p.cols / 64));
+            p.tpr = elem_size == 2 && v > 1 && p.cols >= 128 * p.tsplit ? 8 : 4;  // wavefronts per workgroup of the statistics pass
             p.scratch_bytes = (size_t)p.rows * p.tsplit * 16 + (size_t)p.rows * 3 * 8;
             return p;
         }

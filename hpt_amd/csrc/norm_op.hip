@@ -111,10 +111,10 @@ template <class T, int VEC> void launch_col_split(const NormPlan& p, const NormA
         transposed_stats_kernel<KIND, T, VEC>
             <<<dim3(rg, (unsigned)t.S, batch), dim3(64 * nw), (size_t)nw * VEC * 64 * sizeof(Part), st>>>(t);
     transposed_finalize_kernel<KIND, T><<<dim3((unsigned)((t.R + 15) / 16), 1, batch), dim3(16, 16), 0, st>>>(t);
-    // apply: enough axis chunks for ~2048 workgroups, at least 16 positions each
-    int64_t want = (2048 + (int64_t)rg * batch - 1) / ((int64_t)rg * batch);
-    int64_t chunks = std::max<int64_t>(1, std::min<int64_t>(want, (t.cols + 15) / 16));
-    chunks = std::min<int64_t>(chunks, 65535);
+    // apply: sixteen positions of the axis per workgroup, one batch of four loads per thread; what runs at one time is then
+    // one stretch of memory (f32 [8192, 4096] over axis 0, all three passes, 16 / 32 / 48 positions: 65.2, 70.7, 67.4 us;
+    // [32768, 1024] 66.3, 68.4, 68.6; f16 [8190, 4097] 42.0, 43.1, 43.1)
+    int64_t chunks = std::min<int64_t>((t.cols + 15) / 16, 65535);
     const int chunk = (int)((t.cols + chunks - 1) / chunks);
     chunks = (t.cols + chunk - 1) / chunk;
     if constexpr (VEC > 1) {

@@ -95,7 +95,7 @@ __global__ void __launch_bounds__(1024) transposed_stats_kernel(const Transposed
     // lanes past the last row keep going (they meet the others at the barrier below) on row 0
     const bool valid = (blockIdx.x * 64 + lane) * VEC < a.R;
     const int r0 = valid ? (UA ? min((int)(blockIdx.x * 64 + lane) * VEC, a.R - VEC) : (int)(blockIdx.x * 64 + lane) * VEC) : 0;
-    // Columns are dealt out round-robin over all P = 4 S wavefronts that share these
+    // Columns are dealt out round-robin over all P = S NW wavefronts that share these
     // rows: wavefront p takes columns p, p + P, ... Wavefronts running at the same time
     // then read neighbouring columns, which keeps a power-of-two column pitch from
     // sending them all to the same memory channels.
@@ -184,17 +184,48 @@ __global__ void __launch_bounds__(1024) transposed_stats_kernel(const Transposed
             }
         }
     };
+    // Batches of kBatch columns, two alternating: the next one is on its way while this one is folded. A wavefront alone
+    // on its SIMD is enough then, and the fewer wavefronts read side by side the better the rows of memory they open are
+    // used (softmax over axis 0, this pass alone, us: f32 [8190, 4097] two workgroups per compute unit without the second
+    // batch 32.1, one 36.1, with it 32.1 and 26.1; [32768, 1024] 33.4 -> 23.3. Two-byte elements, twice the arithmetic
+    // per byte, take shorter batches and twice the wavefronts: f16 [8190, 4097] 19.4 -> 15.4).
+    // (The last round's loads are repeated, not left out: behind a test the wait before the fold would be a full one.)
+    constexpr int kBatch = KIND != NORM_LAYERNORM && sizeof(T) == 2 ? 4 : 8;
     const int64_t stepb = (int64_t)P * a.sa;
     const T* p = base + (int64_t)pid * a.sa;
     int c = pid;
-    for (; c + 7 * P < a.cols; c += 8 * P) {  // eight columns in flight per lane
-        Pack<T, VEC> v[8];
+    auto load_batch = [&](Pack<T, VEC>(&v)[kBatch], const T* q) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) v[i] = UA ? load_pack_unaligned<T, VEC>(p + i * stepb) : load_pack<T, VEC>(p + i * stepb);
-        p += 8 * stepb;
-        // keep the scheduler from sinking loads into the arithmetic: all eight stay in flight
+        for (int i = 0; i < kBatch; ++i) v[i] = UA ? load_pack_unaligned<T, VEC>(q + i * stepb) : load_pack<T, VEC>(q + i * stepb);
+        // keep the scheduler from sinking loads into the arithmetic
         __builtin_amdgcn_sched_barrier(0);
-        fold(v, std::integral_constant<int, 8>{});
+    };
+    if (c + (kBatch - 1) * P < a.cols) {
+        Pack<T, VEC> va[kBatch], vb[kBatch];
+        load_batch(va, p);
+        // folds `now` while `next` comes in; false after the last whole batch
+        auto step = [&](Pack<T, VEC>(&now)[kBatch], Pack<T, VEC>(&next)[kBatch]) {
+            const bool more = c + (2 * kBatch - 1) * P < a.cols;
+            load_batch(next, more ? p + kBatch * stepb : p);
+            fold(now, std::integral_constant<int, kBatch>{});
+            __builtin_amdgcn_sched_barrier(0);
+            p += kBatch * stepb;
+            c += kBatch * P;
+            return more;
+        };
+        while (step(va, vb) && step(vb, va)) {
+        }
+    }
+    // the rest: four together, then one at a time
+    if constexpr (kBatch > 4) {
+        if (c + 3 * P < a.cols) {
+            Pack<T, VEC> v[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] = UA ? load_pack_unaligned<T, VEC>(p + i * stepb) : load_pack<T, VEC>(p + i * stepb);
+            p += 4 * stepb;
+            c += 4 * P;
+            fold(v, std::integral_constant<int, 4>{});
+        }
     }
     for (; c < a.cols; c += P) {
         Pack<T, VEC> v = UA ? load_pack_unaligned<T, VEC>(p) : load_pack<T, VEC>(p);
@@ -415,7 +446,9 @@ __global__ void __launch_bounds__(256) col_apply_kernel(const TransposedArgs a, 
     const Pack<CT, VEC> p1 = UA ? load_pack_unaligned<CT, VEC>(pp + a.R) : *reinterpret_cast<const Pack<CT, VEC>*>(pp + a.R);
     const T* in = (const T*)a.in + (int64_t)blockIdx.z * a.bi + r0;
     T* out = (T*)a.out + (int64_t)blockIdx.z * a.cols * a.R + r0;
-    const int c_end = min(a.cols, (int)(blockIdx.y + 1) * chunk);
+    // (the axis from its end backwards: what the statistics pass read last is read first)
+    const int block = gridDim.y - 1 - blockIdx.y;
+    const int c_end = min(a.cols, (block + 1) * chunk);
     auto fetch = [&](int c) {
         if constexpr (UA) return load_pack_unaligned<T, VEC>(in + (int64_t)c * a.sa);
         else return load_pack<T, VEC>(in + (int64_t)c * a.sa);
@@ -441,7 +474,7 @@ __global__ void __launch_bounds__(256) col_apply_kernel(const TransposedArgs a, 
             else if constexpr (VEC > 1) store_pack_stream<T, VEC>(dst, o);
             else dst[0] = o.v[0];
         };
-        int c = blockIdx.y * chunk + ty;
+        int c = block * chunk + ty;
         for (; c + 12 < c_end; c += 16) {  // four positions in flight per thread (thread rows are 4 apart)
             Pack<T, VEC> v[4];
 #pragma unroll
