@@ -251,7 +251,9 @@ __global__ void __launch_bounds__(1024) row_reg_kernel(const NormArgs a) {
     // Rows that take 512 or 1024 threads leave room for one or two workgroups per compute unit, so
     // nothing else hides a row's load -> reduce -> reduce -> store chain: there (PF) the prefetch
     // pays for every type (f32 [3355, 10000] softmax: 3.2 TB/s without).
-    constexpr bool kPrefetch = ((sizeof(T) == 2 && NCHUNK * UV <= ((kSoft || GB) ? 32 : 16)) || PF) && !kRes;
+    // (layernorm(x + residual) holds the residual's vectors as well: with gamma / beta in LDS there is room, and the two reads
+    // per write wait less - f16 [13107, 5120] 86.6 -> 75.7 us, [8192, 4096] 41.4 -> 35.4, [32768, 1024] 38.6 -> 34.3, [10000, 8192] 91.7 -> 83.5)
+    constexpr bool kPrefetch = ((sizeof(T) == 2 && NCHUNK * UV <= ((kSoft || GB) ? 32 : 16)) || PF) && (!kRes || GBL);
     const int64_t row_step = (int64_t)gridDim.x * a.rpb;
     Pack<T, VEC> raw[NCHUNK];
     Pack<T, UV> raw_res[kRes ? NCHUNK : 1];
