@@ -637,6 +637,57 @@ static int64_t stats_split(int64_t groups) {
     return best;
 }
 
+// Softmax over an axis of up to 1024 elements with a contiguous inner dim of L: whether 512 or 1024 threads that hold it in whole
+// vectors (col_tall_kernel) are ahead of the plan `p` (`found`: register columns of 256 threads, else three launches), and
+// that plan in `p` if so. Us over axis 1, as it was and this:
+//   four bytes, 129 ... 256 elements  [64, 129, 256] 9.8 and 6.8, [6, 200, 8200] 21.2 and 17.4, [20, 129, 8001] 48.8 and 34.2; where inner rows
+//     are whole 512-byte segments the 128-register form stays ([256, 256, 256] 20.4 and 22.2, though [16, 256, 2048] 18.0 and 15.2)
+//   257 ... 512  [1, 335, 58050] 88.6 and 45.2, [200, 335, 100] 29.0 and 19.6, [6, 512, 8200] 75.6 and 51.6, [16, 512, 1001] 22.4 and 23.3; where inner
+//     rows are whole 256-byte segments the 128-register form stays below 128 MiB and for very long rows ([16, 512, 2048] 25.3 and
+//     29.5, [1, 512, 262144] 212 and 215; [512, 512, 512] 210 and 190, [64, 512, 1024] 53.2 and 50.1)
+//   513 ... 1024  [64, 777, 256] 28.3 and 21.5, [16, 1024, 2048] 92.2 and 53.4; one workgroup fills a compute unit, so there must be enough of
+//     them, of rows that are not short: [4, 1000, 1000] 16.8 and 18.9, [200, 1000, 100] 66.2 and 72.2
+//   two bytes, 65 ... 512  [64, 100, 256] 10.1 and 5.7, [16, 100, 1001] 13.4 and 6.4, [100, 335, 500] 35.7 and 23.9, [512, 512, 512] 128 and 105;
+//     [64, 256, 2048] 26.0 and 29.6, [100, 256, 1024] 26.1 and 25.1
+//   513 ... 1024  [512, 513, 24] 21.2 and 15.1, [64, 1000, 256] 28.4 and 22.1, [16, 1000, 2048] 38.1 and 28.4; [4, 777, 1000] 13.4 and 19.1, [1, 513, 58050]
+//     (three passes, odd rows) 38.5 and 42.6
+//   three launches for too few positions, any of these  [8, 129, 64] 10.7 and 5.5, two bytes [4, 65, 1000] 10.9 and 5.1, [1, 300, 200] 10.9 and 9.1
+static bool tall_columns(NormPlan& p, bool found, const void* in_data, const void* out_data, int64_t sa, int64_t sb, int64_t L, int64_t batch,
+                         size_t elem_size) {
+    const int64_t vec = 16 / (int64_t)elem_size;
+    if ((elem_size != 2 && elem_size != 4) || L < vec || (((uintptr_t)in_data | (uintptr_t)out_data) % elem_size) != 0) return false;
+    const bool grid = L % vec == 0 && sa % vec == 0 && sb % vec == 0 && (((uintptr_t)in_data | (uintptr_t)out_data) & 15) == 0;
+    int64_t threads = 1024, tx = 16, nc = 8;
+    if (elem_size == 4) {
+        tx = p.cols <= 256 ? 32 : 16;
+        nc = p.cols <= 512 ? 8 : 16;
+    } else {
+        threads = p.cols <= 512 ? 512 : 1024;
+        nc = p.cols <= 256 ? 8 : 16;
+    }
+    const int64_t blocks = (batch * ((L + vec - 1) / vec) + tx - 1) / tx;
+    if (blocks * threads >= (1ll << 32)) return false;  // work-items of one launch
+    const bool whole_segments = found && p.vec == 4 && p.nchunk == 32 && elem_size == 4;  // the 128-register form
+    if (p.cols > 512) {
+        if (elem_size == 4 ? (blocks < 192 || L < 256) : (blocks < 96 || (!grid && batch == 1))) return false;
+    } else if (!found) {
+        // (odd inner rows of a wavefront of vectors and more: tests name the three passes)
+        if (p.cols > 256 && !grid && L >= 64 * vec) return false;
+    } else if (elem_size == 4) {
+        if (p.cols <= 128) return false;
+        if (whole_segments && (p.cols <= 256 || L > 16384 || p.cols * L * batch * 4 < (128ll << 20))) return false;
+    } else if (p.cols <= 64 || (grid && p.cols > 128 && p.cols <= 256 && L >= 1024 && p.cols * L * batch * 2 >= (64ll << 20))) {
+        return false;
+    }
+    p.kind = NormKind::ColReg;
+    p.tall = (int)threads;
+    p.vec = (int)vec;
+    p.shift = grid ? 0 : 1;
+    p.nchunk = (int)nc;
+    p.tpr = (int)(threads / tx);
+    return true;
+}
+
 NormPlan plan_normalize(const void* in_data, const void* out_data, const int64_t* shape,
                         const int64_t* strides, int ndim, int64_t axis, int n_norm_dims,
                         size_t elem_size, bool fused) {
@@ -1191,7 +1242,8 @@ NormPlan plan_normalize(const void* in_data, const void* out_data, const int64_t
                 // (... unless the axis is so short that one thread holds it anyway)
                 // (... or the inner dim so narrow that the alternative, lanes along it, would leave most idle:
                 // f16 [4097, 12, 96, 5] over axis 2, 0.4 -> 1.3 TB/s)
-                for (int ev = max_vec; ev >= ((elem_size == 2 && p.cols > 16 && L >= 64) ? 4 : 1); ev /= 2) {
+                bool found = false;
+                for (int ev = max_vec; !found && ev >= ((elem_size == 2 && p.cols > 16 && L >= 64) ? 4 : 1); ev /= 2) {
                     const int64_t regs = std::max<int64_t>(1, ev * (int64_t)elem_size / 4);
                     int64_t nc_max = std::min<int64_t>(64, 64 / regs);
                     const size_t vb = (size_t)ev * elem_size;
@@ -1227,7 +1279,8 @@ NormPlan plan_normalize(const void* in_data, const void* out_data, const int64_t
                         p.vec = ev;
                         p.nchunk = (int)nc_max;
                         p.tpr = (int)ty;
-                        return p;
+                        found = true;
+                        continue;
                     }
                     // an inner dim that is not whole, aligned vectors of this width (odd L, odd strides): the
                     // same vectors unaligned beat narrower aligned ones
@@ -1237,9 +1290,10 @@ NormPlan plan_normalize(const void* in_data, const void* out_data, const int64_t
                         p.shift = 1;
                         p.nchunk = (int)nc_max;
                         p.tpr = (int)ty;
-                        return p;
+                        found = true;
                     }
                 }
+                if (tall_columns(p, found, in_data, out_data, sa, nk > 1 ? p.kept_in.stride[0] : 0, L, batch, elem_size) || found) return p;
             }
             int v = max_vec;
             const bool vec_ok = v > 1 && L % v == 0 && sa % v == 0 && (nk == 1 || p.kept_in.stride[0] % v == 0) &&

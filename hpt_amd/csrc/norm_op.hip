@@ -155,6 +155,37 @@ template <class T, int EV, bool WIDE = false> void launch_col_reg(const NormPlan
     col_reg_kernel<KIND, T, EV, NC><<<grid, dim3(256), 0, st>>>(c);
 }
 
+// NT threads, TX of them along the inner dim, NC vectors each.
+template <class T, int NT, int TX, int NC> bool launch_col_tall_as(const NormPlan& p, const ColRegArgs& c, hipStream_t st) {
+    if (p.tall != NT || p.tpr != NT / TX || p.nchunk != NC || c.cols > NT / TX * NC) return false;
+    const dim3 grid((unsigned)((c.total + TX - 1) / TX));
+    if (p.shift) col_tall_kernel<KIND, T, NT, TX, NC, true><<<grid, dim3(NT), 0, st>>>(c);
+    else col_tall_kernel<KIND, T, NT, TX, NC><<<grid, dim3(NT), 0, st>>>(c);
+    return true;
+}
+
+template <class T> void launch_col_tall(const NormPlan& p, const NormArgs& a, hipStream_t st) {
+    constexpr int EV = 16 / sizeof(T);
+    ColRegArgs c{};
+    const int nk = p.kept_in.n;
+    c.in = a.in;
+    c.out = a.out;
+    c.sa = a.sa;
+    c.bi = nk > 1 ? p.kept_in.stride[0] : 0;
+    c.L = p.kept_in.size[nk - 1];
+    c.nvec = (c.L + EV - 1) / EV;
+    c.total = (nk > 1 ? p.kept_in.size[0] : 1) * c.nvec;
+    c.cols = (int)p.cols;
+    if (c.L < EV || p.vec != EV || (!p.shift && c.L % EV != 0)) fail(HPT_ERR_KERNEL, "col-reg: inner rows of %lld elements are not whole vectors", (long long)c.L);
+    bool done = false;
+    if constexpr (sizeof(T) == 4) {
+        done = launch_col_tall_as<T, 1024, 32, 8>(p, c, st) || launch_col_tall_as<T, 1024, 16, 8>(p, c, st) || launch_col_tall_as<T, 1024, 16, 16>(p, c, st);
+    } else if constexpr (sizeof(T) == 2) {
+        done = launch_col_tall_as<T, 512, 16, 8>(p, c, st) || launch_col_tall_as<T, 512, 16, 16>(p, c, st) || launch_col_tall_as<T, 1024, 16, 16>(p, c, st);
+    }
+    if (!done) fail(HPT_ERR_KERNEL, "col-reg: no kernel of %d threads holds an axis of %d in %d rows of %d vectors", p.tall, c.cols, p.tpr, p.nchunk);
+}
+
 // The transposed forms (kinds 0..2 only).
 template <class T> void launch_transposed(const NormPlan& p, const NormArgs& a, hipStream_t st) {
     constexpr int FULL = 16 / sizeof(T);
@@ -271,6 +302,10 @@ template <class T> void launch_t(const NormPlan& p, NormArgs a, hipStream_t st) 
     }
     if (p.kind == NormKind::ColReg) {
         if constexpr (KIND == NORM_SOFTMAX || KIND == NORM_LOGSOFTMAX) {
+            if (p.tall) {
+                launch_col_tall<T>(p, a, st);
+                return;
+            }
             switch (p.vec) {
                 case 1: launch_col_reg<T, 1>(p, a, st); break;
                 case 2: if constexpr (FULL >= 2) launch_col_reg<T, 2>(p, a, st); break;

@@ -683,6 +683,146 @@ __global__ void __launch_bounds__(256) col_reg_kernel(const ColRegArgs a) {
         }
 }
 
+// ---- the same for a LONGER axis: more threads, not narrower vectors ---------------------------
+// col_reg_kernel's 256 threads hold 65 ... 1024 elements of the axis only as pieces of 2 ... 8 bytes, or in 128 registers each.
+// Here 512 or 1024 threads hold them as whole vectors: TX lanes along the inner dim (256- or 512-byte segments of every inner
+// row), NT / TX thread rows of NC vectors. 64 registers or fewer per thread leave room for two workgroups of 1024 per compute
+// unit, one loading while the other stores. Bound by memory: the same kernel without its arithmetic takes as long (f32 512^3
+// over axis 1 189 us, at 5.7 TB/s; with col_reg_kernel 210).
+// Segments that are neighbours in an inner row go to one XCD, in pairs (workgroups i and i + 8): 199 -> 190 us there, and
+// unaligned segments share the line between them (f32 [512, 65538] over axis 0 91.0 -> 84.9).
+// (device us, softmax over axis 1, col_reg_kernel -> this: f32 [64, 512, 1024] 54.4 -> 50.6, [1, 335, 58050] 89.2 -> 45.2,
+// [16, 1000, 2048] 90.8 -> 56.6, [64, 200, 1000] 32.3 -> 23.1, f16 [256, 320, 500] 86.2 -> 49.7, [300, 130, 500] 25.4 -> 20.2)
+template <int KIND, class T, int NT, int TX, int NC, bool UA = false>
+__global__ void __launch_bounds__(NT) col_tall_kernel(const ColRegArgs a) {
+    static_assert(KIND == NORM_SOFTMAX || KIND == NORM_LOGSOFTMAX, "a softmax kernel");
+    using CT = typename Elem<T>::Wide;
+    using ST = typename StatType<T>::type;
+    constexpr bool kLog = KIND == NORM_LOGSOFTMAX;
+    constexpr int EV = 16 / sizeof(T), TY = NT / TX, NW = NT / 64;
+    static_assert(TX <= 64 && TX * EV <= NT, "a thread for every place of the segment");
+    __shared__ __align__(16) ST part_raw[NW * TX * EV];
+    __shared__ __align__(16) ST res_raw[TX * EV];
+    const int tx = threadIdx.x % TX, ty = threadIdx.x / TX;
+    int64_t blk = blockIdx.x;
+    if (blk < (int64_t)(gridDim.x & ~15u)) blk = (blk & ~(int64_t)15) | ((blk & 7) << 1) | ((blk >> 3) & 1);
+    const int64_t g = blk * TX + tx;
+    const bool valid = g < a.total;
+    int64_t b = 0, q = 0;
+    if (valid) {
+        if (((uint64_t)(g | a.nvec) >> 32) == 0) {
+            b = (uint32_t)g / (uint32_t)a.nvec;
+            q = (uint32_t)g - (uint32_t)b * (uint32_t)a.nvec;
+        } else {
+            b = g / a.nvec;
+            q = g - b * a.nvec;
+        }
+    }
+    const int64_t e0 = UA ? min(q * EV, a.L - EV) : q * EV;
+    const int skip = (int)(q * EV - e0);  // UA: leading elements that belong to the vector before
+    const T* in = (const T*)a.in + b * a.bi + e0;
+    const int mine = valid ? (a.cols - ty + TY - 1) / TY : 0;  // this thread's axis positions: ty, ty + TY, ...
+    Pack<T, EV> raw[NC];
+#pragma unroll
+    for (int i = 0; i < NC; ++i)
+        if (i < mine) {
+            const T* src = in + (int64_t)(ty + i * TY) * a.sa;
+            if constexpr (UA) raw[i] = load_pack_unaligned<T, EV>(src);
+            else raw[i] = load_pack_stream<T, EV>(src);
+        }
+    // (nothing looks inside a loaded value before every load is out: see col_reg_kernel)
+#pragma unroll
+    for (int i = 0; i < NC; ++i) forget_pack(raw[i]);
+    // All-reduce over the thread rows: a butterfly inside the wavefront, then one thread per place folds the wavefronts.
+    // (The sums stay in the wide type on the way: sixteen wavefronts' f32 totals added one after the other put the error of f32
+    // [64, 256, 3072] over axis 1 at 8.3e-8 of the norm, where col_reg_kernel, whose threads' totals are f32, has 6.8e-8. As it is,
+    // [64, 256, 300] 3.9e-8 against 6.1e-8; it costs nothing.)
+    auto across = [&](auto(&v)[EV], auto op) {
+        using V = typename std::remove_reference<decltype(v[0])>::type;
+        V* part = reinterpret_cast<V*>(part_raw);
+        V* res = reinterpret_cast<V*>(res_raw);
+#pragma unroll
+        for (int d = TX; d < 64; d <<= 1)
+#pragma unroll
+            for (int k = 0; k < EV; ++k) v[k] = op(v[k], shfl_xor_any(v[k], d));
+        if ((threadIdx.x & 63) < TX) {
+#pragma unroll
+            for (int k = 0; k < EV; ++k) part[((threadIdx.x >> 6) * TX + tx) * EV + k] = v[k];
+        }
+        __syncthreads();
+        if ((int)threadIdx.x < TX * EV) {
+            V r = part[threadIdx.x];
+#pragma unroll
+            for (int w = 1; w < NW; ++w) r = op(r, part[w * TX * EV + threadIdx.x]);
+            res[threadIdx.x] = r;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < EV; ++k) v[k] = res[tx * EV + k];
+    };
+    CT m[EV], kk[EV], sf[EV];
+    ST s[EV];  // this thread's sum of exponentials, carried in the wider type
+#pragma unroll
+    for (int k = 0; k < EV; ++k) {
+        m[k] = neg_inf<CT>();
+        s[k] = 0;
+    }
+#pragma unroll
+    for (int i = 0; i < NC; ++i)
+        if (i < mine)
+#pragma unroll
+            for (int k = 0; k < EV; ++k) m[k] = MaxC<CT>::comb(m[k], Elem<T>::widen(raw[i].v[k]));
+    across(m, [](CT x, CT y) { return MaxC<CT>::comb(x, y); });
+#pragma unroll
+    for (int i = 0; i < NC; ++i) forget_pack(raw[i]);
+    constexpr bool kKeepExp = std::is_same<T, CT>::value && !kLog;
+#pragma unroll
+    for (int i = 0; i < NC; ++i)
+        if (i < mine)
+#pragma unroll
+            for (int k = 0; k < EV; ++k) {
+                const CT e = exp_ct<T>(Elem<T>::widen(raw[i].v[k]) - m[k]);
+                s[k] += (ST)e;
+                if constexpr (kKeepExp) raw[i].v[k] = Elem<T>::narrow(e);
+            }
+    across(s, [](ST x, ST y) { return x + y; });
+#pragma unroll
+    for (int k = 0; k < EV; ++k) sf[k] = (CT)s[k];
+#pragma unroll
+    for (int i = 0; i < NC; ++i) forget_pack(raw[i]);
+    int ty_st = ty, mine_st = mine;
+    asm volatile("" : "+v"(ty_st), "+v"(mine_st));
+    T* out = (T*)a.out + b * a.cols * a.L + e0;
+#pragma unroll
+    for (int k = 0; k < EV; ++k) kk[k] = kLog ? log_ct<T>(sf[k]) : (CT)1 / sf[k];
+#pragma unroll
+    for (int i = 0; i < NC; ++i)
+        if (i < mine_st) {
+            Pack<T, EV> o;
+#pragma unroll
+            for (int k = 0; k < EV; ++k) {
+                if constexpr (kKeepExp) {
+                    o.v[k] = Elem<T>::narrow(Elem<T>::widen(raw[i].v[k]) * kk[k]);
+                } else {
+                    const CT d = Elem<T>::widen(raw[i].v[k]) - m[k];
+                    o.v[k] = Elem<T>::narrow(kLog ? d - kk[k] : exp_ct<T>(d) * kk[k]);
+                }
+            }
+            T* dst = out + (int64_t)(ty_st + i * TY) * a.L;
+            if constexpr (UA) {
+                if (skip == 0) {
+                    store_pack_unaligned_stream<T, EV>(dst, o);
+                } else {
+#pragma unroll
+                    for (int k = 0; k < EV; ++k)
+                        if (k >= skip) dst[k] = o.v[k];
+                }
+            } else {
+                store_pack_stream<T, EV>(dst, o);
+            }
+        }
+}
+
 // ---- the same, for a NARROW inner dim: the slab is walked as a flat array --------------------
 // softmax over axis 0 of a contiguous [cols, L] slab with L = 3, 8, 33, 100: lanes along the inner
 // dim would leave most of a wavefront idle. Thread t instead owns elements [t * VEC, t * VEC + VEC)
