@@ -103,6 +103,24 @@ static int legal_vec(const void* data, size_t elem_size, int64_t inner_len, cons
 // hold 8 such blocks.
 constexpr int64_t kBlocksToFill = 2048;
 constexpr int64_t kComputeUnits = 256;  // MI355X
+
+// Slices of the reduced range for `groups` workgroups that share it: the count that fills one, two, three or four rounds of
+// compute units to nine tenths, or the one that comes closest.
+static int64_t full_rounds(int64_t groups) {
+    int64_t best = 1;
+    double best_fill = 0;
+    for (int64_t r = 1; r <= 4; ++r) {
+        const int64_t S = r * kComputeUnits / groups;
+        const double fill = (double)(S * groups) / (double)(r * kComputeUnits);
+        if (S >= 1 && fill > best_fill) {
+            best = S;
+            best_fill = fill;
+        }
+        if (fill >= 0.9) break;
+    }
+    return best;
+}
+
 // Column reductions below this take the plans for small inputs; the partials of those that are split stay below
 // the second figure.
 constexpr int64_t kSmallColBytes = 8ll << 20;
@@ -367,15 +385,23 @@ ReducePlan plan_reduce(const void* data, const int64_t* shape, const int64_t* st
             // vector slot is one (row phase, column) pair, so no fold inside the workgroup is needed and
             // the partials are [slice][phase][K].
             const int64_t phases = full / g;
-            const int64_t xb = (kp + 1023) / 1024;
-            if (slabs_aligned && kp > tmax && p.R >= 16 * phases && xb <= 65535 && kin * phases <= kI32) {
+            // One slab of four-byte elements and more: workgroups of 256 threads, one per compute unit (rows of more than 128 of
+            // them: 512 threads); a thousand threads each left a fifth of the units idle at xb = 5 (us, sum over axis 0: f32 [8190, 4097]
+            // 31.2 -> 26.2, [4097, 8190] 31.1 -> 25.2, [2700, 5001] 19.8 -> 14.5, [700, 50257] the same). Several slabs keep the large ones (i32
+            // [12, 128, 4225] over axis 1 11.2, 12.2 in small ones; f32 [16, 512, 4097] 30.2, 32.8 and, as unaligned columns, 32.5). Shorter
+            // elements, whose periods are eight rows and more, are faster as unaligned columns, below, where those take them (f16
+            // [8190, 4097] 21.9 as it was, 18.5 in small workgroups, 16.4 there; [16, 512, 4097] over axis 1 22.5 and 19.0).
+            const bool one_slab = outer == 1 && elem_size >= 4;
+            const int64_t width = !one_slab ? 1024 : (kp + 255) / 256 > 128 ? 512 : 256;
+            const int64_t xb = (kp + width - 1) / width;
+            if (slabs_aligned && kp > tmax && p.R >= 16 * phases && xb <= 65535 && kin * phases <= kI32 && (elem_size >= 4 || p.R < 256)) {
                 p.flat_t = (int)(((kp + xb - 1) / xb + 63) / 64 * 64);
                 p.flat_xb = (int)xb;
                 p.flat_phases = (int)phases;
                 p.vec = full;
                 const int64_t periods = p.R / phases;
                 int64_t cap = std::max<int64_t>(1, (int64_t)((64ll << 20) / acc_size) / (p.K * phases));
-                int64_t slices = std::min<int64_t>(periods / 4, std::max<int64_t>(1, 256 / (outer * xb)));
+                int64_t slices = std::min<int64_t>(periods / 4, one_slab ? full_rounds(xb) : std::max<int64_t>(1, 256 / (outer * xb)));
                 slices = std::max<int64_t>(1, std::min(slices, cap));
                 p.split = (int)(slices * phases);
                 p.bx = p.flat_t;
@@ -618,23 +644,6 @@ static bool lds_row_shape(NormPlan& p, int64_t nvec, size_t elem_size, bool shif
     p.lds_rows = 1;
     p.rpb = 1;
     return true;
-}
-
-// Slices of the axis for `groups` column groups: the count that fills one, two, three or four rounds of compute units to nine
-// tenths, or the one that comes closest.
-static int64_t stats_split(int64_t groups) {
-    int64_t best = 1;
-    double best_fill = 0;
-    for (int64_t r = 1; r <= 4; ++r) {
-        const int64_t S = r * kComputeUnits / groups;
-        const double fill = (double)(S * groups) / (double)(r * kComputeUnits);
-        if (S >= 1 && fill > best_fill) {
-            best = S;
-            best_fill = fill;
-        }
-        if (fill >= 0.9) break;
-    }
-    return best;
 }
 
 // Softmax over an axis of up to 1024 elements with a contiguous inner dim of L: whether 512 or 1024 threads that hold it in whole
@@ -1350,7 +1359,7 @@ NormPlan plan_normalize(const void* in_data, const void* out_data, const int64_t
             // One workgroup per compute unit for the statistics pass (its loads are in flight two batches deep), or the
             // few rounds of them that leave the fewest units idle.
             const int64_t groups = (L + 64 * v - 1) / (64 * v) * batch;
-            p.tsplit = (int)std::min(stats_split(groups), std::max<int64_t>(1, p.cols / 32));
+            p.tsplit = (int)std::min(full_rounds(groups), std::max<int64_t>(1, p.cols / 32));
             // (beyond 64 partials per row the finalize pass grows: 64 columns each then, f32 [4100, 63] 11.7 -> 10.6 us)
             if (p.tsplit > 64) p.tsplit = (int)std::max<int64_t>(64, std::min<int64_t>(p.tsplit, p.cols / 64));
             p.tpr = elem_size == 2 && v > 1 && p.cols >= 128 * p.tsplit ? 8 : 4;  // wavefronts per workgroup of the statistics pass
