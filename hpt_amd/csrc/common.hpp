@@ -108,6 +108,8 @@ struct ReducePlan {
     int flat_xb = 0;    // > 0: a period of the flat walk is wider than a workgroup and spans this many of them;
                         // `split` then counts the partials per output (slices x row phases)
     int flat_phases = 1;  // rows per period in that case
+    int flat_w = 0;     // > 0: launched in workgroups of this many threads and flat_slices slices (no more than split / flat_phases)
+    int flat_slices = 0;
     bool small_split = false;  // Col: split although the input is small, for speed alone; a plan without partials exists (spare_scratch = false)
 };
 

@@ -385,15 +385,9 @@ ReducePlan plan_reduce(const void* data, const int64_t* shape, const int64_t* st
             // vector slot is one (row phase, column) pair, so no fold inside the workgroup is needed and
             // the partials are [slice][phase][K].
             const int64_t phases = full / g;
-            // One slab of four-byte elements and more: workgroups of 256 threads, one per compute unit (rows of more than 128 of
-            // them: 512 threads); a thousand threads each left a fifth of the units idle at xb = 5 (us, sum over axis 0: f32 [8190, 4097]
-            // 31.2 -> 26.2, [4097, 8190] 31.1 -> 25.2, [2700, 5001] 19.8 -> 14.5, [700, 50257] the same). Several slabs keep the large ones (i32
-            // [12, 128, 4225] over axis 1 11.2, 12.2 in small ones; f32 [16, 512, 4097] 30.2, 32.8 and, as unaligned columns, 32.5). Shorter
-            // elements, whose periods are eight rows and more, are faster as unaligned columns, below, where those take them (f16
-            // [8190, 4097] 21.9 as it was, 18.5 in small workgroups, 16.4 there; [16, 512, 4097] over axis 1 22.5 and 19.0).
-            const bool one_slab = outer == 1 && elem_size >= 4;
-            const int64_t width = !one_slab ? 1024 : (kp + 255) / 256 > 128 ? 512 : 256;
-            const int64_t xb = (kp + width - 1) / width;
+            // (Shorter elements, whose periods are eight rows and more, are faster as unaligned columns, below, where those take
+            // them: us, sum over axis 0, f16 [8190, 4097] 21.9 and 16.4, [2700, 5001] 19.1 and 10.8; [16, 512, 4097] over axis 1 22.5 and 19.0.)
+            const int64_t xb = (kp + 1023) / 1024;
             if (slabs_aligned && kp > tmax && p.R >= 16 * phases && xb <= 65535 && kin * phases <= kI32 && (elem_size >= 4 || p.R < 256)) {
                 p.flat_t = (int)(((kp + xb - 1) / xb + 63) / 64 * 64);
                 p.flat_xb = (int)xb;
@@ -401,9 +395,18 @@ ReducePlan plan_reduce(const void* data, const int64_t* shape, const int64_t* st
                 p.vec = full;
                 const int64_t periods = p.R / phases;
                 int64_t cap = std::max<int64_t>(1, (int64_t)((64ll << 20) / acc_size) / (p.K * phases));
-                int64_t slices = std::min<int64_t>(periods / 4, one_slab ? full_rounds(xb) : std::max<int64_t>(1, 256 / (outer * xb)));
+                int64_t slices = std::min<int64_t>(periods / 4, std::max<int64_t>(1, 256 / (outer * xb)));
                 slices = std::max<int64_t>(1, std::min(slices, cap));
                 p.split = (int)(slices * phases);
+                // One slab of four-byte elements and more is launched in workgroups of 256 threads (rows of more than 128 of them:
+                // 512), one per compute unit, which leave fewer partials than the plan has room for (scratch is sized, and refused,
+                // by `split`): a thousand threads each left a fifth of the units idle at xb = 5, and most of the fold was partials. Us,
+                // sum over axis 0: f32 [8190, 4097] 31.2 -> 26.2, [4097, 8190] 31.1 -> 25.2, [2700, 5001] 19.8 -> 14.5, [700, 50257] the same.
+                // Several slabs keep the large ones (i32 [12, 128, 4225] over axis 1 11.2, 12.2 in small ones).
+                if (outer == 1 && elem_size >= 4) {
+                    p.flat_w = (kp + 255) / 256 > 128 ? 512 : 256;
+                    p.flat_slices = (int)std::min(slices, full_rounds((kp + p.flat_w - 1) / p.flat_w));
+                }
                 p.bx = p.flat_t;
                 p.by = 1;
                 p.chunk = 0;
@@ -605,6 +608,7 @@ std::string describe(const ReducePlan& p) {
             break;
     }
     s = buf;
+    if (p.flat_w) s += "as=" + std::to_string(p.flat_w) + "x" + std::to_string(p.flat_slices * p.flat_phases) + " ";
     describe_dims(s, "kept", p.kept);
     s += " ";
     describe_dims(s, "red", p.red);

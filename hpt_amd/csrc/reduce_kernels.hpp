@@ -1252,9 +1252,10 @@ void launch_reduce_t(const ReducePlan& p, const void* in, void* out, const Reduc
             a.kin = (int)kin;
             a.vecs = (int)(kin * p.flat_phases / FULL);
             a.phases = p.flat_phases;
-            a.slices = p.split / p.flat_phases;
-            col_flat_wide_kernel<Op, FULL><<<dim3((unsigned)p.flat_xb, (unsigned)outer, (unsigned)a.slices),
-                                             dim3((unsigned)p.flat_t), 0, st>>>(a);
+            a.slices = p.flat_w ? p.flat_slices : p.split / p.flat_phases;
+            const int width = p.flat_w ? p.flat_w : p.flat_t;
+            col_flat_wide_kernel<Op, FULL><<<dim3((unsigned)((a.vecs + width - 1) / width), (unsigned)outer, (unsigned)a.slices),
+                                             dim3((unsigned)width), 0, st>>>(a);
         }
     } else if (p.flat_t > 0) {
         if constexpr (FULL > 1) {
@@ -1334,14 +1335,15 @@ if (p.unaligned)             col_flat_kernel<Op, FULL, true><<<dim3(1, (unsigned
             else col_reduce_kernel<Op, 1><<<grid, block, smem, st>>>(a);
         }
     }
-    if (p.split > 1) {
+    const int split = p.flat_w ? p.flat_slices * p.flat_phases : p.split;
+    if (split > 1) {
         int fy = 1;  // thread rows sharing an output's partials: about two partials per thread
-        while (fy < 16 && fy * 2 < p.split) fy <<= 1;
+        while (fy < 16 && fy * 2 < split) fy <<= 1;
         // (swapped kept dims: the partials are in the kernel's numbering, the outputs in the caller's)
         const int64_t kin = p.kept_swapped ? p.kept.size[1] : p.K;
         const int64_t oso = p.kept_swapped ? 1 : 0, osi = p.kept_swapped ? p.kept.size[0] : 1;
         finish_cols_kernel<Op><<<dim3((unsigned)((p.K + 63) / 64)), dim3(64, (unsigned)fy),
-                                 fy > 1 ? (size_t)fy * 64 * sizeof(Acc) : 0, st>>>(sc.partial, out, p.K, p.split,
+                                 fy > 1 ? (size_t)fy * 64 * sizeof(Acc) : 0, st>>>(sc.partial, out, p.K, split,
                                                                                     init_out, count, kin, oso, osi);
     }
 }
