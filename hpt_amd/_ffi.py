@@ -124,6 +124,22 @@ def lib() -> C.CDLL:
     return _lib
 
 
+_calls = None
+
+
+def calls():
+    """The native module of the calls that return a fresh tensor (csrc/pycalls.cpp); it is linked to libhpt_hip.so."""
+    global _calls
+    if _calls is None:
+        lib()  # (says what is missing when nothing has been built)
+        try:
+            from . import _calls as module
+        except ImportError as e:
+            raise ImportError(f"hpt_amd._calls cannot be loaded ({e}): build it with `python -m hpt_amd.build`") from e
+        _calls = module
+    return _calls
+
+
 def check(status: int) -> None:
     if status != OK:
         msg = lib().hpt_hip_last_error().decode("utf-8", "replace")

@@ -13,6 +13,7 @@ import concurrent.futures as cf
 import os
 import subprocess
 import sys
+import sysconfig
 from pathlib import Path
 
 ROOT = Path(__file__).resolve().parent
@@ -92,8 +93,27 @@ def build(force: bool = False, jobs: int | None = None, verbose: bool = True) ->
         r = subprocess.run(cmd, capture_output=True, text=True)
         if r.returncode != 0:
             raise RuntimeError("link failed:\n" + r.stderr)
+    build_calls(force)
     build_host_test(force)
     return LIB
+
+
+CALLS_SRC = CSRC / "pycalls.cpp"
+CALLS = ROOT / f"_calls{sysconfig.get_config_var('EXT_SUFFIX')}"
+
+
+def build_calls(force: bool = False) -> Path:
+    """hpt_amd._calls: the interpreter's side of the ABI, compiled with the host compiler alone."""
+    deps = [CALLS_SRC, INCLUDE / "hpt_hip.h"]
+    if not force and CALLS.exists() and CALLS.stat().st_mtime > max(d.stat().st_mtime for d in deps):
+        return CALLS
+    cmd = [os.environ.get("CXX", "g++"), "-std=c++17", "-O2", "-Wall", "-shared", "-fPIC", "-fvisibility=hidden", f"-I{INCLUDE}",
+           f"-I{sysconfig.get_paths()['include']}", str(CALLS_SRC), "-o", str(CALLS), f"-L{LIB.parent}", "-lhpt_hip",
+           "-Wl,-rpath,$ORIGIN/lib", "-Wl,-rpath-link,/opt/rocm/lib"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("building hpt_amd._calls failed:\n" + r.stderr)
+    return CALLS
 
 
 HOST_TEST_SRC = ROOT.parent / "tests" / "cpp" / "host_api_test.cpp"

@@ -139,20 +139,26 @@ class _DeviceStorage(_StreamTracked):
         if ordered:
             self.touch(0)
 
+    @classmethod
+    def adopt(cls, device: int, ptr: int, nbytes: int, stream: int) -> "_DeviceStorage":
+        """The memory of a result that a native call has allocated and queued work for on `stream`."""
+        st = cls.__new__(cls)
+        st.ptr, st.nbytes, st.device = ptr, nbytes, device
+        st.pending = {stream}
+        return st
+
     def __del__(self):
         if not self.ptr:
             return
-        free = "hpt_hip_free"
-        if self.pending == _DEFAULT_STREAM_ONLY:
-            free = "hpt_hip_free_ordered"  # the next owner's work queues up behind what is still running
-        else:
+        ordered = self.pending == _DEFAULT_STREAM_ONLY  # the next owner's work queues up behind what is still running
+        if not ordered:
             try:
                 self.wait()  # kernels still queued on a caller's stream may use the block
             except Exception:
                 pass  # (interpreter shutdown, or the device is gone: nothing more can be waited for)
         try:
             # the block always goes back to the allocator, whatever the wait did
-            getattr(_ffi.lib(), free)(self.device, C.c_void_p(self.ptr), self.nbytes, ALIGN)
+            _ffi.calls().free(self.device, self.ptr, self.nbytes, ordered)
         except Exception:
             pass
         self.ptr = 0
@@ -187,6 +193,13 @@ def _touch(stream, *tensors) -> None:
         st = getattr(t, "_storage", None) if t is not None else None
         if isinstance(st, _StreamTracked):
             st.touch(stream)
+
+
+def _native_stream(stream) -> int:
+    """The stream of a call that goes through the native module, or -1: given in a form that ctypes sorts out."""
+    if stream is None:
+        return 0
+    return stream if type(stream) is int and stream >= 0 else -1
 
 
 _OUT_DTYPES = {}
@@ -247,6 +260,22 @@ class Tensor:
         """empty() for the output of a call that is about to be queued on `stream`."""
         st = _DeviceStorage(device, math.prod(shape) * dtype.size, ordered=_stream_key(stream) == 0)
         return cls(st, st.ptr, shape, _contiguous_strides(shape), dtype, "hip", device)
+
+    @classmethod
+    def _adopt(cls, answer, device: int, stream: int, *used) -> "Tensor":
+        """The tensor of a native call's answer: (address, bytes, shape, strides, dtype code) of memory whose first use has been
+        queued on `stream`, as the use of the tensors `used` has - or the status of a call that failed."""
+        if type(answer) is int:
+            check(answer)
+        ptr, nbytes, shape, strides, code = answer
+        t = cls.__new__(cls)
+        t._storage = _DeviceStorage.adopt(device, ptr, nbytes, stream)
+        t.ptr, t.shape, t.strides, t.dtype = ptr, shape, strides, DTYPES[code]
+        t.backend, t.device, t.parent = "hip", device, None
+        for u in used:
+            if u is not None and isinstance(u._storage, _StreamTracked):
+                u._storage.pending.add(stream)
+        return t
 
     @classmethod
     def from_raw(cls, ptr: int, shape, dtype: DType, device: int = 0, strides=None) -> "Tensor":
@@ -470,8 +499,13 @@ class Tensor:
         """static_scratch: go through hpt_hip_reduce_static (no device allocation inside the call;
         pass `out` as well to keep this wrapper from allocating the result)."""
         self._require_hip("reduce")
-        l = _ffi.lib()
         axes = _as_axes(axes)
+        k = _native_stream(stream)
+        if out is None and not static_scratch and k >= 0 and init_out:
+            answer = _ffi.calls().reduce(self, k, op, axes, keep_dims)
+            if answer is not None:
+                return Tensor._adopt(answer, self.device, k, self)
+        l = _ffi.lib()
         out_dtype = _reduce_out_dtype(op, self.dtype)
         flat_shape = self._reduce_shape(axes, False)
         final_shape = self._reduce_shape(axes, True) if keep_dims else flat_shape
@@ -499,10 +533,15 @@ class Tensor:
 
     def _argreduce(self, is_max: bool, axis, keep_dims: bool, stream=None) -> "Tensor":
         self._require_hip("argreduce")
-        l = _ffi.lib()
         axes = _as_axes(axis)
         if len(axes) != 1:
             raise ParamError(_ffi.ERR_PARAM, "argmax/argmin reduce exactly one axis")
+        k = _native_stream(stream)
+        if k >= 0:
+            answer = _ffi.calls().argreduce(self, k, is_max, axes, keep_dims)
+            if answer is not None:
+                return Tensor._adopt(answer, self.device, k, self)
+        l = _ffi.lib()
         flat_shape = self._reduce_shape(axes, False)
         final_shape = self._reduce_shape(axes, True) if keep_dims else flat_shape
         res = Tensor._result(flat_shape, i64, self.device, stream)
@@ -586,6 +625,11 @@ class Tensor:
         self._require_hip("softmax")
         # NormalizationOps::Output = Tensor<FloatBinaryType<T>>: a non-float input is promoted inside the
         # kernel (one launch, no promoted copy), as the reference promotes inside the op
+        k = _native_stream(stream)
+        if out is None and k >= 0:
+            answer = _ffi.calls().softmax(self, k, log, int(axis))
+            if answer is not None:
+                return Tensor._adopt(answer, self.device, k, self)
         res = self._norm_out(out, self._float_binary_type(), stream)
         vin, k1 = self._c_view()
         vout, k2 = res._c_view()
@@ -615,6 +659,14 @@ class Tensor:
             # (the fused add + layernorm takes float tensors; the promoted copy is kept alive by `_touch`)
             return self.astype(ft, stream=stream).layernorm(normalized_shape, gamma, beta, eps, stream=stream,
                                                             residual=residual, out=out)
+        k = _native_stream(stream)
+        if out is None and k >= 0:
+            for t, what in ((gamma, "gamma"), (beta, "beta"), (residual, "residual")):
+                if t is not None:
+                    t._require_hip("layernorm " + what)
+            answer = _ffi.calls().layernorm(self, k, len(ns), gamma, beta, float(eps), residual)
+            if answer is not None:
+                return Tensor._adopt(answer, self.device, k, self, gamma, beta, residual)
         res = self._norm_out(out, ft, stream)
         vin, k1 = self._c_view()
         vout, k2 = res._c_view()
@@ -649,6 +701,11 @@ class Tensor:
         `scores.mul_(scaling)`, fill -inf where key > query, `softmax(-1)` of
         hpt-examples/examples/transformer/main.rs:233-246 in one pass; the masked part is never read."""
         self._require_hip("softmax_causal")
+        k = _native_stream(stream)
+        if k >= 0:
+            answer = _ffi.calls().softmax_causal(self, k, log, float(scale), int(causal_offset))
+            if answer is not None:
+                return Tensor._adopt(answer, self.device, k, self)
         res = Tensor._result(self.shape, self.dtype, self.device, stream)
         vin, k1 = self._c_view()
         vout, k2 = res._c_view()
