@@ -903,7 +903,7 @@ static void run_layernorm(int dev, void* stream, const hpt_view* in, const hpt_v
     if (residual && (c.plan.kind == NormKind::Transposed || c.plan.kind == NormKind::TransposedTile))
         demote_to_generic(c.plan);
     // shifted rows: the residual's rows must be misaligned like the output's
-    if (c.plan.shift && residual && (((uintptr_t)residual->data ^ (uintptr_t)out->data) & 15) != 0) demote_to_generic(c.plan);
+    if (c.plan.shift && !c.plan.ua_rows && residual && (((uintptr_t)residual->data ^ (uintptr_t)out->data) & 15) != 0) demote_to_generic(c.plan);
     // vector loads of gamma / beta / residual need 16-byte alignment too (the shifted streaming
     // kernel reads gamma / beta element by element and the residual with the rows' own shift)
     if (c.plan.vec > 1 && !c.plan.shift &&

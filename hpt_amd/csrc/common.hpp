@@ -162,6 +162,7 @@ struct NormPlan {
                         // thread), 2 = gamma / beta read from L2 for every row (rows too long for either)
     int tile_rows = 0;  // RowReg, > 0: short back-to-back rows; the plain kinds stage this many rows per workgroup in LDS
     int shift = 0;      // RowStream: rows start off 16-byte boundaries; aligned vectors, masked at both ends
+    int ua_rows = 0;    // RowReg with shift: the rows are taken as unaligned vectors from their start on
     bool wide_sum = false;  // TransposedTile softmax of f32 rows: every exponential is added in f64
     int tsplit = 1;     // Transposed: workgroups sharing the axis in the statistics pass
     size_t scratch_bytes = 0;  // Transposed: partial statistics (rows * tsplit * 24 bytes at most)

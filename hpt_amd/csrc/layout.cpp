@@ -901,7 +901,20 @@ NormPlan plan_normalize(const void* in_data, const void* out_data, const int64_t
                     p.shift = 1;
                     return p;
                 }
-                if (same && nvs > ((n_norm_dims > 0 && elem_size == 2) ? 1024 : 2048)) {
+                // Two-byte rows and f32 layernorm rows as unaligned vectors from the row's start on, whatever the alignments of input,
+                // output and residual: no masks but at a row's last vector, and gamma / beta per column as in aligned rows. Us, aligned
+                // vectors that contain the row and this: bf16 [17616, 2202] softmax 40.9 and 33.0, [28550, 805] log_softmax 21.2 and 18.2,
+                // causal [32, 1001, 1001] 26.9 and 20.7; f16 layernorm [8190, 4097] 59.7 and 33.7, [14245, 561] 14.4 and 11.2, [2000, 12001]
+                // (streamed) 31.4 and 22.7; f32 layernorm [8190, 4097] 60.4 and 49.6, [3000, 9001] (streamed) 61.6 and 43.9. The f32 softmax
+                // is as fast as that of aligned rows ([16000, 2051] 45.3, [16000, 2052] 47.2).
+                const int64_t nvu = (p.cols + max_vec - 1) / max_vec;
+                if ((elem_size == 2 || (elem_size == 4 && n_norm_dims > 0)) && ((uintptr_t)in_data % elem_size) == 0 && ((uintptr_t)out_data % elem_size) == 0 &&
+                    nvu <= (elem_size == 4 ? 4096 : 2048)) {
+                    v = max_vec;
+                    p.vec = v;
+                    p.shift = 1;
+                    p.ua_rows = 1;
+                } else if (same && nvs > ((n_norm_dims > 0 && elem_size == 2) ? 1024 : 2048)) {
                     p.kind = NormKind::RowStream;
                     p.vec = max_vec;
                     p.shift = 1;
@@ -909,14 +922,15 @@ NormPlan plan_normalize(const void* in_data, const void* out_data, const int64_t
                     p.rpb = 1;
                     return p;
                 }
-                if (same) {
+                if (same && !p.ua_rows) {
                     v = max_vec;
                     p.vec = v;
                     p.shift = 1;
                 }
             }
             // vector loads per row (shifted rows: one more than the row's own length needs)
-            int64_t nv = p.shift ? (p.cols + 2 * (v - 1)) / v : p.cols / (v / p.sstride);
+            int64_t nv = p.ua_rows ? (p.cols + v - 1) / v : p.shift ? (p.cols + 2 * (v - 1)) / v : p.cols / (v / p.sstride);
+            const bool masks = p.shift && !p.ua_rows;  // the kernel masks both ends of every row
             // Few, very long contiguous rows: share each row among workgroups. (One workgroup per
             // row would leave a chip of 256 compute units mostly idle.)
             if (sa == 1 && !p.shift && p.rows <= 128 && p.cols >= 16384 && p.cols % v == 0) {
@@ -951,7 +965,9 @@ NormPlan plan_normalize(const void* in_data, const void* out_data, const int64_t
             // 3.5 -> 4.6, [4096, 8192] 4.7 -> 5.0, [2730, 12288] 3.2 -> 4.6, [2048, 16384] 3.8 -> 4.6; [65536, 1024]
             // 5.0 -> 5.4, [32768, 2048] 4.6 -> 5.3, [74898, 896] 4.5 -> 5.2, [104857, 640] 4.5 -> 4.9 (shorter rows lose:
             // [131072, 512] 4.9 -> 4.5).
-            if (ln_half && p.sstride == 1 && !p.shift && nv * v >= 640 && nv * v <= 16384) {
+            // (With a residual's vectors beside the row's, gamma / beta in registers spill from the third vector on: beyond 256
+            // elements, us: f16 [14245, 560] 20.9 -> 12.5, [14245, 561] 28.9 -> 13.9, [30000, 384] 22.8 -> 16.4; bf16 [30000, 256] 11.4, 14.8 this way.)
+            if (ln_half && p.sstride == 1 && !masks && nv * v >= (fused ? 264 : 640) && nv * v <= 16384) {
                 p.gb_lds = 1;
                 ln_half = false;
             }
@@ -1053,7 +1069,7 @@ NormPlan plan_normalize(const void* in_data, const void* out_data, const int64_t
                 // [44739, 1500] 4.2 -> 4.9, f32 [8190, 4097] 4.4 -> 5.3, [16000, 2051] 4.3 -> 5.5; layernorm, which
                 // carries the masks and the unaligned gamma / beta besides, only up to what it had: more spills.)
                 if (v == max_vec && v > 1 && p.sstride == 1 && !p.tile_rows) {
-                    const int maxc = n_norm_dims > 0 && p.shift ? (elem_size == 2 ? 2 : 4)
+                    const int maxc = n_norm_dims > 0 && masks ? (elem_size == 2 ? 2 : 4)
                                                                 : elem_size == 2 ? (ln_half ? 3 : 4)
                                                                 : (n_norm_dims > 0 ? (fused ? 4 : 6) : 8);
                     // (layernorm(x + residual) holds the residual's vectors beside the row's: with five or six
@@ -1393,6 +1409,7 @@ void demote_to_generic(NormPlan& p) {
     p.flat_t = 0;
     p.vec = 1;
     p.shift = 0;
+    p.ua_rows = 0;
     p.sstride = 1;
     p.nchunk = 1;
     p.scratch_bytes = 0;

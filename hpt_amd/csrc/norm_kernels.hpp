@@ -164,8 +164,13 @@ __device__ __forceinline__ void row_all_reduce_n(A (&v)[N], int tpr, int ty, A* 
 // in its vector, and a thread keeps IL (max, sum) pairs. IL = 2 vectors: a thread's vectors all hold the same VEC
 // numbers (threads per row are even), its neighbour the other VEC, and only threads two apart are folded together. Loads and stores are those of a plain row (softmax over the middle axis of a contiguous
 // [B, C, 2], [B, C, 4], [B, C, 8 heads]).
-template <int KIND, class T, int VEC, int NCHUNK, int SS = 1, bool SHIFT = false, bool PF = false, int GB = 0, int IL = 1>
+// UA (VEC > 1, SS = 1): rows off the vector grid as unaligned vectors from the row's start on, the last one from its end
+// backwards: it holds what the vector before it ends with once more, which counts and is stored there. A thread's columns
+// are the same in every row, so gamma / beta stay where they are for aligned rows, and only the wavefront that
+// holds a row's last vector masks anything.
+template <int KIND, class T, int VEC, int NCHUNK, int SS = 1, bool SHIFT = false, bool PF = false, int GB = 0, int IL = 1, bool UA = false>
 __global__ void __launch_bounds__(1024) row_reg_kernel(const NormArgs a) {
+    static_assert(!UA || (VEC > 1 && SS == 1 && !SHIFT && IL == 1 && GB <= 1), "UA is a full-vector mode of plain rows");
     constexpr int ML = IL < 0 ? -IL : 0;  // interleaved softmaxes whose number is no divisor of the vector (3, 5, 6, 7)
     static_assert(IL == 1 || (!norm_is_layer(KIND) && !norm_is_causal(KIND) && SS == 1 && !SHIFT && VEC > 1 &&
                               (ML ? (ML >= 3 && ML <= 7 && VEC % ML != 0) : (VEC % IL == 0 || IL % VEC == 0))),
@@ -185,7 +190,10 @@ __global__ void __launch_bounds__(1024) row_reg_kernel(const NormArgs a) {
     const int tpr = a.tpr;
     const int tx = threadIdx.x & (tpr - 1);
     const int ty = threadIdx.x >> a.tpr_log2;
-    const int nv = SHIFT ? (int)((a.cols + 2 * (VEC - 1)) / VEC) : (int)(a.cols / UV);  // SHIFT: upper bound
+    const int nv = SHIFT ? (int)((a.cols + 2 * (VEC - 1)) / VEC) : UA ? (int)((a.cols + VEC - 1) / VEC) : (int)(a.cols / UV);  // SHIFT: upper bound
+    // UA: first column of vector iv, and how many columns of the last vector belong to the one before
+    auto first_of = [&](int iv) -> int { return UA ? min(iv * VEC, (int)a.cols - VEC) : iv * UV; };
+    const int twice = UA ? nv * VEC - (int)a.cols : 0;
     // Vector c of this thread. ML: only the largest multiple of ML lanes of a row take part, so that all of a lane's
     // vectors start at the same place modulo ML, (tx * VEC) % ML; the other lanes hold nothing.
     const int tstep = ML ? tpr / (ML ? ML : 1) * ML : tpr;
@@ -234,8 +242,13 @@ __global__ void __launch_bounds__(1024) row_reg_kernel(const NormArgs a) {
                 }
             } else if (iv < nv) {
                 if constexpr (VEC > 1) {
-                    if (a.gamma) gam[c] = load_pack<T, UV>((const T*)a.gamma + (int64_t)iv * UV);
-                    if (a.beta) bet[c] = load_pack<T, UV>((const T*)a.beta + (int64_t)iv * UV);
+                    if constexpr (UA) {
+                        if (a.gamma) gam[c] = load_pack_unaligned<T, UV>((const T*)a.gamma + first_of(iv));
+                        if (a.beta) bet[c] = load_pack_unaligned<T, UV>((const T*)a.beta + first_of(iv));
+                    } else {
+                        if (a.gamma) gam[c] = load_pack<T, UV>((const T*)a.gamma + (int64_t)iv * UV);
+                        if (a.beta) bet[c] = load_pack<T, UV>((const T*)a.beta + (int64_t)iv * UV);
+                    }
                 } else {
                     if (a.gamma) gam[c].v[0] = ((const T*)a.gamma)[iv];
                     if (a.beta) bet[c].v[0] = ((const T*)a.beta)[iv];
@@ -283,11 +296,13 @@ __global__ void __launch_bounds__(1024) row_reg_kernel(const NormArgs a) {
         for (int c = 0; c < NCHUNK; ++c) {
             const int iv = vec_of(c);
             if (iv < nv_row) {
-                if constexpr (VEC > 1) raw[c] = load_pack_stream<T, VEC>(in_row + (int64_t)iv * VEC);
+                if constexpr (UA) raw[c] = load_pack_unaligned<T, VEC>(in_row + first_of(iv));
+                else if constexpr (VEC > 1) raw[c] = load_pack_stream<T, VEC>(in_row + (int64_t)iv * VEC);
                 else raw[c].v[0] = in_row[(int64_t)iv * a.sa];
                 if constexpr (kRes) {
                     const T* res_row = (const T*)a.residual + row * a.cols - m;
-                    if constexpr (VEC > 1) raw_res[c] = load_pack_stream<T, UV>(res_row + (int64_t)iv * UV);
+                    if constexpr (UA) raw_res[c] = load_pack_unaligned<T, UV>(res_row + first_of(iv));
+                    else if constexpr (VEC > 1) raw_res[c] = load_pack_stream<T, UV>(res_row + (int64_t)iv * UV);
                     else raw_res[c].v[0] = res_row[iv];
                 }
             }
@@ -303,8 +318,13 @@ __global__ void __launch_bounds__(1024) row_reg_kernel(const NormArgs a) {
                 g.v[j] = Elem<T>::narrow((CT)1);
                 b.v[j] = Elem<T>::narrow((CT)0);
             }
-            if (a.gamma) g = load_pack<T, UV>((const T*)a.gamma + (int64_t)i * UV);
-            if (a.beta) b = load_pack<T, UV>((const T*)a.beta + (int64_t)i * UV);
+            if constexpr (UA) {
+                if (a.gamma) g = load_pack_unaligned<T, UV>((const T*)a.gamma + first_of(i));
+                if (a.beta) b = load_pack_unaligned<T, UV>((const T*)a.beta + first_of(i));
+            } else {
+                if (a.gamma) g = load_pack<T, UV>((const T*)a.gamma + (int64_t)i * UV);
+                if (a.beta) b = load_pack<T, UV>((const T*)a.beta + (int64_t)i * UV);
+            }
             store_pack<T, UV>(lds_gamma + (size_t)i * UV, g);
             store_pack<T, UV>(lds_beta + (size_t)i * UV, b);
         }
@@ -320,7 +340,7 @@ __global__ void __launch_bounds__(1024) row_reg_kernel(const NormArgs a) {
         // is element j of vector iv inside the row (and, for the causal kinds, kept)?
         auto inside = [&](int iv, int j) -> bool {
             if constexpr (SHIFT) return (unsigned)(iv * UV + j - sh) < (unsigned)limit;
-            else return iv < nv && (!kCausal || iv * UV + j < limit);
+            else return iv < nv && (!kCausal || first_of(iv) + j < limit);
         };
 
         CT x[NCHUNK][UV];
@@ -355,6 +375,13 @@ __global__ void __launch_bounds__(1024) row_reg_kernel(const NormArgs a) {
                 if constexpr (kRes) e = have ? Elem<T>::widen(Elem<T>::narrow(e + Elem<T>::widen(raw_res[c].v[j]))) : fill;
                 if constexpr (kCausal) e = have ? Elem<T>::widen(Elem<T>::narrow(e * scale_t)) : fill;
                 x[c][j] = e;
+            }
+            if constexpr (UA) {
+                if (iv == nv - 1) {
+#pragma unroll
+                    for (int j = 0; j < UV; ++j)
+                        if (j < twice) x[c][j] = fill;
+                }
             }
         }
         if constexpr (kPrefetch) issue_loads(row0 + row_step);
@@ -457,12 +484,20 @@ __global__ void __launch_bounds__(1024) row_reg_kernel(const NormArgs a) {
 #pragma unroll
             for (int c = 0; c < NCHUNK; ++c) {
                 const bool in_row_c = (c * tpr + tx) < nv;
+                auto square = [&](auto last) {
 #pragma unroll
-                for (int j = 0; j < UV; ++j) {
-                    const bool in_row_e = SHIFT ? inside(c * tpr + tx, j) : in_row_c;
-                    const CT d = in_row_e ? (x[c][j] - mean_hi) - mean_lo : (CT)0;
-                    x[c][j] = d;
-                    q += d * d;
+                    for (int j = 0; j < UV; ++j) {
+                        const bool in_row_e = SHIFT ? inside(c * tpr + tx, j) : decltype(last)::value ? j >= twice : in_row_c;
+                        const CT d = in_row_e ? (x[c][j] - mean_hi) - mean_lo : (CT)0;
+                        x[c][j] = d;
+                        q += d * d;
+                    }
+                };
+                if constexpr (UA) {
+                    if (c * tpr + tx == nv - 1) square(std::true_type{});
+                    else square(std::false_type{});
+                } else {
+                    square(std::false_type{});
                 }
             }
             const ST var = row_all_reduce<SumC<ST>>((ST)q, tpr, ty, ssmem) * (ST)a.inv_cols;
@@ -530,7 +565,19 @@ __global__ void __launch_bounds__(1024) row_reg_kernel(const NormArgs a) {
                         }
                     }
                 } else if (iv < nv) {
-                    if constexpr (VEC > 1) {
+                    if constexpr (UA) {
+                        Pack<T, UV> o;
+#pragma unroll
+                        for (int j = 0; j < UV; ++j) o.v[j] = Elem<T>::narrow(x[c][j]);
+                        T* dst = out_row + first_of(iv);
+                        if (twice == 0 || iv < nv - 1) {
+                            store_pack_unaligned_stream<T, UV>(dst, o);
+                        } else {
+#pragma unroll
+                            for (int j = 0; j < UV; ++j)
+                                if (j >= twice) dst[j] = o.v[j];
+                        }
+                    } else if constexpr (VEC > 1) {
                         Pack<T, UV> o;
 #pragma unroll
                         for (int j = 0; j < UV; ++j) o.v[j] = Elem<T>::narrow(x[c][j]);

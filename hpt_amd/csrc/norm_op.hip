@@ -21,24 +21,24 @@ inline int ilog2(int v) {
     return l;
 }
 
-template <class T, int VEC, int SS = 1, bool SHIFT = false, bool PF = false>
+template <class T, int VEC, int SS = 1, bool SHIFT = false, bool PF = false, bool UA = false>
 void launch_row_reg(const NormPlan& p, const NormArgs& a, dim3 grid, dim3 block, hipStream_t st) {
     // (3, 5, 6 and 7 vectors per thread: rows of whole vectors whose length is 3, 5, 6 or 7 times a power of
     // two - 768, 1536, 2560, 3072, 3584, 5120, 6144 ... - without idle lanes; full-vector rows only)
     if constexpr (VEC > 1 && SS == 1) {
         switch (p.nchunk) {
-            case 3: row_reg_kernel<KIND, T, VEC, 3, SS, SHIFT, PF><<<grid, block, 0, st>>>(a); return;
-            case 5: row_reg_kernel<KIND, T, VEC, 5, SS, SHIFT, PF><<<grid, block, 0, st>>>(a); return;
-            case 6: row_reg_kernel<KIND, T, VEC, 6, SS, SHIFT, PF><<<grid, block, 0, st>>>(a); return;
-            case 7: row_reg_kernel<KIND, T, VEC, 7, SS, SHIFT, PF><<<grid, block, 0, st>>>(a); return;
+            case 3: row_reg_kernel<KIND, T, VEC, 3, SS, SHIFT, PF, 0, 1, UA><<<grid, block, 0, st>>>(a); return;
+            case 5: row_reg_kernel<KIND, T, VEC, 5, SS, SHIFT, PF, 0, 1, UA><<<grid, block, 0, st>>>(a); return;
+            case 6: row_reg_kernel<KIND, T, VEC, 6, SS, SHIFT, PF, 0, 1, UA><<<grid, block, 0, st>>>(a); return;
+            case 7: row_reg_kernel<KIND, T, VEC, 7, SS, SHIFT, PF, 0, 1, UA><<<grid, block, 0, st>>>(a); return;
             default: break;
         }
     }
     switch (p.nchunk) {
-        case 1: row_reg_kernel<KIND, T, VEC, 1, SS, SHIFT, PF><<<grid, block, 0, st>>>(a); break;
-        case 2: row_reg_kernel<KIND, T, VEC, 2, SS, SHIFT, PF><<<grid, block, 0, st>>>(a); break;
-        case 4: row_reg_kernel<KIND, T, VEC, 4, SS, SHIFT, PF><<<grid, block, 0, st>>>(a); break;
-        case 8: row_reg_kernel<KIND, T, VEC, 8, SS, SHIFT, PF><<<grid, block, 0, st>>>(a); break;
+        case 1: row_reg_kernel<KIND, T, VEC, 1, SS, SHIFT, PF, 0, 1, UA><<<grid, block, 0, st>>>(a); break;
+        case 2: row_reg_kernel<KIND, T, VEC, 2, SS, SHIFT, PF, 0, 1, UA><<<grid, block, 0, st>>>(a); break;
+        case 4: row_reg_kernel<KIND, T, VEC, 4, SS, SHIFT, PF, 0, 1, UA><<<grid, block, 0, st>>>(a); break;
+        case 8: row_reg_kernel<KIND, T, VEC, 8, SS, SHIFT, PF, 0, 1, UA><<<grid, block, 0, st>>>(a); break;
         default: fail(HPT_ERR_KERNEL, "row_reg: unsupported chunk count %d", p.nchunk);
     }
 }
@@ -441,14 +441,38 @@ template <class T> void launch_t(const NormPlan& p, NormArgs a, hipStream_t st) 
         }
         if (norm_is_layer(KIND) && grid.x > (unsigned)p.max_blocks) grid.x = (unsigned)p.max_blocks;
         if constexpr (FULL > 1) {
+            // Rows off the vector grid: two-byte types and the f32 layernorms as unaligned vectors, the others as the aligned vectors
+            // that contain them.
+            constexpr bool kUnaligned = sizeof(T) == 2 || (sizeof(T) == 4 && norm_is_layer(KIND));
             if (p.vec == FULL && p.shift) {
-                // shifted rows: a thread's gamma / beta fit every row it walks only if those rows share
-                // their misalignment, i.e. the row step is a whole number of vectors
-                if (norm_is_layer(KIND) && (int64_t)grid.x * p.rpb < p.rows) {
-                    if (grid.x >= (unsigned)FULL) grid.x -= grid.x % FULL;
-                    else fail(HPT_ERR_KERNEL, "row_reg: shifted rows need a row step of whole vectors");
+                if constexpr (kUnaligned) {
+                    if (!p.ua_rows || a.cols < FULL) fail(HPT_ERR_KERNEL, "row_reg: no kernel for shifted rows of this type");
+                    if constexpr (sizeof(T) == 2 && norm_is_layer(KIND)) {
+                        if (p.gb_lds == 1 && p.nchunk >= 3 && p.nchunk <= 4) {
+                            const size_t smem = 2 * (size_t)((p.cols + FULL - 1) / FULL) * FULL * sizeof(T);
+                            if (p.tpr >= 512 && grid.x > 512u) grid.x = 512u;
+                            if (p.nchunk == 3) row_reg_kernel<KIND, T, FULL, 3, 1, false, false, 1, 1, true><<<grid, block, smem, st>>>(a);
+                            else row_reg_kernel<KIND, T, FULL, 4, 1, false, false, 1, 1, true><<<grid, block, smem, st>>>(a);
+                            return;
+                        }
+                    }
+                    if constexpr (KIND != NORM_ADD_LAYERNORM) {
+                        if (p.tpr >= 512 && (sizeof(T) >= 4 || p.tpr == 1024 || norm_is_layer(KIND))) {
+                            if (grid.x > 512u) grid.x = 512u;
+                            launch_row_reg<T, FULL, 1, false, true, true>(p, a, grid, block, st);
+                            return;
+                        }
+                    }
+                    launch_row_reg<T, FULL, 1, false, false, true>(p, a, grid, block, st);
+                } else {
+                    // shifted rows: a thread's gamma / beta fit every row it walks only if those rows share
+                    // their misalignment, i.e. the row step is a whole number of vectors
+                    if (norm_is_layer(KIND) && (int64_t)grid.x * p.rpb < p.rows) {
+                        if (grid.x >= (unsigned)FULL) grid.x -= grid.x % FULL;
+                        else fail(HPT_ERR_KERNEL, "row_reg: shifted rows need a row step of whole vectors");
+                    }
+                    launch_row_reg<T, FULL, 1, true>(p, a, grid, block, st);
                 }
-                launch_row_reg<T, FULL, 1, true>(p, a, grid, block, st);
                 return;
             }
         }
