@@ -140,7 +140,16 @@ __global__ void __launch_bounds__(1024) row_lean_kernel(const RowLeanArgs a) {
 #pragma unroll
                 for (int u = 0; u < 4; ++u) fold(v[u], iv + u * tpr);
             }
-            for (; iv < i1; iv += tpr) fold(load(iv), iv);
+            // the up to three that are left, together: one after the other each waits a memory latency. (Those beyond the
+            // row's share load its last vector once more.)
+            if (iv < i1) {
+                Pack<T, VEC> v[3];
+#pragma unroll
+                for (int u = 0; u < 3; ++u) v[u] = load(min(iv + u * tpr, i1 - 1));
+#pragma unroll
+                for (int u = 0; u < 3; ++u)
+                    if (iv + u * tpr < i1) fold(v[u], iv + u * tpr);
+            }
         } else {
 #pragma unroll 4
             for (; iv < i1; iv += tpr) fold_in<Op>(acc, p[(int64_t)iv * a.sr], iv);
@@ -225,7 +234,14 @@ __global__ void __launch_bounds__(256) row_mod_kernel(const RowModArgs a) {
 #pragma unroll
             for (int u = 0; u < 4; ++u) fold(v[u], iv + u * act);
         }
-        for (; iv < nvec; iv += act) fold(load_pack_unaligned<T, VEC>(p + (int64_t)iv * VEC), iv);
+        if (iv < nvec) {  // the up to three that are left, together
+            Pack<T, VEC> v[3];
+#pragma unroll
+            for (int u = 0; u < 3; ++u) v[u] = load_pack_unaligned<T, VEC>(p + (int64_t)min(iv + u * act, nvec - 1) * VEC);
+#pragma unroll
+            for (int u = 0; u < 3; ++u)
+                if (iv + u * act < nvec) fold(v[u], iv + u * act);
+        }
         // the lane's vector places as outputs: place j is output (tx * VEC + j) % L
         const int r = tx * VEC % L;
 #pragma unroll
