@@ -873,6 +873,16 @@ NormPlan plan_normalize(const void* in_data, const void* out_data, const int64_t
                 if (vi == max_vec && out_ok) {
                     v = max_vec;
                     p.sstride = 2;
+                } else if ((elem_size == 2 ? p.cols >= 640 : elem_size == 4 && p.cols > 6144) && (p.cols + uv - 1) / uv <= 4096 && ((uintptr_t)in_data % elem_size) == 0 &&
+                           ((uintptr_t)out_data % elem_size) == 0) {
+                    // Off the vector grid: the same vectors unaligned, for two-byte rows and the longest of four bytes (us, every second of
+                    // the stored, single elements and this: bf16 [3456, 7897] layernorm 26.9 and 19.1, softmax 21.6 and 16.8, [1920, 1763] 6.9 and
+                    // 5.3, f16 [2000, 16383] 37.1 and 26.9, but [768, 955] 5.0 and 5.5; f32 [2000, 16383] softmax 53.6 and 47.6, but [3456, 7897]
+                    // 32.3 and 35.7).
+                    v = max_vec;
+                    p.sstride = 2;
+                    p.shift = 1;
+                    p.ua_rows = 1;
                 }
             }
             p.vec = v;
@@ -929,7 +939,7 @@ NormPlan plan_normalize(const void* in_data, const void* out_data, const int64_t
                 }
             }
             // vector loads per row (shifted rows: one more than the row's own length needs)
-            int64_t nv = p.ua_rows ? (p.cols + v - 1) / v : p.shift ? (p.cols + 2 * (v - 1)) / v : p.cols / (v / p.sstride);
+            int64_t nv = p.ua_rows ? (p.cols + v / p.sstride - 1) / (v / p.sstride) : p.shift ? (p.cols + 2 * (v - 1)) / v : p.cols / (v / p.sstride);
             const bool masks = p.shift && !p.ua_rows;  // the kernel masks both ends of every row
             // Few, very long contiguous rows: share each row among workgroups. (One workgroup per
             // row would leave a chip of 256 compute units mostly idle.)
@@ -1139,6 +1149,7 @@ NormPlan plan_normalize(const void* in_data, const void* out_data, const int64_t
                 if (p.sstride == 2) {  // the streaming kernel gathers stride-2 rows element by element
                     p.vec = 1;
                     p.sstride = 1;
+                    p.shift = p.ua_rows = 0;
                 }
             }
             return p;

@@ -164,13 +164,13 @@ __device__ __forceinline__ void row_all_reduce_n(A (&v)[N], int tpr, int ty, A* 
 // in its vector, and a thread keeps IL (max, sum) pairs. IL = 2 vectors: a thread's vectors all hold the same VEC
 // numbers (threads per row are even), its neighbour the other VEC, and only threads two apart are folded together. Loads and stores are those of a plain row (softmax over the middle axis of a contiguous
 // [B, C, 2], [B, C, 4], [B, C, 8 heads]).
-// UA (VEC > 1, SS = 1): rows off the vector grid as unaligned vectors from the row's start on, the last one from its end
-// backwards: it holds what the vector before it ends with once more, which counts and is stored there. A thread's columns
+// UA (VEC > 1): rows off the vector grid as unaligned vectors from the row's start on, the last one from its end
+// backwards (SS = 2: so that it ends with the row's last element, which is then an odd place of it): it holds what the vector before it ends with once more, which counts and is stored there. A thread's columns
 // are the same in every row, so gamma / beta stay where they are for aligned rows, and only the wavefront that
 // holds a row's last vector masks anything.
 template <int KIND, class T, int VEC, int NCHUNK, int SS = 1, bool SHIFT = false, bool PF = false, int GB = 0, int IL = 1, bool UA = false>
 __global__ void __launch_bounds__(1024) row_reg_kernel(const NormArgs a) {
-    static_assert(!UA || (VEC > 1 && SS == 1 && !SHIFT && IL == 1 && GB <= 1), "UA is a full-vector mode of plain rows");
+    static_assert(!UA || (VEC > 1 && !SHIFT && IL == 1 && GB <= 1), "UA is a full-vector mode of plain rows");
     constexpr int ML = IL < 0 ? -IL : 0;  // interleaved softmaxes whose number is no divisor of the vector (3, 5, 6, 7)
     static_assert(IL == 1 || (!norm_is_layer(KIND) && !norm_is_causal(KIND) && SS == 1 && !SHIFT && VEC > 1 &&
                               (ML ? (ML >= 3 && ML <= 7 && VEC % ML != 0) : (VEC % IL == 0 || IL % VEC == 0))),
@@ -190,10 +190,10 @@ __global__ void __launch_bounds__(1024) row_reg_kernel(const NormArgs a) {
     const int tpr = a.tpr;
     const int tx = threadIdx.x & (tpr - 1);
     const int ty = threadIdx.x >> a.tpr_log2;
-    const int nv = SHIFT ? (int)((a.cols + 2 * (VEC - 1)) / VEC) : UA ? (int)((a.cols + VEC - 1) / VEC) : (int)(a.cols / UV);  // SHIFT: upper bound
+    const int nv = SHIFT ? (int)((a.cols + 2 * (VEC - 1)) / VEC) : UA ? (int)((a.cols + UV - 1) / UV) : (int)(a.cols / UV);  // SHIFT: upper bound
     // UA: first column of vector iv, and how many columns of the last vector belong to the one before
-    auto first_of = [&](int iv) -> int { return UA ? min(iv * VEC, (int)a.cols - VEC) : iv * UV; };
-    const int twice = UA ? nv * VEC - (int)a.cols : 0;
+    auto first_of = [&](int iv) -> int { return UA ? min(iv * UV, (int)a.cols - UV) : iv * UV; };
+    const int twice = UA ? nv * UV - (int)a.cols : 0;
     // Vector c of this thread. ML: only the largest multiple of ML lanes of a row take part, so that all of a lane's
     // vectors start at the same place modulo ML, (tx * VEC) % ML; the other lanes hold nothing.
     const int tstep = ML ? tpr / (ML ? ML : 1) * ML : tpr;
@@ -296,7 +296,7 @@ __global__ void __launch_bounds__(1024) row_reg_kernel(const NormArgs a) {
         for (int c = 0; c < NCHUNK; ++c) {
             const int iv = vec_of(c);
             if (iv < nv_row) {
-                if constexpr (UA) raw[c] = load_pack_unaligned<T, VEC>(in_row + first_of(iv));
+                if constexpr (UA) raw[c] = load_pack_unaligned<T, VEC>(in_row + first_of(iv) * SS - (SS == 2 && iv == nv - 1 ? 1 : 0));
                 else if constexpr (VEC > 1) raw[c] = load_pack_stream<T, VEC>(in_row + (int64_t)iv * VEC);
                 else raw[c].v[0] = in_row[(int64_t)iv * a.sa];
                 if constexpr (kRes) {
@@ -343,6 +343,10 @@ __global__ void __launch_bounds__(1024) row_reg_kernel(const NormArgs a) {
             else return iv < nv && (!kCausal || first_of(iv) + j < limit);
         };
 
+        auto element = [&](int c, int iv, int j) -> T {
+            if constexpr (UA && SS == 2) return iv == nv - 1 ? raw[c].v[j * 2 + 1] : raw[c].v[j * 2];
+            else return raw[c].v[j * SS];
+        };
         CT x[NCHUNK][UV];
 #pragma unroll
         for (int c = 0; c < NCHUNK; ++c) {
@@ -362,14 +366,14 @@ __global__ void __launch_bounds__(1024) row_reg_kernel(const NormArgs a) {
                 if (c_lo + tpr * UV <= limit) {
 #pragma unroll
                     for (int j = 0; j < UV; ++j)
-                        x[c][j] = Elem<T>::widen(Elem<T>::narrow(Elem<T>::widen(raw[c].v[j * SS]) * scale_t));
+                        x[c][j] = Elem<T>::widen(Elem<T>::narrow(Elem<T>::widen(element(c, iv, j)) * scale_t));
                     continue;
                 }
             }
 #pragma unroll
             for (int j = 0; j < UV; ++j) {
                 const bool have = valid && inside(iv, j);
-                CT e = have ? Elem<T>::widen(raw[c].v[j * SS]) : fill;
+                CT e = have ? Elem<T>::widen(element(c, iv, j)) : fill;
                 // the fused forms round the intermediate (in + residual, scale * in) to the tensor's
                 // dtype, as the separate add / mul_ of the unfused sequence would have stored it
                 if constexpr (kRes) e = have ? Elem<T>::widen(Elem<T>::narrow(e + Elem<T>::widen(raw_res[c].v[j]))) : fill;

@@ -444,6 +444,20 @@ template <class T> void launch_t(const NormPlan& p, NormArgs a, hipStream_t st) 
             // Rows off the vector grid: two-byte types and the f32 layernorms as unaligned vectors, the others as the aligned vectors
             // that contain them.
             constexpr bool kUnaligned = sizeof(T) == 2 || (sizeof(T) == 4 && norm_is_layer(KIND));
+            if constexpr (sizeof(T) <= 4) {
+                if (p.vec == FULL && p.ua_rows && p.sstride == 2) {
+                    if (a.cols < FULL) fail(HPT_ERR_KERNEL, "row_reg: rows of %lld elements hold no vector", (long long)a.cols);
+                    if constexpr (KIND != NORM_ADD_LAYERNORM) {
+                        if (p.tpr >= 512 && (sizeof(T) >= 4 || norm_is_layer(KIND))) {
+                            if (grid.x > 512u) grid.x = 512u;
+                            launch_row_reg<T, FULL, 2, false, true, true>(p, a, grid, block, st);
+                            return;
+                        }
+                    }
+                    launch_row_reg<T, FULL, 2, false, false, true>(p, a, grid, block, st);
+                    return;
+                }
+            }
             if (p.vec == FULL && p.shift) {
                 if constexpr (kUnaligned) {
                     if (!p.ua_rows || a.cols < FULL) fail(HPT_ERR_KERNEL, "row_reg: no kernel for shifted rows of this type");
@@ -522,6 +536,15 @@ template <class T> void launch_t(const NormPlan& p, NormArgs a, hipStream_t st) 
                 (sizeof(T) >= 4 || p.tpr == 1024 || norm_is_layer(KIND))) {
                 if (grid.x > 512u) grid.x = 512u;
                 launch_row_reg<T, FULL, 1, false, true>(p, a, grid, block, st);
+                return;
+            }
+        }
+        if constexpr (FULL > 1 && KIND != NORM_ADD_LAYERNORM) {
+            // (every second element: the same walk; us, [:, ::2] of the stored: f32 [1472, 15296] layernorm 38.4 -> 36.3, softmax 37.2 ->
+            // 36.0, f16 [597, 14904] layernorm 11.1 -> 9.1, but its softmax 7.7 -> 8.2)
+            if (p.vec == FULL && p.sstride == 2 && p.tpr >= 512 && (sizeof(T) >= 4 || norm_is_layer(KIND))) {
+                if (grid.x > 512u) grid.x = 512u;
+                launch_row_reg<T, FULL, 2, false, true>(p, a, grid, block, st);
                 return;
             }
         }

@@ -80,6 +80,34 @@ def test_unaligned_rows(hpt, dev, dtype, shape):
             assert u.numpy().tobytes() == want.numpy().tobytes(), what
 
 
+# every second element of the rows: odd pitches, odd first elements, the row's last element the last of the memory or not, 512 threads per
+# row and more (whose workgroups walk the rows), aligned and not, and rows too long for the registers
+@pytest.mark.parametrize("dtype", ["f16", "bf16", "f32"])
+@pytest.mark.parametrize("rows,stored,first", [(5, 129, 0), (9, 130, 1), (33, 263, 0), (3, 1027, 2), (2100, 517, 1), (2100, 1279, 0), (9, 1281, 0), (600, 7897, 0), (5, 12287, 0), (5, 12291, 0), (3, 8190, 1), (530, 8192, 0), (2, 16385, 0),
+                                               (2, 32767, 0), (2, 32770, 1)])
+def test_every_second_element(hpt, dev, dtype, rows, stored, first):
+    rng = np.random.default_rng(stored + first)
+    x = (rng.standard_normal((rows, stored)) * 2).astype(np.float32)
+    x[-1, -1] = x[-1, -2] = 25
+    x[0, first] = 25
+    a, dt = _store(hpt, dtype, x)
+    t = hpt.Tensor.from_numpy(a, dt).to_hip(dev)[:, first::2]
+    v = _wide(hpt, dtype, a)[:, first::2]
+    cols = v.shape[1]
+    what = f"{dtype} [{rows}, {stored}][:, {first}::2] {hpt.normalize_plan(t, 1)[:40]}"
+    for log in (False, True):
+        _check(hpt, dtype, (t.log_softmax(1) if log else t.softmax(1)).numpy(), _softmax(v, log), f"{what} softmax log={log}")
+    (ga, _), (ba, _), (ra, _) = (_store(hpt, dtype, rng.normal(m, 0.1, n).astype(np.float32)) for m, n in ((1, cols), (0, cols), (0, (rows, cols))))
+    tg, tb, tr = (hpt.Tensor.from_numpy(u, dt).to_hip(dev) for u in (ga, ba, ra))
+    g, b = _wide(hpt, dtype, ga), _wide(hpt, dtype, ba)
+    _check(hpt, dtype, t.layernorm([cols], tg, tb, 1e-5).numpy(), _layernorm(v, g, b), f"{what} layernorm")
+    s = _wide(hpt, dtype, _store(hpt, dtype, (v + _wide(hpt, dtype, ra)).astype(np.float32))[0])
+    _check(hpt, dtype, t.add_layernorm(tr, [cols], tg, tb, 1e-5).numpy(), _layernorm(s, g, b), f"{what} add_layernorm")
+    got = t.softmax_causal(1.0, cols - rows if cols > rows else 3).numpy()
+    kept = np.arange(cols)[None, :] <= np.arange(rows)[:, None] + (cols - rows if cols > rows else 3)
+    _check(hpt, dtype, got, _softmax(np.where(kept, v, -np.inf), False), f"{what} causal")
+
+
 @pytest.mark.parametrize("dtype", ["f16", "bf16"])
 @pytest.mark.parametrize("heads,queries,keys", [(3, 40, 131), (2, 300, 301), (4, 9, 805), (1, 70, 2202), (2, 5, 4097), (1, 3, 9001)])
 def test_causal_rows(hpt, dev, dtype, heads, queries, keys):
