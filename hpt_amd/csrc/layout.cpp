@@ -873,12 +873,12 @@ NormPlan plan_normalize(const void* in_data, const void* out_data, const int64_t
                 if (vi == max_vec && out_ok) {
                     v = max_vec;
                     p.sstride = 2;
-                } else if ((elem_size == 2 ? p.cols >= 640 : elem_size == 4 && p.cols > 6144) && (p.cols + uv - 1) / uv <= 4096 && ((uintptr_t)in_data % elem_size) == 0 &&
+                } else if (elem_size == 2 && p.cols >= 640 && (p.cols + uv - 1) / uv <= 4096 && ((uintptr_t)in_data % elem_size) == 0 &&
                            ((uintptr_t)out_data % elem_size) == 0) {
-                    // Off the vector grid: the same vectors unaligned, for two-byte rows and the longest of four bytes (us, every second of
-                    // the stored, single elements and this: bf16 [3456, 7897] layernorm 26.9 and 19.1, softmax 21.6 and 16.8, [1920, 1763] 6.9 and
-                    // 5.3, f16 [2000, 16383] 37.1 and 26.9, but [768, 955] 5.0 and 5.5; f32 [2000, 16383] softmax 53.6 and 47.6, but [3456, 7897]
-                    // 32.3 and 35.7).
+                    // Two-byte rows off the vector grid: the same vectors unaligned (us, every second of the stored, single elements and
+                    // this: bf16 [3456, 7897] layernorm 26.9 and 19.1, softmax 21.6 and 16.8, [1920, 1763] 6.9 and 5.3, f16 [2000, 16383] 37.1
+                    // and 26.9, but [768, 955] 5.0 and 5.5. f32 goes either way: softmax [2000, 16383] 53.6 and 47.6, with sums over more
+                    // elements of a lane, [3456, 7897] 32.3 and 35.7).
                     v = max_vec;
                     p.sstride = 2;
                     p.shift = 1;

@@ -444,11 +444,11 @@ template <class T> void launch_t(const NormPlan& p, NormArgs a, hipStream_t st) 
             // Rows off the vector grid: two-byte types and the f32 layernorms as unaligned vectors, the others as the aligned vectors
             // that contain them.
             constexpr bool kUnaligned = sizeof(T) == 2 || (sizeof(T) == 4 && norm_is_layer(KIND));
-            if constexpr (sizeof(T) <= 4) {
+            if constexpr (sizeof(T) == 2) {
                 if (p.vec == FULL && p.ua_rows && p.sstride == 2) {
                     if (a.cols < FULL) fail(HPT_ERR_KERNEL, "row_reg: rows of %lld elements hold no vector", (long long)a.cols);
-                    if constexpr (KIND != NORM_ADD_LAYERNORM) {
-                        if (p.tpr >= 512 && (sizeof(T) >= 4 || norm_is_layer(KIND))) {
+                    if constexpr (KIND == NORM_LAYERNORM) {
+                        if (p.tpr >= 512) {
                             if (grid.x > 512u) grid.x = 512u;
                             launch_row_reg<T, FULL, 2, false, true, true>(p, a, grid, block, st);
                             return;
