@@ -655,8 +655,11 @@ static bool lds_row_shape(NormPlan& p, int64_t nvec, size_t elem_size, bool shif
 // that plan in `p` if so. Us over axis 1, as it was and this:
 //   four bytes, 129 ... 256 elements  [64, 129, 256] 9.8 and 6.8, [6, 200, 8200] 21.2 and 17.4, [20, 129, 8001] 48.8 and 34.2; where inner rows
 //     are whole 512-byte segments the 128-register form stays ([256, 256, 256] 20.4 and 22.2, though [16, 256, 2048] 18.0 and 15.2)
-//   257 ... 512  [1, 335, 58050] 88.6 and 45.2, [200, 335, 100] 29.0 and 19.6, [6, 512, 8200] 75.6 and 51.6, [16, 512, 1001] 22.4 and 23.3; where inner
-//     rows are whole 256-byte segments the 128-register form stays below 128 MiB and for very long rows ([16, 512, 2048] 25.3 and
+//   257 ... 512  [1, 335, 58050] 88.6 and 45.2, [200, 335, 100] 29.0 and 19.6, [6, 512, 8200] 75.6 and 51.6; odd inner rows
+//     of 28 ... 50 MB in all go either way and stay ([16, 512, 1001] 22.3 and 23.9, [128, 512, 129] 23.9 and 27.6,
+//     [8, 512, 3001] 28.2 and 30.7, [24, 400, 1001] 22.2 and 24.0, [24, 335, 1001] 19.9 and 20.1, but [11, 512, 1001] 18.8 and 17.1, [64, 512, 501]
+//     54.6 and 42.5, [64, 300, 257] 16.0 and 15.7, [256, 512, 65] 24.7 and 22.6); where inner rows
+//     are whole 256-byte segments the 128-register form stays below 128 MiB and for very long rows ([16, 512, 2048] 25.3 and
 //     29.5, [1, 512, 262144] 212 and 215; [512, 512, 512] 210 and 190, [64, 512, 1024] 53.2 and 50.1)
 //   513 ... 1024  [64, 777, 256] 28.3 and 21.5, [16, 1024, 2048] 92.2 and 53.4; one workgroup fills a compute unit, so there must be enough of
 //     them, of rows that are not short: [4, 1000, 1000] 16.8 and 18.9, [200, 1000, 100] 66.2 and 72.2
@@ -689,6 +692,8 @@ static bool tall_columns(NormPlan& p, bool found, const void* in_data, const voi
     } else if (elem_size == 4) {
         if (p.cols <= 128) return false;
         if (whole_segments && (p.cols <= 256 || L > 16384 || p.cols * L * batch * 4 < (128ll << 20))) return false;
+        const int64_t bytes = p.cols * L * batch * 4;
+        if (!grid && p.cols > 320 && L >= 96 && bytes >= (27ll << 20) && bytes < (52ll << 20)) return false;
     } else if (p.cols <= 64 || (grid && p.cols > 128 && p.cols <= 256 && L >= 1024 && p.cols * L * batch * 2 >= (64ll << 20))) {
         return false;
     }

@@ -79,6 +79,7 @@ def test_tall_columns_of_views(hpt, dev, dtype, shape, cut):
 @pytest.mark.parametrize("dtype,shape,want", [
     ("f32", (8, 128, 1000), None), ("f32", (8, 129, 1000), (32, 8)), ("f32", (8, 256, 1000), (32, 8)), ("f32", (8, 256, 1024), None),
     ("f32", (8, 257, 1000), (64, 8)), ("f32", (16, 512, 2048), None), ("f32", (64, 512, 1024), (64, 8)), ("f32", (1, 512, 262144), None), ("f32", (8, 512, 1001), (64, 8)),
+    ("f32", (16, 512, 1001), None), ("f32", (32, 512, 1001), (64, 8)), ("f32", (24, 321, 1001), None), ("f32", (24, 320, 1001), (64, 8)), ("f32", (16, 512, 1000), (64, 8)), ("f32", (256, 512, 65), (64, 8)),
     ("f32", (8, 513, 4000), (64, 16)), ("f32", (2, 513, 1000), None), ("f32", (8, 1025, 4000), None), ("f32", (2, 40, 30), (32, 8)), ("f32", (1, 300, 259), None),
     ("f16", (8, 64, 10000), None), ("f16", (8, 65, 1000), (32, 8)), ("f16", (8, 257, 1000), (32, 16)), ("bf16", (64, 256, 2048), None), ("f16", (16, 1000, 2048), (64, 16)),
     ("bf16", (1, 513, 58050), None), ("f16", (4, 777, 1000), None), ("f64", (8, 200, 1000), None),
