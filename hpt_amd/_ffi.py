@@ -6,6 +6,7 @@ loading fails with an instruction to build it.
 from __future__ import annotations
 
 import ctypes as C
+import warnings
 from pathlib import Path
 
 LIB_PATH = Path(__file__).resolve().parent / "lib" / "libhpt_hip.so"
@@ -124,18 +125,21 @@ def lib() -> C.CDLL:
     return _lib
 
 
-_calls = None
+_calls = ()  # not looked for yet
 
 
 def calls():
-    """The native module of the calls that return a fresh tensor (csrc/pycalls.cpp); it is linked to libhpt_hip.so."""
+    """The native module of the calls that return a fresh tensor (csrc/pycalls.cpp), which is linked to libhpt_hip.so. It is built for one
+    interpreter; under another, or where it was not built, None: every call then goes through ctypes, as those do that it does not take."""
     global _calls
-    if _calls is None:
+    if _calls == ():
         lib()  # (says what is missing when nothing has been built)
         try:
             from . import _calls as module
         except ImportError as e:
-            raise ImportError(f"hpt_amd._calls cannot be loaded ({e}): build it with `python -m hpt_amd.build`") from e
+            module = None
+            warnings.warn(f"hpt_amd._calls cannot be loaded ({e}), calls go through ctypes and take some microseconds longer: "
+                          "build it with `python -m hpt_amd.build`", RuntimeWarning, stacklevel=2)
         _calls = module
     return _calls
 
