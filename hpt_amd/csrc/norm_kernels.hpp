@@ -490,20 +490,27 @@ __global__ void __launch_bounds__(1024) row_reg_kernel(const NormArgs a) {
 #pragma unroll
             for (int c = 0; c < NCHUNK; ++c) {
                 const bool in_row_c = (c * tpr + tx) < nv;
-                auto square = [&](auto last) {
+                auto square = [&](int j, bool in_row_e) {
+                    const CT d = in_row_e ? (x[c][j] - mean_hi) - mean_lo : (CT)0;
+                    x[c][j] = d;
+                    q += d * d;
+                };
+                if constexpr (UA) {
+                    if (c * tpr + tx == nv - 1) {
+#pragma unroll
+                        for (int j = 0; j < UV; ++j) square(j, j >= twice);
+                    } else {
+#pragma unroll
+                        for (int j = 0; j < UV; ++j) square(j, in_row_c);
+                    }
+                } else {
 #pragma unroll
                     for (int j = 0; j < UV; ++j) {
-                        const bool in_row_e = SHIFT ? inside(c * tpr + tx, j) : decltype(last)::value ? j >= twice : in_row_c;
+                        const bool in_row_e = SHIFT ? inside(c * tpr + tx, j) : in_row_c;
                         const CT d = in_row_e ? (x[c][j] - mean_hi) - mean_lo : (CT)0;
                         x[c][j] = d;
                         q += d * d;
                     }
-                };
-                if constexpr (UA) {
-                    if (c * tpr + tx == nv - 1) square(std::true_type{});
-                    else square(std::false_type{});
-                } else {
-                    square(std::false_type{});
                 }
             }
             const ST var = row_all_reduce<SumC<ST>>((ST)q, tpr, ty, ssmem) * (ST)a.inv_cols;
