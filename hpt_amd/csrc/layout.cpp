@@ -104,12 +104,12 @@ static int legal_vec(const void* data, size_t elem_size, int64_t inner_len, cons
 constexpr int64_t kBlocksToFill = 2048;
 constexpr int64_t kComputeUnits = 256;  // MI355X
 
-// Slices of the reduced range for `groups` workgroups that share it: the count that fills one, two, three or four rounds of
+// Slices of the reduced range for `groups` workgroups that share it: the count that fills one, two ... `most` rounds of
 // compute units to nine tenths, or the one that comes closest.
-static int64_t full_rounds(int64_t groups) {
+static int64_t full_rounds(int64_t groups, int64_t most = 4) {
     int64_t best = 1;
     double best_fill = 0;
-    for (int64_t r = 1; r <= 4; ++r) {
+    for (int64_t r = 1; r <= most; ++r) {
         const int64_t S = r * kComputeUnits / groups;
         const double fill = (double)(S * groups) / (double)(r * kComputeUnits);
         if (S >= 1 && fill > best_fill) {
@@ -1359,7 +1359,7 @@ NormPlan plan_normalize(const void* in_data, const void* out_data, const int64_t
             const int64_t lanes = L / max_vec;
             bool wide = vec_ok && L > 1024 * max_vec;
             if (elem_size == 4) wide = vec_ok ? L > 1024 || (L >= 512 && all_bytes < (64ll << 20)) : L >= 768 && batch == 1;
-            else if (elem_size == 2) wide = vec_ok ? L >= 320 && (all_bytes < (48ll << 20) || lanes * 3 >= (lanes + 63) / 64 * 64 * 2) : L >= 768 && batch == 1;
+            else if (elem_size == 2) wide = vec_ok ? L >= 320 && (all_bytes < (44ll << 20) || lanes * 3 >= (lanes + 63) / 64 * 64 * 2) : L >= 768 && batch == 1;
             if (max_vec > 1 && !wide && sa == L && ((uintptr_t)in_data % elem_size) == 0 &&
                 ((uintptr_t)out_data % elem_size) == 0 && batch * p.cols * L * (int64_t)elem_size >= (8ll << 20)) {
                 // (slabs that start off 16-byte boundaries take the same vectors unaligned: `shift`)
@@ -1393,11 +1393,18 @@ NormPlan plan_normalize(const void* in_data, const void* out_data, const int64_t
                 p.shift = 1;
             }
             // One workgroup per compute unit for the statistics pass (its loads are in flight two batches deep), or the
-            // few rounds of them that leave the fewest units idle.
+            // two if they leave fewer units idle (not three: f64 [1344, 8248], 7 and 11 slices, 60.3 and 64.3 us, f32 [1344, 16500] 55.6 and 57.5).
             const int64_t groups = (L + 64 * v - 1) / (64 * v) * batch;
-            p.tsplit = (int)std::min(full_rounds(groups), std::max<int64_t>(1, p.cols / 32));
-            // (beyond 64 partials per row the finalize pass grows: 64 columns each then, f32 [4100, 63] 11.7 -> 10.6 us)
-            if (p.tsplit > 64) p.tsplit = (int)std::max<int64_t>(64, std::min<int64_t>(p.tsplit, p.cols / 64));
+            if (v > 1) {
+                p.tsplit = (int)std::min(full_rounds(groups, 2), std::max<int64_t>(1, p.cols / 32));
+                // (beyond 64 partials per row the finalize pass grows: 64 columns each then, f32 [8122, 76] 16.3 -> 15.9 us)
+                if (p.tsplit > 64) p.tsplit = (int)std::max<int64_t>(64, std::min<int64_t>(p.tsplit, p.cols / 64));
+            } else {
+                // Single elements, of which a wavefront has little to read and its last lanes often nothing: two workgroups per unit, up to
+                // 64 partials per row, 128 of a long axis (us, full rounds and this: f16 [2056, 271] 10.1 and 9.2, [4270, 268] 12.1 and 11.3, f32 [7353,
+                // 79] 14.4 and 13.3, [4100, 63] 64 10.8, 128 11.2; [13675, 122] 64 17.3, 128 16.6).
+                p.tsplit = (int)std::max<int64_t>(1, std::min<int64_t>({512 / groups, p.cols / 32, p.cols >= 10000 ? 128 : 64}));
+            }
             p.tpr = elem_size == 2 && v > 1 && p.cols >= 128 * p.tsplit ? 8 : 4;  // wavefronts per workgroup of the statistics pass
             p.scratch_bytes = (size_t)p.rows * p.tsplit * 16 + (size_t)p.rows * 3 * 8;
             return p;
@@ -1456,6 +1463,7 @@ std::string describe(const NormPlan& p) {
              names[(int)p.kind], p.sstride == 2 ? "-step2" : (p.flat_t ? (p.shift ? "-flat-unaligned" : "-flat") : (p.shift ? ((p.kind == NormKind::RowSplit || p.kind == NormKind::ColReg || p.kind == NormKind::ColSplit || p.kind == NormKind::Transposed || p.kind == NormKind::TransposedTile) ? "-unaligned" : (p.lds_rows ? "-lds-shift" : "-shift")) : (p.gb_lds == 2 ? "-l2gb" : p.gb_lds ? "-ldsgb" : (p.raw_rows ? "-raw" : (p.lds_rows ? "-lds" : ""))))), p.tile_rows ? "+tile" : (p.interleave > 1 ? "-interleaved" : p.interleave < 0 ? "-modular" : p.group_tile ? "-group-tile" : (p.slab_tile ? "-slab" : "")), (long long)p.rows, (long long)p.cols, p.vec, p.tpr, p.rpb,
              p.nchunk, (long long)p.out_axis_stride);
     std::string s = buf;
+    if (p.kind == NormKind::ColSplit || p.kind == NormKind::Transposed) s += "split=" + std::to_string(p.tsplit) + " ";
     if (p.kind == NormKind::RowReg) s += "max_blocks=" + std::to_string(p.max_blocks) + " ";  // (layernorm walks its rows)
     describe_dims(s, "rows_in", p.kept_in);
     s += " ";

@@ -114,7 +114,12 @@ template <class T, int VEC> void launch_col_split(const NormPlan& p, const NormA
     // apply: sixteen positions of the axis per workgroup, one batch of four loads per thread; what runs at one time is then
     // one stretch of memory (f32 [8192, 4096] over axis 0, all three passes, 16 / 32 / 48 positions: 65.2, 70.7, 67.4 us;
     // [32768, 1024] 66.3, 68.4, 68.6; f16 [8190, 4097] 42.0, 43.1, 43.1)
-    int64_t chunks = std::min<int64_t>((t.cols + 15) / 16, 65535);
+    // (Twelve where sixteen unaligned positions span 256 KiB and a line or less: the workgroups that run together then start almost in
+    // step with the memory's interleaving. f32 [2047, 4097] 30.5 -> 28.2 us, [8190, 4097] 77.3 -> 75.5, f16 [2047, 8193] 29.1 -> 27.5; with
+    // aligned rows, with other multiples of 256 KiB and two lines off it there is no difference.)
+    const int64_t span = 16 * t.sa * (int64_t)sizeof(T) - (256 << 10);
+    const int64_t most = ua && span >= 0 && span <= 128 ? 12 : 16;
+    int64_t chunks = std::min<int64_t>((t.cols + most - 1) / most, 65535);
     const int chunk = (int)((t.cols + chunks - 1) / chunks);
     chunks = (t.cols + chunk - 1) / chunk;
     if constexpr (VEC > 1) {

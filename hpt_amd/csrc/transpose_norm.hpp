@@ -188,9 +188,12 @@ __global__ void __launch_bounds__(1024) transposed_stats_kernel(const Transposed
     // on its SIMD is enough then, and the fewer wavefronts read side by side the better the rows of memory they open are
     // used (softmax over axis 0, this pass alone, us: f32 [8190, 4097] two workgroups per compute unit without the second
     // batch 32.1, one 36.1, with it 32.1 and 26.1; [32768, 1024] 33.4 -> 23.3. Two-byte elements, twice the arithmetic
-    // per byte, take shorter batches and twice the wavefronts: f16 [8190, 4097] 19.4 -> 15.4).
+    // per byte, take shorter batches and twice the wavefronts: f16 [8190, 4097] 19.4 -> 15.4; single elements, a few bytes of a line each, the
+    // long ones). The second batch costs registers, f32 softmax 64 -> 111 and layernorm as many, so four wavefronts fit a SIMD
+    // instead of eight; no plan has more than two there. Transposed rows, all three passes, us: f32 [30000, 500] softmax 61.1 -> 51.5, layernorm
+    // 47.0 -> 44.6, f16 [16384, 1024] layernorm 28.8 -> 25.3, [30000, 500] 44.8 -> 35.9, [8192, 8192] no difference.
     // (The last round's loads are repeated, not left out: behind a test the wait before the fold would be a full one.)
-    constexpr int kBatch = KIND != NORM_LAYERNORM && sizeof(T) == 2 ? 4 : 8;
+    constexpr int kBatch = KIND != NORM_LAYERNORM && sizeof(T) == 2 && VEC > 1 ? 4 : 8;
     const int64_t stepb = (int64_t)P * a.sa;
     const T* p = base + (int64_t)pid * a.sa;
     int c = pid;
@@ -216,21 +219,25 @@ __global__ void __launch_bounds__(1024) transposed_stats_kernel(const Transposed
         while (step(va, vb) && step(vb, va)) {
         }
     }
-    // the rest: four together, then one at a time
-    if constexpr (kBatch > 4) {
-        if (c + 3 * P < a.cols) {
-            Pack<T, VEC> v[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) v[i] = UA ? load_pack_unaligned<T, VEC>(p + i * stepb) : load_pack<T, VEC>(p + i * stepb);
-            p += 4 * stepb;
-            c += 4 * P;
-            fold(v, std::integral_constant<int, 4>{});
-        }
-    }
-    for (; c < a.cols; c += P) {
-        Pack<T, VEC> v = UA ? load_pack_unaligned<T, VEC>(p) : load_pack<T, VEC>(p);
-        p += stepb;
-        fold(&v, std::integral_constant<int, 1>{});
+    // the rest, fewer than a batch: four, two and one of them, all loaded before any is folded (one after the other each waits a memory
+    // latency); a part that is not there repeats the last column's load and is left out of the fold
+    if (c < a.cols) {
+        const int left = (a.cols - 1 - c) / P + 1;
+        Pack<T, VEC> v[kBatch - 1];
+        auto load_part = [&](int slot, int n, int first) {
+            for (int i = 0; i < n; ++i) {
+                const T* q = p + min(first + i, left - 1) * stepb;
+                v[slot + i] = UA ? load_pack_unaligned<T, VEC>(q) : load_pack<T, VEC>(q);
+            }
+        };
+        if constexpr (kBatch > 4) load_part(3, 4, 0);
+        load_part(1, 2, left & 4);
+        load_part(0, 1, left - 1);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (kBatch > 4)
+            if (left & 4) fold(v + 3, std::integral_constant<int, 4>{});
+        if (left & 2) fold(v + 1, std::integral_constant<int, 2>{});
+        if (left & 1) fold(v, std::integral_constant<int, 1>{});
     }
 
     // The wavefronts of a workgroup hold partials of the same rows: they meet in LDS
