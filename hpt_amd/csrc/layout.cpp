@@ -851,10 +851,16 @@ NormPlan plan_normalize(const void* in_data, const void* out_data, const int64_t
                     return p;
                 }
                 p.kind = NormKind::Transposed;
-                // statistics pass: a wavefront covers 64*v rows; enough column splits for
-                // about 2048 wavefronts, each keeping at least 32 columns
+                // statistics pass: a wavefront covers 64*v rows, every one keeps at least 32 columns. Its loads are in flight two batches
+                // deep, so one workgroup per compute unit is enough (us, two and one, stored [columns, rows]: f32 [8192, 8192] softmax 145 and
+                // 130, layernorm 144 and 130, [6000, 6000] 98.4 and 92.7, 92.1 and 89.3; f16 [8192, 8192] layernorm 78.7 and 72.6; f64 [8192, 4096] softmax
+                // 152 and 134, though [6000, 6000] 156 and 166). Two-byte softmax, twice the arithmetic per byte, keeps two (f16 [16384, 4096] 74.7
+                // and 76.7, [6000, 6000] 57.5 and 60.4), unless that many would leave wavefronts too few columns: then what there is fills
+                // one round and not a part of the second (f16 [5001, 4001] softmax, 312 workgroups and 256, 41.3 and 39.0).
                 const int64_t groups = (R + 64 * v - 1) / (64 * v) * batch;
-                int64_t S = std::max<int64_t>(1, std::min<int64_t>(512 / groups, p.cols / 128));
+                const int64_t want = elem_size == 2 && n_norm_dims <= 0 ? 512 / groups : full_rounds(groups, 2);
+                int64_t S = std::max<int64_t>(1, std::min<int64_t>(want, p.cols / 128));
+                if (S < want && S * groups > kComputeUnits && S * groups * 10 < 2 * kComputeUnits * 9) S = kComputeUnits / groups;
                 p.tsplit = (int)std::min<int64_t>(S, 64);
                 p.tpr = 4;  // wavefronts per workgroup of the statistics pass
                 p.scratch_bytes = (size_t)p.rows * p.tsplit * 16 + (size_t)p.rows * 3 * 8;

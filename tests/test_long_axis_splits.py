@@ -21,6 +21,15 @@ def test_slices_of_a_long_axis(hpt, dtype, cols, inner, slices):
     assert hpt.normalize_plan(t, 0).startswith("col-split") and _split(hpt, t, 0) == slices
 
 
+@pytest.mark.parametrize("dtype,cols,rows,softmax,layernorm", [
+    ("f32", 8192, 8192, 8, 8), ("f16", 8192, 8192, 32, 16), ("bf16", 5001, 4001, 32, 32), ("f64", 5001, 1001, 32, 32), ("f32", 16384, 1024, 64, 64),
+    ("f32", 5000, 40000, 3, 3)])
+def test_slices_of_transposed_rows(hpt, dtype, cols, rows, softmax, layernorm):
+    t = hpt.Tensor.from_raw(1 << 40, [cols, rows], getattr(hpt, dtype)).permute([1, 0])
+    assert hpt.normalize_plan(t, 1).startswith("transposed")
+    assert (_split(hpt, t, 1), _split(hpt, t, 0, 1)) == (softmax, layernorm)
+
+
 # 256 wavefronts share an axis of 64 slices: eight columns each and `left` more, some wavefronts one more still
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", ["f32", "f16"])
