@@ -444,7 +444,14 @@ template <class T> void launch_t(const NormPlan& p, NormArgs a, hipStream_t st) 
                 return;
             }
         }
-        if (norm_is_layer(KIND) && grid.x > (unsigned)p.max_blocks) grid.x = (unsigned)p.max_blocks;
+        unsigned walkers = (unsigned)p.max_blocks;
+        if constexpr (KIND == NORM_ADD_LAYERNORM && std::is_same<T, f16_t>::value) {
+            // Three vectors per thread in 96 registers: five workgroups of 256 threads per compute unit and not four (bf16 takes 101), so
+            // four rounds of them where every one still walks some rows (us, 3072 and this: [13107, 5120] 71.5 and 68.6, [20000, 3072] 64.5 and 61.7,
+            // [52428, 1536] 82.8 and 79.8; of 5000 workgroups 30.4 and 33.6, 7000 40.3 and 40.3).
+            if (p.gb_lds == 1 && p.nchunk == 3 && p.tpr < 512 && !p.shift && grid.x >= 7500) walkers = 5120;
+        }
+        if (norm_is_layer(KIND) && grid.x > walkers) grid.x = walkers;
         if constexpr (FULL > 1) {
             // Rows off the vector grid: two-byte types and the f32 layernorms as unaligned vectors, the others as the aligned vectors
             // that contain them.

@@ -32,3 +32,18 @@ def test_walked_rows(hpt, dev, dtype, rows, cols):
         tx, tr = hpt.Tensor.from_numpy(ax, dt).to_hip(dev), hpt.Tensor.from_numpy(ar, dt).to_hip(dev)
         out = tx.layernorm([cols], tg, tb, 1e-5, residual=tr, out={"fresh": None, "x": tx, "residual": tr}[place])
         assert_close(back(out.numpy()), want, HALF_RTOL, half_atol(want, bits), f"{dtype} {rows} x {cols}, {place}")
+
+
+# f16 rows of three vectors per thread: from 7500 workgroups on 5120 of them walk the rows
+@pytest.mark.parametrize("rows,cols", [(30001, 1032), (15001, 2056), (7505, 4104)])
+def test_more_than_five_thousand_workgroups(hpt, dev, rows, cols):
+    rng = np.random.default_rng(cols)
+    ax, ar = (rng.standard_normal((rows, cols), dtype=np.float32).astype(np.float16) for _ in range(2))
+    ag, ab = rng.normal(1, 0.1, cols).astype(np.float16), rng.normal(0, 0.1, cols).astype(np.float16)
+    tx, tr, tg, tb = (hpt.Tensor.from_numpy(v).to_hip(dev) for v in (ax, ar, ag, ab))
+    got = tx.add_layernorm(tr, [cols], tg, tb, 1e-5).numpy()
+    for r in range(0, rows, 4096):
+        s = (ax[r:r + 4096] + ar[r:r + 4096]).astype(np.float64)  # x + residual is rounded to the dtype
+        s -= s.mean(1, keepdims=True)
+        want = s / np.sqrt((s * s).mean(1, keepdims=True) + 1e-5) * ag.astype(np.float64) + ab
+        assert_close(got[r:r + 4096], want, HALF_RTOL, half_atol(want, 11), f"{rows} x {cols}")
