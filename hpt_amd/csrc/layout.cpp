@@ -881,15 +881,20 @@ NormPlan plan_normalize(const void* in_data, const void* out_data, const int64_t
                 const int uv = max_vec / 2;
                 int vi = legal_vec(in_data, elem_size, p.cols * 2, p.kept_in, none, 0, 0);
                 bool out_ok = ((uintptr_t)out_data % (uv * elem_size)) == 0 && p.cols % uv == 0;
+                // few rows of up to 4096 elements: single elements have up to four times the threads, and there is room for all of them (f16
+                // [340, 1763] stored layernorm 4.4, 5.6 as vectors, [389, 3853] 6.1 and 6.6, softmax [340, 1763] 3.8 and 4.2; from 1.3
+                // million elements on, or 0.6 million for softmax of short rows, the vectors are ahead)
+                const int64_t elements = p.rows * p.cols;
+                const bool few = !fused && p.cols <= 4096 && (n_norm_dims > 0 ? elements < 1300000 : p.cols < 1024 && elements < 600000);
                 if (vi == max_vec && out_ok) {
                     v = max_vec;
                     p.sstride = 2;
-                } else if (elem_size == 2 && p.cols >= 640 && (p.cols + uv - 1) / uv <= 4096 && ((uintptr_t)in_data % elem_size) == 0 &&
-                           ((uintptr_t)out_data % elem_size) == 0) {
+                } else if (elem_size == 2 && p.cols >= 640 && (p.cols + uv - 1) / uv <= 4096 && !(fused && n_norm_dims > 0) && !few &&
+                           ((uintptr_t)in_data % elem_size) == 0 && ((uintptr_t)out_data % elem_size) == 0) {
                     // Two-byte rows off the vector grid: the same vectors unaligned (us, every second of the stored, single elements and
-                    // this: bf16 [3456, 7897] layernorm 26.9 and 19.1, softmax 21.6 and 16.8, [1920, 1763] 6.9 and 5.3, f16 [2000, 16383] 37.1
-                    // and 26.9, but [768, 955] 5.0 and 5.5. f32 goes either way: softmax [2000, 16383] 53.6 and 47.6, with sums over more
-                    // elements of a lane, [3456, 7897] 32.3 and 35.7).
+                    // this: f16 [3456, 7897] causal 27.6 and 19.9, layernorm 30.9 and 28.3, [2000, 16383] softmax 39.8 and 28.8. f32 goes either way:
+                    // softmax [2000, 16383] 53.6 and 47.6, with sums over more elements of a lane, [3456, 7897] 32.3 and 35.7; x + residual keeps
+                    // single elements, its four vectors spill: f16 [3456, 7897] 35.2, 52.1 as vectors, [7598, 3853] 30.1, 54.8).
                     v = max_vec;
                     p.sstride = 2;
                     p.shift = 1;

@@ -552,10 +552,13 @@ template <class T> void launch_t(const NormPlan& p, NormArgs a, hipStream_t st) 
             }
         }
         if constexpr (FULL > 1 && KIND != NORM_ADD_LAYERNORM) {
-            // (every second element: the same walk; us, [:, ::2] of the stored: f32 [1472, 15296] layernorm 38.4 -> 36.3, softmax 37.2 ->
-            // 36.0, f16 [597, 14904] layernorm 11.1 -> 9.1, but its softmax 7.7 -> 8.2)
-            if (p.vec == FULL && p.sstride == 2 && p.tpr >= 512 && (sizeof(T) >= 4 || norm_is_layer(KIND))) {
-                if (grid.x > 512u) grid.x = 512u;
+            // (every second element: the same walk, where a workgroup has more than one row. us, [:, ::2] of the stored, without and with: f32
+            // of 1024 threads, or 512 with eight vectors, [1472, 15296] layernorm 36.2 and 34.5, causal 24.2 and 21.7, [2000, 10240] causal 19.9 and 17.6,
+            // f16 layernorm [1000, 16384] 14.7 and 11.8, [4000, 8704] 28.1 and 25.5; but of 512 threads with four vectors, three of whose workgroups
+            // fit a unit, f32 [3456, 8192] softmax 31.0 and 32.4, f64 layernorm [3456, 8192] 77.0 and 84.4, and f16 softmax [597, 14904] 7.7 and 8.2)
+            const bool walked = sizeof(T) == 4 ? p.tpr == 1024 || (p.tpr == 512 && p.nchunk == 8) : sizeof(T) == 2 && norm_is_layer(KIND) && p.tpr >= 512;
+            if (p.vec == FULL && p.sstride == 2 && grid.x > 512u && walked) {
+                grid.x = 512u;
                 launch_row_reg<T, FULL, 2, false, true>(p, a, grid, block, st);
                 return;
             }

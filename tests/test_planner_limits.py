@@ -28,3 +28,12 @@ def test_small_transposed_plans(hpt, dtype, cols, rows, softmax, layernorm):
     t = hpt.Tensor.from_raw(1 << 40, [cols, rows], getattr(hpt, dtype)).permute([1, 0])
     assert hpt.normalize_plan(t, 1).split()[0] == softmax
     assert hpt.normalize_plan(t, 0, 1).split()[0] == layernorm
+
+
+# every second element of two-byte rows off the vector grid: few rows stay with single elements, which have more threads
+@pytest.mark.parametrize("rows,stored,softmax,layernorm", [
+    (340, 1763, "rowreg", "rowreg"), (850, 1763, "rowreg-step2", "rowreg"), (2268, 1763, "rowreg-step2", "rowreg-step2"), (389, 3853, "rowreg-step2", "rowreg"),
+    (1038, 3853, "rowreg-step2", "rowreg-step2"), (50, 9001, "rowreg-step2", "rowreg-step2")])
+def test_every_second_element_of_few_rows(hpt, rows, stored, softmax, layernorm):
+    t = hpt.Tensor.from_raw(1 << 40, [rows, stored], hpt.f16)[:, ::2]
+    assert (hpt.normalize_plan(t, 1).split()[0], hpt.normalize_plan(t, 0, 1).split()[0]) == (softmax, layernorm)
