@@ -548,9 +548,9 @@ struct NormCall {
 static int norm_out_dtype(int in_dtype) { return reduce_out_dtype(HPT_MEAN, in_dtype); }
 
 // A non-float input is promoted inside the kernel; the plan is made for the output's element size and
-// cut down to what the promoting kernel runs. `float_only`: the fused kinds.
+// cut down to what the promoting kernel runs. `float_only`: the fused kinds; `residual`: where the other operand of theirs starts.
 static NormCall prepare_norm(const hpt_view* in, const void* out_data, int64_t axis, int n_norm_dims,
-                             bool float_only = false) {
+                             bool float_only = false, const void* residual = nullptr) {
     check_view(in, "normalize input", false);
     if (float_only && !is_float_dtype(in->dtype))
         fail(HPT_ERR_DTYPE, "this fused normalisation needs a float dtype, got %s", dtype_name(in->dtype));
@@ -565,7 +565,7 @@ static NormCall prepare_norm(const hpt_view* in, const void* out_data, int64_t a
     }
     NormCall c;
     c.plan = plan_normalize(in->data, out_data, in->shape, in->strides, in->ndim, axis, n_norm_dims,
-                            dtype_size(norm_out_dtype(in->dtype)), float_only);
+                            dtype_size(norm_out_dtype(in->dtype)), float_only, residual);
     if (!is_float_dtype(in->dtype)) restrict_to_row_stream(c.plan);
     NormArgs& a = c.args;
     memset(&a, 0, sizeof a);
@@ -867,7 +867,7 @@ static void run_layernorm(int dev, void* stream, const hpt_view* in, const hpt_v
     const int odt = norm_out_dtype(in->dtype);
     check_out(out, odt, view_size(in), "layernorm output");
     check_alias(in, out, true, "layernorm", "the input");
-    NormCall c = prepare_norm(in, out->data, 0, n_norm_dims, residual != nullptr);
+    NormCall c = prepare_norm(in, out->data, 0, n_norm_dims, residual != nullptr, residual ? residual->data : nullptr);
     const hpt_view* gb[2] = {gamma, beta};
     const char* names[2] = {"layernorm gamma", "layernorm beta"};
     for (int k = 0; k < 2; ++k) {

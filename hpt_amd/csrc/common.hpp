@@ -173,7 +173,7 @@ struct NormPlan {
 // causal softmax, which the plain softmax's register + LDS kernels do not implement.
 NormPlan plan_normalize(const void* in_data, const void* out_data, const int64_t* shape,
                         const int64_t* strides, int ndim, int64_t axis, int n_norm_dims,
-                        size_t elem_size, bool fused = false);
+                        size_t elem_size, bool fused = false, const void* residual = nullptr);
 
 std::string describe(const NormPlan& p);
 

@@ -708,7 +708,7 @@ static bool tall_columns(NormPlan& p, bool found, const void* in_data, const voi
 
 NormPlan plan_normalize(const void* in_data, const void* out_data, const int64_t* shape,
                         const int64_t* strides, int ndim, int64_t axis, int n_norm_dims,
-                        size_t elem_size, bool fused) {
+                        size_t elem_size, bool fused, const void* residual) {
     NormPlan p;
     int64_t total = 1;
     for (int i = 0; i < ndim; ++i) total *= shape[i];
@@ -933,9 +933,31 @@ NormPlan plan_normalize(const void* in_data, const void* out_data, const int64_t
                 // causal [32, 1001, 1001] 26.9 and 20.7; f16 layernorm [8190, 4097] 59.7 and 33.7, [14245, 561] 14.4 and 11.2, [2000, 12001]
                 // (streamed) 31.4 and 22.7; f32 layernorm [8190, 4097] 60.4 and 49.6, [3000, 9001] (streamed) 61.6 and 43.9. The f32 softmax
                 // is as fast as that of aligned rows ([16000, 2051] 45.3, [16000, 2052] 47.2).
+                // Where the masks fit the registers and there is no row to prefetch, or no gain in it, whole aligned lines are ahead of
+                // stores across them: f32 layernorm up to 256 threads per row ([10695, 561] 12.3 and 13.4 us, [7751, 774] 12.2 and 13.3,
+                // [4552, 1318] 12.3 and 13.2, [485, 3090] 6.1 and 6.6; 512 threads [1464, 4097] 15.8 and 12.6, but few rows [336, 4458]
+                // 6.5 and 6.9), f32 x + residual up to three vectors per thread ([8000, 750] 15.6 and 16.3, [4304, 1394] 15.8 and 16.6; four
+                // spill, [1941, 3090] 20.4 and 16.9), two-byte softmax of 512 threads ([5224, 9571] 43.6 and 46.9, [857, 14001] 15.2 and 16.5,
+                // but [61, 12292], whose rows are four elements off, 6.2 and 5.6, and one row per workgroup [59, 12531] 6.3 and 5.9) and large inputs of
+                // 256 ([6816, 7335] log_softmax 37.7 and 41.4, [9043, 5529] 36.2 and 39.0; [1635, 7335] 13.7 and 13.3).
+                // Input and output off the grid by different amounts took single elements: they stay where stores across lines cost more than
+                // they save, short rows (f32 layernorm [61855, 97] 15.5 and 17.4, x + residual [55813, 215] 17.7 and 19.4, f16 x + residual [68181, 176]
+                // 21.8 and 23.2; [45627, 263] 27.3 and 24.2), and layernorm of few (f32 [1425, 263] 4.3 and 5.2, [178, 2100] 4.9 and 5.5).
                 const int64_t nvu = (p.cols + max_vec - 1) / max_vec;
-                if ((elem_size == 2 || (elem_size == 4 && n_norm_dims > 0)) && ((uintptr_t)in_data % elem_size) == 0 && ((uintptr_t)out_data % elem_size) == 0 &&
-                    nvu <= (elem_size == 4 ? 4096 : 2048)) {
+                bool unaligned = (elem_size == 2 || (elem_size == 4 && n_norm_dims > 0)) && ((uintptr_t)in_data % elem_size) == 0 &&
+                                 ((uintptr_t)out_data % elem_size) == 0 && nvu <= (elem_size == 4 ? 4096 : 2048);
+                if (unaligned && same && (((uintptr_t)residual ^ (uintptr_t)(residual ? out_data : nullptr)) & 15) == 0) {
+                    const int64_t quarter = pow2_ceil((nvs + 3) / 4);  // threads that hold the row in three or four vectors each
+                    if (elem_size == 4 && !fused) unaligned = p.cols <= 256 || nvs > (p.rows <= 512 ? 2048 : 1024);
+                    else if (elem_size == 4) unaligned = p.cols <= 512 || nvs > 2048 || (nvs > 3 * quarter && quarter != 128);
+                    else if (n_norm_dims <= 0 && !fused && nvs <= 2048 && p.cols % 4 != 0)
+                        unaligned = nvu > 1024 ? p.rows <= 512 : nvu <= 512 || p.rows * p.cols * 2 < (48ll << 20);
+                } else if (unaligned && !same && n_norm_dims > 0) {
+                    if (fused) unaligned = p.cols >= 256 || (elem_size == 4 && p.cols >= 128 && p.cols % 4 == 0);
+                    else unaligned = (elem_size == 2 || (p.cols >= 128 && (p.cols <= 192 || p.cols >= 256))) &&
+                                     (p.cols >= (elem_size == 2 ? 1024 : 4096) || p.rows * p.cols * (int64_t)elem_size >= (3ll << 20));
+                }
+                if (unaligned) {
                     v = max_vec;
                     p.vec = v;
                     p.shift = 1;
@@ -993,7 +1015,10 @@ NormPlan plan_normalize(const void* in_data, const void* out_data, const int64_t
             // [131072, 512] 4.9 -> 4.5).
             // (With a residual's vectors beside the row's, gamma / beta in registers spill from the third vector on: beyond 256
             // elements, us: f16 [14245, 560] 20.9 -> 12.5, [14245, 561] 28.9 -> 13.9, [30000, 384] 22.8 -> 16.4; bf16 [30000, 256] 11.4, 14.8 this way.)
-            if (ln_half && p.sstride == 1 && !masks && nv * v >= (fused ? 264 : 640) && nv * v <= 16384) {
+            // (Few unaligned rows that would take four vectors per thread keep them in registers, two vectors and twice the threads: f16 [121, 6149] 5.9
+            // and 6.5, [428, 7001] 7.9 and 8.1; not three: [250, 3000] 6.3 and 5.6.)
+            const bool few_unaligned = p.ua_rows && !fused && p.rows <= 512 && nv > 3 * pow2_ceil((nv + 3) / 4);
+            if (ln_half && p.sstride == 1 && !masks && nv * v >= (fused ? 264 : 640) && nv * v <= 16384 && !few_unaligned) {
                 p.gb_lds = 1;
                 ln_half = false;
             }
@@ -1444,6 +1469,7 @@ void demote_to_generic(NormPlan& p) {
     p.vec = 1;
     p.shift = 0;
     p.ua_rows = 0;
+    p.tall = 0;
     p.sstride = 1;
     p.nchunk = 1;
     p.scratch_bytes = 0;
@@ -1474,6 +1500,7 @@ std::string describe(const NormPlan& p) {
              names[(int)p.kind], p.sstride == 2 ? "-step2" : (p.flat_t ? (p.shift ? "-flat-unaligned" : "-flat") : (p.shift ? ((p.kind == NormKind::RowSplit || p.kind == NormKind::ColReg || p.kind == NormKind::ColSplit || p.kind == NormKind::Transposed || p.kind == NormKind::TransposedTile) ? "-unaligned" : (p.lds_rows ? "-lds-shift" : "-shift")) : (p.gb_lds == 2 ? "-l2gb" : p.gb_lds ? "-ldsgb" : (p.raw_rows ? "-raw" : (p.lds_rows ? "-lds" : ""))))), p.tile_rows ? "+tile" : (p.interleave > 1 ? "-interleaved" : p.interleave < 0 ? "-modular" : p.group_tile ? "-group-tile" : (p.slab_tile ? "-slab" : "")), (long long)p.rows, (long long)p.cols, p.vec, p.tpr, p.rpb,
              p.nchunk, (long long)p.out_axis_stride);
     std::string s = buf;
+    if (p.ua_rows) s += "unaligned ";
     if (p.kind == NormKind::ColSplit || p.kind == NormKind::Transposed) s += "split=" + std::to_string(p.tsplit) + " ";
     if (p.kind == NormKind::RowReg) s += "max_blocks=" + std::to_string(p.max_blocks) + " ";  // (layernorm walks its rows)
     describe_dims(s, "rows_in", p.kept_in);

@@ -21,29 +21,84 @@ inline int ilog2(int v) {
     return l;
 }
 
-template <class T, int VEC, int SS = 1, bool SHIFT = false, bool PF = false, bool UA = false>
+// The row kernel of full vectors for the numbers of vectors per thread that the plan has in this form.
+template <class T, int SS, bool SHIFT, bool PF, bool UA, int... NC>
+void launch_row_of(const NormPlan& p, const NormArgs& a, dim3 grid, dim3 block, hipStream_t st) {
+    const bool done = ((p.nchunk == NC && (row_reg_kernel<KIND, T, 16 / sizeof(T), NC, SS, SHIFT, PF, 0, 1, UA><<<grid, block, 0, st>>>(a), true)) || ...);
+    if (!done) fail(HPT_ERR_KERNEL, "row_reg: no kernel of %d vectors per thread in this form", p.nchunk);
+}
+
+template <class T, int VEC, int SS = 1, bool PF = false>
 void launch_row_reg(const NormPlan& p, const NormArgs& a, dim3 grid, dim3 block, hipStream_t st) {
     // (3, 5, 6 and 7 vectors per thread: rows of whole vectors whose length is 3, 5, 6 or 7 times a power of
     // two - 768, 1536, 2560, 3072, 3584, 5120, 6144 ... - without idle lanes; full-vector rows only)
     if constexpr (VEC > 1 && SS == 1) {
         switch (p.nchunk) {
-            case 3: row_reg_kernel<KIND, T, VEC, 3, SS, SHIFT, PF, 0, 1, UA><<<grid, block, 0, st>>>(a); return;
-            case 5: row_reg_kernel<KIND, T, VEC, 5, SS, SHIFT, PF, 0, 1, UA><<<grid, block, 0, st>>>(a); return;
-            case 6: row_reg_kernel<KIND, T, VEC, 6, SS, SHIFT, PF, 0, 1, UA><<<grid, block, 0, st>>>(a); return;
-            case 7: row_reg_kernel<KIND, T, VEC, 7, SS, SHIFT, PF, 0, 1, UA><<<grid, block, 0, st>>>(a); return;
+            case 3: row_reg_kernel<KIND, T, VEC, 3, SS, false, PF><<<grid, block, 0, st>>>(a); return;
+            case 5: row_reg_kernel<KIND, T, VEC, 5, SS, false, PF><<<grid, block, 0, st>>>(a); return;
+            case 6: row_reg_kernel<KIND, T, VEC, 6, SS, false, PF><<<grid, block, 0, st>>>(a); return;
+            case 7: row_reg_kernel<KIND, T, VEC, 7, SS, false, PF><<<grid, block, 0, st>>>(a); return;
             default: break;
         }
     }
     switch (p.nchunk) {
-        case 1: row_reg_kernel<KIND, T, VEC, 1, SS, SHIFT, PF, 0, 1, UA><<<grid, block, 0, st>>>(a); break;
-        case 2: row_reg_kernel<KIND, T, VEC, 2, SS, SHIFT, PF, 0, 1, UA><<<grid, block, 0, st>>>(a); break;
-        case 4: row_reg_kernel<KIND, T, VEC, 4, SS, SHIFT, PF, 0, 1, UA><<<grid, block, 0, st>>>(a); break;
-        case 8: row_reg_kernel<KIND, T, VEC, 8, SS, SHIFT, PF, 0, 1, UA><<<grid, block, 0, st>>>(a); break;
+        case 1: row_reg_kernel<KIND, T, VEC, 1, SS, false, PF><<<grid, block, 0, st>>>(a); break;
+        case 2: row_reg_kernel<KIND, T, VEC, 2, SS, false, PF><<<grid, block, 0, st>>>(a); break;
+        case 4: row_reg_kernel<KIND, T, VEC, 4, SS, false, PF><<<grid, block, 0, st>>>(a); break;
+        case 8: row_reg_kernel<KIND, T, VEC, 8, SS, false, PF><<<grid, block, 0, st>>>(a); break;
         default: fail(HPT_ERR_KERNEL, "row_reg: unsupported chunk count %d", p.nchunk);
     }
 }
 
 // Few, very long rows: several workgroups per row.
+// Rows off the vector grid as unaligned vectors (two-byte types, f32 layernorms).
+template <class T> void launch_row_unaligned(const NormPlan& p, const NormArgs& a, dim3 grid, dim3 block, hipStream_t st) {
+    constexpr int FULL = 16 / sizeof(T);
+    if (a.cols < FULL) fail(HPT_ERR_KERNEL, "row_reg: rows of %lld elements hold no vector", (long long)a.cols);
+    if constexpr (sizeof(T) == 2) {
+        if (p.sstride == 2) {
+            // (every second element; x + residual has no such plan: its four vectors spill)
+            if constexpr (KIND == NORM_ADD_LAYERNORM) {
+                fail(HPT_ERR_KERNEL, "row_reg: no kernel for every second element of x + residual");
+            } else if constexpr (KIND == NORM_LAYERNORM) {
+                if (p.tpr >= 512) {
+                    if (grid.x > 512u) grid.x = 512u;
+                    launch_row_of<T, 2, false, true, true, 4>(p, a, grid, block, st);
+                } else {
+                    launch_row_of<T, 2, false, false, true, 4>(p, a, grid, block, st);
+                }
+            } else {
+                launch_row_of<T, 2, false, false, true, 2, 4>(p, a, grid, block, st);
+            }
+            return;
+        }
+        if constexpr (norm_is_layer(KIND)) {
+            if (p.gb_lds == 1) {
+                const size_t smem = 2 * (size_t)((p.cols + FULL - 1) / FULL) * FULL * sizeof(T);
+                if (p.tpr >= 512 && grid.x > 512u) grid.x = 512u;
+                if (p.nchunk == 3) row_reg_kernel<KIND, T, FULL, 3, 1, false, false, 1, 1, true><<<grid, block, smem, st>>>(a);
+                else if (p.nchunk == 4) row_reg_kernel<KIND, T, FULL, 4, 1, false, false, 1, 1, true><<<grid, block, smem, st>>>(a);
+                else fail(HPT_ERR_KERNEL, "row_reg: no kernel of %d vectors per thread in this form", p.nchunk);
+                return;
+            }
+        }
+        if constexpr (KIND == NORM_ADD_LAYERNORM) launch_row_of<T, 1, false, false, true, 2>(p, a, grid, block, st);
+        else if constexpr (KIND == NORM_LAYERNORM) launch_row_of<T, 1, false, false, true, 2, 3>(p, a, grid, block, st);
+        else launch_row_of<T, 1, false, false, true, 2, 3, 4>(p, a, grid, block, st);
+    } else if constexpr (sizeof(T) == 4 && KIND == NORM_ADD_LAYERNORM) {
+        launch_row_of<T, 1, false, false, true, 2, 3, 4>(p, a, grid, block, st);
+    } else if constexpr (sizeof(T) == 4 && KIND == NORM_LAYERNORM) {
+        if (p.tpr >= 512) {
+            if (grid.x > 512u) grid.x = 512u;
+            launch_row_of<T, 1, false, true, true, 3, 4, 5, 6>(p, a, grid, block, st);
+        } else {
+            launch_row_of<T, 1, false, false, true, 2, 3, 4, 5>(p, a, grid, block, st);
+        }
+    } else {
+        fail(HPT_ERR_KERNEL, "row_reg: rows of this type are no unaligned vectors");
+    }
+}
+
 template <class T, int VEC, bool UA> void launch_row_split(const NormPlan& p, const NormArgs& a, hipStream_t st) {
     RowSplitArgs r{};
     r.in = a.in;
@@ -453,52 +508,24 @@ template <class T> void launch_t(const NormPlan& p, NormArgs a, hipStream_t st) 
         }
         if (norm_is_layer(KIND) && grid.x > walkers) grid.x = walkers;
         if constexpr (FULL > 1) {
-            // Rows off the vector grid: two-byte types and the f32 layernorms as unaligned vectors, the others as the aligned vectors
-            // that contain them.
-            constexpr bool kUnaligned = sizeof(T) == 2 || (sizeof(T) == 4 && norm_is_layer(KIND));
-            if constexpr (sizeof(T) == 2) {
-                if (p.vec == FULL && p.ua_rows && p.sstride == 2) {
-                    if (a.cols < FULL) fail(HPT_ERR_KERNEL, "row_reg: rows of %lld elements hold no vector", (long long)a.cols);
-                    if constexpr (KIND == NORM_LAYERNORM) {
-                        if (p.tpr >= 512) {
-                            if (grid.x > 512u) grid.x = 512u;
-                            launch_row_reg<T, FULL, 2, false, true, true>(p, a, grid, block, st);
-                            return;
-                        }
-                    }
-                    launch_row_reg<T, FULL, 2, false, false, true>(p, a, grid, block, st);
-                    return;
-                }
+            // Rows off the vector grid: as unaligned vectors, or as the aligned vectors that contain them.
+            if (p.vec == FULL && p.ua_rows) {
+                launch_row_unaligned<T>(p, a, grid, block, st);
+                return;
             }
             if (p.vec == FULL && p.shift) {
-                if constexpr (kUnaligned) {
-                    if (!p.ua_rows || a.cols < FULL) fail(HPT_ERR_KERNEL, "row_reg: no kernel for shifted rows of this type");
-                    if constexpr (sizeof(T) == 2 && norm_is_layer(KIND)) {
-                        if (p.gb_lds == 1 && p.nchunk >= 3 && p.nchunk <= 4) {
-                            const size_t smem = 2 * (size_t)((p.cols + FULL - 1) / FULL) * FULL * sizeof(T);
-                            if (p.tpr >= 512 && grid.x > 512u) grid.x = 512u;
-                            if (p.nchunk == 3) row_reg_kernel<KIND, T, FULL, 3, 1, false, false, 1, 1, true><<<grid, block, smem, st>>>(a);
-                            else row_reg_kernel<KIND, T, FULL, 4, 1, false, false, 1, 1, true><<<grid, block, smem, st>>>(a);
-                            return;
-                        }
-                    }
-                    if constexpr (KIND != NORM_ADD_LAYERNORM) {
-                        if (p.tpr >= 512 && (sizeof(T) >= 4 || p.tpr == 1024 || norm_is_layer(KIND))) {
-                            if (grid.x > 512u) grid.x = 512u;
-                            launch_row_reg<T, FULL, 1, false, true, true>(p, a, grid, block, st);
-                            return;
-                        }
-                    }
-                    launch_row_reg<T, FULL, 1, false, false, true>(p, a, grid, block, st);
-                } else {
-                    // shifted rows: a thread's gamma / beta fit every row it walks only if those rows share
-                    // their misalignment, i.e. the row step is a whole number of vectors
-                    if (norm_is_layer(KIND) && (int64_t)grid.x * p.rpb < p.rows) {
-                        if (grid.x >= (unsigned)FULL) grid.x -= grid.x % FULL;
-                        else fail(HPT_ERR_KERNEL, "row_reg: shifted rows need a row step of whole vectors");
-                    }
-                    launch_row_reg<T, FULL, 1, true>(p, a, grid, block, st);
+                // shifted rows: a thread's gamma / beta fit every row it walks only if those rows share
+                // their misalignment, i.e. the row step is a whole number of vectors
+                if (norm_is_layer(KIND) && (int64_t)grid.x * p.rpb < p.rows) {
+                    if (grid.x >= (unsigned)FULL) grid.x -= grid.x % FULL;
+                    else fail(HPT_ERR_KERNEL, "row_reg: shifted rows need a row step of whole vectors");
                 }
+                // (the plan's numbers of vectors: two-byte rows of 512 threads, layernorm rows while the masks fit beside them)
+                if constexpr (sizeof(T) == 2 && (KIND == NORM_SOFTMAX || KIND == NORM_LOGSOFTMAX)) launch_row_of<T, 1, true, false, false, 3, 4>(p, a, grid, block, st);
+                else if constexpr (sizeof(T) == 2) fail(HPT_ERR_KERNEL, "row_reg: two-byte rows of this kind are unaligned vectors");
+                else if constexpr (sizeof(T) == 4 && KIND == NORM_ADD_LAYERNORM) launch_row_of<T, 1, true, false, false, 2, 3>(p, a, grid, block, st);
+                else if constexpr (norm_is_layer(KIND)) launch_row_of<T, 1, true, false, false, 2, 3, 4>(p, a, grid, block, st);
+                else launch_row_of<T, 1, true, false, false, 2, 3, 4, 5, 6, 7, 8>(p, a, grid, block, st);
                 return;
             }
         }
@@ -547,7 +574,7 @@ template <class T> void launch_t(const NormPlan& p, NormArgs a, hipStream_t st) 
             if (p.vec == FULL && p.sstride == 1 && p.tpr >= 512 &&
                 (sizeof(T) >= 4 || p.tpr == 1024 || norm_is_layer(KIND))) {
                 if (grid.x > 512u) grid.x = 512u;
-                launch_row_reg<T, FULL, 1, false, true>(p, a, grid, block, st);
+                launch_row_reg<T, FULL, 1, true>(p, a, grid, block, st);
                 return;
             }
         }
@@ -556,11 +583,26 @@ template <class T> void launch_t(const NormPlan& p, NormArgs a, hipStream_t st) 
             // of 1024 threads, or 512 with eight vectors, [1472, 15296] layernorm 36.2 and 34.5, causal 24.2 and 21.7, [2000, 10240] causal 19.9 and 17.6,
             // f16 layernorm [1000, 16384] 14.7 and 11.8, [4000, 8704] 28.1 and 25.5; but of 512 threads with four vectors, three of whose workgroups
             // fit a unit, f32 [3456, 8192] softmax 31.0 and 32.4, f64 layernorm [3456, 8192] 77.0 and 84.4, and f16 softmax [597, 14904] 7.7 and 8.2)
-            const bool walked = sizeof(T) == 4 ? p.tpr == 1024 || (p.tpr == 512 && p.nchunk == 8) : sizeof(T) == 2 && norm_is_layer(KIND) && p.tpr >= 512;
-            if (p.vec == FULL && p.sstride == 2 && grid.x > 512u && walked) {
-                grid.x = 512u;
-                launch_row_reg<T, FULL, 2, false, true>(p, a, grid, block, st);
-                return;
+            if (p.vec == FULL && p.sstride == 2 && grid.x > 512u) {
+                if constexpr (sizeof(T) == 4 && KIND == NORM_LAYERNORM) {
+                    if (p.tpr == 1024) {
+                        grid.x = 512u;
+                        launch_row_of<T, 2, false, true, false, 4>(p, a, grid, block, st);
+                        return;
+                    }
+                } else if constexpr (sizeof(T) == 4) {
+                    if (p.tpr == 1024 || (p.tpr == 512 && p.nchunk == 8)) {
+                        grid.x = 512u;
+                        launch_row_of<T, 2, false, true, false, 4, 8>(p, a, grid, block, st);
+                        return;
+                    }
+                } else if constexpr (sizeof(T) == 2 && KIND == NORM_LAYERNORM) {
+                    if (p.tpr >= 512) {
+                        grid.x = 512u;
+                        launch_row_of<T, 2, false, true, false, 4>(p, a, grid, block, st);
+                        return;
+                    }
+                }
             }
         }
         if (p.vec == FULL && p.sstride == 2 && FULL > 1) launch_row_reg<T, FULL, 2>(p, a, grid, block, st);
