@@ -653,20 +653,26 @@ static bool lds_row_shape(NormPlan& p, int64_t nvec, size_t elem_size, bool shif
 // Softmax over an axis of up to 1024 elements with a contiguous inner dim of L: whether 512 or 1024 threads that hold it in whole
 // vectors (col_tall_kernel) are ahead of the plan `p` (`found`: register columns of 256 threads, else three launches), and
 // that plan in `p` if so. Us over axis 1, as it was and this:
-//   four bytes, 129 ... 256 elements  [64, 129, 256] 9.8 and 6.8, [6, 200, 8200] 21.2 and 17.4, [20, 129, 8001] 48.8 and 34.2; where inner rows
-//     are whole 512-byte segments the 128-register form stays ([256, 256, 256] 20.4 and 22.2, though [16, 256, 2048] 18.0 and 15.2)
-//   257 ... 512  [1, 335, 58050] 88.6 and 45.2, [200, 335, 100] 29.0 and 19.6, [6, 512, 8200] 75.6 and 51.6; odd inner rows
-//     of 28 ... 50 MB in all go either way and stay ([16, 512, 1001] 22.3 and 23.9, [128, 512, 129] 23.9 and 27.6,
-//     [8, 512, 3001] 28.2 and 30.7, [24, 400, 1001] 22.2 and 24.0, [24, 335, 1001] 19.9 and 20.1, but [11, 512, 1001] 18.8 and 17.1, [64, 512, 501]
-//     54.6 and 42.5, [64, 300, 257] 16.0 and 15.7, [256, 512, 65] 24.7 and 22.6); where inner rows
+//   four bytes, 129 ... 256 elements  [64, 129, 256] 9.8 and 6.8, [6, 200, 8200] 21.2 and 17.4, [20, 129, 8001] 48.8 and 34.2; where inner rows are
+//     whole 256-byte segments the register columns read what they need of every line too, and stay once there is more than a round of
+//     workgroups ([730, 256, 64] 20.1 and 25.7, [1930, 256, 64] 47.4 and 53.5, [21, 138, 3136] 14.9 and 19.4; 98 shapes 0.98x, below a round 1.03x). In 257 ... 399
+//     workgroups ([16, 222, 2240] 13.8 and 15.4, 24 shapes 1.02x with eight slower) and inner rows of a few vectors ([8181, 208, 12] 33.2 and 43.3)
+//     likewise
+//   257 ... 512  [1, 335, 58050] 88.6 and 45.2, [200, 335, 100] 29.0 and 19.6, [6, 512, 8200] 75.6 and 51.6; odd inner rows of 27 ... 52 MiB in all stay for
+//     inputs that the last-level cache still holds ([16, 512, 1001] 22.3 and 23.9, [128, 512, 129] 23.9 and 27.6, [8, 512, 3001] 28.2 and 30.7, [24, 400,
+//     1001] 22.2 and 24.0); from memory they would gain there too (260 shapes 1.25x). Where inner rows
 //     are whole 256-byte segments the 128-register form stays below 128 MiB and for very long rows ([16, 512, 2048] 25.3 and
 //     29.5, [1, 512, 262144] 212 and 215; [512, 512, 512] 210 and 190, [64, 512, 1024] 53.2 and 50.1)
 //   513 ... 1024  [64, 777, 256] 28.3 and 21.5, [16, 1024, 2048] 92.2 and 53.4; one workgroup fills a compute unit, so there must be enough of
 //     them, of rows that are not short: [4, 1000, 1000] 16.8 and 18.9, [200, 1000, 100] 66.2 and 72.2
-//   two bytes, 65 ... 512  [64, 100, 256] 10.1 and 5.7, [16, 100, 1001] 13.4 and 6.4, [100, 335, 500] 35.7 and 23.9, [512, 512, 512] 128 and 105;
-//     [64, 256, 2048] 26.0 and 29.6, [100, 256, 1024] 26.1 and 25.1
-//   513 ... 1024  [512, 513, 24] 21.2 and 15.1, [64, 1000, 256] 28.4 and 22.1, [16, 1000, 2048] 38.1 and 28.4; [4, 777, 1000] 13.4 and 19.1, [1, 513, 58050]
-//     (three passes, odd rows) 38.5 and 42.6
+//   two bytes, 65 ... 256  [64, 100, 256] 10.1 and 5.7, [16, 100, 1001] 13.4 and 6.4; [64, 256, 2048] 26.0 and 29.6, [100, 256, 1024] 26.1 and 25.1
+//   257 ... 512  [100, 335, 500] 35.7 and 23.9, [512, 512, 512] 128 and 105; not with inner rows of a few vectors ([4200, 311, 16] 23.4 and 29.1, [2207,
+//     342, 27] 32.9 and 39.4), more than a round of workgroups where they are whole 128-byte segments ([22, 455, 3392] 28.0 and 31.6), or few
+//     workgroups where the register columns' pieces are aligned and these are not ([18, 410, 180] 13.3 and 14.7)
+//   513 ... 1024  [512, 513, 24] 21.2 and 15.1, [64, 1000, 256] 28.4 and 22.1, [16, 1000, 2048] 38.1 and 28.4; [4, 777, 1000] 13.4 and 19.1; three
+//     launches for odd rows of 512 and more ([19, 596, 3822] 60.4 and 70.6, [1, 513, 58050] 38.5 and 42.6), for very long ones, and the flat walk where
+//     the last of several rounds is a fifth empty ([536, 896, 180] 121.8 and 149.0); where three launches have whole vectors of wide inner rows, they are
+//     ahead in 257 ... 399 workgroups and 513 ... 899 (8 and 10 shapes 0.89x and 1.00x, then 27 0.96x; up to a round 24 1.11x, 400 ... 512 1.15x)
 //   three launches for too few positions, any of these  [8, 129, 64] 10.7 and 5.5, two bytes [4, 65, 1000] 10.9 and 5.1, [1, 300, 200] 10.9 and 9.1
 static bool tall_columns(NormPlan& p, bool found, const void* in_data, const void* out_data, int64_t sa, int64_t sb, int64_t L, int64_t batch,
                          size_t elem_size) {
@@ -684,18 +690,26 @@ static bool tall_columns(NormPlan& p, bool found, const void* in_data, const voi
     const int64_t blocks = (batch * ((L + vec - 1) / vec) + tx - 1) / tx;
     if (blocks * threads >= (1ll << 32)) return false;  // work-items of one launch
     const bool whole_segments = found && p.vec == 4 && p.nchunk == 32 && elem_size == 4;  // the 128-register form
+    const int64_t bytes = p.cols * L * batch * (int64_t)elem_size;
+    // (the compute units that got a workgroup more than the others are waited for: 257 ... 400 of them, and two-byte ones of 1024 threads, of which
+    // a unit holds one, whenever the last round is a fifth empty)
+    const bool part_of_a_round = blocks > kComputeUnits && blocks < 400;
+    const int64_t rounds = (blocks + kComputeUnits - 1) / kComputeUnits;
     if (p.cols > 512) {
-        if (elem_size == 4 ? (blocks < 192 || L < 256) : (blocks < 96 || (!grid && batch == 1))) return false;
+        if (elem_size == 4 ? (blocks < 192 || L < 256) : blocks < 96) return false;
+        if (elem_size == 2 && !grid && (L >= 64 * vec || ((p.cols * L) % vec == 0 && rounds > 1 && blocks * 5 < rounds * kComputeUnits * 4))) return false;
+        if (elem_size == 2 && grid && L >= 320 && (part_of_a_round || (blocks > 2 * kComputeUnits && blocks < 900) || (L > 8192 && blocks > kComputeUnits))) return false;
     } else if (!found) {
         // (odd inner rows of a wavefront of vectors and more: tests name the three passes)
         if (p.cols > 256 && !grid && L >= 64 * vec) return false;
     } else if (elem_size == 4) {
-        if (p.cols <= 128) return false;
-        if (whole_segments && (p.cols <= 256 || L > 16384 || p.cols * L * batch * 4 < (128ll << 20))) return false;
-        const int64_t bytes = p.cols * L * batch * 4;
+        if (p.cols <= 128 || L <= 16) return false;
+        if (whole_segments && (p.cols <= 256 || L > 16384 || bytes < (128ll << 20))) return false;
+        if (p.cols <= 256 && grid && (L % 64 == 0 ? blocks > kComputeUnits : part_of_a_round)) return false;
         if (!grid && p.cols > 320 && L >= 96 && bytes >= (27ll << 20) && bytes < (52ll << 20)) return false;
-    } else if (p.cols <= 64 || (grid && p.cols > 128 && p.cols <= 256 && L >= 1024 && p.cols * L * batch * 2 >= (64ll << 20))) {
-        return false;
+    } else {
+        if (p.cols <= 64 || (grid && p.cols > 128 && p.cols <= 256 && L >= 1024 && bytes >= (64ll << 20))) return false;
+        if (p.cols > 256 && (L <= 32 || (L % 64 == 0 && blocks > kComputeUnits) || (!grid && !p.shift && blocks < 128))) return false;
     }
     p.kind = NormKind::ColReg;
     p.tall = (int)threads;
