@@ -144,8 +144,8 @@ __device__ __forceinline__ void row_all_reduce_n(A (&v)[N], int tpr, int ty, A* 
 // same cache lines as a scalar gather with a fraction of the instructions. (A
 // 16-byte aligned vector that holds one valid element never leaves that element's
 // page, so the unused half of the last vector is safe to touch.)
-// SHIFT (VEC > 1, SS = 1; f32 softmax and eight-byte types, the others take UA below): rows whose START is only
-// element-aligned (odd row lengths: 197, 4097, 50257). A row is covered by the 16-byte ALIGNED vectors that contain it: vector iv holds the
+// SHIFT (VEC > 1, SS = 1): rows whose START is only
+// element-aligned (odd row lengths: 197, 4097, 50257; which rows take this and which UA, below, is the plan's choice). A row is covered by the 16-byte ALIGNED vectors that contain it: vector iv holds the
 // row's elements iv * VEC - m ... + VEC - 1, m = the row's misalignment in elements; positions
 // outside the row are masked, whole vectors are stored whole and the two end vectors element by
 // element. Input, output and residual rows share m (the caller checks bases and pitches mod 16
@@ -490,12 +490,12 @@ __global__ void __launch_bounds__(1024) row_reg_kernel(const NormArgs a) {
 #pragma unroll
             for (int c = 0; c < NCHUNK; ++c) {
                 const bool in_row_c = (c * tpr + tx) < nv;
-                auto square = [&](int j, bool in_row_e) {
-                    const CT d = in_row_e ? (x[c][j] - mean_hi) - mean_lo : (CT)0;
-                    x[c][j] = d;
-                    q += d * d;
-                };
                 if constexpr (UA) {
+                    auto square = [&](int j, bool in_row_e) {
+                        const CT d = in_row_e ? (x[c][j] - mean_hi) - mean_lo : (CT)0;
+                        x[c][j] = d;
+                        q += d * d;
+                    };
                     if (c * tpr + tx == nv - 1) {
 #pragma unroll
                         for (int j = 0; j < UV; ++j) square(j, j >= twice);
@@ -504,6 +504,8 @@ __global__ void __launch_bounds__(1024) row_reg_kernel(const NormArgs a) {
                         for (int j = 0; j < UV; ++j) square(j, in_row_c);
                     }
                 } else {
+                    // (not through that lambda: it costs aligned rows registers, f16 of four vectors 93 -> 97 and a fifth wavefront, f32 [2441, 12288]
+                    // 46.4 -> 59.1 us by spills)
 #pragma unroll
                     for (int j = 0; j < UV; ++j) {
                         const bool in_row_e = SHIFT ? inside(c * tpr + tx, j) : in_row_c;

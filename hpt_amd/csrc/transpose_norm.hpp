@@ -189,7 +189,7 @@ __global__ void __launch_bounds__(1024) transposed_stats_kernel(const Transposed
     // used (softmax over axis 0, this pass alone, us: f32 [8190, 4097] two workgroups per compute unit without the second
     // batch 32.1, one 36.1, with it 32.1 and 26.1; [32768, 1024] 33.4 -> 23.3. Two-byte elements, twice the arithmetic
     // per byte, take shorter batches and twice the wavefronts: f16 [8190, 4097] 19.4 -> 15.4; single elements, a few bytes of a line each, the
-    // long ones). The second batch costs registers, f32 softmax 64 -> 111 and layernorm as many, so four wavefronts fit a SIMD
+    // long ones). The second batch costs registers, f32 softmax 52 -> 93 and layernorm 64 -> 111, so four or five wavefronts fit a SIMD
     // instead of eight; no plan has more than two there. Transposed rows, all three passes, us: f32 [30000, 500] softmax 61.1 -> 51.5, layernorm
     // 47.0 -> 44.6, f16 [16384, 1024] layernorm 28.8 -> 25.3, [30000, 500] 44.8 -> 35.9, [8192, 8192] no difference.
     // (The last round's loads are repeated, not left out: behind a test the wait before the fold would be a full one.)
@@ -693,9 +693,10 @@ __global__ void __launch_bounds__(256) col_reg_kernel(const ColRegArgs a) {
 // ---- the same for a LONGER axis: more threads, not narrower vectors ---------------------------
 // col_reg_kernel's 256 threads hold 65 ... 1024 elements of the axis only as pieces of 2 ... 8 bytes, or in 128 registers each.
 // Here 512 or 1024 threads hold them as whole vectors: TX lanes along the inner dim (256- or 512-byte segments of every inner
-// row), NT / TX thread rows of NC vectors. 64 registers or fewer per thread leave room for two workgroups of 1024 per compute
-// unit, one loading while the other stores. Bound by memory: the same kernel without its arithmetic takes as long (f32 512^3
-// over axis 1 189 us, at 5.7 TB/s; with col_reg_kernel 210).
+// row), NT / TX thread rows of NC vectors. Four-byte elements with NC = 8 take 62 ... 64 registers per thread, which leave room for two
+// workgroups of 1024 per compute unit, one loading while the other stores, two-byte ones with NC = 8 take 68 (three workgroups of 512); NC = 16
+// takes 94 ... 100, room for two workgroups of 512 but only one of 1024 (which the plan's rules on the count of workgroups follow). Bound by memory: the same kernel
+// without its arithmetic takes as long (f32 512^3 over axis 1 189 us, at 5.7 TB/s; with col_reg_kernel 210).
 // Segments that are neighbours in an inner row go to one XCD, in pairs (workgroups i and i + 8): 199 -> 190 us there, and
 // unaligned segments share the line between them (f32 [512, 65538] over axis 0 91.0 -> 84.9).
 // (device us, softmax over axis 1, col_reg_kernel -> this: f32 [64, 512, 1024] 54.4 -> 50.6, [1, 335, 58050] 89.2 -> 45.2,
