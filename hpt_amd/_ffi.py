@@ -9,6 +9,8 @@ import ctypes as C
 import warnings
 from pathlib import Path
 
+ALIGN = 64  # every tensor's mem_layout alignment (hpt/src/lib.rs:560)
+
 LIB_PATH = Path(__file__).resolve().parent / "lib" / "libhpt_hip.so"
 
 # hpt_status
@@ -125,19 +127,29 @@ def lib() -> C.CDLL:
     return _lib
 
 
-_calls = ()  # not looked for yet
+class _ThroughCtypes:
+    """In the place of the native module where there is none: takes no call, so that every caller goes the long way, and frees through ctypes."""
+    reduce = argreduce = softmax = layernorm = softmax_causal = staticmethod(lambda *_: None)
+
+    @staticmethod
+    def free(device, ptr, nbytes, ordered):
+        entry = lib().hpt_hip_free_ordered if ordered else lib().hpt_hip_free
+        return entry(device, C.c_void_p(ptr), nbytes, ALIGN)
+
+
+_calls = None
 
 
 def calls():
     """The native module of the calls that return a fresh tensor (csrc/pycalls.cpp), which is linked to libhpt_hip.so. It is built for one
-    interpreter; under another, or where it was not built, None: every call then goes through ctypes, as those do that it does not take."""
+    interpreter; under another, or where it was not built, calls go through ctypes, as those do that it does not take."""
     global _calls
-    if _calls == ():
+    if _calls is None:
         lib()  # (says what is missing when nothing has been built)
         try:
             from . import _calls as module
         except ImportError as e:
-            module = None
+            module = _ThroughCtypes
             warnings.warn(f"hpt_amd._calls cannot be loaded ({e}), calls go through ctypes and take some microseconds longer: "
                           "build it with `python -m hpt_amd.build`", RuntimeWarning, stacklevel=2)
         _calls = module

@@ -27,7 +27,7 @@ import numpy as np
 from . import _ffi
 from ._ffi import ParamError, ShapeError, check, make_view
 
-ALIGN = 64  # every tensor's mem_layout alignment (hpt/src/lib.rs:560)
+ALIGN = _ffi.ALIGN
 
 
 class DType:
@@ -158,12 +158,7 @@ class _DeviceStorage(_StreamTracked):
                 pass  # (interpreter shutdown, or the device is gone: nothing more can be waited for)
         try:
             # the block always goes back to the allocator, whatever the wait did
-            native = _ffi.calls()
-            if native is not None:
-                native.free(self.device, self.ptr, self.nbytes, ordered)
-            else:
-                free = _ffi.lib().hpt_hip_free_ordered if ordered else _ffi.lib().hpt_hip_free
-                free(self.device, C.c_void_p(self.ptr), self.nbytes, ALIGN)
+            _ffi.calls().free(self.device, self.ptr, self.nbytes, ordered)
         except Exception:
             pass
         self.ptr = 0
@@ -201,12 +196,10 @@ def _touch(stream, *tensors) -> None:
 
 
 def _native_stream(stream) -> int:
-    """The stream of a call that goes through the native module, or -1: given in a form that ctypes sorts out, or there is no such module."""
+    """The stream of a call that goes through the native module, or -1: given in a form that ctypes sorts out."""
     if stream is None:
-        k = 0
-    else:
-        k = stream if type(stream) is int and stream >= 0 else -1
-    return k if _ffi.calls() is not None else -1
+        return 0
+    return stream if type(stream) is int and stream >= 0 else -1
 
 
 _OUT_DTYPES = {}

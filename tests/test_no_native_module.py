@@ -12,9 +12,9 @@ def without(hpt, monkeypatch):
     from hpt_amd import _ffi
     monkeypatch.setitem(sys.modules, "hpt_amd._calls", None)
     monkeypatch.delattr(hpt, "_calls", raising=False)
-    monkeypatch.setattr(_ffi, "_calls", ())
+    monkeypatch.setattr(_ffi, "_calls", None)
     with pytest.warns(RuntimeWarning, match="_calls cannot be loaded"):
-        assert _ffi.calls() is None
+        assert _ffi.calls() is _ffi._ThroughCtypes
     return _ffi
 
 
@@ -59,9 +59,9 @@ def test_results_and_memory(hpt, dev, without):
     for f in calls:
         f()
     assert live() == before  # nothing of theirs stays allocated
-    without._calls = ()
+    without._calls = None
     del sys.modules["hpt_amd._calls"]
-    assert without.calls() is not None
+    assert without.calls() is not without._ThroughCtypes
     assert [f().numpy().tobytes() for f in calls] == got
 
 
