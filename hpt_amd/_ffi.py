@@ -149,7 +149,7 @@ def calls():
         try:
             from . import _calls as module
         except ImportError as e:
-            module = _ThroughCtypes
+            module = _calls = _ThroughCtypes  # (before the warning, which a program may have made an error)
             warnings.warn(f"hpt_amd._calls cannot be loaded ({e}), calls go through ctypes and take some microseconds longer: "
                           "build it with `python -m hpt_amd.build`", RuntimeWarning, stacklevel=2)
         _calls = module

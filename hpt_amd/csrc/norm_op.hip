@@ -50,7 +50,6 @@ void launch_row_reg(const NormPlan& p, const NormArgs& a, dim3 grid, dim3 block,
     }
 }
 
-// Few, very long rows: several workgroups per row.
 // Rows off the vector grid as unaligned vectors (two-byte types, f32 layernorms).
 template <class T> void launch_row_unaligned(const NormPlan& p, const NormArgs& a, dim3 grid, dim3 block, hipStream_t st) {
     constexpr int FULL = 16 / sizeof(T);
@@ -99,6 +98,7 @@ template <class T> void launch_row_unaligned(const NormPlan& p, const NormArgs& 
     }
 }
 
+// Few, very long rows: several workgroups per row.
 template <class T, int VEC, bool UA> void launch_row_split(const NormPlan& p, const NormArgs& a, hipStream_t st) {
     RowSplitArgs r{};
     r.in = a.in;

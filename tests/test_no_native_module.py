@@ -2,6 +2,7 @@
 memory goes back to the allocator, and results and errors are the same."""
 import ctypes as C
 import sys
+import warnings
 
 import numpy as np
 import pytest
@@ -32,6 +33,14 @@ def test_blocks_are_freed(without, monkeypatch, pending, entry):
     st.pending = set(pending)
     del st
     assert calls[-1] == (entry, 0, 4096, 640, tensor.ALIGN), calls
+
+
+def test_the_warning_as_an_error(without):
+    without._calls = None
+    with pytest.raises(RuntimeWarning), warnings.catch_warnings():
+        warnings.simplefilter("error")
+        without.calls()
+    assert without.calls() is without._ThroughCtypes
 
 
 def test_errors(hpt, without):
