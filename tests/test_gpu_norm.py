@@ -472,7 +472,7 @@ WIDE_ROW_CASES = [
     ("bf16 rows of 1500 (8-byte row starts): shifted, 64 x 3", "bf16", [4400, 1500]),
     ("f32 rows of 2051: shifted, 128 x 5", np.float32, [2300, 2051]),
     ("f32 rows of 3001: shifted, 256 x 3", np.float32, [2100, 3001]),
-    # two-byte layernorm rows of 513 ... 1024 shifted vectors: 512 threads, two vectors each, rows walked
+    # two-byte layernorm rows of 513 ... 1024 vectors off the grid (more rows of them than workgroups: test_gpu_walked_rows_off_grid.py)
     ("f16 rows of 4097: layernorm from registers, 512 threads", np.float16, [2100, 4097]),
     ("bf16 rows of 8185: the longest such row", "bf16", [1500, 8185]),
     ("f16 rows of 6148 (rows start on 8-byte boundaries)", np.float16, [1300, 6148]),

@@ -1,6 +1,7 @@
 """Rows off the vector grid as unaligned vectors, the last one from the row's end backwards: softmax, log_softmax, layernorm, layernorm of
 a sum and the causal softmax at row lengths either side of vectors, threads per row, vectors per thread and the forms that follow;
-rows whose input and output are misaligned by different amounts; more rows than one round of workgroups; in place."""
+rows whose input and output are misaligned by different amounts; in place. Which of them are unaligned vectors and which masked aligned ones is the
+plan's choice; test_gpu_walked_rows_off_grid.py asserts it, with more rows than one round of workgroups."""
 import numpy as np
 import pytest
 
