@@ -666,12 +666,16 @@ static bool lds_row_shape(NormPlan& p, int64_t nvec, size_t elem_size, bool shif
 //   513 ... 1024  [64, 777, 256] 28.3 and 21.5, [16, 1024, 2048] 92.2 and 53.4; one workgroup fills a compute unit, so there must be enough of
 //     them, of rows that are not short: [4, 1000, 1000] 16.8 and 18.9, [200, 1000, 100] 66.2 and 72.2
 //   two bytes, 65 ... 256  [64, 100, 256] 10.1 and 5.7, [16, 100, 1001] 13.4 and 6.4; [64, 256, 2048] 26.0 and 29.6, [100, 256, 1024] 26.1 and 25.1
-//   257 ... 512  [100, 335, 500] 35.7 and 23.9, [512, 512, 512] 128 and 105; not with inner rows of a few vectors ([4200, 311, 16] 23.4 and 29.1, [2207,
-//     342, 27] 32.9 and 39.4), more than a round of workgroups where they are whole 128-byte segments ([22, 455, 3392] 28.0 and 31.6), or few
-//     workgroups where the register columns' pieces are aligned and these are not ([18, 410, 180] 13.3 and 14.7)
+//   257 ... 512  [100, 335, 500] 35.7 and 23.9, [512, 512, 512] 128 and 105; not with inner rows of up to 32 elements that
+//     the register columns take in pieces of four, or short odd ones ([4200, 311, 16] 23.4 and 29.1, [2289, 334, 28] 32.6 and 38.9, [489, 353, 11] 11.9 and 16.3;
+//     others [2032, 330, 10] 21.6 and 15.4, [5810, 323, 17] 56.7 and 51.1), nor, where they are whole 128-byte segments, with the second of a unit's two
+//     workgroups in less than half of the units ([22, 455, 3392] 28.0 and 31.6, [15, 415, 2624] 18.6 and 20.0; but [18, 259, 2816], 396 workgroups, 16.0 and
+//     14.6, [866, 477, 64] 24.5 and 22.0), or few workgroups where the register columns' pieces are aligned and these are not ([18, 410, 180] 13.3 and 14.7)
 //   513 ... 1024  [512, 513, 24] 21.2 and 15.1, [64, 1000, 256] 28.4 and 22.1, [16, 1000, 2048] 38.1 and 28.4; [4, 777, 1000] 13.4 and 19.1; three
-//     launches for odd rows of 512 and more ([19, 596, 3822] 60.4 and 70.6, [1, 513, 58050] 38.5 and 42.6), for very long ones, and the flat walk where
-//     the last of several rounds is a fifth empty ([536, 896, 180] 121.8 and 149.0); where three launches have whole vectors of wide inner rows, they are
+//     launches for odd rows of 1024 and more ([19, 596, 3822] 60.4 and 70.6, [1, 513, 58050] 38.5 and 42.6, [20, 1000, 1501] 40.6 and 51.3; up to 640
+//     elements within a round [12, 600, 2051] 27.0 and 23.1), for very long ones, and the flat walk where the last of several rounds is a fifth empty
+//     ([536, 896, 180] 121.8 and 149.0), for odd rows of 512 ... 1023 a third ([40, 777, 1001] 46.7 and 56.5, but [90, 600, 517] 53.3 and 46.1, [180, 777, 517]
+//     149 and 108; below 64 [966, 544, 35] 47.0 and 38.3); where three launches have whole vectors of wide inner rows, they are
 //     ahead in 257 ... 399 workgroups and 513 ... 899 (8 and 10 shapes 0.89x and 1.00x, then 27 0.96x; up to a round 24 1.11x, 400 ... 512 1.15x)
 //   three launches for too few positions, any of these  [8, 129, 64] 10.7 and 5.5, two bytes [4, 65, 1000] 10.9 and 5.1, [1, 300, 200] 10.9 and 9.1
 static bool tall_columns(NormPlan& p, bool found, const void* in_data, const void* out_data, int64_t sa, int64_t sb, int64_t L, int64_t batch,
@@ -697,7 +701,11 @@ static bool tall_columns(NormPlan& p, bool found, const void* in_data, const voi
     const int64_t rounds = (blocks + kComputeUnits - 1) / kComputeUnits;
     if (p.cols > 512) {
         if (elem_size == 4 ? (blocks < 192 || L < 256) : blocks < 96) return false;
-        if (elem_size == 2 && !grid && (L >= 64 * vec || ((p.cols * L) % vec == 0 && rounds > 1 && blocks * 5 < rounds * kComputeUnits * 4))) return false;
+        if (elem_size == 2 && !grid && L >= 64 && L < 64 * vec && (p.cols * L) % vec == 0 && rounds > 1 && blocks * 5 < rounds * kComputeUnits * 4) return false;
+        if (elem_size == 2 && !grid && L >= 64 * vec) {
+            if (batch == 1 || (rounds > 1 && blocks * 3 < rounds * kComputeUnits * 2)) return false;
+            if (L >= 128 * vec && (rounds > 1 || p.cols > 640)) return false;  // (what else there is has unaligned vectors there, not the flat walk)
+        }
         if (elem_size == 2 && grid && L >= 320 && (part_of_a_round || (blocks > 2 * kComputeUnits && blocks < 900) || (L > 8192 && blocks > kComputeUnits))) return false;
     } else if (!found) {
         // (odd inner rows of a wavefront of vectors and more: tests name the three passes)
@@ -709,7 +717,9 @@ static bool tall_columns(NormPlan& p, bool found, const void* in_data, const voi
         if (!grid && p.cols > 320 && L >= 96 && bytes >= (27ll << 20) && bytes < (52ll << 20)) return false;
     } else {
         if (p.cols <= 64 || (grid && p.cols > 128 && p.cols <= 256 && L >= 1024 && bytes >= (64ll << 20))) return false;
-        if (p.cols > 256 && (L <= 32 || (L % 64 == 0 && blocks > kComputeUnits) || (!grid && !p.shift && blocks < 128))) return false;
+        const bool short_rows = L <= 32 && L != 24 && (L % 4 == 0 || (L < 16 && L % 2 == 1));
+        const bool half_a_round = (blocks > kComputeUnits && blocks < 360) || (blocks > 2 * kComputeUnits && blocks < 600);
+        if (p.cols > 256 && (short_rows || (L % 64 == 0 && half_a_round) || (!grid && !p.shift && blocks < 128 && L > 32))) return false;
     }
     p.kind = NormKind::ColReg;
     p.tall = (int)threads;
@@ -903,12 +913,13 @@ NormPlan plan_normalize(const void* in_data, const void* out_data, const int64_t
                 if (vi == max_vec && out_ok) {
                     v = max_vec;
                     p.sstride = 2;
-                } else if (elem_size == 2 && p.cols >= 640 && (p.cols + uv - 1) / uv <= 4096 && !(fused && n_norm_dims > 0) && !few &&
+                } else if (elem_size == 2 && p.cols >= 640 && (p.cols + uv - 1) / uv <= 4096 && !(fused && n_norm_dims > 0 && p.cols <= 8192) && !few &&
                            ((uintptr_t)in_data % elem_size) == 0 && ((uintptr_t)out_data % elem_size) == 0) {
                     // Two-byte rows off the vector grid: the same vectors unaligned (us, every second of the stored, single elements and
                     // this: f16 [3456, 7897] causal 27.6 and 19.9, layernorm 30.9 and 28.3, [2000, 16383] softmax 39.8 and 28.8. f32 goes either way:
                     // softmax [2000, 16383] 53.6 and 47.6, with sums over more elements of a lane, [3456, 7897] 32.3 and 35.7; x + residual keeps
-                    // single elements, its four vectors spill: f16 [3456, 7897] 35.2, 52.1 as vectors, [7598, 3853] 30.1, 54.8).
+                    // single elements up to 1024 threads' eight, its four vectors spill: f16 [3456, 7897] 35.2, 52.1 as vectors, [7598, 3853] 30.1, 54.8, though bf16
+                    // [1745, 10870] 36.2 and 32.7; longer rows would stream: bf16 [110, 23911] 16.4, 10.2 as vectors, f16 [71, 23142] 15.1 and 10.8).
                     v = max_vec;
                     p.sstride = 2;
                     p.shift = 1;
@@ -947,27 +958,20 @@ NormPlan plan_normalize(const void* in_data, const void* out_data, const int64_t
                 // causal [32, 1001, 1001] 26.9 and 20.7; f16 layernorm [8190, 4097] 59.7 and 33.7, [14245, 561] 14.4 and 11.2, [2000, 12001]
                 // (streamed) 31.4 and 22.7; f32 layernorm [8190, 4097] 60.4 and 49.6, [3000, 9001] (streamed) 61.6 and 43.9. The f32 softmax
                 // is as fast as that of aligned rows ([16000, 2051] 45.3, [16000, 2052] 47.2).
-                // Where the masks fit the registers and there is no row to prefetch, or no gain in it, whole aligned lines are ahead of
-                // stores across them: f32 layernorm up to 256 threads per row ([10695, 561] 12.3 and 13.4 us, [7751, 774] 12.2 and 13.3,
-                // [4552, 1318] 12.3 and 13.2, [485, 3090] 6.1 and 6.6; 512 threads [1464, 4097] 15.8 and 12.6, but few rows [336, 4458]
-                // 6.5 and 6.9), f32 x + residual up to three vectors per thread ([8000, 750] 15.6 and 16.3, [4304, 1394] 15.8 and 16.6; four
-                // spill, [1941, 3090] 20.4 and 16.9), two-byte softmax of 512 threads ([5224, 9571] 43.6 and 46.9, [857, 14001] 15.2 and 16.5,
-                // but [61, 12292], whose rows are four elements off, 6.2 and 5.6, and one row per workgroup [59, 12531] 6.3 and 5.9) and large inputs of
-                // 256 ([6816, 7335] log_softmax 37.7 and 41.4, [9043, 5529] 36.2 and 39.0; [1635, 7335] 13.7 and 13.3).
+                // The masked aligned vectors, whose stores are whole lines, are ahead for f32 layernorm of few rows alone ([485, 3090] 6.1 and 6.6 us,
+                // [336, 4458] 6.5 and 6.9). With more rows and inputs that come from memory they are level, 46 shapes 0.99x, and with inputs
+                // that the last-level cache holds behind: f32 layernorm [7163, 1015] 13.4 and 12.3, [2603, 2161] 13.4 and 10.9, x + residual [2545, 1238]
+                // 10.0 and 9.0, f16 softmax [1131, 16150] 19.4 and 16.2, [5806, 7142] 0.81x (from memory 42 two-byte shapes 1.01x, x + residual 40 shapes 0.94x).
                 // Input and output off the grid by different amounts took single elements: they stay where stores across lines cost more than
-                // they save, short rows (f32 layernorm [61855, 97] 15.5 and 17.4, x + residual [55813, 215] 17.7 and 19.4, f16 x + residual [68181, 176]
-                // 21.8 and 23.2; [45627, 263] 27.3 and 24.2), and layernorm of few (f32 [1425, 263] 4.3 and 5.2, [178, 2100] 4.9 and 5.5).
+                // they save, short rows (f32 layernorm [61855, 97] 15.5 and 17.4, x + residual [55813, 215] 17.7 and 19.4; two-byte
+                // x + residual is level from memory and ahead as vectors in the cache, bf16 [142052, 176] 38.6 and 33.7), and layernorm of few (f32 [1425, 263] 4.3 and 5.2, [178, 2100] 4.9 and 5.5).
                 const int64_t nvu = (p.cols + max_vec - 1) / max_vec;
                 bool unaligned = (elem_size == 2 || (elem_size == 4 && n_norm_dims > 0)) && ((uintptr_t)in_data % elem_size) == 0 &&
                                  ((uintptr_t)out_data % elem_size) == 0 && nvu <= (elem_size == 4 ? 4096 : 2048);
-                if (unaligned && same && (((uintptr_t)residual ^ (uintptr_t)(residual ? out_data : nullptr)) & 15) == 0) {
-                    const int64_t quarter = pow2_ceil((nvs + 3) / 4);  // threads that hold the row in three or four vectors each
-                    if (elem_size == 4 && !fused) unaligned = p.cols <= 256 || nvs > (p.rows <= 512 ? 2048 : 1024);
-                    else if (elem_size == 4) unaligned = p.cols <= 512 || nvs > 2048 || (nvs > 3 * quarter && quarter != 128);
-                    else if (n_norm_dims <= 0 && !fused && nvs <= 2048 && p.cols % 4 != 0)
-                        unaligned = nvu > 1024 ? p.rows <= 512 : nvu <= 512 || p.rows * p.cols * 2 < (48ll << 20);
+                if (unaligned && same && elem_size == 4 && !fused) {
+                    unaligned = p.cols <= 256 || p.rows > 512 || nvs > 2048;
                 } else if (unaligned && !same && n_norm_dims > 0) {
-                    if (fused) unaligned = p.cols >= 256 || (elem_size == 4 && p.cols >= 128 && p.cols % 4 == 0);
+                    if (fused) unaligned = elem_size == 2 || p.cols >= 256 || (p.cols >= 128 && p.cols % 4 == 0);
                     else unaligned = (elem_size == 2 || (p.cols >= 128 && (p.cols <= 192 || p.cols >= 256))) &&
                                      (p.cols >= (elem_size == 2 ? 1024 : 4096) || p.rows * p.cols * (int64_t)elem_size >= (3ll << 20));
                 }

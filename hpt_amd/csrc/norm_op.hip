@@ -56,9 +56,9 @@ template <class T> void launch_row_unaligned(const NormPlan& p, const NormArgs& 
     if (a.cols < FULL) fail(HPT_ERR_KERNEL, "row_reg: rows of %lld elements hold no vector", (long long)a.cols);
     if constexpr (sizeof(T) == 2) {
         if (p.sstride == 2) {
-            // (every second element; x + residual has no such plan: its four vectors spill)
+            // (every second element; x + residual, whose four vectors spill, where it would stream otherwise)
             if constexpr (KIND == NORM_ADD_LAYERNORM) {
-                fail(HPT_ERR_KERNEL, "row_reg: no kernel for every second element of x + residual");
+                launch_row_of<T, 2, false, false, true, 4>(p, a, grid, block, st);
             } else if constexpr (KIND == NORM_LAYERNORM) {
                 if (p.tpr >= 512) {
                     if (grid.x > 512u) grid.x = 512u;
@@ -520,10 +520,8 @@ template <class T> void launch_t(const NormPlan& p, NormArgs a, hipStream_t st) 
                     if (grid.x >= (unsigned)FULL) grid.x -= grid.x % FULL;
                     else fail(HPT_ERR_KERNEL, "row_reg: shifted rows need a row step of whole vectors");
                 }
-                // (the plan's numbers of vectors: two-byte rows of 512 threads, layernorm rows while the masks fit beside them)
-                if constexpr (sizeof(T) == 2 && (KIND == NORM_SOFTMAX || KIND == NORM_LOGSOFTMAX)) launch_row_of<T, 1, true, false, false, 3, 4>(p, a, grid, block, st);
-                else if constexpr (sizeof(T) == 2) fail(HPT_ERR_KERNEL, "row_reg: two-byte rows of this kind are unaligned vectors");
-                else if constexpr (sizeof(T) == 4 && KIND == NORM_ADD_LAYERNORM) launch_row_of<T, 1, true, false, false, 2, 3>(p, a, grid, block, st);
+                // (the plan's numbers of vectors: layernorm rows while the masks fit beside them)
+                if constexpr (sizeof(T) == 2 || (sizeof(T) == 4 && KIND == NORM_ADD_LAYERNORM)) fail(HPT_ERR_KERNEL, "row_reg: rows of this type and kind are unaligned vectors");
                 else if constexpr (norm_is_layer(KIND)) launch_row_of<T, 1, true, false, false, 2, 3, 4>(p, a, grid, block, st);
                 else launch_row_of<T, 1, true, false, false, 2, 3, 4, 5, 6, 7, 8>(p, a, grid, block, st);
                 return;

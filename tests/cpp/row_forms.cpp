@@ -23,7 +23,7 @@ static std::set<int> kernels_of(const NormPlan& p, int size, Kind k, std::string
     if (p.vec == full && p.ua_rows) {
         form = "unaligned";
         if (p.cols < full || size == 8 || (p.sstride == 2 && size != 2) || p.gb_lds == 2 || (p.gb_lds == 1 && size != 2)) return {};
-        if (size == 2 && p.sstride == 2) return k == ADD_LAYERNORM ? std::set<int>{} : k == LAYERNORM ? std::set<int>{4} : std::set<int>{2, 4};
+        if (size == 2 && p.sstride == 2) return layer ? std::set<int>{4} : std::set<int>{2, 4};
         if (size == 2 && layer && p.gb_lds) return {3, 4};
         if (size == 2) return k == ADD_LAYERNORM ? std::set<int>{2} : k == LAYERNORM ? std::set<int>{2, 3} : std::set<int>{2, 3, 4};
         if (k == ADD_LAYERNORM) return {2, 3, 4};
@@ -33,8 +33,7 @@ static std::set<int> kernels_of(const NormPlan& p, int size, Kind k, std::string
     if (p.vec == full && p.shift) {
         form = "masked";
         if (p.sstride != 1 || p.gb_lds || (layer && grid * p.rpb < p.rows && grid < full)) return {};
-        if (size == 2) return k == SOFTMAX ? std::set<int>{3, 4} : std::set<int>{};
-        if (size == 4 && k == ADD_LAYERNORM) return {2, 3};
+        if (size == 2 || (size == 4 && k == ADD_LAYERNORM)) return {};
         return layer ? std::set<int>{2, 3, 4} : std::set<int>{2, 3, 4, 5, 6, 7, 8};
     }
     if (layer && p.gb_lds) {

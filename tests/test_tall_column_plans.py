@@ -16,10 +16,12 @@ def _tall(plan):
     ("f32", (500, 256, 64), True), ("f32", (520, 256, 64), False), ("f32", (16, 222, 2244), False), ("f32", (24, 222, 2244), True), ("f32", (8181, 208, 12), False),
     ("f32", (8181, 208, 20), True), ("f32", (1024, 381, 14), False),
     # two bytes, 257 ... 512
-    ("f16", (4200, 311, 16), False), ("f16", (4200, 311, 40), True), ("bf16", (22, 455, 3392), False), ("bf16", (8, 455, 3392), True), ("f16", (18, 410, 180), False),
+    ("f16", (4200, 311, 16), False), ("f16", (4200, 311, 40), True), ("f16", (4200, 311, 10), True), ("f16", (489, 353, 11), False), ("f16", (5810, 323, 17), True),
+    ("bf16", (22, 455, 3392), False), ("f16", (18, 259, 2816), True), ("f16", (15, 415, 2624), False), ("f16", (966, 544, 35), True), ("bf16", (8, 455, 3392), True), ("f16", (18, 410, 180), False),
     ("f16", (180, 410, 180), True),
     # two bytes, beyond 512
-    ("f16", (19, 596, 3821), False), ("f16", (536, 896, 180), False), ("f16", (700, 896, 180), True), ("f16", (98, 1000, 400), False), ("f16", (80, 1000, 400), True),
+    ("f16", (19, 596, 3821), False), ("f16", (20, 1000, 801), True), ("f16", (90, 600, 517), True), ("f16", (40, 777, 1001), False), ("f16", (12, 600, 2051), True),
+    ("f16", (12, 777, 2051), False), ("bf16", (1, 600, 801), False), ("f16", (536, 896, 180), False), ("f16", (700, 896, 180), True), ("f16", (98, 1000, 400), False), ("f16", (80, 1000, 400), True),
     ("f16", (140, 1000, 400), True), ("f16", (190, 1000, 400), False), ("f16", (3, 600, 10000), True), ("f16", (4, 600, 10000), False)])
 def test_where_the_form_is_taken(hpt, dtype, shape, tall):
     plan = hpt.normalize_plan(hpt.Tensor.from_raw(1 << 40, list(shape), getattr(hpt, dtype)), 1)
@@ -27,8 +29,8 @@ def test_where_the_form_is_taken(hpt, dtype, shape, tall):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("dtype,shape", [("f32", (520, 256, 64)), ("f32", (700, 208, 12)), ("f16", (900, 311, 16)), ("bf16", (900, 342, 27)), ("f16", (18, 410, 180)),
-                                         ("f16", (5, 596, 3821)), ("bf16", (270, 640, 200))])
+@pytest.mark.parametrize("dtype,shape", [("f32", (520, 256, 64)), ("f32", (700, 208, 12)), ("f16", (900, 311, 16)), ("bf16", (900, 342, 27)), ("f16", (900, 353, 11)), ("bf16", (300, 290, 10)), ("f16", (18, 410, 180)),
+                                         ("f16", (5, 700, 3821)), ("f16", (5, 596, 3821)), ("bf16", (90, 600, 517)), ("bf16", (270, 640, 200))])
 def test_results_of_the_others(hpt, dev, dtype, shape):
     rng = np.random.default_rng(shape[2])
     x = (rng.standard_normal(shape, dtype=np.float32) * 3)
