@@ -1455,9 +1455,10 @@ NormPlan plan_normalize(const void* in_data, const void* out_data, const int64_t
                 if (p.tsplit > 64) p.tsplit = (int)std::max<int64_t>(64, std::min<int64_t>(p.tsplit, p.cols / 64));
             } else {
                 // Single elements, of which a wavefront has little to read and its last lanes often nothing: two workgroups per unit, up to
-                // 64 partials per row, 128 of a long axis (us, full rounds and this: f16 [2056, 271] 10.1 and 9.2, [4270, 268] 12.1 and 11.3, f32 [7353,
-                // 79] 14.4 and 13.3, [4100, 63] 64 10.8, 128 11.2; [13675, 122] 64 17.3, 128 16.6).
-                p.tsplit = (int)std::max<int64_t>(1, std::min<int64_t>({512 / groups, p.cols / 32, p.cols >= 10000 ? 128 : 64}));
+                // 64 partials per row, 128 or 256 of a long axis (us, full rounds and this: f16 [2056, 271] 10.1 and 9.2, [4270, 268] 12.1 and 11.3, f32 [7353,
+                // 79] 14.4 and 13.3, [4100, 63] 64 10.8, 128 11.2; [13675, 122] 64 17.3, 128 16.6; [138341, 11]
+                // 128 30.4, 256 26.4, [81669, 10] 22.2 and 20.5, f64 [68163, 15] 31.8 and 29.2).
+                p.tsplit = (int)std::max<int64_t>(1, std::min<int64_t>({512 / groups, p.cols / 32, p.cols >= 50000 ? 256 : p.cols >= 10000 ? 128 : 64}));
             }
             p.tpr = elem_size == 2 && v > 1 && p.cols >= 128 * p.tsplit ? 8 : 4;  // wavefronts per workgroup of the statistics pass
             p.scratch_bytes = (size_t)p.rows * p.tsplit * 16 + (size_t)p.rows * 3 * 8;

@@ -268,10 +268,10 @@ __global__ void __launch_bounds__(1024) row_reg_kernel(const NormArgs a) {
     // pays for every type (f32 [3355, 10000] softmax: 3.2 TB/s without).
     // (layernorm(x + residual) holds the residual's vectors as well: with gamma / beta in LDS there is room, and the two reads
     // per write wait less - f16 [13107, 5120] 86.6 -> 75.7 us, [8192, 4096] 41.4 -> 35.4, [32768, 1024] 38.6 -> 34.3, [10000, 8192] 91.7 -> 83.5)
-    // The squares of a layernorm through a function per vector, as unaligned rows need it: for bf16 rows of three vectors with gamma / beta in registers the
-    // compiler keeps fewer values at a time that way (us, the plain loop and this: [47039, 608] 26.8 and 22.6, [16815, 616] 14.5 and 11.8); where
-    // registers are short it costs some, see there.
-    constexpr bool kSquares = std::is_same<T, bf16_t>::value && NCHUNK == 3 && GB == 0 && SS == 1 && !SHIFT;
+    // The squares of a layernorm vector by vector through a function, as unaligned rows need them: what the compiler makes of it is ahead for two-byte rows of two
+    // vectors with gamma / beta in registers, and of three in bf16 (us, the plain loop and this: bf16 [47039, 608] 26.8 and 22.6, [16815, 616] 14.5
+    // and 11.8, f16 [340749, 72] 27.5 and 25.9); elsewhere it costs registers, see there.
+    constexpr bool kSquares = KIND == NORM_LAYERNORM && sizeof(T) == 2 && GB == 0 && SS == 1 && !SHIFT && (NCHUNK == 2 || (NCHUNK == 3 && std::is_same<T, bf16_t>::value));
     constexpr bool kPrefetch = ((sizeof(T) == 2 && NCHUNK * UV <= ((kSoft || GB) ? 32 : 16)) || PF) && (!kRes || GBL);
     const int64_t row_step = (int64_t)gridDim.x * a.rpb;
     Pack<T, VEC> raw[NCHUNK];
@@ -496,17 +496,20 @@ __global__ void __launch_bounds__(1024) row_reg_kernel(const NormArgs a) {
                 const bool in_row_c = (c * tpr + tx) < nv;
                 // (the same arithmetic in two forms, for what the compiler makes of each: see kSquares)
                 if constexpr (UA || kSquares) {
-                    auto square = [&](int j, bool in_row_e) {
-                        const CT d = in_row_e ? (x[c][j] - mean_hi) - mean_lo : (CT)0;
-                        x[c][j] = d;
-                        q += d * d;
+                    auto square = [&](auto last) {
+#pragma unroll
+                        for (int j = 0; j < UV; ++j) {
+                            const bool in_row_e = decltype(last)::value ? j >= twice : in_row_c;
+                            const CT d = in_row_e ? (x[c][j] - mean_hi) - mean_lo : (CT)0;
+                            x[c][j] = d;
+                            q += d * d;
+                        }
                     };
-                    if (UA && c * tpr + tx == nv - 1) {
-#pragma unroll
-                        for (int j = 0; j < UV; ++j) square(j, j >= twice);
+                    if constexpr (UA) {
+                        if (c * tpr + tx == nv - 1) square(std::true_type{});
+                        else square(std::false_type{});
                     } else {
-#pragma unroll
-                        for (int j = 0; j < UV; ++j) square(j, in_row_c);
+                        square(std::false_type{});
                     }
                 } else {
                     // (not through that lambda: it costs aligned rows registers, f16 of four vectors 93 -> 97 and a fifth wavefront, f32 [2441, 12288]

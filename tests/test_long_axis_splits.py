@@ -12,10 +12,10 @@ def _split(hpt, t, *args):
 
 
 # One workgroup per compute unit of 256, or two if they fill the units better: never more, or the scratch of a call outgrows what a
-# capture of before found there. Single elements: two, 64 partials per row of all but the longest axes.
+# capture of before found there. Single elements: two, 64 partials per row of all but long axes.
 @pytest.mark.parametrize("dtype,cols,inner,slices", [
     ("f32", 8190, 4097, 15), ("f64", 1344, 8248, 7), ("f32", 1977, 16400, 7), ("f32", 1300, 40004, 3), ("f16", 2047, 4097, 28), ("f16", 2056, 271, 64),
-    ("f16", 4270, 268, 64), ("f32", 7353, 79, 64), ("f32", 13675, 122, 128), ("f32", 4100, 63, 64), ("f16", 18232, 536, 128)])
+    ("f16", 4270, 268, 64), ("f32", 7353, 79, 64), ("f32", 13675, 122, 128), ("f32", 4100, 63, 64), ("f32", 138341, 11, 256), ("f64", 49999, 15, 128), ("f16", 18232, 536, 128)])
 def test_slices_of_a_long_axis(hpt, dtype, cols, inner, slices):
     t = hpt.Tensor.from_raw(1 << 40, [cols, inner], getattr(hpt, dtype))
     assert hpt.normalize_plan(t, 0).startswith("col-split") and _split(hpt, t, 0) == slices
