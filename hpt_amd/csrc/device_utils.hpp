@@ -117,6 +117,19 @@ template <class T, int N>
 __device__ __forceinline__ Pack<T, N> load_pack(const T* p) {
     return *reinterpret_cast<const Pack<T, N>*>(p);
 }
+// Which part of the work workgroup i of n takes when neighbouring parts share cache lines. Workgroups are handed to the eight XCDs in turn
+// and each XCD has an L2 of its own: numbered as they come, the two sides of a shared line are fetched twice and written in pieces from
+// two caches. Here 2^run_log2 neighbouring parts follow each other on one XCD; fewer than eight such runs at the end (or, with a large
+// run_log2, all there is) are eight equal shares. A permutation of 0 ... n - 1.
+__device__ __forceinline__ unsigned xcd_order(unsigned i, unsigned n, int run_log2) {
+    const unsigned group = 8u << run_log2;
+    const unsigned base = i & ~(group - 1), j = i - base;
+    if (n - base >= group) return base | ((j & 7) << run_log2) | (j >> 3);
+    const unsigned m = n - base, x = j & 7;
+    return base + x * (m >> 3) + min(x, m & 7) + (j >> 3);
+}
+constexpr int kXcdShares = 28;  // run_log2: eight equal shares of the whole launch
+
 template <class T, int N>
 __device__ __forceinline__ void store_pack(T* p, const Pack<T, N>& v) {
     *reinterpret_cast<Pack<T, N>*>(p) = v;

@@ -186,6 +186,18 @@ template <class T, int VEC> void launch_col_split(const NormPlan& p, const NormA
     col_apply_kernel<KIND, T, VEC><<<dim3(rg, (unsigned)chunks, batch), dim3(256), 0, st>>>(t, chunk);
 }
 
+// How many neighbouring workgroups of the column kernels share an XCD, as xcd_order takes it; `whole`: what is right where inner rows
+// start on cache lines. The others share the lines between them: equal shares of the launch while input and output together fit the last-level
+// cache, runs of 32 (an XCD's units) beyond, which keeps what is in flight in one stretch of memory. Us, softmax over axis 1, as numbered by the
+// hardware (col_reg_kernel) or in pairs (col_tall_kernel) and this: f32 [64, 128, 3249] 56.0 and 48.0, [3000, 40, 250] 60.3 and 52.7, f16 [64, 128, 3249]
+// 29.7 and 25.1; runs of 32 and shares: f32 [46, 300, 301] 13.9 and 11.4, [64, 512, 510] 35.2 and 36.1, [129, 512, 510] 81.9 and 92.9. On
+// cache lines nothing moves ([64, 128, 3136] 40.4 and 40.8).
+static int column_run(const ColRegArgs& c, size_t elem_size, int whole) {
+    if ((c.L * (int64_t)elem_size) % 128 == 0 && (c.sa * (int64_t)elem_size) % 128 == 0 && (((uintptr_t)c.in | (uintptr_t)c.out) & 127) == 0) return whole;
+    const int64_t batch = c.total / c.nvec;
+    return batch * c.cols * c.L * (int64_t)elem_size < (48ll << 20) ? kXcdShares : 5;
+}
+
 // A short strided axis held in registers (softmax kinds).
 // WIDE: twice the vectors per thread (128 registers of raw values instead of 64).
 template <class T, int EV, bool WIDE = false> void launch_col_reg(const NormPlan& p, const NormArgs& a, hipStream_t st) {
@@ -202,10 +214,12 @@ template <class T, int EV, bool WIDE = false> void launch_col_reg(const NormPlan
     c.total = (nk > 1 ? p.kept_in.size[0] : 1) * c.nvec;
     c.cols = (int)p.cols;
     c.ty_log2 = ilog2(p.tpr);  // thread rows per inner position
+    c.run_log2 = column_run(c, sizeof(T), 0);
     if (p.tpr > 16 || c.cols > NC * p.tpr)
         fail(HPT_ERR_KERNEL, "col-reg: axis of %d does not fit %d thread rows of %d vectors", c.cols, p.tpr, NC);
     const int64_t tx = 256 / p.tpr;
     const dim3 grid((unsigned)((c.total + tx - 1) / tx));
+    c.blocks = grid.x;
     if constexpr (EV > 1) {
         if (p.shift) {
             col_reg_kernel<KIND, T, EV, NC, true><<<grid, dim3(256), 0, st>>>(c);
@@ -215,11 +229,29 @@ template <class T, int EV, bool WIDE = false> void launch_col_reg(const NormPlan
     col_reg_kernel<KIND, T, EV, NC><<<grid, dim3(256), 0, st>>>(c);
 }
 
+// Whether the result of col_tall_kernel leaves through the caches. Segments that do not end on 64 bytes share what memory writes at once
+// with their neighbours: non-temporal, both parts go out by themselves. Through the cache, with neighbours on one XCD, they meet there. Us, non-temporal
+// and cached: f32 [512, 512, 510] 333 and 255, [512, 512, 500] 328 and 285, [34, 1000, 1001] 103.9 and 87.8, [32, 512, 510] 25.5 and 17.5, f16 [131, 512, 1000]
+// 81.3 and 67.3. Results of 48 to 96 MiB, which stay in the last-level cache for the most part, are ahead without ([84, 200, 1001]
+// 31.2 and 33.3, [64, 512, 510] 35.2 and 33.3) and two-byte ones up to there ([42, 400, 501] 15.2 and 16.1, [167, 400, 501] 41.4 and 44.9, but aligned vectors
+// [66, 512, 1000] 47.4 and 37.1); whole 64-byte pieces always ([512, 512, 528] 219 and 243).
+template <class T> bool tall_stores_cached(const NormPlan& p, const ColRegArgs& c) {
+    const bool pieces = (c.L * (int64_t)sizeof(T)) % 64 == 0 && ((uintptr_t)c.out & 63) == 0;
+    const int64_t mib = c.total / c.nvec * c.cols * c.L * (int64_t)sizeof(T) >> 20;
+    if (pieces) return false;
+    if (sizeof(T) == 2) return mib >= (p.shift ? 96 : 48);
+    return (mib >= 20 && mib < 48) || mib >= 96;
+}
+
 // NT threads, TX of them along the inner dim, NC vectors each.
-template <class T, int NT, int TX, int NC> bool launch_col_tall_as(const NormPlan& p, const ColRegArgs& c, hipStream_t st) {
+template <class T, int NT, int TX, int NC> bool launch_col_tall_as(const NormPlan& p, ColRegArgs& c, hipStream_t st) {
     if (p.tall != NT || p.tpr != NT / TX || p.nchunk != NC || c.cols > NT / TX * NC) return false;
     const dim3 grid((unsigned)((c.total + TX - 1) / TX));
-    if (p.shift) col_tall_kernel<KIND, T, NT, TX, NC, true><<<grid, dim3(NT), 0, st>>>(c);
+    c.blocks = grid.x;
+    const bool cached = tall_stores_cached<T>(p, c);
+    if (p.shift && cached) col_tall_kernel<KIND, T, NT, TX, NC, true, true><<<grid, dim3(NT), 0, st>>>(c);
+    else if (p.shift) col_tall_kernel<KIND, T, NT, TX, NC, true><<<grid, dim3(NT), 0, st>>>(c);
+    else if (cached) col_tall_kernel<KIND, T, NT, TX, NC, false, true><<<grid, dim3(NT), 0, st>>>(c);
     else col_tall_kernel<KIND, T, NT, TX, NC><<<grid, dim3(NT), 0, st>>>(c);
     return true;
 }
@@ -236,6 +268,7 @@ template <class T> void launch_col_tall(const NormPlan& p, const NormArgs& a, hi
     c.nvec = (c.L + EV - 1) / EV;
     c.total = (nk > 1 ? p.kept_in.size[0] : 1) * c.nvec;
     c.cols = (int)p.cols;
+    c.run_log2 = column_run(c, sizeof(T), 1);
     if (c.L < EV || p.vec != EV || (!p.shift && c.L % EV != 0)) fail(HPT_ERR_KERNEL, "col-reg: inner rows of %lld elements are not whole vectors", (long long)c.L);
     bool done = false;
     if constexpr (sizeof(T) == 4) {

@@ -519,6 +519,8 @@ struct ColRegArgs {
     int64_t L;      // inner length
     int cols;       // axis length (<= NC << ty_log2)
     int ty_log2;    // log2 of the thread rows that share an inner position
+    int run_log2;   // neighbouring workgroups that run on one XCD (see xcd_order); 0: as they come
+    unsigned blocks;  // workgroups of the launch
 };
 
 // Make the compiler forget what it knows about a pack: between two sweeps over the raw values it
@@ -546,7 +548,7 @@ __global__ void __launch_bounds__(256) col_reg_kernel(const ColRegArgs a) {
     const int TX = 256 >> a.ty_log2;
     const int tx = threadIdx.x & (TX - 1);
     const int ty = threadIdx.x >> (8 - a.ty_log2);
-    const int64_t g = (int64_t)blockIdx.x * TX + tx;
+    const int64_t g = (int64_t)(a.run_log2 ? xcd_order(blockIdx.x, a.blocks, a.run_log2) : blockIdx.x) * TX + tx;
     const bool valid = g < a.total;
     int64_t b = 0, q = 0;
     if (valid) {
@@ -697,12 +699,15 @@ __global__ void __launch_bounds__(256) col_reg_kernel(const ColRegArgs a) {
 // workgroups of 1024 per compute unit, one loading while the other stores, two-byte ones with NC = 8 take 68 (three workgroups of 512); NC = 16
 // takes 94 ... 100, room for two workgroups of 512 but only one of 1024 (which the plan's rules on the count of workgroups follow). Bound by memory: the same kernel
 // without its arithmetic takes as long (f32 512^3 over axis 1 189 us, at 5.7 TB/s; with col_reg_kernel 210).
-// Segments that are neighbours in an inner row go to one XCD, in pairs (workgroups i and i + 8): 199 -> 190 us there, and
-// unaligned segments share the line between them (f32 [512, 65538] over axis 0 91.0 -> 84.9).
+// Segments that are neighbours in an inner row go to one XCD, in pairs (workgroups i and i + 8) where inner rows start on cache lines: 199 -> 190 us
+// there. The others share lines and go in longer runs, and CACHED lets the parts of a line meet in the XCD's L2 before memory sees them; column_run
+// and tall_stores_cached in norm_op.hip have the rules (f32 [512, 512, 510] 358 -> 241 us, [16, 1000, 2047] 92 -> 72, [96, 564, 157] 31.7 -> 19.9).
+// (The compiler is held to 64 registers with NC = 8: log_softmax of unaligned four-byte rows took 66, [476, 475, 53] 30.8 us, now 24.7 with three of them
+// spilled.)
 // (device us, softmax over axis 1, col_reg_kernel -> this: f32 [64, 512, 1024] 54.4 -> 50.6, [1, 335, 58050] 89.2 -> 45.2,
 // [16, 1000, 2048] 90.8 -> 56.6, [64, 200, 1000] 32.3 -> 23.1, f16 [256, 320, 500] 86.2 -> 49.7, [300, 130, 500] 25.4 -> 20.2)
-template <int KIND, class T, int NT, int TX, int NC, bool UA = false>
-__global__ void __launch_bounds__(NT) col_tall_kernel(const ColRegArgs a) {
+template <int KIND, class T, int NT, int TX, int NC, bool UA = false, bool CACHED = false>
+__global__ void __launch_bounds__(NT, sizeof(T) == 4 && NC == 8 ? 8 : 1) col_tall_kernel(const ColRegArgs a) {
     static_assert(KIND == NORM_SOFTMAX || KIND == NORM_LOGSOFTMAX, "a softmax kernel");
     using CT = typename Elem<T>::Wide;
     using ST = typename StatType<T>::type;
@@ -712,9 +717,7 @@ __global__ void __launch_bounds__(NT) col_tall_kernel(const ColRegArgs a) {
     __shared__ __align__(16) ST part_raw[NW * TX * EV];
     __shared__ __align__(16) ST res_raw[TX * EV];
     const int tx = threadIdx.x % TX, ty = threadIdx.x / TX;
-    int64_t blk = blockIdx.x;
-    if (blk < (int64_t)(gridDim.x & ~15u)) blk = (blk & ~(int64_t)15) | ((blk & 7) << 1) | ((blk >> 3) & 1);
-    const int64_t g = blk * TX + tx;
+    const int64_t g = (int64_t)(a.run_log2 ? xcd_order(blockIdx.x, a.blocks, a.run_log2) : blockIdx.x) * TX + tx;
     const bool valid = g < a.total;
     int64_t b = 0, q = 0;
     if (valid) {
@@ -819,12 +822,15 @@ __global__ void __launch_bounds__(NT) col_tall_kernel(const ColRegArgs a) {
             T* dst = out + (int64_t)(ty_st + i * TY) * a.L;
             if constexpr (UA) {
                 if (skip == 0) {
-                    store_pack_unaligned_stream<T, EV>(dst, o);
+                    if constexpr (CACHED) store_pack_unaligned<T, EV>(dst, o);
+                    else store_pack_unaligned_stream<T, EV>(dst, o);
                 } else {
 #pragma unroll
                     for (int k = 0; k < EV; ++k)
                         if (k >= skip) dst[k] = o.v[k];
                 }
+            } else if constexpr (CACHED) {
+                store_pack<T, EV>(dst, o);
             } else {
                 store_pack_stream<T, EV>(dst, o);
             }

@@ -1,0 +1,40 @@
+"""Softmax over an axis whose inner rows do not start on cache lines: neighbouring workgroups share the lines between them, and the launches
+number them so that neighbours run on one XCD and choose how results are stored by the size of the result. Sizes on both sides of each of
+those lines, with counts of workgroups that leave the last run partly filled, against numpy in 64 bits."""
+import numpy as np
+import pytest
+
+from conftest import assert_close
+from util import F32_ATOL, F32_RTOL, HALF_RTOL, half_atol
+
+pytestmark = pytest.mark.gpu
+
+
+def _softmax64(x, axis):
+    e = np.exp(x - x.max(axis, keepdims=True))
+    return e / e.sum(axis, keepdims=True)
+
+
+# (shape, dtype): equal shares below 48 MiB, runs of 32 workgroups above; results through the cache from 20 to 48 MiB and from 96 MiB on for four
+# bytes, from 48 (aligned) or 96 MiB on for two
+MIDDLE = [((5, 129, 45), "f32"), ((1, 257, 61), "f32"), ((52, 300, 301), "f32"), ((64, 300, 301), "f32"), ((46, 512, 600), "f32"), ((83, 512, 600), "f32"),
+          ((83, 513, 598), "f32"), ((3, 70, 1001), "f32"), ((101, 64, 2001), "f32"), ((7, 513, 36), "f32"),
+          ((66, 512, 1000), "f16"), ((99, 512, 1001), "f16"), ((40, 200, 1001), "f16"), ((3, 66, 75), "f16")]
+
+
+@pytest.mark.parametrize("shape,dtype", MIDDLE, ids=lambda v: v if isinstance(v, str) else "x".join(map(str, v)))
+def test_softmax_over_the_middle_axis(hpt, dev, shape, dtype):
+    rng = np.random.default_rng(71)
+    x = (rng.standard_normal(shape, dtype=np.float32) * 3).astype(np.float32 if dtype == "f32" else np.float16)
+    x[0, :, 0] = -50
+    x[-1, -1, -1] = 40  # the last element of all dominates its column
+    want = _softmax64(x.astype(np.float64), 1)
+    t = hpt.Tensor.from_numpy(x).to_hip(dev)
+    got = t.softmax(1).numpy().astype(np.float64)
+    half = dtype == "f16"
+    assert_close(got, want, HALF_RTOL if half else F32_RTOL, max(half_atol(want, 11), 6e-8) if half else F32_ATOL, f"{shape} {dtype}")
+    if x.size < 4 << 20:
+        got = t.log_softmax(1).numpy().astype(np.float64)
+        log = x.astype(np.float64) - x.max(1, keepdims=True)
+        log -= np.log(np.exp(log).sum(1, keepdims=True))
+        assert_close(got, log, HALF_RTOL if half else F32_RTOL, half_atol(log, 11) if half else F32_ATOL, f"log {shape} {dtype}")
