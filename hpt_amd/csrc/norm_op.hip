@@ -157,33 +157,43 @@ template <class T, int VEC> void launch_col_split(const NormPlan& p, const NormA
     const unsigned rg = (unsigned)((t.R + 64 * VEC - 1) / (64 * VEC));
     const bool ua = VEC > 1 && p.shift;  // inner rows off the vector grid: unaligned vectors
     if (ua && t.R < VEC) fail(HPT_ERR_KERNEL, "col-split: an inner row of %d elements holds no vector of %d", t.R, VEC);
+    // Inner rows of vectors that do not start on cache lines: neighbours in x share lines, and the grids of the two large passes are dealt to the XCDs in
+    // eight equal parts. Us over axis 0, as numbered by the hardware and this: f32 [8190, 4097] 78.4 and 72.3, [8192, 4112] 78.6 and 73.0, [30000, 1001]
+    // 69.4 and 65.4, f16 [8190, 4097] 43.8 and 40.2, bf16 [2700, 12001] 39.9 and 38.2. Rows that start on lines lose by it ([8192, 4096]
+    // 66.6 and 68.5), and so do inputs below 16 MiB ([2000, 1111] 17.4 and 17.8).
+    const bool on_lines = (t.R * (int64_t)sizeof(T)) % 128 == 0 && (t.sa * (int64_t)sizeof(T)) % 128 == 0 && (((uintptr_t)t.in | (uintptr_t)t.out) & 127) == 0;
+    const bool shared = VEC > 1 && !on_lines && (int64_t)batch * t.cols * t.R * (int64_t)sizeof(T) >= (16ll << 20);
+    auto set_grid = [&](const dim3& g) {
+        t.gx = g.x;
+        t.gy = g.y;
+        const uint64_t n = (uint64_t)g.x * g.y * g.z;
+        t.shared = shared && n < (1ull << 31) ? (unsigned)n : 0;
+        return g;
+    };
+    const dim3 sgrid = set_grid(dim3(rg, (unsigned)t.S, batch));
     if constexpr (VEC > 1) {
         if (ua)
-            transposed_stats_kernel<KIND, T, VEC, true>
-                <<<dim3(rg, (unsigned)t.S, batch), dim3(64 * nw), (size_t)nw * VEC * 64 * sizeof(Part), st>>>(t);
+            transposed_stats_kernel<KIND, T, VEC, true><<<sgrid, dim3(64 * nw), (size_t)nw * VEC * 64 * sizeof(Part), st>>>(t);
     }
     if (!ua)
-        transposed_stats_kernel<KIND, T, VEC>
-            <<<dim3(rg, (unsigned)t.S, batch), dim3(64 * nw), (size_t)nw * VEC * 64 * sizeof(Part), st>>>(t);
+        transposed_stats_kernel<KIND, T, VEC><<<sgrid, dim3(64 * nw), (size_t)nw * VEC * 64 * sizeof(Part), st>>>(t);
     transposed_finalize_kernel<KIND, T><<<dim3((unsigned)((t.R + 15) / 16), 1, batch), dim3(16, 16), 0, st>>>(t);
     // apply: sixteen positions of the axis per workgroup, one batch of four loads per thread; what runs at one time is then
     // one stretch of memory (f32 [8192, 4096] over axis 0, all three passes, 16 / 32 / 48 positions: 65.2, 70.7, 67.4 us;
-    // [32768, 1024] 66.3, 68.4, 68.6; f16 [8190, 4097] 42.0, 43.1, 43.1)
-    // (Twelve where sixteen unaligned positions span 256 KiB and a line or less: the workgroups that run together then start almost in
-    // step with the memory's interleaving. f32 [2047, 4097] 30.5 -> 28.2 us, [8190, 4097] 77.3 -> 75.5, f16 [2047, 8193] 29.1 -> 27.5; with
-    // aligned rows, with other multiples of 256 KiB and two lines off it there is no difference.)
-    const int64_t span = 16 * t.sa * (int64_t)sizeof(T) - (256 << 10);
-    const int64_t most = ua && span >= 0 && span <= 128 ? 12 : 16;
+    // [32768, 1024] 66.3, 68.4, 68.6; f16 [8190, 4097] 42.0, 43.1, 43.1). Where lines are shared eight, so that what an XCD has in flight is a
+    // shorter stretch (8 / 16 positions: f32 [8190, 4097] 71.7 and 73.2, [30000, 1001] 65.4 and 66.3, f16 [8190, 4097] 40.3 and 41.2).
+    const int64_t most = shared ? 8 : 16;
     int64_t chunks = std::min<int64_t>((t.cols + most - 1) / most, 65535);
     const int chunk = (int)((t.cols + chunks - 1) / chunks);
     chunks = (t.cols + chunk - 1) / chunk;
+    const dim3 agrid = set_grid(dim3(rg, (unsigned)chunks, batch));
     if constexpr (VEC > 1) {
         if (ua) {
-            col_apply_kernel<KIND, T, VEC, true><<<dim3(rg, (unsigned)chunks, batch), dim3(256), 0, st>>>(t, chunk);
+            col_apply_kernel<KIND, T, VEC, true><<<agrid, dim3(256), 0, st>>>(t, chunk);
             return;
         }
     }
-    col_apply_kernel<KIND, T, VEC><<<dim3(rg, (unsigned)chunks, batch), dim3(256), 0, st>>>(t, chunk);
+    col_apply_kernel<KIND, T, VEC><<<agrid, dim3(256), 0, st>>>(t, chunk);
 }
 
 // How many neighbouring workgroups of the column kernels share an XCD, as xcd_order takes it; `whole`: what is right where inner rows

@@ -40,7 +40,18 @@ struct TransposedArgs {
     int S;            // workgroups sharing the axis in the statistics pass
     int nw;           // wavefronts per workgroup of the statistics pass
     int y0;           // last pass: column block of blockIdx.y = 0 (a grid has at most 65535 of them)
+    unsigned gx, gy, shared;  // the launch's grid in x and y; > 0: workgroups in all, neighbours in x share cache lines
 };
+
+// Which workgroup of the grid this one is: where neighbours in x share cache lines, the grid is dealt to the XCDs in eight equal parts.
+struct GridPlace {
+    unsigned x, y, z;
+};
+__device__ __forceinline__ GridPlace grid_place(const TransposedArgs& a) {
+    if (!a.shared) return {blockIdx.x, blockIdx.y, blockIdx.z};
+    const unsigned w = xcd_order(blockIdx.x + a.gx * (blockIdx.y + a.gy * blockIdx.z), a.shared, kXcdShares), xy = w / a.gx;
+    return {w - xy * a.gx, xy % a.gy, xy / a.gy};
+}
 
 // Columns that wavefront `pid` of the P that share a row's columns takes (it starts at column pid and steps by P), and
 // columns that the nw wavefronts of workgroup y take together.
@@ -89,19 +100,20 @@ __global__ void __launch_bounds__(1024) transposed_stats_kernel(const Transposed
     extern __shared__ __align__(16) unsigned char smem_raw[];
     const int NW = blockDim.x >> 6;  // wavefronts per workgroup (1...16)
 
+    const GridPlace at = grid_place(a);
     const int lane = threadIdx.x & 63;
     // the wavefront index is uniform: say so, and the column arithmetic stays scalar
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     // lanes past the last row keep going (they meet the others at the barrier below) on row 0
-    const bool valid = (blockIdx.x * 64 + lane) * VEC < a.R;
-    const int r0 = valid ? (UA ? min((int)(blockIdx.x * 64 + lane) * VEC, a.R - VEC) : (int)(blockIdx.x * 64 + lane) * VEC) : 0;
+    const bool valid = (at.x * 64 + lane) * VEC < a.R;
+    const int r0 = valid ? (UA ? min((int)(at.x * 64 + lane) * VEC, a.R - VEC) : (int)(at.x * 64 + lane) * VEC) : 0;
     // Columns are dealt out round-robin over all P = S NW wavefronts that share these
     // rows: wavefront p takes columns p, p + P, ... Wavefronts running at the same time
     // then read neighbouring columns, which keeps a power-of-two column pitch from
     // sending them all to the same memory channels.
     const int P = a.S * NW;
-    const int pid = blockIdx.y * NW + w;
-    const T* base = (const T*)a.in + (int64_t)blockIdx.z * a.bi + r0;
+    const int pid = at.y * NW + w;
+    const T* base = (const T*)a.in + (int64_t)at.z * a.bi + r0;
 
     // per row: softmax (max m, sum of exponentials se); layernorm, of the n columns folded so far:
     //   f32  f64 sums of (x - org) and (x - org)^2, org the first element that the lane sees
@@ -264,18 +276,18 @@ __global__ void __launch_bounds__(1024) transposed_stats_kernel(const Transposed
     }
     __syncthreads();
     if (!valid) return;
-    Part* dst = (Part*)a.stats + ((int64_t)blockIdx.z * a.S + blockIdx.y) * a.R + r0;
+    Part* dst = (Part*)a.stats + ((int64_t)at.z * a.S + at.y) * a.R + r0;
     for (int k = w; k < VEC; k += NW) {
         Part t = sm[k * 64 + lane];
         if constexpr (KIND == NORM_LAYERNORM) {
             // the mean first, as differences from the first wavefront's (f64 elements: and once more from the result, which
             // takes out what a first one far from the others has cost), then the deviations from it
-            auto cnt = [&](int o) { return (double)columns_of_wave(a.cols, P, blockIdx.y * NW + o); };
+            auto cnt = [&](int o) { return (double)columns_of_wave(a.cols, P, at.y * NW + o); };
 #pragma unroll
             for (int pass = 0; pass < (sizeof(CT) == 8 ? 2 : 1); ++pass) {
                 double shift = 0;
                 for (int o = 0; o < NW; ++o) shift += cnt(o) * (sm[(o * VEC + k) * 64 + lane].mean - t.mean);
-                t.mean += shift / (double)columns_of_group(a.cols, P, NW, blockIdx.y);
+                t.mean += shift / (double)columns_of_group(a.cols, P, NW, at.y);
             }
             t.m2 = 0;
             for (int o = 0; o < NW; ++o) {
@@ -444,17 +456,18 @@ __global__ void __launch_bounds__(256) col_apply_kernel(const TransposedArgs a, 
     using CT = typename Elem<T>::Wide;
     constexpr bool kLog = KIND == NORM_LOGSOFTMAX;
     const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-    int r0 = (blockIdx.x * 64 + tx) * VEC;
+    const GridPlace at = grid_place(a);
+    int r0 = (at.x * 64 + tx) * VEC;
     if (r0 >= a.R) return;
     const int skip = UA ? max(r0 - (a.R - VEC), 0) : 0;  // leading elements that belong to the vector before
     r0 -= skip;
-    const CT* pp = (const CT*)a.params + (int64_t)blockIdx.z * 3 * a.R + r0;
+    const CT* pp = (const CT*)a.params + (int64_t)at.z * 3 * a.R + r0;
     const Pack<CT, VEC> p0 = UA ? load_pack_unaligned<CT, VEC>(pp) : *reinterpret_cast<const Pack<CT, VEC>*>(pp);
     const Pack<CT, VEC> p1 = UA ? load_pack_unaligned<CT, VEC>(pp + a.R) : *reinterpret_cast<const Pack<CT, VEC>*>(pp + a.R);
-    const T* in = (const T*)a.in + (int64_t)blockIdx.z * a.bi + r0;
-    T* out = (T*)a.out + (int64_t)blockIdx.z * a.cols * a.R + r0;
+    const T* in = (const T*)a.in + (int64_t)at.z * a.bi + r0;
+    T* out = (T*)a.out + (int64_t)at.z * a.cols * a.R + r0;
     // (the axis from its end backwards: what the statistics pass read last is read first)
-    const int block = gridDim.y - 1 - blockIdx.y;
+    const int block = a.gy - 1 - at.y;
     const int c_end = min(a.cols, (block + 1) * chunk);
     auto fetch = [&](int c) {
         if constexpr (UA) return load_pack_unaligned<T, VEC>(in + (int64_t)c * a.sa);
@@ -489,11 +502,18 @@ __global__ void __launch_bounds__(256) col_apply_kernel(const TransposedArgs a, 
 #pragma unroll
             for (int u = 0; u < 4; ++u) apply(v[u], c + 4 * u);
         }
-        for (; c < c_end; c += 4) apply(fetch(c), c);
+        for (; c + 4 < c_end; c += 8) {
+            Pack<T, VEC> v[2];
+#pragma unroll
+            for (int u = 0; u < 2; ++u) v[u] = fetch(c + 4 * u);
+#pragma unroll
+            for (int u = 0; u < 2; ++u) apply(v[u], c + 4 * u);
+        }
+        if (c < c_end) apply(fetch(c), c);
     };
     // (a walk of its own for the workgroups at the rows' ends: with the test in every store f32 [8190, 4097] takes 2.5 us more)
     if constexpr (UA) {
-        if (blockIdx.x == gridDim.x - 1) {
+        if (at.x == a.gx - 1) {
             walk(std::true_type{});
             return;
         }

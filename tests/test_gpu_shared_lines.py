@@ -38,3 +38,20 @@ def test_softmax_over_the_middle_axis(hpt, dev, shape, dtype):
         log = x.astype(np.float64) - x.max(1, keepdims=True)
         log -= np.log(np.exp(log).sum(1, keepdims=True))
         assert_close(got, log, HALF_RTOL if half else F32_RTOL, half_atol(log, 11) if half else F32_ATOL, f"log {shape} {dtype}")
+
+
+# a long axis 0, three launches: vectors whose rows do not start on lines, eight equal parts from 16 MiB on (with one and several batches)
+LONG = [((2047, 2051), "f32"), ((2048, 2048), "f32"), ((1100, 4100), "f32"), ((1031, 1030), "f32"), ((2, 1500, 1502), "f32"), ((4099, 2051), "f16"), ((2500, 4100), "f16")]
+
+
+@pytest.mark.parametrize("shape,dtype", LONG, ids=lambda v: v if isinstance(v, str) else "x".join(map(str, v)))
+def test_softmax_over_a_long_axis(hpt, dev, shape, dtype):
+    axis = len(shape) - 2
+    x = (np.random.default_rng(72).standard_normal(shape, dtype=np.float32) * 3).astype(np.float32 if dtype == "f32" else np.float16)
+    x[..., -1, -1] = 40
+    want = _softmax64(x.astype(np.float64), axis)
+    t = hpt.Tensor.from_numpy(x).to_hip(dev)
+    half = dtype == "f16"
+    for inplace in (False, True):
+        got = t.softmax(axis, out=t if inplace else None).numpy().astype(np.float64)
+        assert_close(got, want, HALF_RTOL if half else F32_RTOL, max(half_atol(want, 11), 6e-8) if half else F32_ATOL, f"{shape} {dtype} inplace={inplace}")
