@@ -307,8 +307,15 @@ template <class T> void launch_transposed(const NormPlan& p, const NormArgs& a, 
         t.eps = a.eps;
         t.inv_cols = a.inv_cols;
         t.rg_log2 = ilog2(p.tpr);
-        t.share_log2 = p.tpr >= 8 ? 0 : (p.tpr == 4 ? 1 : 2);
         const unsigned blocks = (unsigned)((t.R + p.tpr * FULL - 1) / (p.tpr * FULL));
+        // On the vector grid the workgroups that share a line: one (rgN = 8 and more), two or four. Off it neighbours share a line at any rgN: four, or
+        // eight of two-byte rows (us, softmax, stored [columns, rows]: f32 [2001, 8001] 42.5 and 37.8, [1001, 8191] 21.0 and 18.5, [4001, 4001] 40.1 and
+        // 38.1, f16 [2049, 8191] 26.7 and 23.8, [501, 16001] 14.2 and 12.9). Eight neighbours on one XCD also read and write longer stretches, which
+        // counts where every compute unit has a workgroup: f32 [4096, 4096] 32.3 and 30.8, [3000, 6000] 49.5 and 47.3, two-byte rows of up to 2048 columns f16 [2048, 8192] 17.6 and
+        // 16.3, [2000, 12000] 29.2 and 27.9; not f32 [4000, 2048] 23.6 and 24.5, [1728, 6016] 16.9 and 17.3, f16 [3000, 8000] 34.3 and 35.3, [1024, 8192] 9.7 and 9.8.
+        const bool long_stretch = p.tpr == 4 && (sizeof(T) == 2 ? p.rpb <= 8 && (int64_t)t.R * t.cols >= (16ll << 20) : blocks >= 256 && (int64_t)t.R * t.cols >= (12ll << 20));
+        if (p.shift) t.share_log2 = p.tpr == 2 ? 2 : (sizeof(T) == 2 && p.tpr == 4 ? 3 : 2);
+        else t.share_log2 = p.tpr >= 8 ? 0 : (p.tpr == 4 ? (long_stretch ? 3 : 1) : 2);
         if (p.shift) {
             transposed_tile_kernel<KIND, T, true><<<dim3(blocks, batch), dim3(64u * (unsigned)p.rpb), 0, st>>>(t);
             return;
@@ -355,6 +362,12 @@ template <class T> void launch_transposed(const NormPlan& p, const NormArgs& a, 
         // (more column blocks than a grid has in y, from 2^22 four-byte columns on: one launch after the other)
         for (int blocks = (tiles + 1) / 2; t.y0 < blocks; t.y0 += 65535) {
             const dim3 agrid((rt + 3) / 4, (unsigned)std::min(blocks - t.y0, 65535), batch);
+            // off the vector grid neighbours share lines: eight of them in a row on one XCD (us, softmax, stored [columns, rows]: f32 [8190, 4097]
+            // 103.4 and 94.7, f16 59.0 and 50.4, [8192, 4100] 49.8 and 46.2, [5001, 4001] 37.1 and 37.1)
+            const uint64_t n = (uint64_t)agrid.x * agrid.y * agrid.z;
+            t.gx = agrid.x;
+            t.gy = agrid.y;
+            t.shared = n < (1ull << 31) ? (unsigned)n : 0;
             if (p.shift) transposed_apply_kernel<KIND, T, true><<<agrid, dim3(256), 0, st>>>(t);
             else transposed_apply_kernel<KIND, T><<<agrid, dim3(256), 0, st>>>(t);
         }

@@ -40,7 +40,7 @@ struct TransposedArgs {
     int S;            // workgroups sharing the axis in the statistics pass
     int nw;           // wavefronts per workgroup of the statistics pass
     int y0;           // last pass: column block of blockIdx.y = 0 (a grid has at most 65535 of them)
-    unsigned gx, gy, shared;  // the launch's grid in x and y; > 0: workgroups in all, neighbours in x share cache lines
+    unsigned gx, gy, shared;  // the launch's grid in x and y; > 0: workgroups in all, neighbours share cache lines
 };
 
 // Which workgroup of the grid this one is: where neighbours in x share cache lines, the grid is dealt to the XCDs in eight equal parts.
@@ -384,12 +384,20 @@ __global__ void __launch_bounds__(256) transposed_apply_kernel(const TransposedA
 
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int rg = lane & 7, cl = lane >> 3;
-    int r0 = (blockIdx.x * 4 + w) * TR + rg * VEC;
-    const int c_base = (blockIdx.y + a.y0) * (NC * TC) + cl * VEC;
+    // (UA: pieces of output rows share lines with the next column block's: the columns fastest, eight column blocks in a row on one XCD)
+    GridPlace at{blockIdx.x, blockIdx.y, blockIdx.z};
+    if constexpr (UA) {
+        if (a.shared) {
+            const unsigned n = xcd_order(blockIdx.x + a.gx * (blockIdx.y + a.gy * blockIdx.z), a.shared, 3), xy = n / a.gy;
+            at = {xy % a.gx, n - xy * a.gy, xy / a.gx};
+        }
+    }
+    int r0 = (at.x * 4 + w) * TR + rg * VEC;
+    const int c_base = (at.y + a.y0) * (NC * TC) + cl * VEC;
     if (r0 >= a.R || c_base >= a.cols) return;
     if constexpr (UA) r0 = min(r0, a.R - VEC);
 
-    const CT* pp = (const CT*)a.params + (int64_t)blockIdx.z * 3 * a.R + r0;
+    const CT* pp = (const CT*)a.params + (int64_t)at.z * 3 * a.R + r0;
     auto params = [](const CT* p) { return UA ? load_pack_unaligned<CT, VEC>(p) : load_pack<CT, VEC>(p); };
     auto load = [](const T* p) { return UA ? load_pack_unaligned<T, VEC>(p) : load_pack<T, VEC>(p); };
     const Pack<CT, VEC> p0 = params(pp);
@@ -397,7 +405,7 @@ __global__ void __launch_bounds__(256) transposed_apply_kernel(const TransposedA
     Pack<CT, VEC> p2 = p0;
     if constexpr (KIND == NORM_LAYERNORM) p2 = params(pp + 2 * (int64_t)a.R);
 
-    const T* base = (const T*)a.in + (int64_t)blockIdx.z * a.bi + r0;
+    const T* base = (const T*)a.in + (int64_t)at.z * a.bi + r0;
     Pack<T, VEC> v[NC][VEC], gam[NC], bet[NC];
     bool have[NC];
     int col[NC];
@@ -419,7 +427,7 @@ __global__ void __launch_bounds__(256) transposed_apply_kernel(const TransposedA
         }
     }
 
-    T* out = (T*)a.out + ((int64_t)blockIdx.z * a.R + r0) * a.cols;
+    T* out = (T*)a.out + ((int64_t)at.z * a.R + r0) * a.cols;
 #pragma unroll
     for (int k = 0; k < VEC; ++k)
 #pragma unroll
@@ -1025,7 +1033,7 @@ __global__ void __launch_bounds__(1024) col_flat_apply_kernel(const TransposedAr
 // (CGW = 64 / rgN). A load instruction therefore reads 16 * rgN contiguous bytes per
 // column; a store instruction writes, per row, VEC * CGW consecutive columns.
 //
-// With rgN = 4 (2) a 128-byte line of the input is shared by two (four) workgroups.
+// With rgN = 4 (2) a 128-byte line of the input is shared by two (four) workgroups, off the vector grid by neighbours at any rgN.
 // Workgroups are handed to the eight XCDs (each with its own L2) round-robin, so the
 // row blocks are renumbered to put the parts of a line on workgroups i, i + 8, (i + 16,
 // i + 24): same XCD, dispatched together, and all but the first hit in L2.
@@ -1040,7 +1048,7 @@ struct TileArgs {
     int R;       // rows per batch (contiguous in the input)
     int cols;
     int rg_log2; // log2(rgN), rgN = 2, 4, 8 or 16
-    int share_log2;  // log2 of the workgroups that share a 128-byte line of the input (0, 1 or 2)
+    int share_log2;  // log2 of the neighbouring workgroups that run on one XCD
 };
 
 // All-reduce of VEC row values over every thread that holds a piece of the same rows:

@@ -55,3 +55,21 @@ def test_softmax_over_a_long_axis(hpt, dev, shape, dtype):
     for inplace in (False, True):
         got = t.softmax(axis, out=t if inplace else None).numpy().astype(np.float64)
         assert_close(got, want, HALF_RTOL if half else F32_RTOL, max(half_atol(want, 11), 6e-8) if half else F32_ATOL, f"{shape} {dtype} inplace={inplace}")
+
+
+# stored [columns, rows], normalised along the columns: three launches with unaligned vectors beyond 4096 columns (column blocks of 64 or 128, the last
+# one partly filled; one and two batches), register tiles below; aligned tiles that run eight in a row on an XCD
+TRANSPOSED = [((4500, 701), "f32"), ((4101, 1030), "f16"), ((2, 4200, 259), "f32"), ((1001, 2603), "f32"), ((900, 5003), "f16"), ((3500, 4112), "f32"), ((2048, 8256), "f16")]
+
+
+@pytest.mark.parametrize("shape,dtype", TRANSPOSED, ids=lambda v: v if isinstance(v, str) else "x".join(map(str, v)))
+def test_transposed_rows(hpt, dev, shape, dtype):
+    x = (np.random.default_rng(73).standard_normal(shape, dtype=np.float32) * 3).astype(np.float32 if dtype == "f32" else np.float16)
+    x[..., -1, -1] = 40
+    perm = [0, 2, 1][-len(shape):] if len(shape) == 3 else [1, 0]
+    v = x.astype(np.float64).transpose(perm)
+    t = hpt.Tensor.from_numpy(x).to_hip(dev).permute(perm)
+    half = dtype == "f16"
+    for name, want, got in [("softmax", _softmax64(v, -1), t.softmax(len(shape) - 1)),
+                            ("layernorm", (v - v.mean(-1, keepdims=True)) / np.sqrt(v.var(-1, keepdims=True) + 1e-5), t.layernorm([shape[-2]]))]:
+        assert_close(got.numpy().astype(np.float64), want, HALF_RTOL if half else F32_RTOL, max(half_atol(want, 11), 6e-8) if half else F32_ATOL, f"{name} {shape} {dtype}")
