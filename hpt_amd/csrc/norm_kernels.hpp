@@ -1145,6 +1145,30 @@ template <class CT> struct MomentStatOp {
     }
 };
 
+// (max, sum of exponentials) of `width` neighbouring lanes in each of them, and of a workgroup in every thread: the maximum first, then every side's sum
+// rescaled once and the sums added. (Merged pairwise with SoftStatOp, every step of the butterfly waits for an exponential: statistics
+// and last pass of a split row, us: bf16 [1, 62020] log_softmax 4.7 + 5.0 and 4.4 + 4.6, f32 [5, 33088] 5.2 + 4.9 and 4.6 + 3.6.) smem holds one element per wavefront, 16 at most.
+template <class T, class CT, class ST> __device__ __forceinline__ ST soft_rescale(SoftStat<CT, ST> v, CT m) {
+    return v.s == (ST)0 ? (ST)0 : v.s * (ST)exp_ct<T>(v.m - m);  // a side that has seen nothing must not produce inf - inf
+}
+template <class T, class CT, class ST> __device__ __forceinline__ SoftStat<CT, ST> group_soft(SoftStat<CT, ST> v, int width) {
+    const CT m = group_reduce<MaxC<CT>>(v.m, width);
+    return {m, group_reduce<SumC<ST>>(soft_rescale<T>(v, m), width)};
+}
+template <class T, class CT, class ST> __device__ __forceinline__ SoftStat<CT, ST> block_soft(SoftStat<CT, ST> v, SoftStat<CT, ST>* smem) {
+    const int tid = threadIdx.y * blockDim.x + threadIdx.x, nwaves = (blockDim.x * blockDim.y) >> 6;
+    v = group_soft<T>(v, 64);
+    __syncthreads();  // protect smem from a previous use
+    if ((tid & 63) == 0) smem[tid >> 6] = v;
+    __syncthreads();
+    SoftStat<CT, ST> r{smem[0].m, (ST)0};
+#pragma unroll 4
+    for (int w = 1; w < nwaves; ++w) r.m = MaxC<CT>::comb(r.m, smem[w].m);
+#pragma unroll 4
+    for (int w = 0; w < nwaves; ++w) r.s += soft_rescale<T>(smem[w], r.m);
+    return r;
+}
+
 template <class Op, class S> __device__ __forceinline__ S stat_all_reduce(S v, int tpr, S* smem) {
     if (tpr == 1) return v;
     if (tpr <= 64) return group_reduce<Op>(v, tpr);
@@ -1299,7 +1323,8 @@ __global__ void __launch_bounds__(1024) row_stream_kernel(const NormArgs a) {
                 take(iv, x);
             }
         }
-        st = stat_all_reduce<SoftStatOp<T, CT, ST>>(st, tpr, (SoftStat<CT, ST>*)smem_raw);
+        if (tpr > 64) st = block_soft<T>(st, (SoftStat<CT, ST>*)smem_raw);
+        else if (tpr > 1) st = group_soft<T>(st, tpr);
         if (!valid) return;
         const CT k = kLog ? log_ct<T>((CT)st.s) : (CT)((ST)1 / st.s);
         auto finish = [&](int64_t iv, CT* x) {
@@ -1506,18 +1531,40 @@ template <class T, int VEC, bool UA> __device__ __forceinline__ Pack<T, VEC> row
     else return load_pack<T, VEC>(p);
 }
 
-// the VEC elements of a row from element e0 on, with the residual added where the kind says so
+// The VEC elements of a row from element e0 on, as loaded and as they count: with the residual added where the kind says so.
+template <int KIND, class T, int VEC> struct RowSplitRaw {
+    Pack<T, VEC> v;
+    Pack<T, KIND == NORM_ADD_LAYERNORM ? VEC : 1> r;
+};
 template <int KIND, class T, int VEC, bool UA>
-__device__ __forceinline__ void row_split_load(const RowSplitArgs& a, const T* in_row, int64_t row, int64_t e0,
-                                               typename Elem<T>::Wide (&x)[VEC]) {
-    const Pack<T, VEC> v = row_split_pack<T, VEC, UA>(in_row + e0);
+__device__ __forceinline__ RowSplitRaw<KIND, T, VEC> row_split_load(const RowSplitArgs& a, const T* in_row, int64_t row, int64_t e0) {
+    RowSplitRaw<KIND, T, VEC> x;
+    x.v = row_split_pack<T, VEC, UA>(in_row + e0);
+    if constexpr (KIND == NORM_ADD_LAYERNORM) x.r = row_split_pack<T, VEC, UA>((const T*)a.residual + row * a.cols + e0);
+    return x;
+}
+template <int KIND, class T, int VEC>
+__device__ __forceinline__ void row_split_widen(const RowSplitRaw<KIND, T, VEC>& raw, typename Elem<T>::Wide (&x)[VEC]) {
 #pragma unroll
-    for (int j = 0; j < VEC; ++j) x[j] = Elem<T>::widen(v.v[j]);
-    if constexpr (KIND == NORM_ADD_LAYERNORM) {
-        const Pack<T, VEC> r = row_split_pack<T, VEC, UA>((const T*)a.residual + row * a.cols + e0);
-#pragma unroll
-        for (int j = 0; j < VEC; ++j) x[j] = Elem<T>::widen(Elem<T>::narrow(x[j] + Elem<T>::widen(r.v[j])));
+    for (int j = 0; j < VEC; ++j) {
+        x[j] = Elem<T>::widen(raw.v.v[j]);
+        if constexpr (KIND == NORM_ADD_LAYERNORM) x[j] = Elem<T>::widen(Elem<T>::narrow(x[j] + Elem<T>::widen(raw.r.v[j])));
     }
+}
+// A thread's vectors of its workgroup's slice, four at a time in flight (one after the other each waits a memory latency; those beyond the
+// slice load its last vector once more). Softmax: layernorm, whose f64 sums take longer than the loads, lost by it (us, f32 [16, 300007] 16.5 and
+// 17.1, [16, 300000] 14.6 and 15.1).
+constexpr int kRowSplitBatch = 4;
+template <int KIND, class T, int VEC, bool UA>
+__device__ __forceinline__ void row_split_fetch(const RowSplitArgs& a, const T* in_row, int64_t row, int64_t iv, int64_t v1,
+                                                RowSplitRaw<KIND, T, VEC> (&raw)[kRowSplitBatch]) {
+    constexpr int NB = kRowSplitBatch;
+#pragma unroll
+    for (int u = 0; u < NB; ++u) {
+        const int64_t i = min(iv + u * 256, v1 - 1);
+        raw[u] = row_split_load<KIND, T, VEC, UA>(a, in_row, row, row_split_start<VEC, UA>(i, a.cols));
+    }
+    __builtin_amdgcn_sched_barrier(0);  // (no load sinks into what is done with the others)
 }
 
 // The moments of every thread of a workgroup of four wavefronts as one, in every thread. Sums of differences from the first
@@ -1534,6 +1581,7 @@ __device__ __forceinline__ MomentStat<double> block_moments(MomentStat<double> v
 
 template <int KIND, class T, int VEC, bool UA>
 __global__ void __launch_bounds__(256) row_split_stats_kernel(const RowSplitArgs a) {
+    constexpr int NB = kRowSplitBatch;
     using CT = typename Elem<T>::Wide;
     using ST = typename StatType<T>::type;
     __shared__ __align__(16) unsigned char smem_raw[16 * 3 * sizeof(double)];
@@ -1543,31 +1591,37 @@ __global__ void __launch_bounds__(256) row_split_stats_kernel(const RowSplitArgs
     const int64_t v0 = (int64_t)blockIdx.x * a.chunk_v, v1 = min(nv, v0 + a.chunk_v);
     if constexpr (!norm_is_layer(KIND)) {
         SoftStat<CT, ST> st{neg_inf<CT>(), (ST)0};
-        for (int64_t iv = v0 + threadIdx.x; iv < v1; iv += 256) {
-            CT x[VEC];
-            const int64_t e0 = row_split_start<VEC, UA>(iv, a.cols);
-            row_split_load<KIND, T, VEC, UA>(a, in_row, row, e0, x);
-            if constexpr (UA) {
-                const int skip = (int)(iv * VEC - e0);
+        for (int64_t i0 = v0 + threadIdx.x; i0 < v1; i0 += 256 * NB) {
+            RowSplitRaw<KIND, T, VEC> raw[NB];
+            row_split_fetch<KIND, T, VEC, UA>(a, in_row, row, i0, v1, raw);
 #pragma unroll
-                for (int j = 0; j < VEC; ++j)
-                    if (j < skip) x[j] = neg_inf<CT>();
-            }
-            CT cm = x[0];
+            for (int u = 0; u < NB; ++u) {
+                const int64_t iv = i0 + u * 256;
+                if (iv >= v1) break;
+                CT x[VEC];
+                row_split_widen<KIND, T, VEC>(raw[u], x);
+                if constexpr (UA) {
+                    const int skip = (int)(iv * VEC - row_split_start<VEC, UA>(iv, a.cols));
 #pragma unroll
-            for (int j = 1; j < VEC; ++j) cm = MaxC<CT>::comb(cm, x[j]);
-            if (cm > st.m) {
-                st.s = st.s == (ST)0 ? (ST)0 : st.s * (ST)exp_ct<T>(st.m - cm);
-                st.m = cm;
-            }
-            if (st.m > neg_inf<CT>()) {
-                CT part = 0;
+                    for (int j = 0; j < VEC; ++j)
+                        if (j < skip) x[j] = neg_inf<CT>();
+                }
+                CT cm = x[0];
 #pragma unroll
-                for (int j = 0; j < VEC; ++j) part += exp_ct<T>(x[j] - st.m);
-                st.s += (ST)part;
+                for (int j = 1; j < VEC; ++j) cm = MaxC<CT>::comb(cm, x[j]);
+                if (cm > st.m) {
+                    st.s = st.s == (ST)0 ? (ST)0 : st.s * (ST)exp_ct<T>(st.m - cm);
+                    st.m = cm;
+                }
+                if (st.m > neg_inf<CT>()) {
+                    CT part = 0;
+#pragma unroll
+                    for (int j = 0; j < VEC; ++j) part += exp_ct<T>(x[j] - st.m);
+                    st.s += (ST)part;
+                }
             }
         }
-        st = block_reduce<SoftStatOp<T, CT, ST>>(st, (SoftStat<CT, ST>*)smem_raw);
+        st = block_soft<T>(st, (SoftStat<CT, ST>*)smem_raw);
         if (threadIdx.x == 0) ((SoftStat<CT, ST>*)a.part)[row * a.S + blockIdx.x] = st;
     } else {
         // Per thread: f64 sums around an element of its own (the last of its first vector, which is no other thread's), turned
@@ -1580,7 +1634,7 @@ __global__ void __launch_bounds__(256) row_split_stats_kernel(const RowSplitArgs
         for (int64_t iv = v0 + threadIdx.x; iv < v1; iv += 256) {
             CT x[VEC];
             const int64_t e0 = row_split_start<VEC, UA>(iv, a.cols);
-            row_split_load<KIND, T, VEC, UA>(a, in_row, row, e0, x);
+            row_split_widen<KIND, T, VEC>(row_split_load<KIND, T, VEC, UA>(a, in_row, row, e0), x);
             const int skip = UA ? (int)(iv * VEC - e0) : 0;
             if (n == 0) k = (double)x[VEC - 1];
             n += VEC - skip;
@@ -1608,34 +1662,41 @@ __global__ void __launch_bounds__(256) row_split_stats_kernel(const RowSplitArgs
 // few hundred loads), then re-reads its slice and writes the result.
 template <int KIND, class T, int VEC, bool UA>
 __global__ void __launch_bounds__(256) row_split_apply_kernel(const RowSplitArgs a) {
+    constexpr int NB = kRowSplitBatch;
     using CT = typename Elem<T>::Wide;
     using ST = typename StatType<T>::type;
     __shared__ __align__(16) unsigned char smem_raw[16 * 3 * sizeof(double)];
     const int64_t row = blockIdx.y;
     const T* in_row = (const T*)a.in + offset_of(a.kept_in, row);
     T* out_row = (T*)a.out + row * a.cols;
+    const int64_t nv = row_split_vectors<VEC, UA>(a.cols);
+    const int64_t v0 = (int64_t)blockIdx.x * a.chunk_v, v1 = min(nv, v0 + a.chunk_v);
+    using Part = typename std::conditional<norm_is_layer(KIND), MomentStat<double>, SoftStat<CT, ST>>::type;
+    const Part* parts = (const Part*)a.part + row * a.S;
+    RowSplitRaw<KIND, T, VEC> raw[NB];
     CT p0, p1, p2;
     if constexpr (!norm_is_layer(KIND)) {
-        SoftStat<CT, ST> st{neg_inf<CT>(), (ST)0};
-        for (int i = threadIdx.x; i < a.S; i += 256) st = SoftStatOp<T, CT, ST>::comb(st, ((const SoftStat<CT, ST>*)a.part)[row * a.S + i]);
-        st = block_reduce<SoftStatOp<T, CT, ST>>(st, (SoftStat<CT, ST>*)smem_raw);
+        // the partials and the first batch of the slice are on their way together
+        Part st = parts[min((int)threadIdx.x, a.S - 1)];
+        row_split_fetch<KIND, T, VEC, UA>(a, in_row, row, min(v0 + threadIdx.x, nv - 1), v1, raw);
+        if ((int)threadIdx.x >= a.S) st = {neg_inf<CT>(), (ST)0};
+        for (int i = threadIdx.x + 256; i < a.S; i += 256) st = SoftStatOp<T, CT, ST>::comb(st, parts[i]);
+        st = block_soft<T>(st, (SoftStat<CT, ST>*)smem_raw);
         p0 = st.m;
         p1 = norm_is_log(KIND) ? log_ct<T>((CT)st.s) : (CT)((ST)1 / st.s);
         p2 = 0;
     } else {
         MomentStat<double> st{0, 0, 0};
-        for (int i = threadIdx.x; i < a.S; i += 256) st = MomentStatOp<double>::comb(st, ((const MomentStat<double>*)a.part)[row * a.S + i]);
+        for (int i = threadIdx.x; i < a.S; i += 256) st = MomentStatOp<double>::comb(st, parts[i]);
         st = block_moments(st, (double*)smem_raw);
         p0 = (CT)st.mean;
         p1 = (CT)(st.mean - (double)p0);
         p2 = rsqrt_ct((CT)(st.m2 * a.inv_cols) + (CT)a.eps);
     }
-    const int64_t nv = row_split_vectors<VEC, UA>(a.cols);
-    const int64_t v0 = (int64_t)blockIdx.x * a.chunk_v, v1 = min(nv, v0 + a.chunk_v);
-    for (int64_t iv = v0 + threadIdx.x; iv < v1; iv += 256) {
+    auto finish = [&](const RowSplitRaw<KIND, T, VEC>& from, int64_t iv) {
         CT x[VEC];
         const int64_t e0 = row_split_start<VEC, UA>(iv, a.cols);
-        row_split_load<KIND, T, VEC, UA>(a, in_row, row, e0, x);
+        row_split_widen<KIND, T, VEC>(from, x);
         Pack<T, VEC> o;
         if constexpr (norm_is_layer(KIND)) {
             Pack<T, VEC> g, b;
@@ -1667,6 +1728,19 @@ __global__ void __launch_bounds__(256) row_split_apply_kernel(const RowSplitArgs
             }
         } else if constexpr (VEC > 1) store_pack_stream<T, VEC>(out_row + e0, o);
         else out_row[e0] = o.v[0];
+    };
+    if constexpr (norm_is_layer(KIND)) {
+        for (int64_t iv = v0 + threadIdx.x; iv < v1; iv += 256)
+            finish(row_split_load<KIND, T, VEC, UA>(a, in_row, row, row_split_start<VEC, UA>(iv, a.cols)), iv);
+    } else {
+        for (int64_t i0 = v0 + threadIdx.x; i0 < v1; i0 += 256 * NB) {
+            if (i0 >= v0 + 256 * NB) row_split_fetch<KIND, T, VEC, UA>(a, in_row, row, i0, v1, raw);
+#pragma unroll
+            for (int u = 0; u < NB; ++u) {
+                if (i0 + u * 256 >= v1) break;
+                finish(raw[u], i0 + u * 256);
+            }
+        }
     }
 }
 
