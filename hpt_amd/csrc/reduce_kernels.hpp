@@ -56,6 +56,16 @@ __device__ __forceinline__ void write_out_pack(void* out, int64_t o, const typen
     }
 }
 
+// What is left after a lane's whole batches, up to three loads: f(1), f(2) or f(3) by what the wavefront's first active lane, which has
+// the most, has left. All of them are loaded before any is folded (one after the other each waits a memory latency; behind a test per load the compiler waits too),
+// lanes that have fewer load their last one again, and no wavefront loads what none of its lanes needs.
+template <class F> __device__ __forceinline__ void load_remainder(int left, F f) {
+    const int most = __builtin_amdgcn_readfirstlane(left);
+    if (most == 1) f(std::integral_constant<int, 1>{});
+    else if (most == 2) f(std::integral_constant<int, 2>{});
+    else f(std::integral_constant<int, 3>{});
+}
+
 // ---- lean row kernel ---------------------------------------------------------
 // out[row] = reduce over i in [0, rin) of in[row * row_stride + i * sr].
 struct RowLeanArgs {
@@ -435,33 +445,47 @@ __device__ __forceinline__ void fold_thread_rows(typename Op::Acc (&acc)[VEC], t
     const int bx = blockDim.x, by = blockDim.y;
     const int tx = threadIdx.x, ty = threadIdx.y;
     if (by == 1) return;
-    if (by <= 4) {
+    // The thread rows of one wavefront meet through the lanes, then the wavefronts through LDS: up to four are folded by the first one, more by
+    // a thread per place, all of a place's values on their way before the first is used. Two barriers for sixteen wavefronts, where halving the
+    // thread rows through LDS took two a step (device us, with the loads of col_lean_kernel's remainder together: f32 [40, 28, 26, 26] max over axis 1 6.0 and
+    // 4.2, bf16 [440, 3648] over axis 0 7.1 and 5.5). Pairs all the way, in a fixed order: the result is deterministic.
+    for (int d = bx; d < 64; d <<= 1)
 #pragma unroll
-        for (int j = 0; j < VEC; ++j) smem[((size_t)ty * bx + tx) * VEC + j] = acc[j];
-        __syncthreads();
-        if (ty == 0) {
-            for (int y = 1; y < by; ++y) {
+        for (int j = 0; j < VEC; ++j) acc[j] = Op::comb(acc[j], shfl_xor_any(acc[j], d));
+    const int tid = ty * bx + tx, nw = (bx * by) >> 6, row = bx * VEC;
+    if (nw == 1) return;
+    if ((tid & 63) < bx) {
 #pragma unroll
-                for (int j = 0; j < VEC; ++j) acc[j] = Op::comb(acc[j], smem[((size_t)y * bx + tx) * VEC + j]);
+        for (int j = 0; j < VEC; ++j) smem[(tid >> 6) * row + tx * VEC + j] = acc[j];
+    }
+    __syncthreads();
+    if (nw <= 4) {
+        if (ty == 0)
+            for (int w = 1; w < nw; ++w) {
+#pragma unroll
+                for (int j = 0; j < VEC; ++j) acc[j] = Op::comb(acc[j], smem[w * row + tx * VEC + j]);
             }
-        }
         return;
     }
-    // Many thread rows (a narrow inner dim): halve them step by step; rows [s, 2s) hand their
-    // values to rows [0, s) through LDS. The pairing is fixed, so the result is deterministic.
-    int top = 1;
-    while (top < by) top <<= 1;
-    for (int s = top >> 1; s >= 1; s >>= 1) {
-        if (ty >= s && ty < 2 * s) {
+    auto tree = [&](auto n_tag, int p) {
+        constexpr int N = decltype(n_tag)::value;
+        typename Op::Acc v[N];
 #pragma unroll
-            for (int j = 0; j < VEC; ++j) smem[((size_t)(ty - s) * bx + tx) * VEC + j] = acc[j];
-        }
-        __syncthreads();
-        if (ty < s && ty + s < by) {
+        for (int w = 0; w < N; ++w) v[w] = smem[w * row + p];
 #pragma unroll
-            for (int j = 0; j < VEC; ++j) acc[j] = Op::comb(acc[j], smem[((size_t)ty * bx + tx) * VEC + j]);
-        }
-        __syncthreads();
+        for (int h = N / 2; h >= 1; h >>= 1)
+#pragma unroll
+            for (int w = 0; w < h; ++w) v[w] = Op::comb(v[w], v[w + h]);
+        smem[p] = v[0];  // (nobody else reads this place's values)
+    };
+    for (int p = tid; p < row; p += bx * by) {
+        if (nw == 16) tree(std::integral_constant<int, 16>{}, p);
+        else tree(std::integral_constant<int, 8>{}, p);
+    }
+    __syncthreads();
+    if (ty == 0) {
+#pragma unroll
+        for (int j = 0; j < VEC; ++j) acc[j] = smem[tx * VEC + j];
     }
 }
 
@@ -665,11 +689,28 @@ __global__ void __launch_bounds__(1024) col_lean_kernel(const ColLeanArgs a) {
 #pragma unroll
                 for (int j = 0; j < UV; ++j) fold_in<Op>(acc[j], v[u].v[j * SS], r + u * step);
         }
-        for (; r < a.R; r += step) {
-            const Pack<T, VEC> v = load(base + (int64_t)r * a.rs);
+        if (r + 3 * step < a.R) {
+            Pack<T, VEC> v[4];
 #pragma unroll
-            for (int j = 0; j < UV; ++j) fold_in<Op>(acc[j], v.v[j * SS], r);
+            for (int u = 0; u < 4; ++u) v[u] = load(base + (int64_t)(r + u * step) * a.rs);
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int j = 0; j < UV; ++j) fold_in<Op>(acc[j], v[u].v[j * SS], r + u * step);
+            r += 4 * step;
         }
+        if (r < a.R)
+            load_remainder(1 + (r + step < a.R) + (r + 2 * step < a.R), [&](auto n_tag) {
+                constexpr int N = decltype(n_tag)::value;
+                Pack<T, VEC> v[N];
+#pragma unroll
+                for (int u = 0; u < N; ++u) v[u] = load(base + (int64_t)min(r + u * step, a.R - 1) * a.rs);
+#pragma unroll
+                for (int u = 0; u < N; ++u)
+                    if (r + u * step < a.R)
+#pragma unroll
+                        for (int j = 0; j < UV; ++j) fold_in<Op>(acc[j], v[u].v[j * SS], r + u * step);
+            });
     }
     fold_thread_rows<Op, UV>(acc, (Acc*)smem_raw);
     if (ty == 0 && valid) {
@@ -1036,23 +1077,25 @@ __global__ void __launch_bounds__(1024) finish_cols_kernel(const void* part_, vo
     const bool valid = o < K;
     Acc acc = Op::identity();
     if (valid) {
-        // eight partials in flight per thread (the kernel is a chain of load latencies otherwise)
+        // four partials in flight per thread, those beyond its share the last one again (the kernel is a chain of load latencies)
         const Acc* p = part + o;
-        int s = ty;
-        for (; s + 7 * by < split; s += 8 * by) {
-            Acc v[8];
+        for (int s = ty; s < split; s += 4 * by) {
+            Acc v[4];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) v[u] = p[(int64_t)(s + u * by) * K];
+            for (int u = 0; u < 4; ++u) v[u] = p[(int64_t)min(s + u * by, split - 1) * K];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) acc = Op::comb(acc, v[u]);
+            for (int u = 0; u < 4; ++u)
+                if (s + u * by < split) acc = Op::comb(acc, v[u]);
         }
-        for (; s < split; s += by) acc = Op::comb(acc, p[(int64_t)s * K]);
     }
     if (by > 1) {
         sm[ty * 64 + tx] = acc;
         __syncthreads();
-        if (ty == 0)
-            for (int y = 1; y < by; ++y) acc = Op::comb(acc, sm[y * 64 + tx]);
+        if (ty == 0) {
+#pragma unroll
+            for (int y = 1; y < 16; ++y)
+                if (y < by) acc = Op::comb(acc, sm[y * 64 + tx]);
+        }
     }
     // output o of the kernel's (outer, inner) numbering sits at outer * oso + inner * osi
     if (ty == 0 && valid) write_out<Op>(out, (o / kin) * oso + (o % kin) * osi, acc, init_out, count);
@@ -1297,7 +1340,10 @@ if (p.unaligned)             col_flat_kernel<Op, FULL, true><<<dim3(1, (unsigned
     } else {
         const int64_t kv = p.K / p.vec;
         dim3 block((unsigned)p.bx, (unsigned)p.by);
-        size_t smem = p.by > 1 ? (size_t)p.bx * p.by * (p.vec / p.sstride) * sizeof(Acc) : 0;
+        const int waves = p.bx * p.by / 64;  // what fold_thread_rows takes: 1, 2, 4, 8 or 16 whole wavefronts
+        if (p.by > 1 && (p.bx * p.by % 64 || waves > 16 || (waves & (waves - 1)) || (p.bx & (p.bx - 1)) || p.bx > 64))
+            fail(HPT_ERR_KERNEL, "column reduction: thread rows of %d x %d", p.bx, p.by);
+        size_t smem = waves > 1 ? (size_t)p.bx * waves * (p.vec / p.sstride) * sizeof(Acc) : 0;
         if (p.lean) {
             ColLeanArgs a{};
             const int nk = p.kept.n;
