@@ -235,6 +235,15 @@ ReducePlan plan_reduce(const void* data, const int64_t* shape, const int64_t* st
                 p.tpr = 256;
                 p.rpb = 1;
             }
+            // What is small keeps to one launch, up to 1024 threads per output with four vectors each or more: the second launch costs what
+            // sixteen vectors per thread do (us per call in two launches of 256 threads and in one: argmax of f32 [1, 37568] 10.8 and 7.4, bf16 [10, 116377] 10.9 and
+            // 7.3, sum of all of f32 [4, 104, 12, 12] 10.7 and 7.6; device us of one launch, 256 and 1024 threads: bf16 [28, 46592] argmax 7.3 and
+            // 4.9, f32 [40, 28, 26, 26] over all but the channels 11.4 and 6.8).
+            if (nv <= 16 * 1024 && p.K * nv * 16 <= (4ll << 20)) {
+                p.tpr = std::max(p.tpr, (int)std::min<int64_t>(1024, pow2_ceil((nv + 3) / 4)));
+                p.rpb = std::max(256, p.tpr) / p.tpr;
+                return p;
+            }
             int64_t want = std::max<int64_t>(1, 512 / p.K);  // (never just over two rounds of the compute units)
             int64_t can = nv / (256 * (p.K >= 64 ? 8 : 16));
             int64_t split = std::min<int64_t>(std::min(want, can), 4096);

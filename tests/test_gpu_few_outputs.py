@@ -1,0 +1,46 @@
+"""Reductions whose time is a chain of dependent loads: rows of few outputs that stay in one launch of up to 1024 threads (around the
+16384 vectors and the 4 MiB where a second launch begins), runs of one outer dim walked as one range, and the columns' remainders of one
+to seven rows per lane with one to sixteen wavefronts to fold, against the oracle."""
+import numpy as np
+import pytest
+
+from conftest import assert_close
+from util import F32_ATOL, F32_RTOL, HALF_RTOL, half_acc, half_atol
+
+pytestmark = pytest.mark.gpu
+
+CASES = (
+    # rows: one output and several, the last one-launch length and the first split one, off the vector grid, 1 ... 5 vectors per thread
+    [((1, n), (1,)) for n in (65536, 65537, 65540, 1020, 1028, 4099, 8191)]
+    + [((k, n), (1,)) for k, n in ((16, 65536), (17, 65536), (64, 16384), (65, 16384), (3, 20484), (7, 33333), (500, 2051))]
+    # batch-norm runs: one outer dim, runs of fewer and of more vectors than threads, 1 ... 7 pairs per lane, several outer dims
+    + [((b, c, h), (0, 2)) for b, c, h in ((3, 5, 49), (12, 6, 2401), (40, 28, 676), (2, 64, 676), (17, 3, 1000), (33, 9, 7), (9, 4, 5000))]
+    + [((3, 4, 5, 6, 77), (0, 2, 4)), ((64, 2, 3136), (0, 2))]
+    # columns: remainders after whole batches of eight, 1 ... 16 wavefronts
+    + [((r, c), (0,)) for r in (7, 15, 64 * 8 + 65, 64 * 11, 64 * 13 + 1, 64 * 15 + 3) for c in (24, 64, 260)]
+    + [((8 * 9 + 5, 3000), (0,)), ((1100, 5, 33), (0, 2)), ((300, 8200), (0,))]
+)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float16, np.int32, np.uint8, np.float64], ids=lambda d: np.dtype(d).name)
+@pytest.mark.parametrize("shape,axes", CASES, ids=lambda v: str(v).replace(" ", ""))
+def test_few_outputs(hpt, orc, dev, shape, axes, dtype):
+    rng = np.random.default_rng(17)
+    a = rng.standard_normal(shape).astype(dtype) if np.issubdtype(dtype, np.floating) else rng.integers(0, 100, shape).astype(dtype)
+    t = hpt.Tensor.from_numpy(a).to_hip(dev)
+    axes = list(axes)
+    n = int(np.prod([shape[i] for i in axes]))
+    print(hpt.reduce_plan(t, hpt.SUM, axes), flush=True)
+    assert np.array_equal(t.max(axes).numpy(), a.max(tuple(axes)))
+    if len(axes) == 1:
+        assert np.array_equal(t.argmax(axes[0]).numpy(), orc.argreduce(True, a, axes[0]))
+    s = t.sum(axes).numpy()
+    if dtype == np.float16:
+        want = orc.reduce(orc.SUM, a, axes, acc=half_acc(orc, n)).astype(np.float32)
+        assert_close(s.astype(np.float32), want, HALF_RTOL, half_atol(want, 11), "sum")
+    elif dtype in (np.float32, np.float64):
+        # (sums near zero: the error follows the terms, at most eps sqrt(n) of their size here, not the result)
+        rtol, atol = (F32_RTOL, max(F32_ATOL, 6e-8 * n ** 0.5)) if dtype == np.float32 else (1e-12, 1e-11)
+        assert_close(s, orc.reduce(orc.SUM, a, axes, acc=orc.ACC_F64), rtol, atol, "sum")
+    else:
+        assert np.array_equal(s, orc.reduce(orc.SUM, a, axes))
