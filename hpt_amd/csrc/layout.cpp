@@ -895,7 +895,12 @@ NormPlan plan_normalize(const void* in_data, const void* out_data, const int64_t
                 int64_t S = std::max<int64_t>(1, std::min<int64_t>(want, p.cols / 128));
                 if (S < want && S * groups > kComputeUnits && S * groups * 10 < 2 * kComputeUnits * 9) S = kComputeUnits / groups;
                 p.tsplit = (int)std::min<int64_t>(S, 64);
-                p.tpr = 4;  // wavefronts per workgroup of the statistics pass
+                // Wavefronts per workgroup of the statistics pass: four, one per SIMD, stream a large input. Where half of the compute units
+                // have no workgroup and a wavefront of four would walk 16 ... 63 columns, the pass is that chain of loads and exponentials, and eight halve it
+                // (us, four and eight, softmax, stored [columns, rows]: f16 [6208, 163] 18.1 and 16.3, f32 [7533, 203] 17.4 and 17.0, bf16 [16000, 256] 25.5 and
+                // 20.8; not the f64 sums of layernorm, f16 [6208, 163] 16.5 and 17.0, f32 [12000, 400] 18.3 and 18.9).
+                const int64_t slices = p.tsplit;
+                p.tpr = n_norm_dims <= 0 && slices * groups <= kComputeUnits / 2 && p.cols >= 64 * slices && p.cols < 256 * slices ? 8 : 4;
                 p.scratch_bytes = (size_t)p.rows * p.tsplit * 16 + (size_t)p.rows * 3 * 8;
                 return p;
             }
