@@ -322,8 +322,9 @@ __global__ void __launch_bounds__(256) transposed_finalize_kernel(const Transpos
     const bool ok = r < a.R;
     const int P = a.S;
     const Part* sp = (const Part*)a.stats + (int64_t)blockIdx.z * P * a.R + (ok ? r : 0);
-    // eight partials in flight (the kernel is a chain of load latencies); those beyond the thread's share load the last one again
-    constexpr int NB = 8;
+    // eight partials in flight (the kernel is a chain of load latencies), four of layernorm, which has 64 slices at most (f32 [12000, 400] transposed, all three
+    // passes, 18.6 us, 18.8 with eight; f16 [6208, 163] 16.2 and 16.5); those beyond the thread's share load the last one again
+    constexpr int NB = KIND == NORM_LAYERNORM ? 4 : 8;
     auto each = [&](auto take) {
         for (int p = threadIdx.y; p < P; p += NB * LY) {
             Part t[NB];
