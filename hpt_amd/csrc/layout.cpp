@@ -491,7 +491,11 @@ ReducePlan plan_reduce(const void* data, const int64_t* shape, const int64_t* st
                     return p;
                 }
             }
-            while (p.bx > 16 && xblocks < kComputeUnits && p.R >= 32) {
+            // (Eight lanes, a line of each row, and 128 thread rows where 64 would leave a lane more than twelve rows: up to 2048 of them stay in
+            // one launch. Over axis 0, us per call, sixteen lanes and eight: f16 [1536, 1000] 11.1 and 7.9, [1021, 3001] 10.2 and 7.4, bf16 [1344, 2368] 9.1 and
+            // 7.6, f32 [1400, 900] every second 11.4 and 7.7. Longer columns are more than one compute unit brings in: f32 [2100, 900] 10.9 and
+            // 11.1, f16 [3000, 1200] every second 11.0 and 14.6, [2040, 2000], nearly 8 MiB, 10.9 and 11.4.)
+            while ((p.bx > 16 || (p.bx > 8 && p.vec > 1 && p.R > 768 && p.R <= (bytes <= (7ll << 20) ? 2048 : 1536))) && xblocks < kComputeUnits && p.R >= 32) {
                 p.bx /= 2;
                 xblocks = (kv + p.bx - 1) / p.bx * outer;
             }
