@@ -1124,6 +1124,12 @@ template <class T, class CT, class ST = CT> struct SoftStatOp {
         return r;
     }
 };
+// What the exponentials of a running statistic are taken around: its maximum, or while there is none (nothing but -inf and NaN so far) the
+// lowest finite number, around which -inf adds nothing and a NaN stays in the sum. (Left out until there is a maximum, a NaN before
+// a lane's first finite element was lost, and its row came out finite.)
+template <class CT> __device__ __forceinline__ CT exp_origin(CT m) {
+    return MaxC<CT>::comb(m, sizeof(CT) == 8 ? (CT)-__DBL_MAX__ : (CT)-__FLT_MAX__);
+}
 // running (count, mean, sum of squared deviations)
 template <class CT> struct MomentStat {
     CT n, mean, m2;
@@ -1301,12 +1307,11 @@ __global__ void __launch_bounds__(1024) row_stream_kernel(const NormArgs a) {
                     st.s = st.s == (ST)0 ? (ST)0 : st.s * (ST)exp_ct<T>(st.m - cm);
                     st.m = cm;
                 }
-                if (st.m > neg_inf<CT>()) {
-                    CT part = 0;  // the few elements of one vector add up in the compute type
+                const CT org = exp_origin(st.m);
+                CT part = 0;  // the few elements of one vector add up in the compute type
 #pragma unroll
-                    for (int j = 0; j < VEC; ++j) part += exp_ct<T>(x[j] - st.m);
-                    st.s += (ST)part;
-                }
+                for (int j = 0; j < VEC; ++j) part += exp_ct<T>(x[j] - org);
+                st.s += (ST)part;
             };
             // four vectors in flight per thread (one per iteration left the memory pipeline mostly idle)
             int64_t iv = tx;
@@ -1613,12 +1618,11 @@ __global__ void __launch_bounds__(256) row_split_stats_kernel(const RowSplitArgs
                     st.s = st.s == (ST)0 ? (ST)0 : st.s * (ST)exp_ct<T>(st.m - cm);
                     st.m = cm;
                 }
-                if (st.m > neg_inf<CT>()) {
-                    CT part = 0;
+                const CT org = exp_origin(st.m);
+                CT part = 0;
 #pragma unroll
-                    for (int j = 0; j < VEC; ++j) part += exp_ct<T>(x[j] - st.m);
-                    st.s += (ST)part;
-                }
+                for (int j = 0; j < VEC; ++j) part += exp_ct<T>(x[j] - org);
+                st.s += (ST)part;
             }
         }
         st = block_soft<T>(st, (SoftStat<CT, ST>*)smem_raw);

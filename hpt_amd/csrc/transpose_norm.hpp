@@ -189,10 +189,9 @@ __global__ void __launch_bounds__(1024) transposed_stats_kernel(const Transposed
                     se[k] = se[k] == (ST)0 ? (ST)0 : se[k] * (ST)exp_ct<T>(m[k] - bm);
                     m[k] = bm;
                 }
-                if (m[k] > neg_inf<CT>()) {
+                const CT org = exp_origin(m[k]);
 #pragma unroll
-                    for (int i = 0; i < CNT; ++i) se[k] += (ST)exp_ct<T>(Elem<T>::widen(v[i].v[k]) - m[k]);
-                }
+                for (int i = 0; i < CNT; ++i) se[k] += (ST)exp_ct<T>(Elem<T>::widen(v[i].v[k]) - org);
             }
         }
     };
@@ -939,10 +938,9 @@ __global__ void __launch_bounds__(1024) col_flat_stats_kernel(const TransposedAr
                 s[k] = s[k] == (ST)0 ? (ST)0 : s[k] * (ST)exp_ct<T>(m[k] - bm);
                 m[k] = bm;
             }
-            if (m[k] > neg_inf<CT>()) {
+            const CT org = exp_origin(m[k]);
 #pragma unroll
-                for (int i = 0; i < CNT; ++i) s[k] += (ST)exp_ct<T>(Elem<T>::widen(v[i].v[k]) - m[k]);
-            }
+            for (int i = 0; i < CNT; ++i) s[k] += (ST)exp_ct<T>(Elem<T>::widen(v[i].v[k]) - org);
         }
     };
     if (t < threads) {
