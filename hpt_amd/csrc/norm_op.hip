@@ -171,12 +171,17 @@ template <class T, int VEC> void launch_col_split(const NormPlan& p, const NormA
         return g;
     };
     const dim3 sgrid = set_grid(dim3(rg, (unsigned)t.S, batch));
-    if constexpr (VEC > 1) {
-        if (ua)
-            transposed_stats_kernel<KIND, T, VEC, true><<<sgrid, dim3(64 * nw), (size_t)nw * VEC * 64 * sizeof(Part), st>>>(t);
-    }
-    if (!ua)
-        transposed_stats_kernel<KIND, T, VEC><<<sgrid, dim3(64 * nw), (size_t)nw * VEC * 64 * sizeof(Part), st>>>(t);
+    auto as_grid = [&](auto launch) {  // launch(unaligned, shared)
+        if constexpr (VEC > 1) {
+            if (ua && t.shared) return launch(std::true_type{}, std::true_type{});
+            if (ua) return launch(std::true_type{}, std::false_type{});
+            if (t.shared) return launch(std::false_type{}, std::true_type{});
+        }
+        launch(std::false_type{}, std::false_type{});
+    };
+    as_grid([&](auto unaligned, auto dealt) {
+        transposed_stats_kernel<KIND, T, VEC, decltype(unaligned)::value, decltype(dealt)::value><<<sgrid, dim3(64 * nw), (size_t)nw * VEC * 64 * sizeof(Part), st>>>(t);
+    });
     transposed_finalize_kernel<KIND, T><<<dim3((unsigned)((t.R + 15) / 16), 1, batch), dim3(16, 16), 0, st>>>(t);
     // apply: sixteen positions of the axis per workgroup, one batch of four loads per thread; what runs at one time is then
     // one stretch of memory (f32 [8192, 4096] over axis 0, all three passes, 16 / 32 / 48 positions: 65.2, 70.7, 67.4 us;
@@ -187,13 +192,9 @@ template <class T, int VEC> void launch_col_split(const NormPlan& p, const NormA
     const int chunk = (int)((t.cols + chunks - 1) / chunks);
     chunks = (t.cols + chunk - 1) / chunk;
     const dim3 agrid = set_grid(dim3(rg, (unsigned)chunks, batch));
-    if constexpr (VEC > 1) {
-        if (ua) {
-            col_apply_kernel<KIND, T, VEC, true><<<agrid, dim3(256), 0, st>>>(t, chunk);
-            return;
-        }
-    }
-    col_apply_kernel<KIND, T, VEC><<<agrid, dim3(256), 0, st>>>(t, chunk);
+    as_grid([&](auto unaligned, auto dealt) {
+        col_apply_kernel<KIND, T, VEC, decltype(unaligned)::value, decltype(dealt)::value><<<agrid, dim3(256), 0, st>>>(t, chunk);
+    });
 }
 
 // How many neighbouring workgroups of the column kernels share an XCD, as xcd_order takes it; `whole`: what is right where inner rows

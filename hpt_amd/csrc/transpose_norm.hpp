@@ -43,12 +43,14 @@ struct TransposedArgs {
     unsigned gx, gy, shared;  // the launch's grid in x and y; > 0: workgroups in all, neighbours share cache lines
 };
 
-// Which workgroup of the grid this one is: where neighbours in x share cache lines, the grid is dealt to the XCDs in eight equal parts.
+// Which workgroup of the grid this one is: where neighbours in x share cache lines, the grid is dealt to the XCDs in eight equal parts. (Kernels of
+// their own: behind a test the first loads wait for the arguments twice. All three passes, us, tested and this: softmax over axis 0 of f32 [2040, 2048] 16.5 and
+// 16.1, f16 [3000, 1001] 14.9 and 14.2; layernorm of f32 [12000, 400] transposed 19.5 and 18.8, [6858, 960] 22.3 and 21.2.)
 struct GridPlace {
     unsigned x, y, z;
 };
-__device__ __forceinline__ GridPlace grid_place(const TransposedArgs& a) {
-    if (!a.shared) return {blockIdx.x, blockIdx.y, blockIdx.z};
+template <bool SHARED> __device__ __forceinline__ GridPlace grid_place(const TransposedArgs& a) {
+    if constexpr (!SHARED) return {blockIdx.x, blockIdx.y, blockIdx.z};
     const unsigned w = xcd_order(blockIdx.x + a.gx * (blockIdx.y + a.gy * blockIdx.z), a.shared, kXcdShares), xy = w / a.gx;
     return {w - xy * a.gx, xy % a.gy, xy / a.gy};
 }
@@ -92,7 +94,7 @@ template <int KIND, class T> struct RowPartial {
 // UA: the inner rows are not whole, aligned vectors (an odd inner length): the same vectors unaligned; the last
 // lane of an inner row takes its vector from the row's end backwards, so no load leaves the row, and computes the
 // rows it shares with the lane before a second time (the same bits, stored twice).
-template <int KIND, class T, int VEC = 16 / sizeof(T), bool UA = false>
+template <int KIND, class T, int VEC = 16 / sizeof(T), bool UA = false, bool SHARED = false>
 __global__ void __launch_bounds__(1024) transposed_stats_kernel(const TransposedArgs a) {
     using CT = typename Elem<T>::Wide;
     using Part = typename RowPartial<KIND, T>::type;
@@ -100,7 +102,7 @@ __global__ void __launch_bounds__(1024) transposed_stats_kernel(const Transposed
     extern __shared__ __align__(16) unsigned char smem_raw[];
     const int NW = blockDim.x >> 6;  // wavefronts per workgroup (1...16)
 
-    const GridPlace at = grid_place(a);
+    const GridPlace at = grid_place<SHARED>(a);
     const int lane = threadIdx.x & 63;
     // the wavefront index is uniform: say so, and the column arithmetic stays scalar
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -491,12 +493,12 @@ __global__ void __launch_bounds__(256) transposed_apply_kernel(const TransposedA
 // UA: the last vector of an inner row is taken from the row's end backwards and stores only the elements that the vector
 // before it does not cover. Each element has one writer: `out` may be `in`, and the vector before may belong to another
 // workgroup, which then reads what this one must not have touched.
-template <int KIND, class T, int VEC, bool UA = false>
+template <int KIND, class T, int VEC, bool UA = false, bool SHARED = false>
 __global__ void __launch_bounds__(256) col_apply_kernel(const TransposedArgs a, int chunk) {
     using CT = typename Elem<T>::Wide;
     constexpr bool kLog = KIND == NORM_LOGSOFTMAX;
     const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-    const GridPlace at = grid_place(a);
+    const GridPlace at = grid_place<SHARED>(a);
     int r0 = (at.x * 64 + tx) * VEC;
     if (r0 >= a.R) return;
     const int skip = UA ? max(r0 - (a.R - VEC), 0) : 0;  // leading elements that belong to the vector before
