@@ -1127,9 +1127,20 @@ __global__ void __launch_bounds__(1024) finish_cols_kernel(const void* part_, vo
     const bool valid = o < K;
     Acc acc = Op::identity();
     if (valid) {
-        // four partials in flight per thread, those beyond its share the last one again (the kernel is a chain of load latencies)
+        // Eight partials in flight per thread while it has as many, then four, those beyond its share the last one again (the kernel is a chain of
+        // load latencies). 256 partials, sixteen per thread, us per call, four all the way and this: argmax of f32 [1016800, 33] over axis 0
+        // 32.5 and 31.2, sum of [100000, 200] 20.0 and 19.3; what eight and then one after the other take for four partials per thread: sum of
+        // f32 [32768, 1024] 26.4 and 25.7, [4100, 1000] 9.9 and 9.6.
         const Acc* p = part + o;
-        for (int s = ty; s < split; s += 4 * by) {
+        int s = ty;
+        for (; s + 7 * by < split; s += 8 * by) {
+            Acc v[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) v[u] = p[(int64_t)(s + u * by) * K];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) acc = Op::comb(acc, v[u]);
+        }
+        for (; s < split; s += 4 * by) {
             Acc v[4];
 #pragma unroll
             for (int u = 0; u < 4; ++u) v[u] = p[(int64_t)min(s + u * by, split - 1) * K];

@@ -44,3 +44,26 @@ def test_few_outputs(hpt, orc, dev, shape, axes, dtype):
         assert_close(s, orc.reduce(orc.SUM, a, axes, acc=orc.ACC_F64), rtol, atol, "sum")
     else:
         assert np.array_equal(s, orc.reduce(orc.SUM, a, axes))
+
+
+# columns whose partials a second launch folds, 16 thread rows per output: 51 and 64 partials are up to four per thread, 129 and 141 up to nine, 235 fifteen, 256
+# sixteen (eight loads in flight, then four)
+PARTIALS = [((9000, 260), 51), ((4100, 1000), 64), ((16600, 127), 129), ((17000, 130), 141), ((30000, 100), 235), ((100000, 200), 256), ((200000, 33), 256)]
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.int32], ids=lambda d: np.dtype(d).name)
+@pytest.mark.parametrize("shape,split", PARTIALS, ids=lambda v: str(v).replace(" ", ""))
+def test_partials_of_columns(hpt, orc, dev, shape, split, dtype):
+    rng = np.random.default_rng(split)
+    a = rng.standard_normal(shape).astype(dtype) if dtype == np.float32 else rng.integers(-1000, 1001, shape).astype(dtype)
+    a[rng.integers(0, shape[0], shape[1]), np.arange(shape[1])] = 2000  # the largest of every column somewhere
+    t = hpt.Tensor.from_numpy(a).to_hip(dev)
+    plan = hpt.reduce_plan(t, hpt.SUM, [0])
+    assert f" split={split} " in plan, plan
+    assert np.array_equal(t.max([0]).numpy(), a.max(0))
+    assert np.array_equal(t.argmax(0).numpy(), orc.argreduce(True, a, 0))
+    s = t.sum([0]).numpy()
+    if dtype == np.float32:  # (around 2000 and, as above, at most eps sqrt(n) of the terms)
+        assert_close(s, orc.reduce(orc.SUM, a, [0], acc=orc.ACC_F64), F32_RTOL, 6e-8 * shape[0] ** 0.5, "sum")
+    else:
+        assert np.array_equal(s, a.sum(0, dtype=np.int32))
