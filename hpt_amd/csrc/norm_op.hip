@@ -242,16 +242,18 @@ template <class T, int EV, bool WIDE = false> void launch_col_reg(const NormPlan
 
 // Whether the result of col_tall_kernel leaves through the caches. Segments that do not end on 64 bytes share what memory writes at once
 // with their neighbours: non-temporal, both parts go out by themselves. Through the cache, with neighbours on one XCD, they meet there. Us, non-temporal
-// and cached: f32 [512, 512, 510] 333 and 255, [512, 512, 500] 328 and 285, [34, 1000, 1001] 103.9 and 87.8, [32, 512, 510] 25.5 and 17.5, f16 [131, 512, 1000]
-// 81.3 and 67.3. Results of 48 to 96 MiB, which stay in the last-level cache for the most part, are ahead without ([84, 200, 1001]
-// 31.2 and 33.3, [64, 512, 510] 35.2 and 33.3) and two-byte ones up to there ([42, 400, 501] 15.2 and 16.1, [167, 400, 501] 41.4 and 44.9, but aligned vectors
-// [66, 512, 1000] 47.4 and 37.1); whole 64-byte pieces always ([512, 512, 528] 219 and 243).
+// and cached: f32 [512, 512, 510] 333 and 255, [512, 512, 500] 328 and 285, [46, 1000, 500] 66.0 and 47.9, [116, 512, 500] 74.1 and 51.4, [64, 512, 510] 37.8 and 29.9,
+// [84, 200, 1001] 34.1 and 32.6, [32, 512, 510] 25.5 and 17.5, f16 [131, 512, 1000] 81.3 and 67.3, aligned vectors [66, 512, 1000] 47.4 and 37.1. Not small results,
+// which the last-level cache takes either way (four bytes, below 20 MiB: [67, 256, 250] 12.3 and 14.4, [31, 300, 510] 12.4 and 13.0; but [84, 200, 300] 13.0 and 12.1), nor
+// unaligned two-byte ones below 96 ([42, 400, 501] 15.2 and 16.1, [167, 400, 501] 41.4 and 44.9), nor whole 64-byte pieces ([512, 512, 528] 219 and 243). Four bytes
+// of 48 to 96 MiB from an axis of 160 on, inputs from memory and from the last-level cache (ahead or level: [167, 160, 706] 37.0 and 33.4, 30.7 and 31.0, [75, 208, 1001] 33.5 and
+// 31.1, 30.5 and 27.0; behind: [143, 129, 706] 25.8 and 27.5, 23.1 and 25.0, [59, 129, 2047] 28.8 and 28.8, 24.4 and 27.4, [159, 140, 706] 30.0 and 29.4, 25.3 and 27.3).
 template <class T> bool tall_stores_cached(const NormPlan& p, const ColRegArgs& c) {
     const bool pieces = (c.L * (int64_t)sizeof(T)) % 64 == 0 && ((uintptr_t)c.out & 63) == 0;
     const int64_t mib = c.total / c.nvec * c.cols * c.L * (int64_t)sizeof(T) >> 20;
     if (pieces) return false;
     if (sizeof(T) == 2) return mib >= (p.shift ? 96 : 48);
-    return (mib >= 20 && mib < 48) || mib >= 96;
+    return mib >= 20 && (c.cols >= 160 || mib < 48 || mib >= 96);
 }
 
 // NT threads, TX of them along the inner dim, NC vectors each.

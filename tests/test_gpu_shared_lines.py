@@ -73,3 +73,31 @@ def test_transposed_rows(hpt, dev, shape, dtype):
     for name, want, got in [("softmax", _softmax64(v, -1), t.softmax(len(shape) - 1)),
                             ("layernorm", (v - v.mean(-1, keepdims=True)) / np.sqrt(v.var(-1, keepdims=True) + 1e-5), t.layernorm([shape[-2]]))]:
         assert_close(got.numpy().astype(np.float64), want, HALF_RTOL if half else F32_RTOL, max(half_atol(want, 11), 6e-8) if half else F32_ATOL, f"{name} {shape} {dtype}")
+
+
+# held by 512 and 1024 threads: either side of 20, 48 and 96 MiB and of an axis of 160, where results of four bytes begin to leave through the caches, and of 48
+# (whole vectors) and 96 MiB of two bytes
+STORED = [((40, 300, 401), "f32"), ((44, 300, 402), "f32"), ((44, 300, 404), "f32"), ((100, 159, 801), "f32"), ((99, 160, 801), "f32"), ((129, 200, 1001), "f32"),
+          ((26, 1000, 500), "f32"), ((59, 300, 1400), "f16"), ((60, 300, 1400), "f16"), ((83, 300, 2001), "f16"), ((84, 300, 2001), "f16")]
+
+
+@pytest.mark.parametrize("log", [False, True], ids=["softmax", "log_softmax"])
+@pytest.mark.parametrize("shape,dtype", STORED, ids=lambda v: v if isinstance(v, str) else "x".join(map(str, v)))
+def test_results_through_the_caches(hpt, dev, shape, dtype, log):
+    x = (np.random.default_rng(74).standard_normal(shape, dtype=np.float32) * 3).astype(np.float32 if dtype == "f32" else np.float16)
+    x[-1, -1, -1] = 40
+    t = hpt.Tensor.from_numpy(x).to_hip(dev)
+    plan = hpt.normalize_plan(t, 1)
+    assert plan.startswith("col-reg") and (" tpr=32 " in plan or " tpr=64 " in plan), plan
+    run = t.log_softmax if log else t.softmax
+    fresh = run(1).numpy()
+    half = dtype == "f16"
+    for b in (slice(0, 2), slice(shape[0] // 2, shape[0] // 2 + 1), slice(shape[0] - 2, shape[0])):  # (64 bits of the whole take seconds)
+        d = x[b].astype(np.float64) - x[b].max(1, keepdims=True)
+        e = np.exp(d)
+        want = d - np.log(e.sum(1, keepdims=True)) if log else e / e.sum(1, keepdims=True)
+        assert_close(fresh[b].astype(np.float64), want, HALF_RTOL if half else F32_RTOL, max(half_atol(want, 11), 6e-8) if half else F32_ATOL, f"{shape} {dtype}")
+    if not log:
+        assert abs(fresh.sum(1, dtype=np.float64) - 1).max() < (2.0 ** -10 if half else 1e-5)  # (every column: results are rounded to 2 ** -11 of themselves, and the sum to their statistics)
+    run(1, out=t)
+    assert np.array_equal(t.numpy(), fresh)
