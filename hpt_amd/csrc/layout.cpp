@@ -125,6 +125,9 @@ static int64_t full_rounds(int64_t groups, int64_t most = 4) {
 // the second figure.
 constexpr int64_t kSmallColBytes = 8ll << 20;
 constexpr size_t kSmallColScratch = 1u << 20;
+// Accumulators of a column workgroup's threads, in bytes: more of them take longer to fold than their loads save (argmax of one-byte types, sixteen of eight bytes per
+// thread, over axis 0, us, this and twice as many: u8 [2628, 53] 12.0 and 13.7, [1283, 54] 9.6 and 11.7, [300, 20000] 7.9 and 8.5, [2208, 103] 10.8 and 14.9).
+constexpr size_t kColAccs = 64u << 10;
 
 ReducePlan plan_reduce(const void* data, const int64_t* shape, const int64_t* strides, int ndim,
                        const int64_t* axes, int naxes, size_t elem_size, size_t acc_size, bool heavy, bool spare_scratch) {
@@ -461,7 +464,7 @@ ReducePlan plan_reduce(const void* data, const int64_t* shape, const int64_t* st
             const int64_t base = 64 / p.bx, rp = std::min(need_of(), can);
             if (rp <= 1) return base;
             int64_t by = std::min<int64_t>(pow2_ceil(rp), 1024 / p.bx / base) * base;
-            while (by > base && (size_t)p.bx * by * (p.vec / p.sstride) * acc_size > (64u << 10)) by /= 2;
+            while (by > base && p.bx * by * (p.vec / p.sstride) * acc_size > kColAccs) by /= 2;
             return by;
         };
         columns(ua_ok && kin >= 256 && p.R >= 256);
@@ -495,7 +498,11 @@ ReducePlan plan_reduce(const void* data, const int64_t* shape, const int64_t* st
             // one launch. Over axis 0, us per call, sixteen lanes and eight: f16 [1536, 1000] 11.1 and 7.9, [1021, 3001] 10.2 and 7.4, bf16 [1344, 2368] 9.1 and
             // 7.6, f32 [1400, 900] every second 11.4 and 7.7. Longer columns are more than one compute unit brings in: f32 [2100, 900] 10.9 and
             // 11.1, f16 [3000, 1200] every second 11.0 and 14.6, [2040, 2000], nearly 8 MiB, 10.9 and 11.4.)
-            while ((p.bx > 16 || (p.bx > 8 && p.vec > 1 && p.R > 768 && p.R <= (bytes <= (7ll << 20) ? 2048 : 1536))) && xblocks < kComputeUnits && p.R >= 32) {
+            // The accumulators of one-byte argmin / argmax allow 64 thread rows, so eight lanes up to 1024 rows: u8, argmax, sixteen and eight: [850, 1152] 10.4 and
+            // 8.5, [1000, 256] 9.6 and 8.5; [1200, 900] 11.0 and 14.6, [1600, 397] 10.7 and 13.9, [1821, 144] 10.1 and 14.1.
+            const int64_t most8 = std::min<int64_t>(128, kColAccs / (8 * (p.vec / p.sstride) * acc_size));
+            const bool eight = p.vec > 1 && p.R > 768 && p.R <= most8 * (bytes <= (7ll << 20) ? 16 : 12);
+            while (p.bx > (eight ? 8 : 16) && xblocks < kComputeUnits && p.R >= 32) {
                 p.bx /= 2;
                 xblocks = (kv + p.bx - 1) / p.bx * outer;
             }
@@ -503,7 +510,7 @@ ReducePlan plan_reduce(const void* data, const int64_t* shape, const int64_t* st
             int64_t by = pow2_ceil((p.R + 7) / 8);
             by = std::min(by, rows_per_wave * pow2_ceil((2048 + xblocks - 1) / xblocks));
             by = std::max<int64_t>(rows_per_wave, std::min<int64_t>(by, 1024 / p.bx));
-            while (by > rows_per_wave && (size_t)p.bx * by * uv * acc_size > (64u << 10)) by /= 2;
+            while (by > rows_per_wave && p.bx * by * uv * acc_size > kColAccs) by /= 2;
             p.by = (int)by;
             p.split = 1;
             if ((p.R + by - 1) / by > (p.vec > 1 ? 24 : 48) && spare_scratch) {
@@ -537,7 +544,7 @@ ReducePlan plan_reduce(const void* data, const int64_t* shape, const int64_t* st
                     // with eight), up to 256 workgroups per column block.
                     const int64_t slices = std::min((2048 + xblocks - 1) / xblocks, can);
                     int64_t by_waves = std::min<int64_t>(8, pow2_floor(slices));
-                    while (by_waves > 1 && (size_t)64 * by_waves * uv * acc_size > (64u << 10)) by_waves /= 2;
+                    while (by_waves > 1 && 64 * by_waves * uv * acc_size > kColAccs) by_waves /= 2;
                     p.split = (int)std::min<int64_t>(std::min<int64_t>((slices + by_waves - 1) / by_waves, 256), cap);
                     p.by = (int)by_waves * base_by;
                 } else {

@@ -12,7 +12,7 @@ from util import F32_ATOL, F32_RTOL, HALF_RTOL, half_acc, half_atol
 pytestmark = pytest.mark.gpu
 
 # (shape, reduced axis, view): around one vector more than a lane, two lanes, the row count from which unaligned vectors
-# are taken (64) and from which rows are split (more than 24 per lane of 64 thread rows: 1537), odd and whole rows, stepped
+# are taken (64), thousands of rows, which are split (2048 and 2049, where that begins, are in test_small_column_plans.py), odd and whole rows, stepped
 # rows, a swapped kept dim
 SHAPES = [
     ((6135, 287), 0, None), ((12608, 128), 0, None), ((1536, 128), 0, None), ((1537, 128), 0, None), ((34112, 40), 0, None), ((5440, 45), 0, None), ((37446, 16), 0, None),
