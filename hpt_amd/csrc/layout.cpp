@@ -496,12 +496,17 @@ ReducePlan plan_reduce(const void* data, const int64_t* shape, const int64_t* st
             }
             // (Eight lanes, a line of each row, and 128 thread rows where 64 would leave a lane more than twelve rows: up to 2048 of them stay in
             // one launch. Over axis 0, us per call, sixteen lanes and eight: f16 [1536, 1000] 11.1 and 7.9, [1021, 3001] 10.2 and 7.4, bf16 [1344, 2368] 9.1 and
-            // 7.6, f32 [1400, 900] every second 11.4 and 7.7. Longer columns are more than one compute unit brings in: f32 [2100, 900] 10.9 and
-            // 11.1, f16 [3000, 1200] every second 11.0 and 14.6, [2040, 2000], nearly 8 MiB, 10.9 and 11.4.)
+            // 7.6, f32 [1400, 900] every second 11.4 and 7.7; in two launches and in one [2040, 384] 9.6 and 8.8, [1800, 1001] 9.6 and 7.8. Longer columns are more than one
+            // compute unit brings in: f32 [2100, 900] 10.9 and 11.1, f16 [3000, 1200] every second 11.0 and 14.6. Beyond 1536 rows so are inputs of more than
+            // 7 MiB (f16 [2040, 2000] 10.9 and 11.4), whole vectors of rows that do not start on cache lines, which a block reads as two half lines each (f32 [1800, 300] 9.5 and 10.2,
+            // [2040, 700] 9.8 and 12.3, [2040, 900] every second 9.8 and 12.3, bf16 [2040, 1800] 9.5 and 12.6), and accumulators of eight bytes that fill 64 KiB (argmax of f16 [2040, 1024] 10.2 and 11.6).
             // The accumulators of one-byte argmin / argmax allow 64 thread rows, so eight lanes up to 1024 rows: u8, argmax, sixteen and eight: [850, 1152] 10.4 and
             // 8.5, [1000, 256] 9.6 and 8.5; [1200, 900] 11.0 and 14.6, [1600, 397] 10.7 and 13.9, [1821, 144] 10.1 and 14.1.
-            const int64_t most8 = std::min<int64_t>(128, kColAccs / (8 * (p.vec / p.sstride) * acc_size));
-            const bool eight = p.vec > 1 && p.R > 768 && p.R <= most8 * (bytes <= (7ll << 20) ? 16 : 12);
+            const size_t lane_accs = (p.vec / p.sstride) * acc_size;
+            const bool off_lines = !p.unaligned && (((uintptr_t)data | (uintptr_t)(p.red.stride[0] * (int64_t)elem_size)) & 127) != 0;
+            const int64_t most8 = std::min<int64_t>(16 * std::min<int64_t>(128, kColAccs / (8 * lane_accs)),
+                                                    bytes > (7ll << 20) || off_lines || (acc_size >= 8 && 1024 * lane_accs >= kColAccs) ? 1536 : 2048);
+            const bool eight = p.vec > 1 && p.R > 768 && p.R <= most8;
             while (p.bx > (eight ? 8 : 16) && xblocks < kComputeUnits && p.R >= 32) {
                 p.bx /= 2;
                 xblocks = (kv + p.bx - 1) / p.bx * outer;

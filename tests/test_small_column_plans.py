@@ -11,14 +11,17 @@ SUM, ARGMAX = 0, 14
 # (type, shape, every second element, op, lanes, thread rows, workgroups)
 PLANS = [
     # eight lanes from 769 rows on, whole vectors and not, stepped, up to 2048 rows in one launch
-    ("f32", (768, 500), False, SUM, 16, 64, 1), ("f32", (769, 500), False, SUM, 8, 128, 1), ("f32", (2048, 500), False, SUM, 8, 128, 1), ("f32", (2049, 500), False, SUM, 16, 16, 11),
+    ("f32", (768, 500), False, SUM, 16, 64, 1), ("f32", (769, 500), False, SUM, 8, 128, 1), ("f32", (2048, 512), False, SUM, 8, 128, 1), ("f32", (2049, 512), False, SUM, 16, 16, 11),
     ("f16", (768, 501), False, SUM, 16, 64, 1), ("f16", (769, 501), False, SUM, 8, 128, 1), ("f16", (2048, 501), False, SUM, 8, 128, 1), ("f16", (2049, 501), False, SUM, 16, 16, 11),
     ("f32", (768, 1000), True, SUM, 16, 64, 1), ("f32", (2048, 800), True, SUM, 8, 128, 1), ("f32", (2049, 800), True, SUM, 16, 16, 11),
     # up to 7 MiB, above that up to 1536 rows
     ("f16", (2000, 1835), False, SUM, 8, 128, 1), ("f16", (2000, 1836), False, SUM, 16, 16, 11), ("f32", (2000, 917), False, SUM, 8, 128, 1), ("f32", (2000, 918), False, SUM, 16, 16, 11),
     ("f16", (1536, 2400), False, SUM, 8, 128, 1), ("f16", (1537, 2400), False, SUM, 16, 16, 9),
-    # accumulators of eight bytes: argmax of two bytes as above, of one byte 64 thread rows and up to 1024 rows
-    ("f16", (2048, 501), False, ARGMAX, 8, 128, 1), ("u8", (768, 500), False, ARGMAX, 16, 32, 1), ("u8", (769, 500), False, ARGMAX, 8, 64, 1), ("u8", (1024, 500), False, ARGMAX, 8, 64, 1),
+    # up to 1536 rows of whole vectors that do not start on cache lines
+    ("f32", (1536, 500), False, SUM, 8, 128, 1), ("f32", (1537, 500), False, SUM, 16, 16, 9), ("f16", (1536, 600), False, SUM, 8, 128, 1), ("f16", (1537, 600), False, SUM, 16, 16, 9),
+    ("f32", (1537, 900), True, SUM, 16, 16, 9),
+    # accumulators of eight bytes: argmax of two bytes up to 1536 rows, of one byte 64 thread rows and up to 1024 rows
+    ("f16", (1536, 501), False, ARGMAX, 8, 128, 1), ("f16", (1537, 501), False, ARGMAX, 16, 16, 9), ("f32", (2048, 501), False, ARGMAX, 8, 128, 1), ("u8", (768, 500), False, ARGMAX, 16, 32, 1), ("u8", (769, 500), False, ARGMAX, 8, 64, 1), ("u8", (1024, 500), False, ARGMAX, 8, 64, 1),
     ("u8", (1025, 500), False, ARGMAX, 16, 16, 6), ("u8", (2048, 500), False, ARGMAX, 16, 16, 11), ("u8", (2048, 500), False, SUM, 8, 128, 1), ("i8", (1200, 900), False, ARGMAX, 16, 16, 7),
 ]
 
