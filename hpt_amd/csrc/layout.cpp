@@ -242,8 +242,17 @@ ReducePlan plan_reduce(const void* data, const int64_t* shape, const int64_t* st
             // sixteen vectors per thread do (us per call in two launches of 256 threads and in one: argmax of f32 [1, 37568] 10.8 and 7.4, bf16 [10, 116377] 10.9 and
             // 7.3, sum of all of f32 [4, 104, 12, 12] 10.7 and 7.6; device us of one launch, 256 and 1024 threads: bf16 [28, 46592] argmax 7.3 and
             // 4.9, f32 [40, 28, 26, 26] over all but the channels 11.4 and 6.8).
-            if (nv <= 16 * 1024 && p.K * nv * 16 <= (4ll << 20)) {
-                p.tpr = std::max(p.tpr, (int)std::min<int64_t>(1024, pow2_ceil((nv + 3) / 4)));
+            // (Half as many of one-byte argmin / argmax, whose sixteen elements per vector take longer than their load: u8 [131072] 7.9 and 7.2, [204894] 8.0 and 10.2,
+            // [262128] 8.3 and 12.8.)
+            if (nv <= (elem_size == 1 && acc_size >= 8 ? 8 : 16) * 1024 && p.K * nv * 16 <= (4ll << 20)) {
+                // Not where the first lanes of a row would have four vectors and most of the others three: a wavefront then goes through whole batches and
+                // remainder, twice the instructions to fetch (device us, eight and four per thread: argmax of u8 [30, 3200] 3.1 and 5.6, f32 [30, 800] 2.3 and 3.2; from
+                // 3.5 of them on eight are uneven too, bf16 [30, 960] 2.4 and 2.3). Nor where up to four workgroups would become more, on XCDs that have yet to
+                // fetch all of it: sum of f32 [200, 68] 1.9 and 2.3, [30, 1024] 1.9 and 2.5.
+                const int t4 = (int)std::min<int64_t>(1024, pow2_ceil((nv + 3) / 4));
+                const int rpb4 = std::max(256, t4) / t4;
+                const bool uneven = nv < 1024 && nv > 3 * t4 && 2 * nv <= 7 * t4;
+                if (!uneven && !(blocks <= 4 && (p.K + rpb4 - 1) / rpb4 > 4)) p.tpr = std::max(p.tpr, t4);
                 p.rpb = std::max(256, p.tpr) / p.tpr;
                 return p;
             }
