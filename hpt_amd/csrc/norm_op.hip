@@ -243,17 +243,19 @@ template <class T, int EV, bool WIDE = false> void launch_col_reg(const NormPlan
 // Whether the result of col_tall_kernel leaves through the caches. Segments that do not end on 64 bytes share what memory writes at once
 // with their neighbours: non-temporal, both parts go out by themselves. Through the cache, with neighbours on one XCD, they meet there. Us, non-temporal
 // and cached: f32 [512, 512, 510] 333 and 255, [512, 512, 500] 328 and 285, [46, 1000, 500] 66.0 and 47.9, [116, 512, 500] 74.1 and 51.4, [64, 512, 510] 37.8 and 29.9,
-// [84, 200, 1001] 34.1 and 32.6, [32, 512, 510] 25.5 and 17.5, f16 [131, 512, 1000] 81.3 and 67.3, aligned vectors [66, 512, 1000] 47.4 and 37.1. Not small results,
-// which the last-level cache takes either way (four bytes, below 20 MiB: [67, 256, 250] 12.3 and 14.4, [31, 300, 510] 12.4 and 13.0; but [84, 200, 300] 13.0 and 12.1), nor
-// unaligned two-byte ones below 96 ([42, 400, 501] 15.2 and 16.1, [167, 400, 501] 41.4 and 44.9), nor whole 64-byte pieces ([512, 512, 528] 219 and 243). Four bytes
-// of 48 to 96 MiB from an axis of 160 on, inputs from memory and from the last-level cache (ahead or level: [167, 160, 706] 37.0 and 33.4, 30.7 and 31.0, [75, 208, 1001] 33.5 and
-// 31.1, 30.5 and 27.0; behind: [143, 129, 706] 25.8 and 27.5, 23.1 and 25.0, [59, 129, 2047] 28.8 and 28.8, 24.4 and 27.4, [159, 140, 706] 30.0 and 29.4, 25.3 and 27.3).
+// [84, 200, 1001] 34.1 and 32.6, f16, whole vectors, [131, 512, 1000] 81.3 and 67.3, [66, 512, 1000] 47.4 and 37.1. Whole vectors from 20 MiB of four bytes and 48 of two on (below,
+// where the last-level cache takes either, f32 [67, 256, 250] 12.3 and 14.4), but not whole 64-byte pieces ([512, 512, 528] 219 and 243).
+// Unaligned vectors, of which a row's last one is stored in elements, only of four bytes (f16, 150 MiB: [250, 400, 501] 1.28 times the time, [800, 300, 301] 1.16) and only where a
+// segment is a part of an inner row, so that rows share less than segments do: [655, 256, 50] 21.1 and 23.0, [1273, 256, 37] 23.0 and 24.5, [421, 256, 90] 20.5 and 22.6, but
+// [463, 200, 130] 23.1 and 22.1, [310, 300, 90] 19.7 and 18.9. Those from 34 MiB on (16 vectors of a row per workgroup: 26; ratio cached / non-temporal of 200 columns at 21, 28, 36, 46, 90 MiB, rows of
+// 201: 1.09, 1.10, 0.93, 0.87, 0.90; of 300: 1.06, 0.94, 0.82, 0.85, 0.83), and of 48 to 96 MiB from an axis of 160 on ([167, 160, 706] 37.0 and 33.4, [143, 129, 706] 25.8 and 27.5).
 template <class T> bool tall_stores_cached(const NormPlan& p, const ColRegArgs& c) {
-    const bool pieces = (c.L * (int64_t)sizeof(T)) % 64 == 0 && ((uintptr_t)c.out & 63) == 0;
+    if ((c.L * (int64_t)sizeof(T)) % 64 == 0 && ((uintptr_t)c.out & 63) == 0) return false;
     const int64_t mib = c.total / c.nvec * c.cols * c.L * (int64_t)sizeof(T) >> 20;
-    if (pieces) return false;
-    if (sizeof(T) == 2) return mib >= (p.shift ? 96 : 48);
-    return mib >= 20 && (c.cols >= 160 || mib < 48 || mib >= 96);
+    if (!p.shift) return mib >= (sizeof(T) == 2 ? 48 : 20);
+    const int tx = p.tall / p.tpr;  // vectors of an inner row per workgroup
+    if (sizeof(T) == 2 || 8 * c.L < 9 * tx * (16 / (int)sizeof(T))) return false;
+    return mib >= (tx == 16 ? 26 : 34) && (c.cols >= 160 || mib < 48 || mib >= 96);
 }
 
 // NT threads, TX of them along the inner dim, NC vectors each.
@@ -262,8 +264,13 @@ template <class T, int NT, int TX, int NC> bool launch_col_tall_as(const NormPla
     const dim3 grid((unsigned)((c.total + TX - 1) / TX));
     c.blocks = grid.x;
     const bool cached = tall_stores_cached<T>(p, c);
-    if (p.shift && cached) col_tall_kernel<KIND, T, NT, TX, NC, true, true><<<grid, dim3(NT), 0, st>>>(c);
-    else if (p.shift) col_tall_kernel<KIND, T, NT, TX, NC, true><<<grid, dim3(NT), 0, st>>>(c);
+    if constexpr (sizeof(T) == 4) {
+        if (p.shift && cached) {
+            col_tall_kernel<KIND, T, NT, TX, NC, true, true><<<grid, dim3(NT), 0, st>>>(c);
+            return true;
+        }
+    }
+    if (p.shift) col_tall_kernel<KIND, T, NT, TX, NC, true><<<grid, dim3(NT), 0, st>>>(c);
     else if (cached) col_tall_kernel<KIND, T, NT, TX, NC, false, true><<<grid, dim3(NT), 0, st>>>(c);
     else col_tall_kernel<KIND, T, NT, TX, NC><<<grid, dim3(NT), 0, st>>>(c);
     return true;

@@ -75,10 +75,11 @@ def test_transposed_rows(hpt, dev, shape, dtype):
         assert_close(got.numpy().astype(np.float64), want, HALF_RTOL if half else F32_RTOL, max(half_atol(want, 11), 6e-8) if half else F32_ATOL, f"{name} {shape} {dtype}")
 
 
-# held by 512 and 1024 threads: either side of 20, 48 and 96 MiB and of an axis of 160, where results of four bytes begin to leave through the caches, and of 48
-# (whole vectors) and 96 MiB of two bytes
-STORED = [((40, 300, 401), "f32"), ((44, 300, 402), "f32"), ((44, 300, 404), "f32"), ((100, 159, 801), "f32"), ((99, 160, 801), "f32"), ((129, 200, 1001), "f32"),
-          ((26, 1000, 500), "f32"), ((59, 300, 1400), "f16"), ((60, 300, 1400), "f16"), ((83, 300, 2001), "f16"), ((84, 300, 2001), "f16")]
+# held by 512 and 1024 threads, either side of where results begin to leave through the caches: whole vectors of four bytes from 20 MiB, of two from 48; unaligned ones of
+# four bytes from 34 MiB (26 of more than 256 elements of the axis), where a segment of 128 (64) elements is a part of an inner row, of 48 to 96 MiB from an axis of 160 on
+STORED = [((43, 300, 404), "f32"), ((44, 300, 404), "f32"), ((26, 1000, 500), "f32"), ((59, 300, 1400), "f16"), ((60, 300, 1400), "f16"), ((84, 300, 2001), "f16"),
+          ((56, 300, 402), "f32"), ((57, 300, 402), "f32"), ((330, 300, 71), "f32"), ((330, 300, 73), "f32"), ((44, 200, 1001), "f32"), ((45, 200, 1001), "f32"),
+          ((320, 200, 143), "f32"), ((320, 200, 145), "f32"), ((100, 159, 801), "f32"), ((99, 160, 801), "f32"), ((129, 150, 1301), "f32"), ((129, 200, 1001), "f32")]
 
 
 @pytest.mark.parametrize("log", [False, True], ids=["softmax", "log_softmax"])
