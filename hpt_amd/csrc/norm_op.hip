@@ -225,19 +225,31 @@ template <class T, int EV, bool WIDE = false> void launch_col_reg(const NormPlan
     c.total = (nk > 1 ? p.kept_in.size[0] : 1) * c.nvec;
     c.cols = (int)p.cols;
     c.ty_log2 = ilog2(p.tpr);  // thread rows per inner position
-    c.run_log2 = column_run(c, sizeof(T), 0);
     if (p.tpr > 16 || c.cols > NC * p.tpr)
         fail(HPT_ERR_KERNEL, "col-reg: axis of %d does not fit %d thread rows of %d vectors", c.cols, p.tpr, NC);
     const int64_t tx = 256 / p.tpr;
     const dim3 grid((unsigned)((c.total + tx - 1) / tx));
     c.blocks = grid.x;
+    // (Up to eight bytes per thread of inner rows that a workgroup holds whole share lines at its ends only, and the numbering costs more: us, dealt and as they
+    // come, f32 [472, 176, 9] 11.6 and 10.4, [776, 144, 15] 11.5 and 10.7; but [36, 1000, 157] 17.8 and 23.2, f64 pairs
+    // [100, 60, 33] 12.7 and 15.5.)
+    constexpr bool kNarrow = EV * sizeof(T) <= 8;
+    c.run_log2 = kNarrow && c.nvec < tx ? 0 : column_run(c, sizeof(T), p.shift ? 5 : 0);  // (unaligned with every row on a line: only a batch is off it)
     if constexpr (EV > 1) {
-        if (p.shift) {
-            col_reg_kernel<KIND, T, EV, NC, true><<<grid, dim3(256), 0, st>>>(c);
+        if (p.shift && c.run_log2) {
+            col_reg_kernel<KIND, T, EV, NC, true, true><<<grid, dim3(256), 0, st>>>(c);
             return;
         }
     }
-    col_reg_kernel<KIND, T, EV, NC><<<grid, dim3(256), 0, st>>>(c);
+    if constexpr (EV > 1 && kNarrow) {
+        if (p.shift) {
+            col_reg_kernel<KIND, T, EV, NC, true, false><<<grid, dim3(256), 0, st>>>(c);
+            return;
+        }
+    }
+    if (EV > 1 && p.shift) fail(HPT_ERR_KERNEL, "col-reg: unaligned vectors of %d as they come", EV);
+    if (c.run_log2) col_reg_kernel<KIND, T, EV, NC, false, true><<<grid, dim3(256), 0, st>>>(c);
+    else col_reg_kernel<KIND, T, EV, NC><<<grid, dim3(256), 0, st>>>(c);
 }
 
 // Whether the result of col_tall_kernel leaves through the caches. Segments that do not end on 64 bytes share what memory writes at once

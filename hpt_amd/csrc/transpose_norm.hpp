@@ -599,7 +599,8 @@ template <class T, int N> __device__ __forceinline__ void forget_pack(Pack<T, N>
 // UA: the inner dim is not whole, aligned vectors (an odd length, odd strides): unaligned vectors all the
 // same; the last vector of an inner row is taken from the row's end backwards and stores only the
 // elements that the vector before it does not cover.
-template <int KIND, class T, int EV, int NC, bool UA = false>
+// DEALT: numbered by xcd_order. (A kernel of its own: behind a test the first loads wait longer, f32 [472, 176, 9] 11.6 us, 10.4 without.)
+template <int KIND, class T, int EV, int NC, bool UA = false, bool DEALT = false>
 __global__ void __launch_bounds__(256) col_reg_kernel(const ColRegArgs a) {
     static_assert(KIND == NORM_SOFTMAX || KIND == NORM_LOGSOFTMAX, "a softmax kernel");
     using CT = typename Elem<T>::Wide;
@@ -610,7 +611,7 @@ __global__ void __launch_bounds__(256) col_reg_kernel(const ColRegArgs a) {
     const int TX = 256 >> a.ty_log2;
     const int tx = threadIdx.x & (TX - 1);
     const int ty = threadIdx.x >> (8 - a.ty_log2);
-    const int64_t g = (int64_t)(a.run_log2 ? xcd_order(blockIdx.x, a.blocks, a.run_log2) : blockIdx.x) * TX + tx;
+    const int64_t g = (int64_t)(DEALT ? xcd_order(blockIdx.x, a.blocks, a.run_log2) : blockIdx.x) * TX + tx;
     const bool valid = g < a.total;
     int64_t b = 0, q = 0;
     if (valid) {

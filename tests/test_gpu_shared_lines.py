@@ -102,3 +102,38 @@ def test_results_through_the_caches(hpt, dev, shape, dtype, log):
         assert abs(fresh.sum(1, dtype=np.float64) - 1).max() < (2.0 ** -10 if half else 1e-5)  # (every column: results are rounded to 2 ** -11 of themselves, and the sum to their statistics)
     run(1, out=t)
     assert np.array_equal(t.numpy(), fresh)
+
+
+# held in registers, workgroups dealt to the XCDs and as they come: single elements and pairs of inner rows that a workgroup holds whole and does not, aligned pairs,
+# vectors on cache lines, and rows on lines in batches that are not
+REGISTERS = [((472, 176, 9), "f32", 1), ((36, 1000, 157), "f32", 1), ((600, 100, 13), "f16", 1), ((300, 60, 33), "f64", 1), ((8227, 43, 27), "f32", 2), ((40, 43, 301), "f32", 4),
+             ((817, 13, 37), "f32", 2), ((28, 512, 510), "f32", 2), ((64, 40, 128), "f32", 4), ((500, 43, 20), "f32", 4)]
+
+
+@pytest.mark.parametrize("shape,dtype,vec", REGISTERS, ids=lambda v: str(v).replace(" ", ""))
+def test_register_columns(hpt, dev, shape, dtype, vec):
+    x = (np.random.default_rng(75).standard_normal(shape) * 3).astype({"f32": np.float32, "f16": np.float16, "f64": np.float64}[dtype])
+    x[0, :, 0] = -50
+    x[-1, -1, -1] = 40
+    t = hpt.Tensor.from_numpy(x).to_hip(dev)
+    print(hpt.normalize_plan(t, 1), flush=True)
+    half = dtype == "f16"
+    want = _softmax64(x.astype(np.float64), 1)
+    for inplace in (False, True):
+        got = t.softmax(1, out=t if inplace else None).numpy().astype(np.float64)
+        assert_close(got, want, HALF_RTOL if half else F32_RTOL, max(half_atol(want, 11), 6e-8) if half else F32_ATOL, f"{shape} {dtype} inplace={inplace}")
+
+
+@pytest.mark.parametrize("axis_len", [21, 100])
+@pytest.mark.parametrize("batch_step", [1, 2, 4, 32])
+def test_register_columns_of_batches_off_the_lines(hpt, dev, axis_len, batch_step):
+    """Inner rows of 256 bytes back to back, the batches a few elements apart: unaligned vectors with every row but the batches on cache lines."""
+    b, length = 40000 // axis_len, 64
+    step = axis_len * length + batch_step
+    flat = (np.random.default_rng(76).standard_normal(b * step) * 3).astype(np.float32)
+    base = hpt.Tensor.from_numpy(flat).to_hip(dev)
+    t = hpt.Tensor.from_raw(base.ptr, [b, axis_len, length], hpt.f32, dev, strides=[step, length, 1])
+    plan = hpt.normalize_plan(t, 1)
+    assert plan.startswith("col-reg"), plan
+    x = np.lib.stride_tricks.as_strided(flat, (b, axis_len, length), (step * 4, length * 4, 4)).astype(np.float64)
+    assert_close(t.softmax(1).numpy().astype(np.float64), _softmax64(x, 1), F32_RTOL, F32_ATOL, plan)
