@@ -248,11 +248,11 @@ ReducePlan plan_reduce(const void* data, const int64_t* shape, const int64_t* st
                 // Not where the first lanes of a row would have four vectors and most of the others three: a wavefront then goes through whole batches and
                 // remainder, twice the instructions to fetch (device us, eight and four per thread: argmax of u8 [30, 3200] 3.1 and 5.6, f32 [30, 800] 2.3 and 3.2; from
                 // 3.5 of them on eight are uneven too, bf16 [30, 960] 2.4 and 2.3). Nor where up to four workgroups would become more, on XCDs that have yet to
-                // fetch all of it: sum of f32 [200, 68] 1.9 and 2.3, [30, 1024] 1.9 and 2.5.
+                // fetch all of it: sum of f32 [200, 68] 1.9 and 2.3, [30, 1024] 1.9 and 2.5. (From 1024 vectors on what is in flight counts for more.)
                 const int t4 = (int)std::min<int64_t>(1024, pow2_ceil((nv + 3) / 4));
                 const int rpb4 = std::max(256, t4) / t4;
-                const bool uneven = nv < 1024 && nv > 3 * t4 && 2 * nv <= 7 * t4;
-                if (!uneven && !(blocks <= 4 && (p.K + rpb4 - 1) / rpb4 > 4)) p.tpr = std::max(p.tpr, t4);
+                const bool uneven = nv > 3 * t4 && 2 * nv <= 7 * t4, spread = blocks <= 4 && (p.K + rpb4 - 1) / rpb4 > 4;
+                if (nv >= 1024 || (!uneven && !spread)) p.tpr = std::max(p.tpr, t4);
                 p.rpb = std::max(256, p.tpr) / p.tpr;
                 return p;
             }

@@ -16,9 +16,9 @@ PLANS = [
     ("bf16", (1, 131072), ARGMAX, 1024, 1),
     # four vectors per thread; eight where some lanes would have four and most of the others three
     ("u8", (300, 3072), ARGMAX, 64, 1), ("u8", (300, 3088), ARGMAX, 32, 1), ("u8", (300, 3584), ARGMAX, 32, 1), ("u8", (300, 3600), ARGMAX, 64, 1),
-    ("f32", (100, 800), SUM, 32, 1), ("f32", (100, 3200), SUM, 128, 1), ("f32", (100, 3588), SUM, 256, 1), ("f32", (100, 4096), SUM, 256, 1), ("f32", (100, 6400), SUM, 512, 1),
+    ("f32", (100, 800), SUM, 32, 1), ("f32", (100, 3200), SUM, 128, 1), ("f32", (100, 3588), SUM, 256, 1), ("f32", (100, 4096), SUM, 256, 1), ("f32", (100, 6400), SUM, 512, 1), ("f32", (7, 6400), SUM, 512, 1), ("f32", (5, 13200), SUM, 1024, 1),
     # and where up to four workgroups would become more
-    ("f32", (128, 68), SUM, 8, 1), ("f32", (129, 68), SUM, 4, 1), ("f32", (256, 68), SUM, 4, 1), ("f32", (257, 68), SUM, 8, 1), ("bf16", (30, 2048), ARGMAX, 32, 1),
+    ("f32", (128, 68), SUM, 8, 1), ("f32", (129, 68), SUM, 4, 1), ("f32", (256, 68), SUM, 4, 1), ("f32", (257, 68), SUM, 8, 1), ("bf16", (30, 2048), ARGMAX, 32, 1), ("f32", (7, 4092), SUM, 128, 1),
 ]
 
 
