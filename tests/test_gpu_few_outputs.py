@@ -30,7 +30,15 @@ def test_few_outputs(hpt, orc, dev, shape, axes, dtype):
     t = hpt.Tensor.from_numpy(a).to_hip(dev)
     axes = list(axes)
     n = int(np.prod([shape[i] for i in axes]))
-    print(hpt.reduce_plan(t, hpt.SUM, axes), flush=True)
+    plan = hpt.reduce_plan(t, hpt.SUM, axes)
+    print(plan, flush=True)
+    vectors = -(-n // (16 // a.itemsize))
+    if axes != [0]:  # rows: one launch up to 16384 vectors per output and 4 MiB in all
+        assert plan.startswith("row"), plan
+        if vectors <= 16384 and a.size * a.itemsize <= 4 << 20:
+            assert " split=1(" in plan, plan
+    else:
+        assert plan.startswith("col"), plan
     assert np.array_equal(t.max(axes).numpy(), a.max(tuple(axes)))
     if len(axes) == 1:
         assert np.array_equal(t.argmax(axes[0]).numpy(), orc.argreduce(True, a, axes[0]))

@@ -11,7 +11,9 @@ pytestmark = pytest.mark.gpu
 
 # rows of 16384 elements and more, whole vectors and not: slices of 1024 vectors and more, the last one short; stored [columns, rows]
 ROWS = [(3, 32768), (1, 32772), (2, 40001), (5, 36868), (1, 300007), (100, 16389), (2, 147456)]
-COLUMNS = [(8191, 100), (8192, 100), (8195, 101), (16383, 130), (16400, 129), (6208, 163), (12000, 400)]
+COLUMNS = [(8191, 100), (8192, 100), (8195, 101), (16383, 130), (16400, 129), (6208, 163), (12000, 400), (8195, 160), (8192, 130), (12000, 101), (8192, 8192)]
+# what they take: (f32, f16) wavefronts of a slice, none where a group of lanes per row is ahead of few two-byte rows
+WAVEFRONTS = {(8191, 100): (8, None), (8192, 100): (8, None), (8195, 101): (8, None), (16400, 129): (4, 4), (8192, 8192): (4, 4)}
 
 
 def _values(shape, dtype, axis, seed):
@@ -35,7 +37,13 @@ def test_partials_meet(hpt, dev, kind, shape, dtype):
     t = hpt.Tensor.from_numpy(x).to_hip(dev)
     if kind == "transposed":
         t, x = t.permute([1, 0]), x.T
-    print(hpt.normalize_plan(t, 1), flush=True)
+    plan = hpt.normalize_plan(t, 1)
+    print(plan, flush=True)
+    if kind == "rows":
+        assert plan.startswith("rowsplit"), plan
+    else:
+        waves = WAVEFRONTS.get(shape, (8, 8))[dtype == np.float16]
+        assert plan.startswith("transposed") and f" tpr={waves} " in plan if waves else plan.startswith("generic "), plan
     v = x.astype(np.float64)
     d = v - v.max(1, keepdims=True)
     e = np.exp(d)

@@ -1,4 +1,4 @@
-"""Registers of the layernorm row kernels, as the compiler reports them: a compute unit holds as many wavefronts as fit its registers, so a
+"""Registers of the layernorm row kernels and of tall softmax columns, as the compiler reports them: a compute unit holds as many wavefronts as fit its registers, so a
 change that costs a kernel a few of them costs time although every result stays the same. Compiled here for gfx950, nothing is launched."""
 import re
 import subprocess
@@ -27,6 +27,15 @@ LIMITS = [
     ("row_reg_kernel<NORM_LAYERNORM, float, 4, 4, 1, false, false, 0, 1>", 104, 0),
 ]
 
+COLUMNS = [
+    # softmax over an axis in the middle, f32 [512, 512, 512] and unaligned [476, 475, 53], log_softmax: held to 64 registers, so that two workgroups of 1024
+    # threads share a compute unit
+    ("col_tall_kernel<NORM_SOFTMAX, float, 1024, 16, 8, false, false>", 64, 0),
+    ("col_tall_kernel<NORM_SOFTMAX, float, 1024, 32, 8, true, true>", 64, 0),
+    ("col_tall_kernel<NORM_LOGSOFTMAX, float, 1024, 16, 8, true, false>", 64, 3),
+    ("col_tall_kernel<NORM_LOGSOFTMAX, float, 1024, 32, 8, true, true>", 64, 3),
+]
+
 
 @pytest.fixture(scope="module")
 def report(tmp_path_factory):
@@ -34,7 +43,7 @@ def report(tmp_path_factory):
     if not Path(build.HIPCC).exists():
         pytest.skip("needs hipcc")
     src = tmp_path_factory.mktemp("registers") / "kernels.hip"
-    src.write_text('#include "transpose_norm.hpp"\nnamespace hpt {\n' + "".join(f"template __global__ void {k}(const NormArgs);\n" for k, _, _ in LIMITS) + "}\n")
+    src.write_text('#include "transpose_norm.hpp"\nnamespace hpt {\n' + "".join(f"template __global__ void {k}(const {'ColRegArgs' if k.startswith('col') else 'NormArgs'});\n" for k, _, _ in LIMITS + COLUMNS) + "}\n")
     flags = [f for f in build.FLAGS if not f.startswith("--offload-compress")]
     r = subprocess.run([build.HIPCC, *flags, "--cuda-device-only", "-Rpass-analysis=kernel-resource-usage", "-c", str(src), "-o", "/dev/null"],
                        capture_output=True, text=True, timeout=600)
@@ -52,7 +61,7 @@ def report(tmp_path_factory):
 def _mangled(kernel: str) -> str:
     """The part of a kernel's mangled name that its template arguments make up."""
     name, args = re.match(r"(\w+)<(.*)>", kernel).groups()
-    codes = {"NORM_LAYERNORM": "Li2E", "NORM_ADD_LAYERNORM": "Li3E", "f16_t": "DF16_", "float": "f", "double": "d", "false": "Lb0E", "true": "Lb1E"}
+    codes = {"NORM_SOFTMAX": "Li0E", "NORM_LOGSOFTMAX": "Li1E", "NORM_LAYERNORM": "Li2E", "NORM_ADD_LAYERNORM": "Li3E", "f16_t": "DF16_", "float": "f", "double": "d", "false": "Lb0E", "true": "Lb1E"}
     return name + "I" + "".join(codes.get(a, f"Li{a}E") for a in args.split(", "))
 
 
@@ -61,3 +70,8 @@ def test_layernorm_rows_keep_their_wavefronts(report, kernel, registers, spilled
     match = [v for k, v in report.items() if _mangled(kernel) in k]
     assert len(match) == 1, f"{kernel}: {sorted(report)}"
     assert match[0]["VGPRs"] <= registers and match[0]["VGPRs Spill"] <= spilled, f"{kernel}: {match[0]}"
+
+
+@pytest.mark.parametrize("kernel,registers,spilled", COLUMNS)
+def test_tall_columns_keep_two_workgroups(report, kernel, registers, spilled):
+    test_layernorm_rows_keep_their_wavefronts(report, kernel, registers, spilled)
