@@ -337,8 +337,10 @@ __device__ __forceinline__ void row_step(typename Op::Acc& acc, const typename O
     else fold_in<Op>(acc, p[iv * sr], iv);
 }
 
+// (One-byte argmin / argmax are held to 64 registers, eight wavefronts per SIMD: with what is left over loaded together they took 100, u8 [1000, 64, 4096][:, :32] over
+// axis 2 34.4 us, 31.1 so, in the loop for one run, which rows of 64 vectors and more keep (29.3 without the other in the same kernel); [4000, 64, 200][:, :32] 14.5 there and 11.4.)
 template <class Op, int VEC, bool UA = false>
-__global__ void __launch_bounds__(1024) row_reduce_kernel(const RowArgs a) {
+__global__ void __launch_bounds__(1024, sizeof(typename Op::In) == 1 && sizeof(typename Op::Acc) == 8 ? 8 : 1) row_reduce_kernel(const RowArgs a) {
     static_assert(!UA || VEC > 1, "UA is a full-vector mode");
     using T = typename Op::In;
     using Acc = typename Op::Acc;
@@ -362,7 +364,8 @@ __global__ void __launch_bounds__(1024) row_reduce_kernel(const RowArgs a) {
         const int64_t i1 = min(a.rin_v, i0 + a.ichunk);
         const int64_t ni = i1 - i0;
         const int64_t total = (q1 - q0) * ni;
-        if (q0 < q1 && ni > 0 && a.redo.n <= 1 && sizeof(T) != 2 && total + 4 * tpr < (1ll << 31) && i1 + tpr < (1ll << 31)) {
+        constexpr bool kByteArg = sizeof(T) == 1 && sizeof(Acc) == 8;  // argmin / argmax of one byte: short rows only (see above)
+        if (q0 < q1 && ni > 0 && a.redo.n <= 1 && sizeof(T) != 2 && (!kByteArg || total < 64) && total + 4 * tpr < (1ll << 31) && i1 + tpr < (1ll << 31)) {
             // Outer reduced indices of one dim (the sums of a batch norm: [N, C, H*W] over N and H*W), each with an inner run of ni
             // vectors: the lanes walk the (outer, inner) pairs as ONE flat range, so a run that is not a multiple of the group size wastes no
             // lanes, with four loads in flight per lane and what is left loaded together. A lane's run and place in it advance by
@@ -526,11 +529,19 @@ __device__ __forceinline__ void fold_thread_rows(typename Op::Acc (&acc)[VEC], t
         for (int h = N / 2; h >= 1; h >>= 1)
 #pragma unroll
             for (int w = 0; w < h; ++w) v[w] = Op::comb(v[w], v[w + h]);
-        smem[p] = v[0];  // (nobody else reads this place's values)
+        return v[0];
     };
     for (int p = tid; p < row; p += bx * by) {
-        if (nw == 16) tree(std::integral_constant<int, 16>{}, p);
-        else tree(std::integral_constant<int, 8>{}, p);
+        typename Op::Acc r;
+        if constexpr (sizeof(typename Op::Acc) > 8) {
+            // (four at a time: all sixteen pairs of argmin / argmax of eight-byte types take 64 registers, two of the kernel's eight wavefronts per SIMD:
+            // argmax of f64 [233483, 1, 75] over axis 1 73.8 us, 65.0 so)
+            r = tree(std::integral_constant<int, 4>{}, p);
+#pragma unroll 1
+            for (int w = 4; w < nw; w += 4) r = Op::comb(r, tree(std::integral_constant<int, 4>{}, w * row + p));
+        } else if (nw == 16) r = tree(std::integral_constant<int, 16>{}, p);
+        else r = tree(std::integral_constant<int, 8>{}, p);
+        smem[p] = r;  // (nobody else reads this place's values)
     }
     __syncthreads();
     if (ty == 0) {

@@ -75,3 +75,16 @@ def test_partials_of_columns(hpt, orc, dev, shape, split, dtype):
         assert_close(s, orc.reduce(orc.SUM, a, [0], acc=orc.ACC_F64), F32_RTOL, 6e-8 * shape[0] ** 0.5, "sum")
     else:
         assert np.array_equal(s, a.sum(0, dtype=np.int32))
+
+
+# argmin / argmax over the last axis of a view whose kept dims do not merge: one-byte rows of fewer than 64 vectors walk a lane's remainder together, longer ones
+# one by one; and sixteen wavefronts of eight-byte pairs, which meet four at a time
+@pytest.mark.parametrize("dtype", [np.uint8, np.int8, np.float64, np.int64], ids=lambda d: np.dtype(d).name)
+@pytest.mark.parametrize("shape,axis", [((30, 8, 160), 2), ((30, 8, 1008), 2), ((30, 8, 1024), 2), ((30, 8, 1040), 2), ((30, 8, 4111), 2), ((600, 4, 40), 0), ((1025, 4, 130), 0)], ids=str)
+def test_argreduce_of_views(hpt, orc, dev, shape, axis, dtype):
+    rng = np.random.default_rng(23)
+    a = rng.integers(-100 if np.issubdtype(dtype, np.signedinteger) else 0, 100, shape).astype(dtype)
+    t, v = hpt.Tensor.from_numpy(a).to_hip(dev)[:, :3], a[:, :3]
+    print(hpt.reduce_plan(t, 14, [axis]), flush=True)
+    assert np.array_equal(t.argmax(axis).numpy(), orc.argreduce(True, np.ascontiguousarray(v), axis))
+    assert np.array_equal(t.argmin(axis).numpy(), orc.argreduce(False, np.ascontiguousarray(v), axis))
