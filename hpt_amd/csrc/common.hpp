@@ -110,7 +110,7 @@ struct ReducePlan {
     int flat_phases = 1;  // rows per period in that case
     int flat_w = 0;     // > 0: launched in workgroups of this many threads and flat_slices slices (no more than split / flat_phases)
     int flat_slices = 0;
-    bool small_split = false;  // Col: split although the input is small, for speed alone; a plan without partials exists (spare_scratch = false)
+    bool small_split = false;  // split although the input is small, for speed alone; a plan without partials exists (spare_scratch = false)
 };
 
 // Build the plan for reducing `axes` (already normalised) of a view.

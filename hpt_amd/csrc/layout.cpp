@@ -243,8 +243,10 @@ ReducePlan plan_reduce(const void* data, const int64_t* shape, const int64_t* st
             // 7.3, sum of all of f32 [4, 104, 12, 12] 10.7 and 7.6; device us of one launch, 256 and 1024 threads: bf16 [28, 46592] argmax 7.3 and
             // 4.9, f32 [40, 28, 26, 26] over all but the channels 11.4 and 6.8).
             // (Half as many of one-byte argmin / argmax, whose sixteen elements per vector take longer than their load: u8 [131072] 7.9 and 7.2, [204894] 8.0 and 10.2,
-            // [262128] 8.3 and 12.8.)
-            if (nv <= (elem_size == 1 && acc_size >= 8 ? 8 : 16) * 1024 && p.K * nv * 16 <= (4ll << 20)) {
+            // [262128] 8.3 and 12.8; without scratch to spare they stay in one.)
+            const bool small = nv <= 16 * 1024 && p.K * nv * 16 <= (4ll << 20);
+            p.small_split = small && nv > 8 * 1024 && elem_size == 1 && acc_size >= 8 && spare_scratch;
+            if (small && !p.small_split) {
                 // Not where the first lanes of a row would have four vectors and most of the others three: a wavefront then goes through whole batches and
                 // remainder, twice the instructions to fetch (device us, eight and four per thread: argmax of u8 [30, 3200] 3.1 and 5.6, f32 [30, 800] 2.3 and 3.2; from
                 // 3.5 of them on eight are uneven too, bf16 [30, 960] 2.4 and 2.3). Nor where up to four workgroups would become more, on XCDs that have yet to

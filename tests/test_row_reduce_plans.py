@@ -49,3 +49,43 @@ def test_row_reduce_results(hpt, orc, dev, dtype, shape, op, tpr, launches):
         assert_close(s, orc.reduce(orc.SUM, b, [axis], acc=orc.ACC_F64), F32_RTOL, F32_ATOL, "sum")
     else:
         assert np.array_equal(s, orc.reduce(orc.SUM, b, [axis]))
+
+
+@pytest.mark.gpu
+def test_captured_argmax_takes_no_scratch(hpt, dev):
+    """One-byte argmax of 8193 ... 16384 vectors is split for speed alone: recorded, on a stream that has no scratch, it is one node."""
+    import ctypes as C
+
+    from hpt_amd import _ffi
+    hip, P = C.CDLL("libamdhip64.so"), C.c_void_p
+    hip.hipStreamCreateWithFlags.argtypes = [C.POINTER(P), C.c_uint]
+    hip.hipStreamBeginCapture.argtypes = [P, C.c_int]
+    hip.hipStreamEndCapture.argtypes = [P, C.POINTER(P)]
+    hip.hipGraphGetNodes.argtypes = [P, P, C.POINTER(C.c_size_t)]
+    hip.hipGraphInstantiate.argtypes = [C.POINTER(P), P, P, P, C.c_size_t]
+    hip.hipGraphLaunch.argtypes = [P, P]
+    for f in (hip.hipStreamSynchronize, hip.hipGraphExecDestroy, hip.hipGraphDestroy, hip.hipStreamDestroy):
+        f.argtypes = [P]
+    a = np.random.default_rng(4).integers(0, 200, (2, 204896)).astype(np.uint8)
+    a[0, 204895], a[1, 3] = 250, 250
+    t, out = hpt.Tensor.from_numpy(a).to_hip(dev), hpt.Tensor.empty([2], hpt.i64, dev)
+    assert "split=1(" not in hpt.reduce_plan(t, ARGMAX, [1])
+    s, graph, gexec, n = P(), P(), P(), C.c_size_t()
+    assert hip.hipStreamCreateWithFlags(C.byref(s), 1) == 0
+    vin, k1 = t._c_view()
+    vout, k2 = out._c_view()
+    hpt.synchronize(dev)
+    assert hip.hipStreamBeginCapture(s, 0) == 0
+    try:
+        rc = _ffi.lib().hpt_hip_argreduce(dev, s, 1, C.byref(vin), 1, C.byref(vout))
+    finally:
+        ended = hip.hipStreamEndCapture(s, C.byref(graph))
+    assert rc == 0 and ended == 0 and hip.hipGraphGetNodes(graph, None, C.byref(n)) == 0 and n.value == 1
+    assert hip.hipGraphInstantiate(C.byref(gexec), graph, None, None, 0) == 0
+    for _ in range(3):
+        assert hip.hipGraphLaunch(gexec, s) == 0 and hip.hipStreamSynchronize(s) == 0
+        assert np.array_equal(out.numpy(), [204895, 3])
+        assert np.array_equal(t.argmax(1).numpy(), [204895, 3])  # eagerly, in two launches
+    hip.hipGraphExecDestroy(gexec)
+    hip.hipGraphDestroy(graph)
+    hip.hipStreamDestroy(s)
