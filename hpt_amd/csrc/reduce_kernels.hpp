@@ -337,10 +337,12 @@ __device__ __forceinline__ void row_step(typename Op::Acc& acc, const typename O
     else fold_in<Op>(acc, p[iv * sr], iv);
 }
 
-// (One-byte argmin / argmax are held to 64 registers, eight wavefronts per SIMD: with what is left over loaded together they took 100, u8 [1000, 64, 4096][:, :32] over
-// axis 2 34.4 us, 31.1 so, in the loop for one run, which rows of 64 vectors and more keep (29.3 without the other in the same kernel); [4000, 64, 200][:, :32] 14.5 there and 11.4.)
-template <class Op, int VEC, bool UA = false>
-__global__ void __launch_bounds__(1024, sizeof(typename Op::In) == 1 && sizeof(typename Op::Acc) == 8 ? 8 : 1) row_reduce_kernel(const RowArgs a) {
+// WALK: rows of no or one outer reduced dim go through the flat walk below. One-byte argmin / argmax do below 64 vectors per row only, held to 64 registers, eight wavefronts per SIMD,
+// where what is left over loaded together took 100. With the walk in the same kernel longer rows are slower: u8 over axis 2 [1000, 64, 4096][:, :32] 33.2 us (31.1 held to 64
+// registers) and 28.5 in a kernel without it, [4000, 64, 1024][:, :32] 30.4 and 26.5; [4000, 64, 200][:, :32], which walks, 11.0, 14.5 without.
+template <class Op> constexpr bool kByteArg = sizeof(typename Op::In) == 1 && sizeof(typename Op::Acc) == 8;
+template <class Op, int VEC, bool UA, bool WALK>
+__global__ void __launch_bounds__(1024, kByteArg<Op> && WALK ? 8 : 1) row_reduce_kernel(const RowArgs a) {
     static_assert(!UA || VEC > 1, "UA is a full-vector mode");
     using T = typename Op::In;
     using Acc = typename Op::Acc;
@@ -364,8 +366,7 @@ __global__ void __launch_bounds__(1024, sizeof(typename Op::In) == 1 && sizeof(t
         const int64_t i1 = min(a.rin_v, i0 + a.ichunk);
         const int64_t ni = i1 - i0;
         const int64_t total = (q1 - q0) * ni;
-        constexpr bool kByteArg = sizeof(T) == 1 && sizeof(Acc) == 8;  // argmin / argmax of one byte: short rows only (see above)
-        if (q0 < q1 && ni > 0 && a.redo.n <= 1 && sizeof(T) != 2 && (!kByteArg || total < 64) && total + 4 * tpr < (1ll << 31) && i1 + tpr < (1ll << 31)) {
+        if (WALK && q0 < q1 && ni > 0 && a.redo.n <= 1 && total + 4 * tpr < (1ll << 31) && i1 + tpr < (1ll << 31)) {
             // Outer reduced indices of one dim (the sums of a batch norm: [N, C, H*W] over N and H*W), each with an inner run of ni
             // vectors: the lanes walk the (outer, inner) pairs as ONE flat range, so a run that is not a multiple of the group size wastes no
             // lanes, with four loads in flight per lane and what is left loaded together. A lane's run and place in it advance by
@@ -1356,9 +1357,16 @@ void launch_reduce_t(const ReducePlan& p, const void* in, void* out, const Reduc
                     grid.x = (unsigned)a.xcd_chunk * 8;
                 }
             }
-            if (vec && p.unaligned) row_reduce_kernel<Op, FULL, true><<<grid, block, 0, st>>>(a);
-            else if (vec) row_reduce_kernel<Op, FULL><<<grid, block, 0, st>>>(a);
-            else row_reduce_kernel<Op, 1><<<grid, block, 0, st>>>(a);
+            auto rows = [&](auto walk) {
+                constexpr bool W = decltype(walk)::value;
+                if (vec && p.unaligned) row_reduce_kernel<Op, FULL, true, W><<<grid, block, 0, st>>>(a);
+                else if (vec) row_reduce_kernel<Op, FULL, false, W><<<grid, block, 0, st>>>(a);
+                else row_reduce_kernel<Op, 1, false, W><<<grid, block, 0, st>>>(a);
+            };
+            if constexpr (kByteArg<Op>) {
+                if (a.redo.n <= 1 && std::min(a.rout, a.qchunk) * std::min(a.rin_v, a.ichunk) < 64) rows(std::true_type{});
+                else rows(std::false_type{});
+            } else rows(std::bool_constant<sizeof(T) != 2>{});
         }
         if (p.split > 1 && p.split <= 16)
             finish_rows_thin_kernel<Op><<<dim3((unsigned)((p.K + 255) / 256)), dim3(256), 0, st>>>(sc.partial, out, p.K, p.split,
